@@ -1,0 +1,459 @@
+// One block of out[M, N] = A[M, K] * W[N, K]^T on the matrix cores: the K loop and the fused epilogues that the plain products
+// (gemm.hip) and the products over the rows of routed experts (routed.hip) share.
+//
+// Both operands are contiguous along K, so a 16x32 MFMA fragment of either is "row
+// l % 16, elements (l / 16) * 8 .. + 8".  Two LDS buffers, one barrier per K step.  LDS has 64 banks
+// of 4 bytes; the 16-byte fragment reads of a wave are free of bank conflicts when the row pitch is
+// 32 modulo 64 bytes (measured: pitches of 80 or 144 bytes take twice as long), or, with unpadded
+// rows of 128 bytes, when chunk c of row r lies at position c ^ (r & 7).
+// bfloat16 with K steps of 64: tiles go global -> LDS directly (global_load_lds_dwordx4, a wave's
+// 64 lanes fill 1 KB = 8 unpadded rows in lane order, so the swizzle is applied to the global
+// address), and the next step's tile is in flight while this one is multiplied; only a partial last
+// step goes through registers, where what lies beyond K is masked.  The 32-bit build and K steps of
+// 32 go global -> registers -> LDS (padded rows).
+// Every output element is the sum over K in steps of 32 in ascending order whatever the
+// tile shape or the number of rows, so a row's result does not depend on its batch.
+#pragma once
+#include <type_traits>
+
+#include "common.cuh"
+
+namespace ms {
+
+#ifdef MS_ELEM_HALF
+constexpr int EPC = 8;   // elements per 16-byte chunk
+constexpr int KPAD = 16;  // row padding in elements: rows of 96 (BK 32) or 160 (BK 64) bytes
+#else
+constexpr int EPC = 4;
+constexpr int KPAD = 8;  // rows of 160 bytes (BK 32)
+#endif
+
+enum EpiKind {
+    EPI_STORE_F32 = 0, EPI_STORE_ELEM = 1, EPI_RESIDUAL = 2, EPI_SWIGLU = 3, EPI_QKV_ROPE = 4, EPI_ACT = 5,
+    EPI_EXPERT_GATED = 6, EPI_EXPERT_PLAIN = 7, EPI_EXPERT_DOWN = 8,  // over the rows that chose an expert (routed.hip)
+};
+
+struct NoExperts {
+    __device__ __forceinline__ int source(int m, int) const { return m; }
+    __device__ __forceinline__ int pitch(int K) const { return K; }  // elements from a row of A to the next
+};
+
+struct EpiArgs {
+    void* out;          // [M, ldo]
+    const float* bias;  // [N] or null
+    int ldo;
+    int n_out;          // SWIGLU: number of output columns (intermediate size)
+    int k_per_split;    // K range of one blockIdx.y slice (multiple of 32); K itself without split
+    size_t split_stride;  // STORE_F32 with gridDim.y > 1: elements between the slices' outputs
+    // a factor a row for the finished sums (the RMS norm of rows that came in multiplied by the norm's weight only):
+    // 1 / sqrt(sum over parts of row_ss[part, row] / K + ss_eps)
+    const float* row_ss;  // [ss_parts, M] or null
+    int ss_parts;
+    float ss_eps;
+    int act;            // SWIGLU: the activation on the gate (GateActivation); ACT: the activation (UnaryActivation)
+    // QKV_ROPE: the columns are H query heads, KV key heads and KV value heads of the tile's width; bias added, queries
+    // and keys rotated by the rows' angles (pairs (j, j + half a head)), queries to `out` [M, H * hd], keys and values
+    // into their pages
+    const float* rope_cs;  // [M, hd / 2, 2]: cosine and sine of each row's angles
+    const int* slot_map;   // [M]: page * ps + offset of each row's key and value, or negative: not written
+    elem_t* kpool;         // [pages, KV, ps, hd]
+    elem_t* vpool;         // [pages, KV, hd, ps]
+    int H, KV, ps;
+};
+
+// The block of rows m0 .. m0 + BM and columns n0 .. n0 + BN.  `rows` says which row of A the block's row i is and, for the
+// experts' epilogues, what becomes of it (NoExperts: the rows as they come).
+template <int BM, int BN, int WM, int WN, int BK, int EPI, int STAGES, bool SCALED, class Rows>
+__device__ __forceinline__ void gemm_tile(const elem_t* __restrict__ A, const elem_t* __restrict__ W, int M, int N, int K, const EpiArgs& ep,
+                                          int m0, int n0, int split, const Rows& rows) {
+    static_assert(WM * WN == 4 || WM * WN == 8, "four waves, or eight for the widest tiles");
+    constexpr int NT = 64 * WM * WN;  // threads of the block
+    static_assert(BK % 32 == 0, "K step in MFMA steps of 32");
+#ifdef MS_ELEM_HALF
+    constexpr bool DIRECT = BK == 64;
+#else
+    constexpr bool DIRECT = false;
+#endif
+    constexpr int LDS_LD = DIRECT ? BK : BK + KPAD;
+    constexpr int CPR = BK / EPC;  // chunks per tile row
+    // where chunk `chunk` of tile row `row` lies in a buffer
+    auto at = [](int row, int chunk) { return row * LDS_LD + (DIRECT ? (chunk ^ (row & 7)) : chunk) * EPC; };
+    constexpr int TM = BM / WM / 16, TN = BN / WN / 16;
+    constexpr int A_CHUNKS = BM * CPR / NT, W_CHUNKS = BN * CPR / NT;
+    static_assert(BM * CPR % NT == 0 && BN * CPR % NT == 0, "tile loads divide over the block");
+    static_assert(NT == 256 || !SCALED, "the row factors' shares are dealt to four waves");
+    static_assert(STAGES == 2 || DIRECT, "more than two LDS buffers only with direct loads");
+    static_assert(!SCALED || (STAGES > 2 && EPI == EPI_SWIGLU), "row factors: built for the gated product with several steps in flight");
+    static_assert(256 % BM == 0 || !SCALED, "threads are dealt to the rows");
+    __shared__ float ss_q[SCALED ? 256 / BM : 1][SCALED ? BM : 1];  // the rows' sums of squares, in 256 / BM interleaved shares
+    float ss_v[SCALED ? 8 : 1];
+    int ss_r = 0;
+    __shared__ __attribute__((aligned(16))) elem_t As[STAGES][BM * LDS_LD];
+    __shared__ __attribute__((aligned(16))) elem_t Ws[STAGES][BN * LDS_LD];
+
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int wm = wave / WN, wn = wave % WN;
+    const int r16 = lane & 15, grp = lane >> 4;
+
+    const int k_end = min(K, (split + 1) * ep.k_per_split);
+    // Loads are unconditional, on one straight path: a row beyond the operand reads the last row
+    // (its results are never stored), and only the last K step of a slice, if it is a partial one,
+    // masks what lies beyond the slice.
+    u32x4 ra[A_CHUNKS], rw[W_CHUNKS];
+    const elem_t* pa[A_CHUNKS];
+    const elem_t* pw[W_CHUNKS];
+    // Thread t owns position (t + i * NT) % CPR of tile row (t + i * NT) / CPR; with swizzled rows that
+    // position holds another chunk of K, the same one for every i (NT / CPR rows on is a multiple of 8).
+    const int my_chunk = DIRECT ? (tid % CPR) ^ ((tid / CPR) & 7) : tid % CPR;
+#pragma unroll
+    for (int i = 0; i < A_CHUNKS; ++i) {
+        const int c = tid + i * NT;
+        pa[i] = A + (size_t)rows.source(min(m0 + c / CPR, M - 1), m0) * rows.pitch(K) + my_chunk * EPC;
+    }
+#pragma unroll
+    for (int i = 0; i < W_CHUNKS; ++i) {
+        const int c = tid + i * NT;
+        pw[i] = W + (size_t)min(n0 + c / CPR, N - 1) * K + my_chunk * EPC;
+    }
+    auto load_global = [&](int k0) {
+#pragma unroll
+        for (int i = 0; i < A_CHUNKS; ++i) ra[i] = *reinterpret_cast<const u32x4*>(pa[i] + k0);
+#pragma unroll
+        for (int i = 0; i < W_CHUNKS; ++i) rw[i] = *reinterpret_cast<const u32x4*>(pw[i] + k0);
+    };
+    auto load_global_tail = [&](int k0) {
+        const int kk = k0 + my_chunk * EPC;  // the same K chunk for all of a thread's loads
+        const bool in = kk < k_end;
+        const uint32_t keep = opaque(in ? 0xffffffffu : 0u);
+#pragma unroll
+        for (int i = 0; i < A_CHUNKS; ++i) {
+            u32x4 v = *reinterpret_cast<const u32x4*>(in ? pa[i] + k0 : A);  // the operand's start when beyond the slice
+            ra[i] = (u32x4){v[0] & keep, v[1] & keep, v[2] & keep, v[3] & keep};
+        }
+#pragma unroll
+        for (int i = 0; i < W_CHUNKS; ++i) {
+            u32x4 v = *reinterpret_cast<const u32x4*>(in ? pw[i] + k0 : W);
+            rw[i] = (u32x4){v[0] & keep, v[1] & keep, v[2] & keep, v[3] & keep};
+        }
+    };
+    auto store_lds = [&](int buf) {
+#pragma unroll
+        for (int i = 0; i < A_CHUNKS; ++i) {
+            const int c = tid + i * NT, row = c / CPR;
+            *reinterpret_cast<u32x4*>(&As[buf][at(row, my_chunk)]) = ra[i];
+        }
+#pragma unroll
+        for (int i = 0; i < W_CHUNKS; ++i) {
+            const int c = tid + i * NT, row = c / CPR;
+            *reinterpret_cast<u32x4*>(&Ws[buf][at(row, my_chunk)]) = rw[i];
+        }
+    };
+#ifdef MS_ELEM_HALF
+    // One K step of both tiles straight into LDS buffer `buf`: lane l of a wave's load lands at the wave's
+    // base + 16 l.  Written in assembly: of a load that it knows to write LDS the compiler makes every later
+    // LDS read wait (vmcnt(0)), and nothing would be in flight during the multiplications; the waits are
+    // explicit instead (`step_barrier`).
+    auto load_direct = [&](int k0, int buf) {
+        auto issue = [](const elem_t* g, const elem_t* l) {
+            const uint32_t base = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) const char*)l);
+            asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(g), "s"(base) : "memory", "m0");
+        };
+#pragma unroll
+        for (int i = 0; i < A_CHUNKS; ++i) issue(pa[i] + k0, &As[buf][(i * NT + wave * 64) * EPC]);
+#pragma unroll
+        for (int i = 0; i < W_CHUNKS; ++i) issue(pw[i] + k0, &Ws[buf][(i * NT + wave * 64) * EPC]);
+    };
+#endif
+    // End of a K step: this wave's loads and LDS accesses have completed, then everybody's.
+    auto step_barrier = [&]() {
+        if constexpr (DIRECT) {
+            __builtin_amdgcn_sched_barrier(0);
+            asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+            __builtin_amdgcn_s_barrier();
+            __builtin_amdgcn_sched_barrier(0);
+        } else {
+            __syncthreads();
+        }
+    };
+
+    f32x4 acc[TM][TN];
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+
+    // a slice of K per blockIdx.y: partial sums that the consumer adds in slice order
+    const int k_begin = split * ep.k_per_split;
+    const int nk = ceil_div(k_end - k_begin, BK);
+    const bool partial = (k_end - k_begin) % BK != 0;  // the last step is a partial one
+    auto multiply = [&](int buf) {
+#pragma unroll
+        for (int kk = 0; kk < BK; kk += 32) {
+            Frag fa[TM], fb[TN];
+            if constexpr (DIRECT) {
+#pragma unroll
+                for (int i = 0; i < TM; ++i) fa[i] = frag_load(&As[buf][at(wm * (BM / WM) + i * 16 + r16, kk / EPC + grp)]);
+#pragma unroll
+                for (int j = 0; j < TN; ++j) fb[j] = frag_load(&Ws[buf][at(wn * (BN / WN) + j * 16 + r16, kk / EPC + grp)]);
+            } else {
+#pragma unroll
+                for (int i = 0; i < TM; ++i) fa[i] = frag_load(&As[buf][(wm * (BM / WM) + i * 16 + r16) * LDS_LD + kk + grp * 8]);
+#pragma unroll
+                for (int j = 0; j < TN; ++j) fb[j] = frag_load(&Ws[buf][(wn * (BN / WN) + j * 16 + r16) * LDS_LD + kk + grp * 8]);
+            }
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+                for (int j = 0; j < TN; ++j) mma_16x16x32(acc[i][j], fa[i], fb[j]);
+        }
+    };
+    if constexpr (DIRECT && STAGES > 2) {
+#ifdef MS_ELEM_HALF
+        // A block that is alone on its CU (few tiles: one tile of rows under a weight of a few hundred column
+        // tiles) has nobody to hide its loads behind, and with one step in flight every step costs a trip to
+        // memory.  Here STAGES - 1 steps are in flight: the loads of step kt + STAGES - 1 go out before step
+        // kt is multiplied, and the step's end waits only for the loads of step kt + 1 (a wave's loads
+        // complete in order, so "all but the last (STAGES - 2) steps' loads" is a count).  The launcher
+        // gives this variant whole K steps only.
+        constexpr int PER_STEP = A_CHUNKS + W_CHUNKS;
+        static_assert(PER_STEP * (STAGES - 2) <= 63, "the wait count is a 6-bit field");
+        for (int s = 0; s < STAGES - 1; ++s)
+            if (s < nk) load_direct(k_begin + s * BK, s);
+        if constexpr (SCALED) {
+            // The rows' sums of squares, asked for behind the first K steps and not used before the last one is
+            // multiplied: what they are made of was written by the kernel before this one, a slow read that the
+            // walk over K covers.  Thread (row, q) takes parts q, q + 256 / BM, ...
+            ss_r = min(m0 + tid % BM, M - 1);
+#pragma unroll
+            for (int u = 0; u < 8; ++u) ss_v[u] = ep.row_ss[(size_t)min(tid / BM + u * (256 / BM), ep.ss_parts - 1) * M + ss_r];
+        }
+        // the first step's loads: the earliest of up to STAGES - 1 steps' loads
+        __builtin_amdgcn_sched_barrier(0);
+        if (nk >= STAGES - 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PER_STEP * (STAGES - 2)) : "memory");
+        else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+        for (int kt = 0; kt < nk; ++kt) {
+            const bool more = kt + STAGES - 1 < nk;
+            if (more) load_direct(k_begin + (kt + STAGES - 1) * BK, (kt + STAGES - 1) % STAGES);
+            multiply(kt % STAGES);
+            __builtin_amdgcn_sched_barrier(0);
+            // towards the end fewer steps are in flight behind step kt + 1: wait for everything
+            if (more) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(PER_STEP * (STAGES - 2)) : "memory");
+            else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+            __builtin_amdgcn_s_barrier();
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if constexpr (SCALED) {
+            constexpr int Q = 256 / BM;
+            const int q = tid / BM;
+            float ssum = 0.f;
+#pragma unroll
+            for (int u = 0; u < 8; ++u) ssum += q + u * Q < ep.ss_parts ? ss_v[u] : 0.f;
+            for (int p = q + 8 * Q; p < ep.ss_parts; p += Q) ssum += ep.row_ss[(size_t)p * M + ss_r];  // more than 8 * Q parts: a very wide stream
+            ss_q[q][tid % BM] = ssum;
+            __syncthreads();
+        }
+#endif
+    } else if constexpr (DIRECT) {
+#ifdef MS_ELEM_HALF
+        if (nk == 1 && partial) {
+            load_global_tail(k_begin);
+            store_lds(0);
+        } else {
+            load_direct(k_begin, 0);
+        }
+        step_barrier();
+        for (int kt = 0; kt < nk; ++kt) {
+            const int buf = kt & 1;
+            // the next step: a whole one straight into the other buffer, a partial one into registers
+            const bool tail_next = kt + 2 == nk && partial;
+            if (kt + 1 < nk) {
+                if (tail_next) load_global_tail(k_begin + (kt + 1) * BK);
+                else load_direct(k_begin + (kt + 1) * BK, buf ^ 1);
+            }
+            multiply(buf);
+            if (tail_next) store_lds(buf ^ 1);
+            step_barrier();
+        }
+#endif
+    } else {
+        if (nk == 1 && partial) load_global_tail(k_begin);
+        else load_global(k_begin);
+        store_lds(0);
+        __syncthreads();
+        for (int kt = 0; kt < nk; ++kt) {
+            const int buf = kt & 1;
+            if (kt + 2 < nk || (kt + 2 == nk && !partial)) load_global(k_begin + (kt + 1) * BK);
+            else if (kt + 1 < nk) load_global_tail(k_begin + (kt + 1) * BK);
+            multiply(buf);
+            if (kt + 1 < nk) store_lds(buf ^ 1);
+            __syncthreads();
+        }
+    }
+
+    // Epilogue.  Lane holds rows grp * 4 + e of column r16 in each 16x16 tile: sixteen lanes write
+    // sixteen consecutive elements of a row.  (Four consecutive columns a lane - transposed tiles,
+    // one 8-byte store - measured slower: neighbouring lanes then write to different rows, which
+    // the memory pipeline does not merge.)  A tile wholly inside the output stores without checks:
+    // sixty-four guarded stores cost a third of a whole 2,048 x 9,728 x 896 product.
+    const int row_base = m0 + wm * (BM / WM) + grp * 4;
+    const int col_base = n0 + wn * (BN / WN) + r16;
+    const bool whole = m0 + BM <= M && n0 + BN <= N && (EPI != EPI_SWIGLU || (n0 + BN) / 2 <= ep.n_out);
+    // A tile at the lower edge of an output whose rows come in whole groups of sixteen (a decode step
+    // of 48 requests in a 64-row tile) skips the groups beyond the last row and stores the others
+    // without checks as well.
+    auto emit = [&](auto checked, auto row_groups) {
+        constexpr bool CHECKED = decltype(checked)::value, ROW_GROUPS = decltype(row_groups)::value;
+        if constexpr (EPI == EPI_SWIGLU) {
+            static_assert(TN % 2 == 0, "gate and up tiles come in pairs");
+            elem_t* out = reinterpret_cast<elem_t*>(ep.out);
+#pragma unroll
+            for (int i = 0; i < TM; ++i) {
+                if (ROW_GROUPS && m0 + wm * (BM / WM) + i * 16 >= M) continue;
+                float f[4] = {1.f, 1.f, 1.f, 1.f};  // SCALED: of the rows this lane holds
+                if constexpr (SCALED) {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const int lr = wm * (BM / WM) + i * 16 + grp * 4 + e;
+                        float ssum = 0.f;
+#pragma unroll
+                        for (int qq = 0; qq < 256 / BM; ++qq) ssum += ss_q[qq][lr];
+                        f[e] = 1.0f / sqrtf(ssum / (float)K + ep.ss_eps);
+                    }
+                }
+#pragma unroll
+                for (int j = 0; j < TN; j += 2) {
+                    const int col = (col_base + j * 16 - r16) / 2 + r16;  // tiles 2t, 2t+1 -> output tile t
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const int row = row_base + i * 16 + e;
+                        if (CHECKED && !(row < M && col < ep.n_out)) continue;
+                        float gv = acc[i][j][e], uv = acc[i][j + 1][e];
+                        if constexpr (SCALED) {
+                            gv *= f[e];
+                            uv *= f[e];
+                        }
+                        out[(size_t)row * ep.ldo + col] = from_f32<elem_t>(gate_activation(gv, ep.act) * uv);
+                    }
+                }
+            }
+        } else if constexpr (EPI == EPI_QKV_ROPE) {
+            // The tile's columns are one head (the launcher sees to it), and a wave holds all of them: lane (r16, grp)
+            // has columns r16 + 16 j of rows grp * 4 + e, so both elements of a pair (j, j + TN / 2) are its own.
+            static_assert(WN == 1 && TN % 2 == 0, "a wave holds whole heads");
+            constexpr int HT = TN / 2, hd = BN, half = BN / 2;
+            const int head = n0 / hd;
+            const int kind = head < ep.H ? 0 : (head < ep.H + ep.KV ? 1 : 2);  // query, key or value head
+            float bias_j[TN];
+#pragma unroll
+            for (int j = 0; j < TN; ++j) bias_j[j] = ep.bias ? ep.bias[n0 + j * 16 + r16] : 0.f;
+#pragma unroll
+            for (int i = 0; i < TM; ++i) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const int row = row_base + i * 16 + e;
+                    if (row >= M) continue;
+                    float x[TN];
+#pragma unroll
+                    for (int j = 0; j < TN; ++j) x[j] = bias_j[j] + acc[i][j][e];
+                    if (kind < 2) {
+                        const float* cs = ep.rope_cs + (size_t)row * (2 * half);
+#pragma unroll
+                        for (int j = 0; j < HT; ++j) {
+                            const float c = cs[2 * (j * 16 + r16)], sn = cs[2 * (j * 16 + r16) + 1];
+                            const float x0 = x[j], x1 = x[j + HT];
+                            x[j] = x0 * c - x1 * sn;
+                            x[j + HT] = x0 * sn + x1 * c;
+                        }
+                    }
+                    if (kind == 0) {
+                        elem_t* o = reinterpret_cast<elem_t*>(ep.out) + ((size_t)row * ep.H + head) * hd + r16;
+#pragma unroll
+                        for (int j = 0; j < TN; ++j) o[j * 16] = from_f32<elem_t>(x[j]);
+                    } else {
+                        const int slot = ep.slot_map[row];
+                        if (slot < 0) continue;
+                        const int page = slot / ep.ps, off = slot - page * ep.ps;
+                        if (kind == 1) {
+                            elem_t* o = ep.kpool + (((size_t)page * ep.KV + (head - ep.H)) * ep.ps + off) * hd + r16;
+#pragma unroll
+                            for (int j = 0; j < TN; ++j) o[j * 16] = from_f32<elem_t>(x[j]);
+                        } else {
+                            elem_t* o = ep.vpool + (((size_t)page * ep.KV + (head - ep.H - ep.KV)) * hd + r16) * ep.ps + off;
+#pragma unroll
+                            for (int j = 0; j < TN; ++j) o[(size_t)(j * 16) * ep.ps] = from_f32<elem_t>(x[j]);
+                        }
+                    }
+                }
+            }
+        } else if constexpr (EPI == EPI_EXPERT_GATED || EPI == EPI_EXPERT_PLAIN) {
+            // the activations of the rows that chose the expert, one block of BM rows after the other
+            constexpr int STEP = EPI == EPI_EXPERT_GATED ? 2 : 1;
+            static_assert(TN % STEP == 0, "gate and up tiles come in pairs");
+            elem_t* out = reinterpret_cast<elem_t*>(ep.out);
+#pragma unroll
+            for (int i = 0; i < TM; ++i) {
+                if (ROW_GROUPS && m0 + wm * (BM / WM) + i * 16 >= M) continue;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const int row = row_base + i * 16 + e;
+                    if (CHECKED && row >= M) continue;
+                    const float w = rows.weight(row);
+                    elem_t* o = out + (size_t)rows.slot(row, m0) * ep.ldo;
+#pragma unroll
+                    for (int j = 0; j < TN; j += STEP) {
+                        const int col = STEP == 2 ? (col_base + j * 16 - r16) / 2 + r16 : col_base + j * 16;
+                        if (CHECKED && col >= ep.n_out) continue;
+                        o[col] = from_f32<elem_t>(STEP == 2 ? rows.gated(acc[i][j][e], acc[i][j + STEP - 1][e], w) : rows.plain(acc[i][j][e], w));
+                    }
+                }
+            }
+        } else if constexpr (EPI == EPI_EXPERT_DOWN) {
+#pragma unroll
+            for (int i = 0; i < TM; ++i) {
+                if (ROW_GROUPS && m0 + wm * (BM / WM) + i * 16 >= M) continue;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const int row = row_base + i * 16 + e;
+                    if (CHECKED && row >= M) continue;
+                    float* o = reinterpret_cast<float*>(ep.out) + rows.sum_row(row) * ep.ldo;
+#pragma unroll
+                    for (int j = 0; j < TN; ++j) {
+                        const int col = col_base + j * 16;
+                        if (CHECKED && col >= N) continue;
+                        o[col] = acc[i][j][e];
+                    }
+                }
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < TM; ++i) {
+                if (ROW_GROUPS && m0 + wm * (BM / WM) + i * 16 >= M) continue;
+#pragma unroll
+                for (int j = 0; j < TN; ++j) {
+                    const int col = col_base + j * 16;
+                    const float b = ep.bias ? ep.bias[min(col, N - 1)] : 0.f;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const int row = row_base + i * 16 + e;
+                        if (CHECKED && !(row < M && col < N)) continue;
+                        const size_t o = (size_t)row * ep.ldo + col;
+                        const float v = acc[i][j][e] + b;
+                        if constexpr (EPI == EPI_STORE_F32) reinterpret_cast<float*>(ep.out)[split * ep.split_stride + o] = v;
+                        else if constexpr (EPI == EPI_STORE_ELEM) reinterpret_cast<elem_t*>(ep.out)[o] = from_f32<elem_t>(v);
+                        else if constexpr (EPI == EPI_ACT) reinterpret_cast<elem_t*>(ep.out)[o] = from_f32<elem_t>(unary_activation(v, ep.act));
+                        else reinterpret_cast<float*>(ep.out)[o] += v;  // residual stream, 32-bit
+                    }
+                }
+            }
+        }
+    };
+    const bool cols_whole = n0 + BN <= N && (EPI != EPI_SWIGLU || (n0 + BN) / 2 <= ep.n_out);
+    if (whole) emit(std::false_type{}, std::false_type{});
+    else if (cols_whole && M % 16 == 0) emit(std::false_type{}, std::true_type{});
+    else emit(std::true_type{}, std::false_type{});
+}
+
+
+}  // namespace ms

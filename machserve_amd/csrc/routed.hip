@@ -17,17 +17,26 @@
 // beyond the outputs to choose from (`extra`) are gates that every row has, the sigmoids of their own logits, left behind
 // the experts' weights; the first of them can stand for the expert that every row uses.  A weight may also multiply a gated
 // expert's input instead of its output: act(w gate) * (w up).
-#include "common.cuh"
+#include "gemm_tile.cuh"
 
 namespace ms {
 
 constexpr int MAX_EXPERTS = 1024;
 enum Scoring { SOFTMAX_CHOSEN = 0, SOFTMAX_ALL = 1, SIGMOID = 2 };
 
+// What the router leaves for the products over the chosen rows alone: plane[t, e] numbers the experts that row t uses (chosen, with a
+// weight that is not zero) in ascending order, -1 for the others; sums [top, T, width] will hold the k-th of them's output in plane k, and
+// the rows of planes that row t does not use are zeroed here.
+struct RouteSums {
+    int* plane;   // [T, real], or null: not asked for
+    float* sums;
+    int real, width, T;
+};
+
 // gates[t, e] = the row's weight for expert e, 0 where it was not chosen.  One block a row: a wave a logit in turn.
 __global__ __launch_bounds__(256) void route_kernel(const elem_t* __restrict__ x, const float* __restrict__ w,
                                                     const float* __restrict__ bias, float* __restrict__ gates, int d, int E, int top,
-                                                    int scoring, const float* __restrict__ correction, int extra) {
+                                                    int scoring, const float* __restrict__ correction, int extra, RouteSums rs) {
     const bool softmax_all = scoring == SOFTMAX_ALL;
     __shared__ float z[MAX_EXPERTS];
     __shared__ float score[MAX_EXPERTS];  // SOFTMAX_ALL: the outputs' scores; else `extra` logits
@@ -91,9 +100,7 @@ __global__ __launch_bounds__(256) void route_kernel(const elem_t* __restrict__ x
     __syncthreads();
     if (scoring == SIGMOID) {
         if (threadIdx.x < top && chosen_e[threadIdx.x] < E) g[chosen_e[threadIdx.x]] = 1.0f / (1.0f + expf(-chosen_z[threadIdx.x]));
-        return;
-    }
-    if (threadIdx.x == 0 && softmax_all) {
+    } else if (threadIdx.x == 0 && softmax_all) {
         float sum = 0.f;
         for (int k = 0; k < top; ++k)
             if (chosen_e[k] < E) sum += score[chosen_e[k]];
@@ -106,6 +113,26 @@ __global__ __launch_bounds__(256) void route_kernel(const elem_t* __restrict__ x
         for (int k = 0; k < top; ++k)
             if (chosen_e[k] < E) g[chosen_e[k]] = expf(chosen_z[k] - m) / sum;
     }
+    if (!rs.plane) return;
+    int* pl = rs.plane + (size_t)t * rs.real;
+    for (int e = threadIdx.x; e < rs.real; e += 256) pl[e] = -1;
+    __syncthreads();  // (the weights above are this block's own stores: visible behind the barrier)
+    __shared__ int used;
+    if (wave == 0) {
+        const int e = lane < top ? chosen_e[lane] : MAX_EXPERTS;
+        const bool uses = e < rs.real && g[e] != 0.f;
+        int at = 0;
+        for (int k = 0; k < top; ++k) {
+            const int other = __shfl(uses ? e : MAX_EXPERTS, k, WAVE);
+            at += other < e;
+        }
+        if (uses) pl[e] = at;
+        const unsigned long long all = __ballot(uses);
+        if (lane == 0) used = __popcll(all);
+    }
+    __syncthreads();
+    for (int p = used; p < top; ++p)
+        for (int c = threadIdx.x; c < rs.width; c += 256) rs.sums[((size_t)p * rs.T + t) * rs.width + c] = 0.f;
 }
 
 // act: 0 the exact GELU (erf), 1 its tanh form, 2 SiLU
@@ -183,22 +210,192 @@ __global__ __launch_bounds__(256) void add_scaled_rows_kernel(float* __restrict_
         x[(size_t)t * d + c] += w * to_f32(h[(size_t)t * d + c]);
 }
 
+// ---- products over the rows that chose an expert -------------------------------------------------------------------------
+// Of E experts a row uses `top`, so a product over every expert's columns does E / top times the work (2,048 rows of 2,048, 8
+// experts of 2,816 of which 2 are used, and one that every row uses: up, activation and down 366 + 73 + 366 us a layer where this
+// does it all in a third).  Here a block's tile of rows belongs to one expert: the up product gathers the rows that chose it, applies
+// the activation and the weight in its epilogue (the 32-bit sums of all experts never go through memory), and leaves the
+// activations tile after tile; the down product multiplies them by the expert's own matrix and stores the sums in the planes that
+// the reader adds up, one for each expert that a row uses, in ascending order.  Who reads what is found by the blocks themselves: a step of
+// at most 64 rows has one tile an expert, whose rows a wave finds with one ballot; above, `expert_rows_kernel` lists them
+// and a block finds its expert by a prefix sum over the lists' lengths.  Blocks of tiles that do not exist end at once.
+struct ExpertArgs {
+    const int* plane;     // [T, E]
+    const float* gates;   // [T, ld_gates]
+    const int* rows;      // [E, T] lists of the experts' rows, or null: T <= 64
+    const int* counts;    // [E] their lengths
+    int T, E, ld_gates, top;
+    int routed_tiles, shared_tiles;  // row tiles of the grid: those of the experts (as many as there can be), those of the expert that every row uses
+    int ff, shared;       // columns of an expert, and of the one that every row uses (0: there is none)
+    int width;            // of the rows
+    int shared_gate, weigh_input, act;
+};
+
+__global__ __launch_bounds__(1024) void expert_rows_kernel(const int* __restrict__ plane, int* __restrict__ rows, int* __restrict__ counts, int T, int E) {
+    __shared__ int part[2][16];
+    const int e = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    int n = 0;
+    for (int t0 = 0, turn = 0; t0 < T; t0 += 1024, turn ^= 1) {  // two sets of partial counts in turn: one barrier a round
+        const int t = t0 + threadIdx.x;
+        const bool mine = t < T && plane[(size_t)min(t, T - 1) * E + e] >= 0;
+        const unsigned long long all = __ballot(mine);
+        if (lane == 0) part[turn][wave] = __popcll(all);
+        __syncthreads();
+        int before = n;
+        for (int w = 0; w < 16; ++w) {
+            if (w < wave) before += part[turn][w];
+            n += part[turn][w];
+        }
+        if (mine) rows[(size_t)e * T + before + __popcll(all & ((1ull << lane) - 1))] = t;
+    }
+    if (threadIdx.x == 0) counts[e] = n;
+}
+
+struct ExpertRows {
+    const ExpertArgs& g;
+    const int* list;  // of the expert's rows; null: every row
+    int e, tile;      // e == E: the expert that every row uses
+    int bm;
+    bool gathers;     // A's rows are the step's rows (the up product), else the tiles' activations (the down product)
+    __device__ __forceinline__ int row_of(int m) const { return list ? list[m] : m; }
+    __device__ __forceinline__ int slot(int m, int m0) const { return tile * bm + (m - m0); }
+    __device__ __forceinline__ int source(int m, int m0) const { return gathers ? row_of(m) : slot(m, m0); }
+    __device__ __forceinline__ int pitch(int) const { return gathers ? g.width : max(g.ff, g.shared); }
+    __device__ __forceinline__ float weight(int m) const {
+        if (e == g.E && !g.shared_gate) return 1.0f;
+        return g.gates[(size_t)row_of(m) * g.ld_gates + e];
+    }
+    // as expert_act: the weight on the output, or inside the expert
+    __device__ __forceinline__ float gated(float gv, float uv, float w) const {
+        const float wi = g.weigh_input && e < g.E ? w : 1.0f;
+        return w != 0.f ? expert_activation(wi * gv, g.act) * uv * w : 0.f;
+    }
+    __device__ __forceinline__ float plain(float z, float w) const { return w != 0.f ? expert_activation(z, g.act) * w : 0.f; }
+    __device__ __forceinline__ size_t sum_row(int m) const {
+        const int t = row_of(m);
+        const int p = e == g.E ? g.top : g.plane[(size_t)t * g.E + e];
+        return (size_t)p * g.T + t;
+    }
+};
+
+template <int BM, int BN, int WM, int WN, int BK, int EPI, int STAGES>
+__global__ __launch_bounds__(64 * WM * WN) void expert_gemm_kernel(const elem_t* __restrict__ A, const elem_t* __restrict__ W, void* out, ExpertArgs g) {
+    __shared__ int few[64];
+    const int tiles = g.routed_tiles + g.shared_tiles, lane = threadIdx.x & 63;
+    const int tile = blockIdx.x % tiles;
+    int e = g.E, m0 = (tile - g.routed_tiles) * BM, count = g.T;
+    const int* list = nullptr;
+    if (tile < g.routed_tiles && !g.rows) {
+        e = tile;
+        m0 = 0;
+        const bool mine = lane < g.T && g.plane[(size_t)min(lane, g.T - 1) * g.E + e] >= 0;
+        const unsigned long long all = __ballot(mine);
+        count = __popcll(all);
+        if (mine) few[__popcll(all & ((1ull << lane) - 1))] = lane;
+        list = few;
+    } else if (tile < g.routed_tiles) {
+        // the expert whose tiles hold this one: 64 experts' counts of tiles at a time (none: a tile beyond the lists, no rows)
+        int base = 0;
+        count = m0 = 0;
+        for (int e0 = 0; e0 < g.E; e0 += 64) {
+            const int c = e0 + lane < g.E ? g.counts[e0 + lane] : 0;
+            const int mine = ceil_div(c, BM);
+            int upto = mine;
+#pragma unroll
+            for (int o = 1; o < 64; o <<= 1) {
+                const int v = __shfl_up(upto, o, WAVE);
+                if (lane >= o) upto += v;
+            }
+            const unsigned long long behind = __ballot(base + upto > tile);
+            if (behind) {
+                const int at = __builtin_ctzll(behind);
+                e = e0 + at;
+                count = __shfl(c, at, WAVE);
+                m0 = (tile - (base + __shfl(upto - mine, at, WAVE))) * BM;
+                break;
+            }
+            base += __shfl(upto, 63, WAVE);
+        }
+        list = g.rows + (size_t)e * g.T;
+    }
+    e = __builtin_amdgcn_readfirstlane(e);
+    count = __builtin_amdgcn_readfirstlane(count);
+    m0 = __builtin_amdgcn_readfirstlane(m0);
+    const int cols = e == g.E ? g.shared : g.ff;
+    constexpr int PER = EPI == EPI_EXPERT_GATED ? 2 : 1;  // columns of the up product for one of the activations
+    const int N = EPI == EPI_EXPERT_DOWN ? g.width : PER * cols, K = EPI == EPI_EXPERT_DOWN ? cols : g.width;
+    const int n0 = blockIdx.x / tiles * BN;
+    if (m0 >= count || n0 >= N) return;  // the whole block: these are the block's own numbers
+    __syncthreads();
+    EpiArgs ep{out, nullptr, EPI == EPI_EXPERT_DOWN ? g.width : max(g.ff, g.shared), cols, K, 0};
+    const ExpertRows rows{g, list, e, tile, BM, EPI != EPI_EXPERT_DOWN};
+    const elem_t* own = W + (size_t)e * (EPI == EPI_EXPERT_DOWN ? 1 : PER) * g.ff * g.width;
+    gemm_tile<BM, BN, WM, WN, BK, EPI, STAGES, false>(A, own, count, N, K, ep, m0, n0, 0, rows);
+}
+
+// Rows of a tile: a step of at most 64 rows has one tile an expert; above, the larger tile where the experts' lists can be expected to fill it.
+static int expert_tile_rows(int T, int E, int top) {
+#ifdef MS_ELEM_HALF
+    return T <= 64 || (long)T * top < 96L * E ? 64 : 128;
+#else
+    (void)T; (void)E; (void)top;
+    return 64;
+#endif
+}
+
+static long expert_routed_tiles(int T, int E, int top) {
+    if (T <= 64) return E;
+    const long bm = expert_tile_rows(T, E, top);
+    return min((long)T * top / bm + min((long)E, (long)T * top), (long)E * ceil_div((long)T, bm));
+}
+
+static int check_experts(const char* what, const ExpertArgs& g) {
+    MS_REQUIRE(g.T > 0 && g.E > 0 && g.E <= MAX_EXPERTS && g.top >= 1 && g.top <= 64, "%s: %d rows, %d of %d experts", what, g.T, g.top, g.E);
+    MS_REQUIRE(g.width > 0 && g.width % 64 == 0 && g.ff > 0 && g.ff % 64 == 0 && g.shared >= 0 && g.shared % 64 == 0,
+               "%s: width %d, experts of %d and %d for every row: multiples of 64 are taken", what, g.width, g.ff, g.shared);
+    MS_REQUIRE(g.plane && g.gates && g.ld_gates >= g.E + (g.shared_gate ? 1 : 0), "%s: %d weights a row for %d experts", what, g.ld_gates, g.E);
+    MS_REQUIRE(g.act >= 0 && g.act <= 2, "%s: activation %d", what, g.act);
+    MS_REQUIRE((g.T <= 64) == (g.rows == nullptr) && (g.T <= 64) == (g.counts == nullptr), "%s: lists of rows go with more than 64 of them", what);
+    return 0;
+}
+
+template <int EPI>
+static int launch_experts(const void* a, const void* w, void* out, ExpertArgs g, hipStream_t stream) {
+    MS_REQUIRE((reinterpret_cast<uintptr_t>(a) & 15) == 0 && (reinterpret_cast<uintptr_t>(w) & 15) == 0, "experts: operands must be 16-byte aligned");
+    const int bm = expert_tile_rows(g.T, g.E, g.top);
+    g.routed_tiles = (int)expert_routed_tiles(g.T, g.E, g.top);
+    g.shared_tiles = g.shared ? ceil_div(g.T, bm) : 0;
+    const int N = EPI == EPI_EXPERT_DOWN ? g.width : (EPI == EPI_EXPERT_GATED ? 2 : 1) * max(g.ff, g.shared);
+#define MS_EXPERTS(BM_, BN_, WM_, WN_, BK_, ST_)                                                                                           do {                                                                                                                                       const long nb = (long)(g.routed_tiles + g.shared_tiles) * ceil_div(N, BN_);                                                            hipLaunchKernelGGL((expert_gemm_kernel<BM_, BN_, WM_, WN_, BK_, EPI, ST_>), dim3((unsigned)nb), dim3(64 * WM_ * WN_), 0, stream,                            (const elem_t*)a, (const elem_t*)w, out, g);                                                                        return check_launch("experts " #BM_ "x" #BN_ "x" #BK_);                                                                            } while (0)
+#ifdef MS_ELEM_HALF
+    if (bm == 128) MS_EXPERTS(128, 128, 2, 2, 64, 2);
+    MS_EXPERTS(64, 64, 2, 2, 64, 4);
+#else
+    (void)bm;
+    MS_EXPERTS(64, 64, 2, 2, 32, 2);
+#endif
+#undef MS_EXPERTS
+}
+
 }  // namespace ms
 
 using namespace ms;
 
 extern "C" int ms_route_max_experts() { return MAX_EXPERTS; }
 
-// w [E + extra, d]; gates [T, E + extra]: the weights of the E outputs to choose from, then `extra` gates of every row.
+// w [E + extra, d]; gates [T, E + extra]: the weights of the E outputs to choose from, then `extra` gates of every row.  With `plane`
+// [T, real] (else null) the experts that each row uses among the first `real` outputs are numbered, and the rows of sums [top, T, d] that
+// no expert will write are zeroed.
 extern "C" int ms_route(const void* x, const float* w, const float* bias, float* gates, int T, int d, int E, int top, int scoring,
-                        const float* correction, int extra, hipStream_t stream) {
+                        const float* correction, int extra, int* plane, float* sums, int real, hipStream_t stream) {
     MS_REQUIRE(scoring >= SOFTMAX_CHOSEN && scoring <= SIGMOID, "route: scoring %d", scoring);
     MS_REQUIRE(extra >= 0 && extra <= MAX_EXPERTS && (extra == 0 || (scoring != SOFTMAX_ALL && !bias)),
                "route: %d gates of every row (none with scores over all outputs or a bias)", extra);
     MS_REQUIRE(T > 0 && d > 0 && E > 0 && E <= MAX_EXPERTS, "route: %d rows of %d over %d experts (at most %d)", T, d, E, MAX_EXPERTS);
     MS_REQUIRE(top >= 1 && top <= E && top <= 64, "route: %d of %d experts a row (at most 64)", top, E);
+    MS_REQUIRE((plane == nullptr) == (sums == nullptr) && (!plane || (real > 0 && real <= E)), "route: %d of %d outputs are experts", real, E);
     hipLaunchKernelGGL(route_kernel, dim3(T), dim3(256), 0, stream, (const elem_t*)x, w, bias, gates, d, E, top, scoring, correction,
-                       extra);
+                       extra, RouteSums{plane, sums, real, d, T});
     return check_launch("route");
 }
 
@@ -224,4 +421,38 @@ extern "C" int ms_add_scaled_rows(float* x, const void* h, const float* weights,
     hipLaunchKernelGGL(add_scaled_rows_kernel, dim3(T, ceil_div(d, 1024)), dim3(256), 0, stream, x, (const elem_t*)h, weights, ld_w, first,
                        count, d);
     return check_launch("add_scaled_rows");
+}
+
+// Rows of the activations that ms_experts_up leaves and ms_experts_down reads (a tile's rows one behind the other, tile after tile).
+extern "C" long ms_experts_slots(int T, int E, int top, int shared) {
+    if (T <= 0 || E <= 0 || top <= 0) return 0;
+    const long bm = expert_tile_rows(T, E, top);
+    return (expert_routed_tiles(T, E, top) + (shared > 0 ? ceil_div((long)T, bm) : 0)) * bm;
+}
+
+// rows [E, T], counts [E]: the rows that use each expert, in ascending order.
+extern "C" int ms_expert_rows(const int* plane, int* rows, int* counts, int T, int E, hipStream_t stream) {
+    MS_REQUIRE(plane && rows && counts && T > 0 && E > 0 && E <= MAX_EXPERTS, "expert rows: %d rows of %d experts", T, E);
+    hipLaunchKernelGGL(expert_rows_kernel, dim3(E), dim3(1024), 0, stream, plane, rows, counts, T, E);
+    return check_launch("expert_rows");
+}
+
+// x [T, width]; w: the experts' matrices one behind the other and then that of the expert every row uses (`shared` columns, 0: none), each
+// [cols, width], or with `gated` [2 cols, width] with gate and up rows interleaved in blocks of 16; out [slots, max(ff, shared)].
+extern "C" int ms_experts_up(const void* x, const void* w, void* out, const int* plane, const float* gates, const int* rows, const int* counts,
+                             int T, int E, int ld_gates, int top, int ff, int shared, int width, int gated, int shared_gate, int weigh_input,
+                             int act, hipStream_t stream) {
+    const ExpertArgs g{plane, gates, rows, counts, T, E, ld_gates, top, 0, 0, ff, shared, width, shared_gate, weigh_input, act};
+    if (int rc = check_experts("experts up", g)) return rc;
+    MS_REQUIRE(!weigh_input || gated, "experts up: weights inside experts that are not gated");
+    return gated ? launch_experts<EPI_EXPERT_GATED>(x, w, out, g, stream) : launch_experts<EPI_EXPERT_PLAIN>(x, w, out, g, stream);
+}
+
+// a [slots, max(ff, shared)] as ms_experts_up leaves it; w: the experts' [width, ff] one behind the other,
+// then the shared one's; sums [top (+ 1), T, width]: plane k of row t is the k-th expert that it uses, the last plane the shared one's.
+extern "C" int ms_experts_down(const void* a, const void* w, float* sums, const int* plane, const float* gates, const int* rows, const int* counts,
+                               int T, int E, int ld_gates, int top, int ff, int shared, int width, hipStream_t stream) {
+    const ExpertArgs g{plane, gates, rows, counts, T, E, ld_gates, top, 0, 0, ff, shared, width, 0, 0, 0};
+    if (int rc = check_experts("experts down", g)) return rc;
+    return launch_experts<EPI_EXPERT_DOWN>(a, w, sums, g, stream);
 }

@@ -1336,13 +1336,16 @@ class HipOps:
         return {"experts": self._extra_lib("routed").ms_route_max_experts(), "top": 64}
 
     def route(self, h: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], top: int, correction: Optional[torch.Tensor] = None,
-              softmax_all: bool = False, sigmoid: bool = False, extra_gates: int = 0) -> torch.Tensor:
+              softmax_all: bool = False, sigmoid: bool = False, extra_gates: int = 0, plane: Optional[torch.Tensor] = None,
+              sums: Optional[torch.Tensor] = None) -> torch.Tensor:
         """Float32 ``[T, experts]``: for every row its weight for each expert, the softmax over the ``top`` largest of the
         logits ``h @ w.T + bias`` (32-bit sums, float32 weights; the lower index wins a tie), zero for the others.  With
         ``softmax_all`` the scores are the softmax over all logits, the ``top`` largest of score + ``correction`` are chosen,
         and the weights are the chosen scores over their sum (+ 1e-20).  With ``sigmoid`` the weights are the sigmoids of the
         chosen logits.  ``extra_gates``: that many last rows of ``w`` are no experts but gates of every row, the sigmoids of
-        their logits, left in the last columns (``[T, experts + extra_gates]``)."""
+        their logits, left in the last columns (``[T, experts + extra_gates]``).  ``plane`` int32 ``[T, n]`` receives, for the first
+        ``n`` outputs, the number of each among those that the row uses, in ascending order, or -1; rows of ``sums`` (float32
+        ``[top or more, T, d]``) in planes that a row does not use are zeroed."""
         lib = self._extra_lib("routed")
         T, d = h.shape
         E = w.shape[0] - extra_gates
@@ -1354,8 +1357,41 @@ class HipOps:
             self._want(correction, torch.float32, "route correction", E)
         gates = torch.empty((T, E + extra_gates), dtype=torch.float32, device=h.device)
         self._check(lib, lib.ms_route(_ptr(h), _ptr(w), _ptr(bias), _ptr(gates), _c_int(T), _c_int(d), _c_int(E), _c_int(top),
-                                      _c_int(1 if softmax_all else (2 if sigmoid else 0)), _ptr(correction), _c_int(extra_gates), self._stream()))
+                                      _c_int(1 if softmax_all else (2 if sigmoid else 0)), _ptr(correction), _c_int(extra_gates), _ptr(plane),
+                                      _ptr(sums), _c_int(0 if plane is None else plane.shape[1]), self._stream()))
         return gates
+
+    def routed_experts_takes(self, width: int, ff: int, shared: int, top: int) -> bool:
+        """Whether experts of these sizes run over the rows that chose them (:meth:`routed_experts`): whole K steps of both
+        products, and no more planes than a reader's kernel asks for at once."""
+        return width % 64 == 0 and ff % 64 == 0 and shared % 64 == 0 and top + (shared > 0) <= 16
+
+    def routed_experts(self, h: torch.Tensor, w_router: torch.Tensor, b_router: Optional[torch.Tensor], top: int, w_up: torch.Tensor,
+                       w_down: torch.Tensor, experts: int, ff: int, shared: int, activation: str, gated: bool = False, weigh_input: bool = False,
+                       shared_gate: bool = False, **scoring):
+        """A feed-forward of routed experts over the rows that chose each: ``(sums, gates)``, float32 ``[top (+ 1), T, width]`` whose sum
+        over the first axis is the feed-forward's output, and the rows' weights (:meth:`route`, whose other arguments ``scoring`` are).
+        ``w_up``: the experts' up matrices one behind the other and then that of the expert that every row uses, each ``[cols, width]`` or
+        with ``gated`` gate and up interleaved (:func:`interleave_gate_up`); ``w_down`` flat: each expert's ``[width, cols]`` in the same order."""
+        lib = self._extra_lib("routed")
+        T, d = h.shape
+        self._want(w_up, self.dtype, "experts up", (2 if gated else 1) * (experts * ff + shared), d)
+        self._want(w_down, self.dtype, "experts down", d * (experts * ff + shared))
+        if activation not in self.EXPERT_ACTIVATIONS:
+            raise KernelError(f"experts: activation {activation!r} is not built (built: {', '.join(sorted(self.EXPERT_ACTIVATIONS))})")
+        new = lambda shape, dt: torch.empty(shape, dtype=dt, device=h.device)  # noqa: E731
+        plane, sums = new((T, experts), torch.int32), new((top + (shared > 0), T, d), torch.float32)
+        gates = self.route(h, w_router, b_router, top, extra_gates=int(shared_gate), plane=plane, sums=sums, **scoring)
+        rows = counts = None
+        if T > 64:  # fewer: the products' blocks find an expert's rows themselves
+            rows, counts = new((experts, T), torch.int32), new((experts,), torch.int32)
+            self._check(lib, lib.ms_expert_rows(_ptr(plane), _ptr(rows), _ptr(counts), _c_int(T), _c_int(experts), self._stream()))
+        a = new((self._plan("ms_experts_slots", T, experts, top, shared, lib=lib), max(ff, shared)), self.dtype)
+        sizes = [_ptr(plane), _ptr(gates), _ptr(rows), _ptr(counts)] + [_c_int(v) for v in (T, experts, gates.shape[1], top, ff, shared, d)]
+        self._check(lib, lib.ms_experts_up(_ptr(h), _ptr(w_up), _ptr(a), *sizes, _c_int(int(gated)), _c_int(int(shared_gate)),
+                                           _c_int(int(weigh_input)), _c_int(self.EXPERT_ACTIVATIONS[activation]), self._stream()))
+        self._check(lib, lib.ms_experts_down(_ptr(a), _ptr(w_down), _ptr(sums), *sizes, self._stream()))
+        return sums, gates
 
     def expert_act(self, up: torch.Tensor, gates: torch.Tensor, ff: int, activation: str, experts: Optional[int] = None,
                    gated: bool = False, weigh_input: bool = False, shared_gate: bool = False) -> torch.Tensor:

@@ -129,6 +129,11 @@ class ResidualStream:
             self.x += bias
         self.deferred = (a, w)
 
+    def add_sums(self, sums: torch.Tensor) -> None:
+        """``x += sum(sums)`` for float32 ``sums [P, T, width]`` that a part's last product left; the next reader adds them."""
+        self.open()
+        self.pending = sums
+
     def add_normed_mean(self, branches, eps: float) -> None:
         """``x += mean_i rmsnorm(a_i @ w_i.T) * g_i`` for branches side by side, each given as ``((a, w), g)``: the
         operands of its last product and the weight of its norm."""

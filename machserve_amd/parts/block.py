@@ -77,9 +77,13 @@ class _Branch:
         self.branches = None
         self.weighted = None
         self.scaled = None
+        self.sums = None
 
     def add_linear(self, a, w, bias=None) -> None:
         self.product, self.bias = (a, w), bias
+
+    def add_sums(self, sums) -> None:
+        self.sums = sums
 
     def add_normed_mean(self, branches, eps) -> None:
         self.branches = (list(branches), eps)
@@ -146,7 +150,9 @@ class MultiStreamBlock(Block):
             h = norm.forward(stream.read(mix.w_in))
         out = _Branch(ops)
         part.forward(h, out, ctx)
-        if out.product is not None:
+        if out.sums is not None:
+            sums = out.sums
+        elif out.product is not None:
             sums = ops.linear_split(*out.product)
         elif out.tensor is not None:
             sums = out.tensor.float().contiguous().unsqueeze(0)
@@ -190,6 +196,8 @@ class SandwichBlock(Block):
         stream.flush()  # a norm left pending has added what was pending by now; nothing else may be
         if out.weighted is not None:
             post.add_normed_weighted(stream, out.weighted)
+        elif out.sums is not None:
+            post.add_normed_sums(stream, out.sums)
         elif out.product is not None:
             post.add_normed(stream, *out.product)
         else:
@@ -230,6 +238,8 @@ class PostNormBlock(Block):
             post.add_normed_mean(stream, *out.branches)
         elif out.weighted is not None:
             post.add_normed_weighted(stream, out.weighted)
+        elif out.sums is not None:
+            post.add_normed_sums(stream, out.sums)
         elif out.product is not None:
             post.add_normed(stream, *out.product, bias=out.bias)
         else:
@@ -265,7 +275,9 @@ class SumNormBlock(Block):
         ops = self.rt.ops
         out = _Branch(ops)
         part.forward(stream.value() if getattr(part, "reads_stream", False) else stream.rows(), out, ctx)
-        if out.product is not None:
+        if out.sums is not None:
+            sums = out.sums
+        elif out.product is not None:
             sums = ops.linear_split(*out.product)
         elif out.tensor is not None:
             sums = out.tensor.float().contiguous().unsqueeze(0)

@@ -53,6 +53,10 @@ class RMSNorm(Norm):
             stream.open()
             stream.ops.norm_add_bias(stream.x, stream.ops.linear_split(a, w), bias, self.weight, self.spec.eps)
 
+    def add_normed_sums(self, stream, sums) -> None:
+        """``x += rmsnorm(sum(sums)) * weight`` for a branch whose last product has left its sums, float32 ``[P, T, width]``."""
+        stream.add_normed_sums([(sums, 1.0)], self.weight, self.spec.eps)
+
     def add_normed_mean(self, stream, branches, eps) -> None:
         """``x += rmsnorm((rmsnorm(a) * wa + rmsnorm(b) * wb) / 2) * weight`` for two branches side by side, given as
         ``branches = [((a, w_a), wa), ((b, w_b), wb)]`` with each branch the operands of its last product."""

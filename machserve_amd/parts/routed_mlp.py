@@ -5,7 +5,9 @@ The router's logits are 32-bit sums over 32-bit weights; a row's ``top`` largest
 over the chosen logits alone weighs them.  All experts' up projections are one matrix and their down projections one
 matrix: the up product runs for every expert, one kernel applies the activation and the row's weight for the expert
 (an exact zero for an expert the row did not choose, one for the expert that every row uses), and the down product
-sums the chosen experts' outputs.  A row's result depends on its own logits alone.
+sums the chosen experts' outputs.  A row's result depends on its own logits alone.  Where the kernels take the sizes
+(``routed_experts_takes``) the products run over the rows that chose each expert alone, and what the down product leaves are
+the chosen experts' outputs as sums that are still to be added.
 
 Variants that the spec names: experts with a gate, ``W_down (act(W_gate h) * (W_up h))`` (all gates are the first half of
 the one up matrix); scores that are the softmax over every router output, a correction added for the choice only, and
@@ -18,6 +20,7 @@ from __future__ import annotations
 
 import torch
 
+from ..kernels.ops import interleave_gate_up
 from .base import FeedForward, TensorDecl, require_kernel_sizes
 from .registry import register_feed_forward
 
@@ -73,6 +76,16 @@ class RoutedMlp(FeedForward):
     def load(self, t):
         s = self.spec
         self.w_router, self.b_router, self.w_correction = t["router.weight"], t.get("router.bias"), t.get("correction")
+        if self.shared_gate:  # one more row of the router's matrix, which is no expert to choose
+            self.w_router = torch.cat([self.w_router, t["shared.gate_weight"]], dim=0).contiguous()
+        takes = getattr(self.rt.ops, "routed_experts_takes", None)
+        self.grouped = takes is not None and takes(s.hidden, s.intermediate, s.shared, s.top)
+        if self.grouped:  # every expert's matrices by themselves
+            names = [f"e{e}" for e in range(s.experts)] + (["shared"] if s.shared else [])
+            up = (lambda n: interleave_gate_up(t[f"{n}.gate"], t[f"{n}.up"])) if self.gated else (lambda n: t[f"{n}.up"])
+            self.w_up = torch.cat([up(n) for n in names], dim=0)
+            self.w_down = torch.cat([t[f"{n}.down"].reshape(-1) for n in names])
+            return
         ups, downs = [t[f"e{e}.up"] for e in range(s.experts)], [t[f"e{e}.down"] for e in range(s.experts)]
         if s.shared:
             ups.append(t["shared.up"])
@@ -84,12 +97,22 @@ class RoutedMlp(FeedForward):
         if self.gated:  # every expert's gate, then every expert's up projection
             gates = [t[f"e{e}.gate"] for e in range(s.experts)] + ([t["shared.gate"]] if s.shared else [])
             ups = gates + ([ups[0].new_zeros((fill, s.hidden))] if fill else []) + ups
-        if self.shared_gate:  # one more row of the router's matrix, which is no expert to choose
-            self.w_router = torch.cat([self.w_router, t["shared.gate_weight"]], dim=0).contiguous()
         self.w_up, self.w_down = torch.cat(ups, dim=0).contiguous(), torch.cat(downs, dim=1).contiguous()
 
     def forward(self, h, stream, ctx):
         s, ops = self.spec, self.rt.ops
+        if self.grouped:
+            scoring = {"correction": self.w_correction, "softmax_all": True} if self.scoring == "softmax_all" else {"sigmoid": self.scoring == "sigmoid"}
+            sums, gates = ops.routed_experts(h, self.w_router, self.b_router, s.top, self.w_up, self.w_down, s.experts, s.intermediate, s.shared,
+                                             s.activation, gated=self.gated, weigh_input=self.weigh == "input", shared_gate=self.shared_gate,
+                                             **scoring)
+            if self.identity:
+                ops.add_scaled_rows(sums[0], h, gates, s.experts, self.identity)
+            if hasattr(stream, "add_sums"):
+                stream.add_sums(sums)
+            else:  # a block's own collector that knows finished tensors
+                stream.add(sums.sum(0))
+            return
         if self.scoring == "softmax_all":
             gates = ops.route(h, self.w_router, self.b_router, s.top, correction=self.w_correction, softmax_all=True)
         elif self.scoring == "sigmoid" or self.shared_gate:

@@ -1,0 +1,83 @@
+"""Products over the rows that chose an expert, against the same feed-forward over every expert in 64 bits: steps of one tile an expert
+and of lists, at the edges of both; experts that no row or every row uses; planes that a row does not use."""
+import pytest
+import torch
+
+from emulated_ops import EmulatedOps
+from gpu_util import DEV, assert_close
+
+pytestmark = pytest.mark.gpu
+
+# rows, router outputs, of them experts, used a row, columns of an expert, columns of the expert for every row, width
+SIZES = [(1, 8, 8, 2, 64, 0, 128), (4, 9, 8, 2, 128, 64, 192), (64, 5, 5, 3, 64, 128, 64), (65, 5, 5, 3, 64, 64, 64), (129, 8, 6, 2, 192, 0, 256),
+         (300, 70, 68, 1, 64, 0, 128), (700, 4, 3, 2, 128, 64, 320), (1025, 2, 2, 2, 64, 64, 64), (40, 130, 130, 12, 64, 64, 64)]
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("T,outputs,E,top,ff,shared,width", SIZES)
+@pytest.mark.parametrize("kind", ["gated", "gated, weighed at the input", "plain"])
+def test_products_over_the_rows_that_chose_an_expert(dtype, T, outputs, E, top, ff, shared, width, kind):
+    from machserve_amd.kernels import get_ops
+    from machserve_amd.kernels.ops import interleave_gate_up
+    ops, gated, inside = get_ops(dtype, DEV), kind != "plain", kind.endswith("input")
+    g = torch.Generator().manual_seed(T * 31 + E)
+    rnd = lambda *s: torch.randn(*s, generator=g)  # noqa: E731
+    h = rnd(T, width).to(dtype)
+    shared_gate = bool(shared) and outputs == E
+    router = rnd(outputs + shared_gate, width) * 0.3
+    if E > 2:
+        router[1] = -1e3 * h[T // 2].float() / h[T // 2].float().norm()  # hardly any row, or none, chooses this one
+    cols = [ff] * E + ([shared] if shared else [])
+    gate, up = [(rnd(c, width) * width ** -0.5).to(dtype) for c in cols], [(rnd(c, width) * width ** -0.5).to(dtype) for c in cols]
+    down = [(rnd(width, c) * c ** -0.5).to(dtype) for c in cols]
+    w_up = torch.cat([interleave_gate_up(a, b) if gated else b for a, b in zip(gate, up)])
+    w_down = torch.cat([d.reshape(-1) for d in down])
+    scoring = {"sigmoid": True} if inside else ({"softmax_all": True} if outputs > E else {})
+    sums, gates = ops.routed_experts(h.to(DEV), router.to(DEV), None, top, w_up.to(DEV), w_down.to(DEV), E, ff, shared, "silu", gated=gated,
+                                     weigh_input=inside, shared_gate=shared_gate, **scoring)
+    assert sums.shape == (top + (shared > 0), T, width) and bool(torch.isfinite(sums).all())
+    # the weights themselves: the stand-in's on the CPU (32-bit sums in another order)
+    assert_close(gates, EmulatedOps(torch.float32).route(h.float(), router, None, top, extra_gates=int(shared_gate), **scoring), torch.float32, "weights")
+    w = gates.double().cpu()
+    want = torch.zeros(T, width, dtype=torch.float64)
+    silu = lambda z: z * torch.sigmoid(z)  # noqa: E731
+    for e in range(len(cols)):
+        we = (w[:, e] if e < E or shared_gate else torch.ones(T, dtype=torch.float64))[:, None]
+        wi = we if inside and e < E else 1.0
+        a, b = h.double() @ gate[e].double().T, h.double() @ up[e].double().T
+        z = silu(wi * a) * b * we if gated else silu(b) * we
+        want += z.to(dtype).double() @ down[e].double().T  # the activations are kept in the element type
+    assert_close(sums.sum(0), want, dtype, kind)
+    used = (w[:, :E] != 0).sum(1)
+    for k in range(top):
+        assert not bool(sums[k].cpu()[used <= k].any()), "a plane that a row does not use is zero"
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("T", [3, 200])
+@pytest.mark.parametrize("spec", [dict(gated=True, scoring="sigmoid", weigh="input", shared=64, shared_gate=True), dict(router_bias=True, shared=128),
+                                  dict(gated=True, scoring="softmax_all", correction=True, identity=2), dict(gated=True, shared=64)])
+def test_the_part_gives_what_it_gives_over_every_expert(dtype, T, spec, monkeypatch):
+    """The same part with the same tensors: over the rows that chose an expert, and over every expert."""
+    from machserve_amd.config import RoutedMlpSpec
+    from machserve_amd.kernels import get_ops
+    from machserve_amd.parts import FEED_FORWARDS, Runtime
+    from machserve_amd.parts.base import ResidualStream
+    ops, spec = get_ops(dtype, DEV), dict(spec)
+    width, E, top, ff, shared, bias = 128, 6, 2, 64, spec.pop("shared", 0), spec.pop("router_bias", False)
+    g = torch.Generator().manual_seed(T)
+    h = torch.randn(T, width, generator=g).to(dtype).to(DEV)
+    x = torch.randn(T, width, generator=g).to(DEV)
+    tensors, got = {}, []
+    for takes in (True, False):
+        monkeypatch.setattr(ops, "routed_experts_takes", lambda *a, takes=takes: takes, raising=False)
+        part = FEED_FORWARDS.build(RoutedMlpSpec("routed_mlp", width, E, top, ff, "silu", shared, bias, {}, **spec), Runtime(torch.device(DEV), dtype, ops))
+        for d in part.tensor_decls():
+            if d.name not in tensors:
+                tensors[d.name] = (torch.randn(d.shape, generator=g) * 0.1).to(DEV, torch.float32 if d.role == "vector" else dtype)
+        part.load(tensors)
+        assert part.grouped == takes
+        stream = ResidualStream(x.clone(), ops)
+        part.forward(h, stream, None)
+        got.append(stream.value())
+    assert_close(got[0], got[1], dtype, str(spec))
