@@ -15,7 +15,17 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_kernel(const elem_t* __rest
     arguments_now(A, W, M, N, K, ep.out, ep.bias, ep.ldo, ep.n_out, ep.k_per_split, ep.split_stride);
     if constexpr (SCALED) arguments_now(ep.row_ss, ep.ss_parts, ep.ss_eps);
     const int tiles_m = ceil_div(M, BM);
-    const int tm = blockIdx.x % tiles_m, tn = blockIdx.x / tiles_m;
+    int tile = blockIdx.x;
+    // Blocks go to the eight dies in turn, each die with an L2 of its own.  With a multiple of eight row tiles a die gets the same rows under
+    // every column, and all of W; a contiguous run of the order instead gives it all rows under its own columns.  What
+    // the dies read together is the smaller this way where W has more rows than A (and where the row tiles are no multiple of eight a
+    // die would read everything): 2,048 x 37,888 x 3,584 470 -> 453 us, 1,040 rows 289 -> 272; 2,048 x 2,048 x 5,632 the other
+    // way round, 45.7 against 43.7.  (Tiles of 128 rows are taken where W is small beside them.)
+    if (STAGES == GEMM_PIPED && (tiles_m % 8 != 0 || (BM == 256 && N > 2 * M))) {
+        const int per = gridDim.x / 8, rest = gridDim.x % 8, die = tile % 8;
+        tile = die * per + min(die, rest) + tile / 8;
+    }
+    const int tm = tile % tiles_m, tn = tile / tiles_m;
     gemm_tile<BM, BN, WM, WN, BK, EPI, STAGES, SCALED>(A, W, M, N, K, ep, tm * BM, tn * BN, blockIdx.y, NoExperts{});
 }
 
@@ -23,6 +33,65 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_kernel(const elem_t* __rest
 static int g_gemm_config = 0;  // 0: chosen by shape; else a fixed tile
 #else
 static constexpr int g_gemm_config = 0;
+#endif
+
+#ifdef MS_ELEM_HALF
+// The choice of a tile (and of the K slices, where the reader adds them up) for more than 64 rows and whole K steps: the
+// one whose predicted time is least.  A block of a tile takes `step[n]` us a K step of 64 where n + 1 such blocks share a CU, `slope` more of it in
+// proportion as the chip is full, and `store32` or `store16` for each block a CU to store its sums; `start` is paid once a product.  The
+// numbers are a fit (non-negative least squares, 8 to 15 % off) to the times of 168 products: 96 to 3,001 rows of the projections
+// of the 0.5B, 1.5B and 7B layer sizes and of widths of 1,024 and 2,048, cold operands, one to six slices.  The choice is 2 % slower
+// than the best tile measured, on average; against the rules it replaces (rounds of 128x128 blocks, with borders
+// for wider tiles, in a loop of one burst of loads a step) the products are 1.26 times as fast (geometric mean).
+struct TileCost {
+    int bm, bn, per_cu;
+    float step[4], store32, store16, start, slope;
+};
+enum Tile { TILE_256x256, TILE_256x192, TILE_256x128, TILE_128x128, TILE_64x64, TILE_64x64_DEEP, TILE_COUNT };
+static constexpr TileCost kTiles[TILE_COUNT] = {
+    {256, 256, 1, {1.12f}, 8.64f, 0.85f, 8.26f, 0.22f},
+    {256, 192, 1, {0.96f}, 7.82f, 0.00f, 7.22f, 0.14f},
+    {256, 128, 1, {0.65f}, 5.95f, 1.97f, 4.09f, 0.17f},
+    {128, 128, 2, {0.42f, 0.67f}, 1.99f, 0.12f, 3.70f, 0.31f},
+    {64, 64, 4, {0.27f, 0.29f, 0.40f, 0.51f}, 0.31f, 0.00f, 2.87f, 0.37f},
+    {64, 64, 2, {0.25f, 0.45f}, 0.79f, 0.09f, 2.79f, 0.04f},
+};
+
+static float tile_time(const TileCost& t, int M, int N, int k_per_split, int splits, bool store32) {
+    const long blocks = (long)ceil_div(M, t.bm) * ceil_div(N, t.bn) * splits, cus = compute_units(), round = cus * t.per_cu;
+    const float steps = (float)ceil_div(k_per_split, 64), store = store32 ? t.store32 : t.store16;
+    const long full = blocks / round, rest = blocks % round;
+    float us = t.start + (float)full * (steps * (t.step[t.per_cu - 1] + t.slope) + store * t.per_cu);
+    if (rest) {
+        const float fill = (float)rest / (float)round;
+        us += steps * (t.step[ceil_div(rest, cus) - 1] + t.slope * fill) + store * t.per_cu * fill;
+    }
+    return us;
+}
+
+struct GemmPlan {
+    int tile, splits;
+};
+// The best tile for `splits` slices, or, with splits == 0, the best tile and number of slices: a slice more is a plane of sums more to
+// write and to read again (4.5 TB/s), and never less than three K steps.
+static GemmPlan plan_gemm(int M, int N, int K, int splits, bool store32) {
+    GemmPlan best{0, max(1, splits)};
+    float best_us = INFINITY;
+    for (int s = splits ? splits : 1; s <= (splits ? splits : 6); ++s) {
+        const int per = ceil_div(ceil_div(K, s), 64) * 64;
+        if (splits == 0 && s > 1 && (ceil_div(K, per) != s || per < 192)) continue;
+        for (int i = 0; i < TILE_COUNT; ++i) {
+            const float us = tile_time(kTiles[i], M, N, per, s, store32) + (float)(s - 1) * (float)M * (float)N * (8.0f / 4.5e6f);
+            if (us < best_us) {
+                best_us = us;
+                best = {i, s};
+            }
+        }
+    }
+    return best;
+}
+// products of more than 64 rows over whole K steps: what is planned as above
+static bool planned(int M, int K) { return M > 64 && K % 64 == 0 && g_gemm_config == 0; }
 #endif
 
 template <int EPI>
@@ -59,6 +128,16 @@ static int launch_gemm(const elem_t* A, const elem_t* W, int M, int N, int K, Ep
     if (forced == 5) MS_GEMM(128, 64, 2, 2, 64);
     if (forced == 6) MS_GEMM(64, 64, 2, 2, 64);
     const bool whole_steps = ep.k_per_split % 64 == 0 && K % 64 == 0;
+    if (planned(M, K)) {
+        switch (plan_gemm(M, N, K, (int)ns, EPI == EPI_STORE_F32 || EPI == EPI_RESIDUAL).tile) {
+            case TILE_256x256: MS_GEMM_DEEP(256, 256, 2, 4, 64, GEMM_PIPED);
+            case TILE_256x192: MS_GEMM_DEEP(256, 192, 4, 2, 64, GEMM_PIPED);
+            case TILE_256x128: MS_GEMM_DEEP(256, 128, 4, 2, 64, GEMM_PIPED);
+            case TILE_128x128: MS_GEMM_DEEP(128, 128, 2, 4, 64, GEMM_PIPED);
+            case TILE_64x64: MS_GEMM_DEEP(64, 64, 2, 2, 64, GEMM_PIPED);
+            default: MS_GEMM_DEEP(64, 64, 2, 2, 64, 4);
+        }
+    }
     if (forced == 8 && whole_steps) MS_GEMM_DEEP(64, 64, 2, 2, 64, 4);
     if (forced == 9) MS_GEMM(256, 256, 2, 4, 64);
     // The largest tile that still gives every CU of the chip a block or two, with K steps of 64 (half
@@ -130,15 +209,16 @@ static int plan_tiled_splits(int M, int N, int K) {
     const long round_blocks = 2L * compute_units();  // two 128x128 blocks a CU
     // A very long K under few output tiles (the 7B down projection: K = 18,944, 14 column tiles of 256): tiles of 256x256
     // bring half the bytes of 128x128 tiles from the L2, but one or two thousand rows of them do not fill the chip's round of
-    // one block a CU; with K cut in two to four they do, and the norm that follows adds the slices.  Measured with that
-    // norm: 2,048 rows 374 -> 330 us in two slices (320 in four), 1,024 rows 198 -> 158 in four; shorter K (the 1.5B down
-    // projection, 8,960) and the 0.5B sizes lose by it, and from 4,096 rows on the uncut tiles fill the round themselves.
+    // one block a CU; with K cut in two to four they do, and the norm that follows adds the slices (2,048 rows: 221 us in two slices and
+    // 13 for the second plane, 238 uncut in tiles of 256x128).  Other K, and rows that leave the round less full, as planned
+    // above.
     if (M > 64 && K >= 16384 && g_force_splits == 0) {
         const long t256 = (long)ceil_div(M, 256) * ceil_div(N, 256), cus = compute_units();
         if (t256 * 100 < 72 * cus)
             for (int sl = 2; sl <= 4; ++sl)
                 if (t256 * sl * 100 >= 85 * cus && t256 * sl <= cus) return ceil_div(K, ceil_div(ceil_div(K, sl), 64) * 64);
     }
+    if (planned(M, K) && g_force_splits == 0) return plan_gemm(M, N, K, 0, true).splits;
     if (b128 >= round_blocks * 300 / 512 && g_force_splits == 0) return 1;
     // More than six slices cost more in the consumer's sums than they gain here (with very few tiles - a
     // portion of a few hundred rows - slices of 256 still pay).  With few rows the partial sums are small
@@ -315,6 +395,17 @@ extern "C" int ms_linear_qkv_rope(const void* a, const void* w, const float* bia
 
 // Number of partial sums ms_linear_split_tiled writes for this problem (1 = the complete product).
 extern "C" int ms_tiled_partials(int M, int N, int K) { return plan_tiled_splits(M, N, K); }
+
+// The tile that a product over whole K steps runs in with that many K slices (an index into kTiles), or -1 where it is not planned (up to
+// 64 rows, a partial K step, the 32-bit build).
+extern "C" int ms_tiled_tile(int M, int N, int K, int splits, int store32) {
+#ifdef MS_ELEM_HALF
+    return planned(M, K) ? plan_gemm(M, N, K, max(1, splits), store32 != 0).tile : -1;
+#else
+    (void)M; (void)N; (void)K; (void)splits; (void)store32;
+    return -1;
+#endif
+}
 
 // Whether a product of M rows is better served by the tiled kernel than by the few-rows kernel (which
 // takes at most 64 rows).  The few-rows kernel reads its rows again for every 32 or 64 columns; with

@@ -8,9 +8,9 @@
 // rows of 128 bytes, when chunk c of row r lies at position c ^ (r & 7).
 // bfloat16 with K steps of 64: tiles go global -> LDS directly (global_load_lds_dwordx4, a wave's
 // 64 lanes fill 1 KB = 8 unpadded rows in lane order, so the swizzle is applied to the global
-// address), and the next step's tile is in flight while this one is multiplied; only a partial last
-// step goes through registers, where what lies beyond K is masked.  The 32-bit build and K steps of
-// 32 go global -> registers -> LDS (padded rows).
+// address), and the next step's tile is in flight while this one is multiplied (how far ahead, and with how many buffers, see the
+// loops below); only a partial last step goes through registers, where what lies beyond K is masked.  The 32-bit build and
+// K steps of 32 go global -> registers -> LDS (padded rows).
 // Every output element is the sum over K in steps of 32 in ascending order whatever the
 // tile shape or the number of rows, so a row's result does not depend on its batch.
 #pragma once
@@ -28,14 +28,18 @@ constexpr int EPC = 4;
 constexpr int KPAD = 8;  // rows of 160 bytes (BK 32)
 #endif
 
+constexpr int GEMM_PIPED = 1;  // in the place of a number of LDS buffers: two of them, in phases (see gemm_tile)
+
 enum EpiKind {
     EPI_STORE_F32 = 0, EPI_STORE_ELEM = 1, EPI_RESIDUAL = 2, EPI_SWIGLU = 3, EPI_QKV_ROPE = 4, EPI_ACT = 5,
     EPI_EXPERT_GATED = 6, EPI_EXPERT_PLAIN = 7, EPI_EXPERT_DOWN = 8,  // over the rows that chose an expert (routed.hip)
 };
 
 struct NoExperts {
+    static constexpr bool GATHERS = false;  // A's rows lie one behind the other
     __device__ __forceinline__ int source(int m, int) const { return m; }
-    __device__ __forceinline__ int pitch(int K) const { return K; }  // elements from a row of A to the next
+    __device__ __forceinline__ int pitch(int K) const { return K; }    // elements from a row of A to the next
+    __device__ __forceinline__ int w_pitch(int K) const { return K; }  // ... of W
 };
 
 struct EpiArgs {
@@ -74,6 +78,8 @@ __device__ __forceinline__ void gemm_tile(const elem_t* __restrict__ A, const el
 #else
     constexpr bool DIRECT = false;
 #endif
+    constexpr bool PIPED = STAGES == GEMM_PIPED;
+    constexpr int BUFS = PIPED ? 2 : STAGES;
     constexpr int LDS_LD = DIRECT ? BK : BK + KPAD;
     constexpr int CPR = BK / EPC;  // chunks per tile row
     // where chunk `chunk` of tile row `row` lies in a buffer
@@ -82,14 +88,14 @@ __device__ __forceinline__ void gemm_tile(const elem_t* __restrict__ A, const el
     constexpr int A_CHUNKS = BM * CPR / NT, W_CHUNKS = BN * CPR / NT;
     static_assert(BM * CPR % NT == 0 && BN * CPR % NT == 0, "tile loads divide over the block");
     static_assert(NT == 256 || !SCALED, "the row factors' shares are dealt to four waves");
-    static_assert(STAGES == 2 || DIRECT, "more than two LDS buffers only with direct loads");
+    static_assert(STAGES == 2 || DIRECT, "more than two LDS buffers, and phases, only with direct loads");
     static_assert(!SCALED || (STAGES > 2 && EPI == EPI_SWIGLU), "row factors: built for the gated product with several steps in flight");
     static_assert(256 % BM == 0 || !SCALED, "threads are dealt to the rows");
     __shared__ float ss_q[SCALED ? 256 / BM : 1][SCALED ? BM : 1];  // the rows' sums of squares, in 256 / BM interleaved shares
     float ss_v[SCALED ? 8 : 1];
     int ss_r = 0;
-    __shared__ __attribute__((aligned(16))) elem_t As[STAGES][BM * LDS_LD];
-    __shared__ __attribute__((aligned(16))) elem_t Ws[STAGES][BN * LDS_LD];
+    __shared__ __attribute__((aligned(16))) elem_t As[BUFS][BM * LDS_LD];
+    __shared__ __attribute__((aligned(16))) elem_t Ws[BUFS][BN * LDS_LD];
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wm = wave / WN, wn = wave % WN;
@@ -113,7 +119,7 @@ __device__ __forceinline__ void gemm_tile(const elem_t* __restrict__ A, const el
 #pragma unroll
     for (int i = 0; i < W_CHUNKS; ++i) {
         const int c = tid + i * NT;
-        pw[i] = W + (size_t)min(n0 + c / CPR, N - 1) * K + my_chunk * EPC;
+        pw[i] = W + (size_t)min(n0 + c / CPR, N - 1) * rows.w_pitch(K) + my_chunk * EPC;
     }
     auto load_global = [&](int k0) {
 #pragma unroll
@@ -152,16 +158,54 @@ __device__ __forceinline__ void gemm_tile(const elem_t* __restrict__ A, const el
     // One K step of both tiles straight into LDS buffer `buf`: lane l of a wave's load lands at the wave's
     // base + 16 l.  Written in assembly: of a load that it knows to write LDS the compiler makes every later
     // LDS read wait (vmcnt(0)), and nothing would be in flight during the multiplications; the waits are
-    // explicit instead (`step_barrier`).
+    // explicit instead (`step_barrier`).  The bases are scalars, and so are the operands' with a lane's offset of 32 bits
+    // (a tile's rows lie within 4 GiB): kept a lane, the places in LDS alone took 32 registers, and the 256-row tiles spilled.
+    const int swave = __builtin_amdgcn_readfirstlane(wave);
+    // The first of the eight tile rows that this wave loads in round i.  In phases, the rounds' first half brings the rows that the waves' first
+    // halves of row tiles read.
+    auto a_row = [&](int i) {
+        if constexpr (PIPED) {
+            constexpr int HR = BM / WM / 2;
+            const int at8 = (i % (A_CHUNKS / 2)) * (NT / 64) + swave;
+            return at8 / (HR / 8) * (BM / WM) + (i / (A_CHUNKS / 2)) * HR + at8 % (HR / 8) * 8;
+        } else {
+            return i * (NT / 8) + swave * 8;
+        }
+    };
+    const uint32_t lds_a = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)&As[0][0];
+    const uint32_t lds_w = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)&Ws[0][0];
+    const elem_t* base_a = A + (size_t)rows.source(m0, m0) * rows.pitch(K);
+    const elem_t* base_w = W + (size_t)n0 * rows.w_pitch(K);
+    uint32_t oa[A_CHUNKS], ow[W_CHUNKS];
+    const elem_t* ga[Rows::GATHERS ? A_CHUNKS : 1];
+    if constexpr (DIRECT) {
+#pragma unroll
+        for (int i = 0; i < A_CHUNKS; ++i) {
+            const int m = min(m0 + a_row(i) + lane / 8, M - 1);
+            if constexpr (Rows::GATHERS) ga[i] = A + (size_t)rows.source(m, m0) * rows.pitch(K) + my_chunk * EPC;
+            else oa[i] = ((uint32_t)(m - m0) * (uint32_t)rows.pitch(K) + my_chunk * EPC) * (uint32_t)sizeof(elem_t);
+        }
+#pragma unroll
+        for (int i = 0; i < W_CHUNKS; ++i)
+            ow[i] = ((uint32_t)(min(n0 + (tid + i * NT) / CPR, N - 1) - n0) * (uint32_t)rows.w_pitch(K) + my_chunk * EPC) * (uint32_t)sizeof(elem_t);
+    }
+    // load l of a step: A's rounds, then W's
+    auto load_one = [&](int k0, int buf, int l) {
+        if (l < A_CHUNKS) {
+            const uint32_t to = lds_a + buf * (BM * LDS_LD * (int)sizeof(elem_t)) + a_row(l) * (LDS_LD * (int)sizeof(elem_t));
+            if constexpr (Rows::GATHERS)
+                asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(ga[l] + k0), "s"(to) : "memory", "m0");
+            else
+                asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(oa[l]), "s"(base_a + k0), "s"(to) : "memory", "m0");
+        } else {
+            const int i = l - A_CHUNKS;
+            const uint32_t to = lds_w + buf * (BN * LDS_LD * (int)sizeof(elem_t)) + (i * (NT / 8) + swave * 8) * (LDS_LD * (int)sizeof(elem_t));
+            asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(ow[i]), "s"(base_w + k0), "s"(to) : "memory", "m0");
+        }
+    };
     auto load_direct = [&](int k0, int buf) {
-        auto issue = [](const elem_t* g, const elem_t* l) {
-            const uint32_t base = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) const char*)l);
-            asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(g), "s"(base) : "memory", "m0");
-        };
 #pragma unroll
-        for (int i = 0; i < A_CHUNKS; ++i) issue(pa[i] + k0, &As[buf][(i * NT + wave * 64) * EPC]);
-#pragma unroll
-        for (int i = 0; i < W_CHUNKS; ++i) issue(pw[i] + k0, &Ws[buf][(i * NT + wave * 64) * EPC]);
+        for (int l = 0; l < A_CHUNKS + W_CHUNKS; ++l) load_one(k0, buf, l);
     };
 #endif
     // End of a K step: this wave's loads and LDS accesses have completed, then everybody's.
@@ -207,7 +251,86 @@ __device__ __forceinline__ void gemm_tile(const elem_t* __restrict__ A, const el
                 for (int j = 0; j < TN; ++j) mma_16x16x32(acc[i][j], fa[i], fb[j]);
         }
     };
-    if constexpr (DIRECT && STAGES > 2) {
+    if constexpr (PIPED) {
+#ifdef MS_ELEM_HALF
+        // Two LDS buffers, whole K steps.  What bounds the loop with one burst of loads a step and all of a K chunk's fragments read before they are
+        // multiplied (measured with parts of it left out, 256x256 tiles, 2,048 x 37,888 x 3,584: 493 us; without the loads
+        // 351, without the matrix instructions 410, without both 124): a step waits for its burst, and LDS reads and
+        // matrix instructions add up.  So:
+        // * a step is four phases, (first half of the wave's rows, K chunk 0), (first, 1), (second, 0), (second, 1); in each the wave
+        //   reads the fragments of the next one between groups of this one's matrix instructions;
+        // * W and the first half's rows have been read when phase 0 ends, the second half's when phase 2 ends: the loads of the step
+        //   after the next go out there, in two portions, into the places just read, and have a step and a half to
+        //   come.  The wait at both places is for all but the last step's worth of loads; the two barriers a step say that
+        //   everybody's have come and that everybody has read.
+        // 256x256: 493 -> 429 us (with the order of the tiles); 256x192 of 2,048 x 11,264 x 2,048: 79 us (128x128 tiles in the old loop:
+        // 103); 128x128 of 2,048 x 2,048 x 5,632, one block a CU: 80 -> 60.
+        static_assert(TM % 2 == 0 && A_CHUNKS % 2 == 0, "a wave's rows in two halves");
+        constexpr int TH = TM / 2;
+        Frag fa[2][TH], fb[2][TN];
+        auto fetch_a = [&](int buf, int p, int i) {
+            fa[p & 1][i] = frag_load(&As[buf][at(wm * (BM / WM) + (p / 2 * TH + i) * 16 + r16, (p & 1) * (32 / EPC) + grp)]);
+        };
+        auto fetch_b = [&](int buf, int kk, int j) {
+            fb[kk][j] = frag_load(&Ws[buf][at(wn * (BN / WN) + j * 16 + r16, kk * (32 / EPC) + grp)]);
+        };
+        constexpr int PER_STEP = A_CHUNKS + W_CHUNKS, EARLY = W_CHUNKS + A_CHUNKS / 2;
+        static_assert(PER_STEP <= 63, "the wait count is a 6-bit field");
+        auto load_nth = [&](int k0, int buf, int l) { load_one(k0, buf, l < W_CHUNKS ? A_CHUNKS + l : l - W_CHUNKS); };  // W, first half, second half
+        auto arrive = [&](bool all_but_a_step) {
+            __builtin_amdgcn_sched_barrier(0);
+            if (all_but_a_step) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(PER_STEP) : "memory");
+            else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+            __builtin_amdgcn_s_barrier();
+            __builtin_amdgcn_sched_barrier(0);
+        };
+#pragma unroll
+        for (int l = 0; l < PER_STEP; ++l) load_nth(k_begin, 0, l);
+        if (nk > 1)
+#pragma unroll
+            for (int l = 0; l < PER_STEP; ++l) load_nth(k_begin + BK, 1, l);
+        arrive(nk > 1);
+#pragma unroll
+        for (int i = 0; i < TH; ++i) fetch_a(0, 0, i);
+#pragma unroll
+        for (int j = 0; j < TN; ++j) fetch_b(0, 0, j);
+        constexpr int GR = TH * TN % 4 == 0 ? 4 : 2, GROUPS = TH * TN / GR;  // matrix instructions in groups, each with its share of reads and loads ahead
+        static_assert(TH * TN % GR == 0, "groups of matrix instructions");
+        auto step = [&](int kt, int buf) {
+            const bool more = kt + 2 < nk;
+#pragma unroll
+            for (int p = 0; p < 4; ++p) {
+                const int np = (p + 1) & 3, nbuf = p == 3 ? buf ^ 1 : buf;  // (behind the last step: what is left there, and not used)
+                const int reads = TH + (np < 2 ? TN : 0);
+                // phase 1: the second half's rows of this step have come; phase 3: W and the first half's rows of the next one
+                if (p == 1) arrive(kt + 1 < nk);
+                if (p == 3) arrive(more);
+                const int first = p == 1 ? 0 : EARLY, loads = p == 1 ? EARLY : p == 3 ? PER_STEP - EARLY : 0;
+#pragma unroll
+                for (int g = 0; g < GROUPS; ++g) {
+#pragma unroll
+                    for (int r = 0; r < TH + TN; ++r) {
+                        if (r >= reads || r * GROUPS / reads != g) continue;
+                        if (r < TH) fetch_a(nbuf, np, r);
+                        else fetch_b(nbuf, np, r - TH);
+                    }
+#pragma unroll
+                    for (int l = 0; l < PER_STEP; ++l)
+                        if (l < loads && l * GROUPS / (loads > 0 ? loads : 1) == g && more) load_nth(k_begin + (kt + 2) * BK, buf, first + l);
+#pragma unroll
+                    for (int m = g * GR; m < (g + 1) * GR; ++m) mma_16x16x32(acc[p / 2 * TH + m / TN][m % TN], fa[p & 1][m / TN], fb[p & 1][m % TN]);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+        };
+        int kt = 0;
+        for (; kt + 1 < nk; kt += 2) {
+            step(kt, 0);
+            step(kt + 1, 1);
+        }
+        if (kt < nk) step(kt, 0);
+#endif
+    } else if constexpr (DIRECT && STAGES > 2) {
 #ifdef MS_ELEM_HALF
         // A block that is alone on its CU (few tiles: one tile of rows under a weight of a few hundred column
         // tiles) has nobody to hide its loads behind, and with one step in flight every step costs a trip to

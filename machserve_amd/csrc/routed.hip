@@ -148,11 +148,11 @@ constexpr int ACT_COLS = 2048;  // columns of a row that a block takes
 template <int V>  // columns a thread takes at once: 4 where an expert's columns and the row are multiples of four
 __global__ __launch_bounds__(256) void expert_act_kernel(const float* __restrict__ up, const float* __restrict__ gates,
                                                          elem_t* __restrict__ out, int n, int E, int ff, int act, int ld_gates, int gated,
-                                                         int weigh_input, int shared_gate) {
+                                                         int weigh_input, int shared_gate, int interleaved) {
     const int t = blockIdx.x, c0 = blockIdx.y * ACT_COLS, c1 = min(n, c0 + ACT_COLS);
     const float* g = gates + (size_t)t * ld_gates;
     const float shared_w = shared_gate ? g[E] : 1.0f;
-    if (gated) {  // up [T, 2 n]: the gates' columns, then the up projections'
+    if (gated) {  // up [T, 2 n]: the gates' columns, then the up projections', or both in blocks of 16 in turn
         const float* row = up + (size_t)t * 2 * n;
 #pragma unroll 2
         for (int c = c0 + threadIdx.x * V; c < c1; c += 256 * V) {
@@ -166,9 +166,10 @@ __global__ __launch_bounds__(256) void expert_act_kernel(const float* __restrict
             };
             if constexpr (V == 4) {
                 float4 a = (float4){0.f, 0.f, 0.f, 0.f}, b = a;
+                const int at = interleaved ? c / 16 * 32 + c % 16 : c;
                 if (w != 0.f) {
-                    a = *reinterpret_cast<const float4*>(row + c);
-                    b = *reinterpret_cast<const float4*>(row + n + c);
+                    a = *reinterpret_cast<const float4*>(row + at);
+                    b = *reinterpret_cast<const float4*>(row + at + (interleaved ? 16 : n));
                 }
                 o[0] = from_f32<elem_t>(value(a.x, b.x));
                 o[1] = from_f32<elem_t>(value(a.y, b.y));
@@ -251,16 +252,18 @@ __global__ __launch_bounds__(1024) void expert_rows_kernel(const int* __restrict
     if (threadIdx.x == 0) counts[e] = n;
 }
 
+template <bool GATHERS_>  // A's rows are the step's rows (the up product), else the tiles' activations (the down product)
 struct ExpertRows {
+    static constexpr bool GATHERS = GATHERS_;
     const ExpertArgs& g;
     const int* list;  // of the expert's rows; null: every row
     int e, tile;      // e == E: the expert that every row uses
     int bm;
-    bool gathers;     // A's rows are the step's rows (the up product), else the tiles' activations (the down product)
     __device__ __forceinline__ int row_of(int m) const { return list ? list[m] : m; }
     __device__ __forceinline__ int slot(int m, int m0) const { return tile * bm + (m - m0); }
-    __device__ __forceinline__ int source(int m, int m0) const { return gathers ? row_of(m) : slot(m, m0); }
-    __device__ __forceinline__ int pitch(int) const { return gathers ? g.width : max(g.ff, g.shared); }
+    __device__ __forceinline__ int source(int m, int m0) const { return GATHERS ? row_of(m) : slot(m, m0); }
+    __device__ __forceinline__ int pitch(int) const { return GATHERS ? g.width : max(g.ff, g.shared); }
+    __device__ __forceinline__ int w_pitch(int) const { return GATHERS ? g.width : g.E * g.ff + g.shared; }
     __device__ __forceinline__ float weight(int m) const {
         if (e == g.E && !g.shared_gate) return 1.0f;
         return g.gates[(size_t)row_of(m) * g.ld_gates + e];
@@ -328,8 +331,8 @@ __global__ __launch_bounds__(64 * WM * WN) void expert_gemm_kernel(const elem_t*
     if (m0 >= count || n0 >= N) return;  // the whole block: these are the block's own numbers
     __syncthreads();
     EpiArgs ep{out, nullptr, EPI == EPI_EXPERT_DOWN ? g.width : max(g.ff, g.shared), cols, K, 0};
-    const ExpertRows rows{g, list, e, tile, BM, EPI != EPI_EXPERT_DOWN};
-    const elem_t* own = W + (size_t)e * (EPI == EPI_EXPERT_DOWN ? 1 : PER) * g.ff * g.width;
+    const ExpertRows<EPI != EPI_EXPERT_DOWN> rows{g, list, e, tile, BM};
+    const elem_t* own = W + (size_t)e * g.ff * (EPI == EPI_EXPERT_DOWN ? 1 : PER * g.width);  // its columns, or its rows
     gemm_tile<BM, BN, WM, WN, BK, EPI, STAGES, false>(A, own, count, N, K, ep, m0, n0, 0, rows);
 }
 
@@ -368,7 +371,7 @@ static int launch_experts(const void* a, const void* w, void* out, ExpertArgs g,
     const int N = EPI == EPI_EXPERT_DOWN ? g.width : (EPI == EPI_EXPERT_GATED ? 2 : 1) * max(g.ff, g.shared);
 #define MS_EXPERTS(BM_, BN_, WM_, WN_, BK_, ST_)                                                                                           do {                                                                                                                                       const long nb = (long)(g.routed_tiles + g.shared_tiles) * ceil_div(N, BN_);                                                            hipLaunchKernelGGL((expert_gemm_kernel<BM_, BN_, WM_, WN_, BK_, EPI, ST_>), dim3((unsigned)nb), dim3(64 * WM_ * WN_), 0, stream,                            (const elem_t*)a, (const elem_t*)w, out, g);                                                                        return check_launch("experts " #BM_ "x" #BN_ "x" #BK_);                                                                            } while (0)
 #ifdef MS_ELEM_HALF
-    if (bm == 128) MS_EXPERTS(128, 128, 2, 2, 64, 2);
+    if (bm == 128) MS_EXPERTS(128, 128, 2, 4, 64, GEMM_PIPED);
     MS_EXPERTS(64, 64, 2, 2, 64, 4);
 #else
     (void)bm;
@@ -401,16 +404,17 @@ extern "C" int ms_route(const void* x, const float* w, const float* bias, float*
 
 // n: columns of the output; with `gated`, up has 2 n columns.  ld_gates: numbers a row of gates has (>= E).
 extern "C" int ms_expert_act(const float* up, const float* gates, void* out, int T, int n, int E, int ff, int act, int ld_gates, int gated,
-                             int weigh_input, int shared_gate, hipStream_t stream) {
+                             int weigh_input, int shared_gate, int interleaved, hipStream_t stream) {
+    MS_REQUIRE(!interleaved || (gated && n % 16 == 0 && ff % 4 == 0), "expert_act: %d gated columns in blocks of 16", n);
     MS_REQUIRE(T > 0 && n > 0 && E >= 0 && ff > 0 && (long)E * ff <= n && ld_gates >= E, "expert_act: %d columns for %d experts of %d", n, E, ff);
     MS_REQUIRE(act >= 0 && act <= 2, "expert_act: activation %d", act);
     MS_REQUIRE(!weigh_input || gated, "expert_act: weights inside experts that are not gated");
     MS_REQUIRE(!shared_gate || ld_gates > E, "expert_act: %d weights a row for %d experts and a gate", ld_gates, E);
     const dim3 grid(T, ceil_div(n, ACT_COLS));
     if (n % 4 == 0 && ff % 4 == 0) hipLaunchKernelGGL(expert_act_kernel<4>, grid, dim3(256), 0, stream, up, gates, (elem_t*)out, n, E, ff, act, ld_gates, gated,
-                                                       weigh_input, shared_gate);
+                                                       weigh_input, shared_gate, interleaved);
     else hipLaunchKernelGGL(expert_act_kernel<1>, grid, dim3(256), 0, stream, up, gates, (elem_t*)out, n, E, ff, act, ld_gates, gated,
-                                                       weigh_input, shared_gate);
+                                                       weigh_input, shared_gate, interleaved);
     return check_launch("expert_act");
 }
 
@@ -448,7 +452,7 @@ extern "C" int ms_experts_up(const void* x, const void* w, void* out, const int*
     return gated ? launch_experts<EPI_EXPERT_GATED>(x, w, out, g, stream) : launch_experts<EPI_EXPERT_PLAIN>(x, w, out, g, stream);
 }
 
-// a [slots, max(ff, shared)] as ms_experts_up leaves it; w: the experts' [width, ff] one behind the other,
+// a [slots, max(ff, shared)] as ms_experts_up leaves it; w [width, E * ff + shared]: the experts' down matrices side by side,
 // then the shared one's; sums [top (+ 1), T, width]: plane k of row t is the k-th expert that it uses, the last plane the shared one's.
 extern "C" int ms_experts_down(const void* a, const void* w, float* sums, const int* plane, const float* gates, const int* rows, const int* counts,
                                int T, int E, int ld_gates, int top, int ff, int shared, int width, hipStream_t stream) {

@@ -1362,9 +1362,15 @@ class HipOps:
         return gates
 
     def routed_experts_takes(self, width: int, ff: int, shared: int, top: int) -> bool:
-        """Whether experts of these sizes run over the rows that chose them (:meth:`routed_experts`): whole K steps of both
+        """Whether experts of these sizes may run over the rows that chose them (:meth:`routed_experts`): whole K steps of both
         products, and no more planes than a reader's kernel asks for at once."""
         return width % 64 == 0 and ff % 64 == 0 and shared % 64 == 0 and top + (shared > 0) <= 16
+
+    def routed_experts_runs(self, rows: int) -> bool:
+        """Whether a step of so many rows runs so.  In 32-bit a step of up to :attr:`SKINNY_ROWS` rows runs over every expert instead:
+        there the weight-streaming products, whose waves share K, are the faster ones (11.6 against 12.7 ms for a pass of decode steps
+        of Livovik layers) and the more exact."""
+        return self.dtype != torch.float32 or rows > self.SKINNY_ROWS
 
     def routed_experts(self, h: torch.Tensor, w_router: torch.Tensor, b_router: Optional[torch.Tensor], top: int, w_up: torch.Tensor,
                        w_down: torch.Tensor, experts: int, ff: int, shared: int, activation: str, gated: bool = False, weigh_input: bool = False,
@@ -1372,11 +1378,11 @@ class HipOps:
         """A feed-forward of routed experts over the rows that chose each: ``(sums, gates)``, float32 ``[top (+ 1), T, width]`` whose sum
         over the first axis is the feed-forward's output, and the rows' weights (:meth:`route`, whose other arguments ``scoring`` are).
         ``w_up``: the experts' up matrices one behind the other and then that of the expert that every row uses, each ``[cols, width]`` or
-        with ``gated`` gate and up interleaved (:func:`interleave_gate_up`); ``w_down`` flat: each expert's ``[width, cols]`` in the same order."""
+        with ``gated`` gate and up interleaved (:func:`interleave_gate_up`); ``w_down [width, columns]``: the down matrices side by side in the same order."""
         lib = self._extra_lib("routed")
         T, d = h.shape
         self._want(w_up, self.dtype, "experts up", (2 if gated else 1) * (experts * ff + shared), d)
-        self._want(w_down, self.dtype, "experts down", d * (experts * ff + shared))
+        self._want(w_down, self.dtype, "experts down", d, experts * ff + shared)
         if activation not in self.EXPERT_ACTIVATIONS:
             raise KernelError(f"experts: activation {activation!r} is not built (built: {', '.join(sorted(self.EXPERT_ACTIVATIONS))})")
         new = lambda shape, dt: torch.empty(shape, dtype=dt, device=h.device)  # noqa: E731
@@ -1394,12 +1400,12 @@ class HipOps:
         return sums, gates
 
     def expert_act(self, up: torch.Tensor, gates: torch.Tensor, ff: int, activation: str, experts: Optional[int] = None,
-                   gated: bool = False, weigh_input: bool = False, shared_gate: bool = False) -> torch.Tensor:
+                   gated: bool = False, weigh_input: bool = False, shared_gate: bool = False, interleaved: bool = False) -> torch.Tensor:
         """``act(up[t, c]) * gates[t, c // ff]`` in the element type for float32 ``up [T, n]``; the columns beyond
         ``experts * ff`` (an expert every row uses) carry weight one.  ``experts``: how many of the gates' columns are
         experts with columns here (None: all).  ``gated``: ``up`` is ``[T, 2 n]``, the experts' gates and then their up
         projections, and the result ``act(gate) * up * weight``, or with ``weigh_input`` ``act(weight gate) * (weight up)`` for the
-        experts' columns.  ``shared_gate``: the columns beyond the experts carry ``gates[t, experts]`` instead of one."""
+        experts' columns.  ``interleaved``: gate and up columns come in blocks of 16 in turn (:func:`interleave_gate_up`).  ``shared_gate``: the columns beyond the experts carry ``gates[t, experts]`` instead of one."""
         lib = self._extra_lib("routed")
         T, n = up.shape
         if gated:
@@ -1416,7 +1422,7 @@ class HipOps:
         out = torch.empty((T, n), dtype=self.dtype, device=up.device)
         self._check(lib, lib.ms_expert_act(_ptr(up), _ptr(gates), _ptr(out), _c_int(T), _c_int(n), _c_int(E), _c_int(ff),
                                            _c_int(self.EXPERT_ACTIVATIONS[activation]), _c_int(gates.shape[1]), _c_int(int(gated)),
-                                           _c_int(int(weigh_input)), _c_int(int(shared_gate)), self._stream()))
+                                           _c_int(int(weigh_input)), _c_int(int(shared_gate)), _c_int(int(interleaved)), self._stream()))
         return out
 
     def add_scaled_rows(self, x: torch.Tensor, h: torch.Tensor, weights: torch.Tensor, first: int, count: int) -> None:

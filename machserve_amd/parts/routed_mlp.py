@@ -80,11 +80,11 @@ class RoutedMlp(FeedForward):
             self.w_router = torch.cat([self.w_router, t["shared.gate_weight"]], dim=0).contiguous()
         takes = getattr(self.rt.ops, "routed_experts_takes", None)
         self.grouped = takes is not None and takes(s.hidden, s.intermediate, s.shared, s.top)
-        if self.grouped:  # every expert's matrices by themselves
+        if self.grouped:  # an expert's gate and up rows in blocks of 16 in turn, so that one tile of the up product holds both
             names = [f"e{e}" for e in range(s.experts)] + (["shared"] if s.shared else [])
             up = (lambda n: interleave_gate_up(t[f"{n}.gate"], t[f"{n}.up"])) if self.gated else (lambda n: t[f"{n}.up"])
             self.w_up = torch.cat([up(n) for n in names], dim=0)
-            self.w_down = torch.cat([t[f"{n}.down"].reshape(-1) for n in names])
+            self.w_down = torch.cat([t[f"{n}.down"] for n in names], dim=1).contiguous()
             return
         ups, downs = [t[f"e{e}.up"] for e in range(s.experts)], [t[f"e{e}.down"] for e in range(s.experts)]
         if s.shared:
@@ -101,7 +101,7 @@ class RoutedMlp(FeedForward):
 
     def forward(self, h, stream, ctx):
         s, ops = self.spec, self.rt.ops
-        if self.grouped:
+        if self.grouped and ops.routed_experts_runs(h.shape[0]):
             scoring = {"correction": self.w_correction, "softmax_all": True} if self.scoring == "softmax_all" else {"sigmoid": self.scoring == "sigmoid"}
             sums, gates = ops.routed_experts(h, self.w_router, self.b_router, s.top, self.w_up, self.w_down, s.experts, s.intermediate, s.shared,
                                              s.activation, gated=self.gated, weigh_input=self.weigh == "input", shared_gate=self.shared_gate,
@@ -122,7 +122,8 @@ class RoutedMlp(FeedForward):
         up = ops.linear(h, self.w_up, None, out_f32=True)
         if self.gated or self.identity or self.shared_gate:
             a = ops.expert_act(up, gates, s.intermediate, s.activation, experts=s.experts, gated=self.gated,
-                               weigh_input=self.weigh == "input", shared_gate=self.shared_gate)
+                               weigh_input=self.weigh == "input", shared_gate=self.shared_gate,
+                               **({"interleaved": True} if self.grouped and self.gated else {}))
         else:
             a = ops.expert_act(up, gates, s.intermediate, s.activation)
         stream.add_linear(a, self.w_down)

@@ -31,7 +31,7 @@ def test_products_over_the_rows_that_chose_an_expert(dtype, T, outputs, E, top, 
     gate, up = [(rnd(c, width) * width ** -0.5).to(dtype) for c in cols], [(rnd(c, width) * width ** -0.5).to(dtype) for c in cols]
     down = [(rnd(width, c) * c ** -0.5).to(dtype) for c in cols]
     w_up = torch.cat([interleave_gate_up(a, b) if gated else b for a, b in zip(gate, up)])
-    w_down = torch.cat([d.reshape(-1) for d in down])
+    w_down = torch.cat(down, dim=1)
     scoring = {"sigmoid": True} if inside else ({"softmax_all": True} if outputs > E else {})
     sums, gates = ops.routed_experts(h.to(DEV), router.to(DEV), None, top, w_up.to(DEV), w_down.to(DEV), E, ff, shared, "silu", gated=gated,
                                      weigh_input=inside, shared_gate=shared_gate, **scoring)
@@ -70,7 +70,7 @@ def test_the_part_gives_what_it_gives_over_every_expert(dtype, T, spec, monkeypa
     x = torch.randn(T, width, generator=g).to(DEV)
     tensors, got = {}, []
     for takes in (True, False):
-        monkeypatch.setattr(ops, "routed_experts_takes", lambda *a, takes=takes: takes, raising=False)
+        monkeypatch.setattr(ops, "routed_experts_takes", lambda *a, takes=takes: takes)
         part = FEED_FORWARDS.build(RoutedMlpSpec("routed_mlp", width, E, top, ff, "silu", shared, bias, {}, **spec), Runtime(torch.device(DEV), dtype, ops))
         for d in part.tensor_decls():
             if d.name not in tensors:

@@ -1,0 +1,47 @@
+"""The tiles that products of more than 64 rows run in: every one at sizes that are no multiple of it, with one K step, two, three and
+more (odd and even), in each epilogue; and a row's sums, which are the same whatever tile its batch runs in."""
+import pytest
+import torch
+
+from gpu_util import DEV, assert_close
+
+pytestmark = pytest.mark.gpu
+
+# rows, columns, K, the tile of the plain product: 256x256, 256x192, 256x128, 128x128, 64x64, 64x64 with four buffers
+SIZES = [(1537, 8200, 1024, 0), (1537, 8200, 1088, 0), (1000, 8200, 1024, 1), (1025, 8200, 1088, 1), (700, 6152, 1024, 2), (511, 8200, 1088, 2),
+         (1000, 4104, 320, 3), (513, 8200, 384, 3), (193, 4104, 64, 4), (65, 2056, 64, 4), (1537, 130, 64, 4), (130, 8200, 192, 4),
+         (65, 40, 64, 5), (193, 40, 192, 5), (127, 40, 128, 5)]
+
+
+def rnd(shape, dtype, seed, scale=1.0):
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    return (torch.randn(shape, generator=g, device=DEV) * scale).to(dtype)
+
+
+def ops_for(dtype):
+    from machserve_amd.kernels import get_ops
+    return get_ops(dtype, DEV)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M,N,K,tile", SIZES)
+def test_products_in_every_tile(dtype, M, N, K, tile):
+    from machserve_amd.kernels.ops import interleave_gate_up
+    ops = ops_for(dtype)
+    assert ops._plan("ms_tiled_tile", M, N, K, 1, 1) == tile, "the sizes are those of another tile"
+    a, w, bias, x = rnd((M, K), dtype, 1), rnd((N, K), dtype, 2, K ** -0.5), rnd((N,), torch.float32, 3), rnd((M, N), torch.float32, 4)
+    ref = a.float() @ w.float().T
+    out = ops.linear(a, w, None, out_f32=True)
+    assert_close(out, ref, torch.float32, "32-bit sums")
+    assert_close(ops.linear(a, w, bias), ref + bias, dtype, "element type, with bias")
+    assert_close(ops.linear_split(a, w).sum(0), ref, torch.float32, "sums in slices of K")
+    assert_close(ops.linear_act(a, w, "relu2"), torch.relu(ref) ** 2, dtype, "activation in the epilogue")
+    x1 = x.clone()
+    pending = ops.linear_residual(a, w, x1)
+    assert_close(x1 if pending is None else x1 + pending.sum(0), x + ref, torch.float32, "added to the stream")
+    gate, up = w[:N // 2].contiguous(), w[N // 2:N // 2 * 2].contiguous()
+    z, u = a.float() @ gate.float().T, a.float() @ up.float().T
+    assert_close(ops.linear_swiglu(a, interleave_gate_up(gate, up), N // 2), z * torch.sigmoid(z) * u, dtype, "gated product")
+    # the same rows in a batch of another size, another tile: the same sums bit for bit
+    some = ops.linear(a[:65].contiguous(), w, None, out_f32=True)
+    assert torch.equal(some, out[:65])
