@@ -189,6 +189,18 @@ static int launch_gemm(const elem_t* A, const elem_t* W, int M, int N, int K, Ep
     if ((long)ceil_div(M, 64) * ceil_div(N, 64) * ns <= round_blocks && whole_steps && ep.k_per_split >= 256) MS_GEMM_DEEP(64, 64, 2, 2, 64, 4);
     MS_GEMM(64, 64, 2, 2, 64);
 #else
+    // Whole K steps straight to LDS, three or two of them in flight (the loop through registers waits for a trip to memory every step:
+    // 1,024 x 2,048 x 2,048 in 512 tiles of 64x64 90 -> 69 us); where the 64x64 tiles are less than two a CU, four times as many of
+    // 32x32 (512 x 896 x 4,864 118 -> 50 us, 512 x 896 x 896 25 -> 12; at two a CU 69 against 75).  The sums keep their order.
+    if (K % 32 == 0) {
+        const bool few = (long)ceil_div(M, 64) * ceil_div(N, 64) < 2L * compute_units();
+        if constexpr (EPI == EPI_SWIGLU) {  // gate and up columns lie side by side: 32 columns a wave
+            if (few) MS_GEMM_DEEP(32, 64, 2, 2, 32, 4);
+        } else {
+            if (few) MS_GEMM_DEEP(32, 32, 2, 2, 32, 4);
+        }
+        MS_GEMM_DEEP(64, 64, 2, 2, 32, 3);
+    }
     MS_GEMM(64, 64, 2, 2, 32);
 #endif
 #undef MS_GEMM

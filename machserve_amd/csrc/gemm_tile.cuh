@@ -9,8 +9,9 @@
 // bfloat16 with K steps of 64: tiles go global -> LDS directly (global_load_lds_dwordx4, a wave's
 // 64 lanes fill 1 KB = 8 unpadded rows in lane order, so the swizzle is applied to the global
 // address), and the next step's tile is in flight while this one is multiplied (how far ahead, and with how many buffers, see the
-// loops below); only a partial last step goes through registers, where what lies beyond K is masked.  The 32-bit build and
-// K steps of 32 go global -> registers -> LDS (padded rows).
+// loops below); only a partial last step goes through registers, where what lies beyond K is masked.  K steps of 32 of
+// two-byte elements, and in 32-bit whatever has a partial last step, go global -> registers -> LDS (padded rows); the other
+// products of the 32-bit build go straight to LDS as well (its K steps of 32 are rows of 128 bytes too).
 // Every output element is the sum over K in steps of 32 in ascending order whatever the
 // tile shape or the number of rows, so a row's result does not depend on its batch.
 #pragma once
@@ -76,7 +77,7 @@ __device__ __forceinline__ void gemm_tile(const elem_t* __restrict__ A, const el
 #ifdef MS_ELEM_HALF
     constexpr bool DIRECT = BK == 64;
 #else
-    constexpr bool DIRECT = false;
+    constexpr bool DIRECT = STAGES > 2;
 #endif
     constexpr bool PIPED = STAGES == GEMM_PIPED;
     constexpr int BUFS = PIPED ? 2 : STAGES;
@@ -154,7 +155,6 @@ __device__ __forceinline__ void gemm_tile(const elem_t* __restrict__ A, const el
             *reinterpret_cast<u32x4*>(&Ws[buf][at(row, my_chunk)]) = rw[i];
         }
     };
-#ifdef MS_ELEM_HALF
     // One K step of both tiles straight into LDS buffer `buf`: lane l of a wave's load lands at the wave's
     // base + 16 l.  Written in assembly: of a load that it knows to write LDS the compiler makes every later
     // LDS read wait (vmcnt(0)), and nothing would be in flight during the multiplications; the waits are
@@ -207,7 +207,6 @@ __device__ __forceinline__ void gemm_tile(const elem_t* __restrict__ A, const el
 #pragma unroll
         for (int l = 0; l < A_CHUNKS + W_CHUNKS; ++l) load_one(k0, buf, l);
     };
-#endif
     // End of a K step: this wave's loads and LDS accesses have completed, then everybody's.
     auto step_barrier = [&]() {
         if constexpr (DIRECT) {
@@ -230,15 +229,27 @@ __device__ __forceinline__ void gemm_tile(const elem_t* __restrict__ A, const el
     const int k_begin = split * ep.k_per_split;
     const int nk = ceil_div(k_end - k_begin, BK);
     const bool partial = (k_end - k_begin) % BK != 0;  // the last step is a partial one
+    // 8 elements of a tile's row, of the K chunk of 32 at kk, in swizzled rows: one 16-byte chunk, or in 32-bit two
+    auto tile_frag = [&](const elem_t* t, int row, int kk) {
+#ifdef MS_ELEM_HALF
+        return frag_load(&t[at(row, kk / EPC + grp)]);
+#else
+        Frag f;
+        const f32x4 x = *reinterpret_cast<const f32x4*>(&t[at(row, kk / EPC + 2 * grp)]), y = *reinterpret_cast<const f32x4*>(&t[at(row, kk / EPC + 2 * grp + 1)]);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) { f.v[e] = x[e]; f.v[4 + e] = y[e]; }
+        return f;
+#endif
+    };
     auto multiply = [&](int buf) {
 #pragma unroll
         for (int kk = 0; kk < BK; kk += 32) {
             Frag fa[TM], fb[TN];
             if constexpr (DIRECT) {
 #pragma unroll
-                for (int i = 0; i < TM; ++i) fa[i] = frag_load(&As[buf][at(wm * (BM / WM) + i * 16 + r16, kk / EPC + grp)]);
+                for (int i = 0; i < TM; ++i) fa[i] = tile_frag(As[buf], wm * (BM / WM) + i * 16 + r16, kk);
 #pragma unroll
-                for (int j = 0; j < TN; ++j) fb[j] = frag_load(&Ws[buf][at(wn * (BN / WN) + j * 16 + r16, kk / EPC + grp)]);
+                for (int j = 0; j < TN; ++j) fb[j] = tile_frag(Ws[buf], wn * (BN / WN) + j * 16 + r16, kk);
             } else {
 #pragma unroll
                 for (int i = 0; i < TM; ++i) fa[i] = frag_load(&As[buf][(wm * (BM / WM) + i * 16 + r16) * LDS_LD + kk + grp * 8]);
@@ -331,7 +342,6 @@ __device__ __forceinline__ void gemm_tile(const elem_t* __restrict__ A, const el
         if (kt < nk) step(kt, 0);
 #endif
     } else if constexpr (DIRECT && STAGES > 2) {
-#ifdef MS_ELEM_HALF
         // A block that is alone on its CU (few tiles: one tile of rows under a weight of a few hundred column
         // tiles) has nobody to hide its loads behind, and with one step in flight every step costs a trip to
         // memory.  Here STAGES - 1 steps are in flight: the loads of step kt + STAGES - 1 go out before step
@@ -377,7 +387,6 @@ __device__ __forceinline__ void gemm_tile(const elem_t* __restrict__ A, const el
             ss_q[q][tid % BM] = ssum;
             __syncthreads();
         }
-#endif
     } else if constexpr (DIRECT) {
 #ifdef MS_ELEM_HALF
         if (nk == 1 && partial) {

@@ -375,7 +375,7 @@ static int launch_experts(const void* a, const void* w, void* out, ExpertArgs g,
     MS_EXPERTS(64, 64, 2, 2, 64, 4);
 #else
     (void)bm;
-    MS_EXPERTS(64, 64, 2, 2, 32, 2);
+    MS_EXPERTS(64, 64, 2, 2, 32, 3);
 #endif
 #undef MS_EXPERTS
 }

@@ -45,3 +45,21 @@ def test_products_in_every_tile(dtype, M, N, K, tile):
     # the same rows in a batch of another size, another tile: the same sums bit for bit
     some = ops.linear(a[:65].contiguous(), w, None, out_f32=True)
     assert torch.equal(some, out[:65])
+
+
+# 32-bit: tiles of 32x32 (gated products 32x64) and 64x64 with whole K steps, one to many of them, and a partial last step
+@pytest.mark.parametrize("M,N,K", [(65, 40, 32), (97, 130, 64), (130, 200, 96), (501, 896, 160), (1025, 2056, 32), (1100, 2050, 352), (200, 136, 104)])
+def test_32_bit_products_in_every_tile(M, N, K):
+    from machserve_amd.kernels.ops import interleave_gate_up
+    ops = ops_for(torch.float32)
+    a, w, x = rnd((M, K), torch.float32, 5), rnd((N, K), torch.float32, 6, K ** -0.5), rnd((M, N), torch.float32, 7)
+    ref = (a.double() @ w.double().T).float()
+    out = ops.linear(a, w, None, out_f32=True)
+    assert_close(out, ref, torch.float32, "sums")
+    x1 = x.clone()
+    assert ops.linear_residual(a, w, x1) is None
+    assert_close(x1, x + ref, torch.float32, "added to the stream")
+    gate, up = w[:N // 2].contiguous(), w[N // 2:N // 2 * 2].contiguous()
+    z, u = a.double() @ gate.double().T, a.double() @ up.double().T
+    assert_close(ops.linear_swiglu(a, interleave_gate_up(gate, up), N // 2), z * torch.sigmoid(z) * u, torch.float32, "gated product")
+    assert torch.equal(ops.linear(a[:65].contiguous(), w, None, out_f32=True), out[:65]), "a row's sums do not depend on its batch"
