@@ -5,6 +5,7 @@
 // kernels (crates/mach-model/src/kernels.rs:5772-5798, 6416-6455, 131-160).
 //
 // A block's loop over K and its epilogues are in gemm_tile.cuh; here are the choice of the tile and the entry points.
+#include "gemm_plan.h"
 #include "gemm_tile.cuh"
 
 namespace ms {
@@ -36,39 +37,6 @@ static constexpr int g_gemm_config = 0;
 #endif
 
 #ifdef MS_ELEM_HALF
-// The choice of a tile (and of the K slices, where the reader adds them up) for more than 64 rows and whole K steps: the
-// one whose predicted time is least.  A block of a tile takes `step[n]` us a K step of 64 where n + 1 such blocks share a CU, `slope` more of it in
-// proportion as the chip is full, and `store32` or `store16` for each block a CU to store its sums; `start` is paid once a product.  The
-// numbers are a fit (non-negative least squares, 8 to 15 % off) to the times of 168 products: 96 to 3,001 rows of the projections
-// of the 0.5B, 1.5B and 7B layer sizes and of widths of 1,024 and 2,048, cold operands, one to six slices.  The choice is 2 % slower
-// than the best tile measured, on average; against the rules it replaces (rounds of 128x128 blocks, with borders
-// for wider tiles, in a loop of one burst of loads a step) the products are 1.26 times as fast (geometric mean).
-struct TileCost {
-    int bm, bn, per_cu;
-    float step[4], store32, store16, start, slope;
-};
-enum Tile { TILE_256x256, TILE_256x192, TILE_256x128, TILE_128x128, TILE_64x64, TILE_64x64_DEEP, TILE_COUNT };
-static constexpr TileCost kTiles[TILE_COUNT] = {
-    {256, 256, 1, {1.12f}, 8.64f, 0.85f, 8.26f, 0.22f},
-    {256, 192, 1, {0.96f}, 7.82f, 0.00f, 7.22f, 0.14f},
-    {256, 128, 1, {0.65f}, 5.95f, 1.97f, 4.09f, 0.17f},
-    {128, 128, 2, {0.42f, 0.67f}, 1.99f, 0.12f, 3.70f, 0.31f},
-    {64, 64, 4, {0.27f, 0.29f, 0.40f, 0.51f}, 0.31f, 0.00f, 2.87f, 0.37f},
-    {64, 64, 2, {0.25f, 0.45f}, 0.79f, 0.09f, 2.79f, 0.04f},
-};
-
-static float tile_time(const TileCost& t, int M, int N, int k_per_split, int splits, bool store32) {
-    const long blocks = (long)ceil_div(M, t.bm) * ceil_div(N, t.bn) * splits, cus = compute_units(), round = cus * t.per_cu;
-    const float steps = (float)ceil_div(k_per_split, 64), store = store32 ? t.store32 : t.store16;
-    const long full = blocks / round, rest = blocks % round;
-    float us = t.start + (float)full * (steps * (t.step[t.per_cu - 1] + t.slope) + store * t.per_cu);
-    if (rest) {
-        const float fill = (float)rest / (float)round;
-        us += steps * (t.step[ceil_div(rest, cus) - 1] + t.slope * fill) + store * t.per_cu * fill;
-    }
-    return us;
-}
-
 struct GemmPlan {
     int tile, splits;
 };
@@ -81,7 +49,8 @@ static GemmPlan plan_gemm(int M, int N, int K, int splits, bool store32) {
         const int per = ceil_div(ceil_div(K, s), 64) * 64;
         if (splits == 0 && s > 1 && (ceil_div(K, per) != s || per < 192)) continue;
         for (int i = 0; i < TILE_COUNT; ++i) {
-            const float us = tile_time(kTiles[i], M, N, per, s, store32) + (float)(s - 1) * (float)M * (float)N * (8.0f / 4.5e6f);
+            const long blocks = (long)ceil_div(M, kTiles[i].bm) * ceil_div(N, kTiles[i].bn) * s;
+            const float us = tile_time(kTiles[i], blocks, per, store32) + (float)(s - 1) * (float)M * (float)N * (8.0f / 4.5e6f);
             if (us < best_us) {
                 best_us = us;
                 best = {i, s};

@@ -38,7 +38,7 @@ enum EpiKind {
 
 struct NoExperts {
     static constexpr bool GATHERS = false;  // A's rows lie one behind the other
-    __device__ __forceinline__ int source(int m, int) const { return m; }
+    __device__ __forceinline__ int source(int m) const { return m; }
     __device__ __forceinline__ int pitch(int K) const { return K; }    // elements from a row of A to the next
     __device__ __forceinline__ int w_pitch(int K) const { return K; }  // ... of W
 };
@@ -115,7 +115,7 @@ __device__ __forceinline__ void gemm_tile(const elem_t* __restrict__ A, const el
 #pragma unroll
     for (int i = 0; i < A_CHUNKS; ++i) {
         const int c = tid + i * NT;
-        pa[i] = A + (size_t)rows.source(min(m0 + c / CPR, M - 1), m0) * rows.pitch(K) + my_chunk * EPC;
+        pa[i] = A + (size_t)rows.source(min(m0 + c / CPR, M - 1)) * rows.pitch(K) + my_chunk * EPC;
     }
 #pragma unroll
     for (int i = 0; i < W_CHUNKS; ++i) {
@@ -174,7 +174,7 @@ __device__ __forceinline__ void gemm_tile(const elem_t* __restrict__ A, const el
     };
     const uint32_t lds_a = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)&As[0][0];
     const uint32_t lds_w = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)&Ws[0][0];
-    const elem_t* base_a = A + (size_t)rows.source(m0, m0) * rows.pitch(K);
+    const elem_t* base_a = A + (size_t)rows.source(m0) * rows.pitch(K);
     const elem_t* base_w = W + (size_t)n0 * rows.w_pitch(K);
     uint32_t oa[A_CHUNKS], ow[W_CHUNKS];
     const elem_t* ga[Rows::GATHERS ? A_CHUNKS : 1];
@@ -182,7 +182,7 @@ __device__ __forceinline__ void gemm_tile(const elem_t* __restrict__ A, const el
 #pragma unroll
         for (int i = 0; i < A_CHUNKS; ++i) {
             const int m = min(m0 + a_row(i) + lane / 8, M - 1);
-            if constexpr (Rows::GATHERS) ga[i] = A + (size_t)rows.source(m, m0) * rows.pitch(K) + my_chunk * EPC;
+            if constexpr (Rows::GATHERS) ga[i] = A + (size_t)rows.source(m) * rows.pitch(K) + my_chunk * EPC;
             else oa[i] = ((uint32_t)(m - m0) * (uint32_t)rows.pitch(K) + my_chunk * EPC) * (uint32_t)sizeof(elem_t);
         }
 #pragma unroll
@@ -519,45 +519,6 @@ __device__ __forceinline__ void gemm_tile(const elem_t* __restrict__ A, const el
                     }
                 }
             }
-        } else if constexpr (EPI == EPI_EXPERT_GATED || EPI == EPI_EXPERT_PLAIN) {
-            // the activations of the rows that chose the expert, one block of BM rows after the other
-            constexpr int STEP = EPI == EPI_EXPERT_GATED ? 2 : 1;
-            static_assert(TN % STEP == 0, "gate and up tiles come in pairs");
-            elem_t* out = reinterpret_cast<elem_t*>(ep.out);
-#pragma unroll
-            for (int i = 0; i < TM; ++i) {
-                if (ROW_GROUPS && m0 + wm * (BM / WM) + i * 16 >= M) continue;
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const int row = row_base + i * 16 + e;
-                    if (CHECKED && row >= M) continue;
-                    const float w = rows.weight(row);
-                    elem_t* o = out + (size_t)rows.slot(row, m0) * ep.ldo;
-#pragma unroll
-                    for (int j = 0; j < TN; j += STEP) {
-                        const int col = STEP == 2 ? (col_base + j * 16 - r16) / 2 + r16 : col_base + j * 16;
-                        if (CHECKED && col >= ep.n_out) continue;
-                        o[col] = from_f32<elem_t>(STEP == 2 ? rows.gated(acc[i][j][e], acc[i][j + STEP - 1][e], w) : rows.plain(acc[i][j][e], w));
-                    }
-                }
-            }
-        } else if constexpr (EPI == EPI_EXPERT_DOWN) {
-#pragma unroll
-            for (int i = 0; i < TM; ++i) {
-                if (ROW_GROUPS && m0 + wm * (BM / WM) + i * 16 >= M) continue;
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const int row = row_base + i * 16 + e;
-                    if (CHECKED && row >= M) continue;
-                    float* o = reinterpret_cast<float*>(ep.out) + rows.sum_row(row) * ep.ldo;
-#pragma unroll
-                    for (int j = 0; j < TN; ++j) {
-                        const int col = col_base + j * 16;
-                        if (CHECKED && col >= N) continue;
-                        o[col] = acc[i][j][e];
-                    }
-                }
-            }
         } else {
 #pragma unroll
             for (int i = 0; i < TM; ++i) {
@@ -581,6 +542,50 @@ __device__ __forceinline__ void gemm_tile(const elem_t* __restrict__ A, const el
             }
         }
     };
+    if constexpr (EPI == EPI_EXPERT_GATED || EPI == EPI_EXPERT_PLAIN || EPI == EPI_EXPERT_DOWN) {
+        // Half of the tiles are the last of an expert's rows: groups of sixteen that exist store without checks, those that do not are skipped.
+        // up: the activations of the rows that chose the expert; down: their sums, each row's in its plane.
+        constexpr int STEP = EPI == EPI_EXPERT_GATED ? 2 : 1;
+        static_assert(TN % STEP == 0, "gate and up tiles come in pairs");
+        using Out = std::conditional_t<EPI == EPI_EXPERT_DOWN, float, elem_t>;
+        auto emit_group = [&](auto checked, int i) {
+            constexpr bool CHECKED = decltype(checked)::value;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int row = row_base + i * 16 + e;
+                if (CHECKED && row >= M) continue;
+                Out* o = reinterpret_cast<Out*>(ep.out) + rows.out_row(row, m0) * ep.ldo;
+#pragma unroll
+                for (int j = 0; j < TN; j += STEP) {
+                    const int col = STEP == 2 ? (col_base + j * 16 - r16) / 2 + r16 : col_base + j * 16;
+                    if (CHECKED && col >= ep.n_out) continue;
+                    o[col] = from_f32<Out>(acc[i][j][e]);
+                }
+            }
+        };
+        if constexpr (EPI != EPI_EXPERT_DOWN)  // in place, before the stores: the code of each activation is there once
+            rows.with_activation([&](auto act) {
+#pragma unroll
+                for (int i = 0; i < TM; ++i) {
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const float w = rows.weight(row_base + i * 16 + e, m0);
+#pragma unroll
+                        for (int j = 0; j < TN; j += STEP)
+                            acc[i][j][e] = STEP == 2 ? rows.gated(act, acc[i][j][e], acc[i][j + STEP - 1][e], w) : rows.plain(act, acc[i][j][e], w);
+                    }
+                }
+            });
+        const int lower = m0 + wm * (BM / WM);
+#pragma unroll
+        for (int i = 0; i < TM; ++i) {
+            if (lower + i * 16 >= M) break;
+            if (lower + i * 16 + 16 <= M && n0 + BN <= N) emit_group(std::false_type{}, i);
+            else emit_group(std::true_type{}, i);
+        }
+        return;
+    }
     const bool cols_whole = n0 + BN <= N && (EPI != EPI_SWIGLU || (n0 + BN) / 2 <= ep.n_out);
     if (whole) emit(std::false_type{}, std::false_type{});
     else if (cols_whole && M % 16 == 0) emit(std::false_type{}, std::true_type{});

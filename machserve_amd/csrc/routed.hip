@@ -17,6 +17,7 @@
 // beyond the outputs to choose from (`extra`) are gates that every row has, the sigmoids of their own logits, left behind
 // the experts' weights; the first of them can stand for the expert that every row uses.  A weight may also multiply a gated
 // expert's input instead of its output: act(w gate) * (w up).
+#include "gemm_plan.h"
 #include "gemm_tile.cuh"
 
 namespace ms {
@@ -214,7 +215,7 @@ __global__ __launch_bounds__(256) void add_scaled_rows_kernel(float* __restrict_
 // ---- products over the rows that chose an expert -------------------------------------------------------------------------
 // Of E experts a row uses `top`, so a product over every expert's columns does E / top times the work (2,048 rows of 2,048, 8
 // experts of 2,816 of which 2 are used, and one that every row uses: up, activation and down 366 + 73 + 366 us a layer where this
-// does it all in a third).  Here a block's tile of rows belongs to one expert: the up product gathers the rows that chose it, applies
+// does it all in 179 + 83).  Here a block's tile of rows belongs to one expert: the up product gathers the rows that chose it, applies
 // the activation and the weight in its epilogue (the 32-bit sums of all experts never go through memory), and leaves the
 // activations tile after tile; the down product multiplies them by the expert's own matrix and stores the sums in the planes that
 // the reader adds up, one for each expert that a row uses, in ascending order.  Who reads what is found by the blocks themselves: a step of
@@ -227,6 +228,7 @@ struct ExpertArgs {
     const int* counts;    // [E] their lengths
     int T, E, ld_gates, top;
     int routed_tiles, shared_tiles;  // row tiles of the grid: those of the experts (as many as there can be), those of the expert that every row uses
+    int routed_slots;     // rows of the activations before those of the expert that every row uses
     int ff, shared;       // columns of an expert, and of the one that every row uses (0: there is none)
     int width;            // of the rows
     int shared_gate, weigh_input, act;
@@ -257,98 +259,171 @@ struct ExpertRows {
     static constexpr bool GATHERS = GATHERS_;
     const ExpertArgs& g;
     const int* list;  // of the expert's rows; null: every row
-    int e, tile;      // e == E: the expert that every row uses
-    int bm;
+    int e, first;     // e == E: the expert that every row uses; where its activations begin
+    const int* of_row;  // LDS: the weight of each of the tile's rows (up), the row of its sums (down)
     __device__ __forceinline__ int row_of(int m) const { return list ? list[m] : m; }
-    __device__ __forceinline__ int slot(int m, int m0) const { return tile * bm + (m - m0); }
-    __device__ __forceinline__ int source(int m, int m0) const { return GATHERS ? row_of(m) : slot(m, m0); }
+    __device__ __forceinline__ int slot(int m) const { return first + m; }
+    __device__ __forceinline__ int source(int m) const { return GATHERS ? row_of(m) : slot(m); }
     __device__ __forceinline__ int pitch(int) const { return GATHERS ? g.width : max(g.ff, g.shared); }
     __device__ __forceinline__ int w_pitch(int) const { return GATHERS ? g.width : g.E * g.ff + g.shared; }
-    __device__ __forceinline__ float weight(int m) const {
-        if (e == g.E && !g.shared_gate) return 1.0f;
-        return g.gates[(size_t)row_of(m) * g.ld_gates + e];
+    __device__ __forceinline__ float weight(int m, int m0) const { return __int_as_float(of_row[m - m0]); }
+    __device__ __forceinline__ size_t out_row(int m, int m0) const { return GATHERS ? slot(m) : of_row[m - m0]; }
+    template <typename F>
+    __device__ __forceinline__ void with_activation(F f) const {
+        if (g.act == 0) f(std::integral_constant<int, 0>{});
+        else if (g.act == 1) f(std::integral_constant<int, 1>{});
+        else f(std::integral_constant<int, 2>{});
     }
     // as expert_act: the weight on the output, or inside the expert
-    __device__ __forceinline__ float gated(float gv, float uv, float w) const {
+    template <int ACT>
+    __device__ __forceinline__ float gated(std::integral_constant<int, ACT>, float gv, float uv, float w) const {
         const float wi = g.weigh_input && e < g.E ? w : 1.0f;
-        return w != 0.f ? expert_activation(wi * gv, g.act) * uv * w : 0.f;
+        return w != 0.f ? expert_activation(wi * gv, ACT) * uv * w : 0.f;
     }
-    __device__ __forceinline__ float plain(float z, float w) const { return w != 0.f ? expert_activation(z, g.act) * w : 0.f; }
-    __device__ __forceinline__ size_t sum_row(int m) const {
-        const int t = row_of(m);
-        const int p = e == g.E ? g.top : g.plane[(size_t)t * g.E + e];
-        return (size_t)p * g.T + t;
+    template <int ACT>
+    __device__ __forceinline__ float plain(std::integral_constant<int, ACT>, float z, float w) const {
+        return w != 0.f ? expert_activation(z, ACT) * w : 0.f;
     }
 };
 
 template <int BM, int BN, int WM, int WN, int BK, int EPI, int STAGES>
 __global__ __launch_bounds__(64 * WM * WN) void expert_gemm_kernel(const elem_t* __restrict__ A, const elem_t* __restrict__ W, void* out, ExpertArgs g) {
     __shared__ int few[64];
-    const int tiles = g.routed_tiles + g.shared_tiles, lane = threadIdx.x & 63;
-    const int tile = blockIdx.x % tiles;
-    int e = g.E, m0 = (tile - g.routed_tiles) * BM, count = g.T;
-    const int* list = nullptr;
-    if (tile < g.routed_tiles && !g.rows) {
-        e = tile;
-        m0 = 0;
-        const bool mine = lane < g.T && g.plane[(size_t)min(lane, g.T - 1) * g.E + e] >= 0;
-        const unsigned long long all = __ballot(mine);
-        count = __popcll(all);
-        if (mine) few[__popcll(all & ((1ull << lane) - 1))] = lane;
-        list = few;
-    } else if (tile < g.routed_tiles) {
-        // the expert whose tiles hold this one: 64 experts' counts of tiles at a time (none: a tile beyond the lists, no rows)
-        int base = 0;
-        count = m0 = 0;
-        for (int e0 = 0; e0 < g.E; e0 += 64) {
-            const int c = e0 + lane < g.E ? g.counts[e0 + lane] : 0;
-            const int mine = ceil_div(c, BM);
-            int upto = mine;
-#pragma unroll
-            for (int o = 1; o < 64; o <<= 1) {
-                const int v = __shfl_up(upto, o, WAVE);
-                if (lane >= o) upto += v;
-            }
-            const unsigned long long behind = __ballot(base + upto > tile);
-            if (behind) {
-                const int at = __builtin_ctzll(behind);
-                e = e0 + at;
-                count = __shfl(c, at, WAVE);
-                m0 = (tile - (base + __shfl(upto - mine, at, WAVE))) * BM;
-                break;
-            }
-            base += __shfl(upto, 63, WAVE);
-        }
-        list = g.rows + (size_t)e * g.T;
-    }
-    e = __builtin_amdgcn_readfirstlane(e);
-    count = __builtin_amdgcn_readfirstlane(count);
-    m0 = __builtin_amdgcn_readfirstlane(m0);
-    const int cols = e == g.E ? g.shared : g.ff;
     constexpr int PER = EPI == EPI_EXPERT_GATED ? 2 : 1;  // columns of the up product for one of the activations
+    constexpr int GROUP = BM >= 256 ? 4 : 1024 / BM;      // tiles of rows that go over the columns together
+    const int lane = threadIdx.x & 63;
+    int e = g.E, m0 = 0, count = g.T, first = g.routed_slots, col;
+    const int* list = nullptr;
+    if (!g.rows) {
+        const int tiles = g.routed_tiles + g.shared_tiles, tile = blockIdx.x % tiles;
+        col = blockIdx.x / tiles;
+        if (tile < g.routed_tiles) {
+            e = tile;
+            first = tile * 64;
+            const bool mine = lane < g.T && g.plane[(size_t)min(lane, g.T - 1) * g.E + e] >= 0;
+            const unsigned long long all = __ballot(mine);
+            count = __popcll(all);
+            if (mine) few[__popcll(all & ((1ull << lane) - 1))] = lane;
+            list = few;
+        }
+    } else {
+        // The blocks of one XCD (every 8th) take a run of the tiles that there are, first of the expert that every row uses, then of the others; in it
+        // GROUP tiles, mostly of one or two experts, go over the columns together and share both operands in the XCD's L2.
+        const int cols_all = EPI == EPI_EXPERT_DOWN ? ceil_div(g.width, BN) : ceil_div(PER * g.shared, BN);
+        const int cols_one = EPI == EPI_EXPERT_DOWN ? ceil_div(g.width, BN) : ceil_div(PER * g.ff, BN);
+        const int xcd = blockIdx.x & 7, run_all = ceil_div(g.shared_tiles * cols_all, 8);
+        int nth = blockIdx.x >> 3, tiles = g.shared_tiles, cols = cols_all, run = run_all;
+        const bool routed = nth >= run_all;
+        if (routed) {
+            nth -= run_all;
+            tiles = 0;
+            for (int e0 = 0; e0 < g.E; e0 += 64) {
+                int mine = e0 + lane < g.E ? ceil_div(g.counts[e0 + lane], BM) : 0;
+#pragma unroll
+                for (int o = 1; o < 64; o <<= 1) mine += __shfl_xor(mine, o, WAVE);
+                tiles += mine;
+            }
+            tiles = __builtin_amdgcn_readfirstlane(tiles);
+            cols = cols_one;
+            run = ceil_div(tiles * cols, 8);
+        }
+        const int at = xcd * run + nth;
+        if (nth >= run || at >= tiles * cols) return;
+        const int group = at / (GROUP * cols), in = at - group * (GROUP * cols), size = min(GROUP, tiles - group * GROUP);
+        const int tile = group * GROUP + in % size;
+        col = in / size;
+        if (routed) {
+            // the expert whose tiles hold this one, 64 experts' counts at a time
+            int base = 0, slots = 0;
+            count = 0;
+            for (int e0 = 0; e0 < g.E; e0 += 64) {
+                const int c = e0 + lane < g.E ? g.counts[e0 + lane] : 0;
+                const int mine = ceil_div(c, BM), own = ceil_div(c, 64) * 64;
+                int upto = mine, upto_slots = own;
+#pragma unroll
+                for (int o = 1; o < 64; o <<= 1) {
+                    const int v = __shfl_up(upto, o, WAVE), u = __shfl_up(upto_slots, o, WAVE);
+                    if (lane >= o) {
+                        upto += v;
+                        upto_slots += u;
+                    }
+                }
+                const unsigned long long behind = __ballot(base + upto > tile);
+                if (behind) {
+                    const int l = __builtin_ctzll(behind);
+                    e = e0 + l;
+                    count = __shfl(c, l, WAVE);
+                    m0 = (tile - (base + __shfl(upto - mine, l, WAVE))) * BM;
+                    first = slots + __shfl(upto_slots - own, l, WAVE);
+                    break;
+                }
+                base += __shfl(upto, 63, WAVE);
+                slots += __shfl(upto_slots, 63, WAVE);
+            }
+            list = g.rows + (size_t)e * g.T;
+        } else {
+            m0 = tile * BM;
+        }
+    }
+    // Into scalar registers for good (the tile's loads take their bases from there): seen through, the compiler may keep them in vector ones.
+    auto scalar = [](int v) {
+        asm volatile("" : "+v"(v));
+        return __builtin_amdgcn_readfirstlane(v);
+    };
+    e = scalar(e), count = scalar(count), m0 = scalar(m0), first = scalar(first), col = scalar(col);
+    const int cols = e == g.E ? g.shared : g.ff;
     const int N = EPI == EPI_EXPERT_DOWN ? g.width : PER * cols, K = EPI == EPI_EXPERT_DOWN ? cols : g.width;
-    const int n0 = blockIdx.x / tiles * BN;
+    const int n0 = col * BN;
     if (m0 >= count || n0 >= N) return;  // the whole block: these are the block's own numbers
     __syncthreads();
-    EpiArgs ep{out, nullptr, EPI == EPI_EXPERT_DOWN ? g.width : max(g.ff, g.shared), cols, K, 0};
-    const ExpertRows<EPI != EPI_EXPERT_DOWN> rows{g, list, e, tile, BM};
+    // What the epilogue needs of each row, read once by the whole block: read row by row between the stores the two dependent loads
+    // were 9 to 12 us of a block's 35 to 72.
+    __shared__ int of_row[BM];
+    int own_e = e;
+    asm volatile("" : "+v"(own_e));  // a copy for the branches: what they merge is kept in vector registers
+    for (int i = threadIdx.x; i < BM; i += 64 * WM * WN) {
+        const int m = min(m0 + i, count - 1), t = list ? list[m] : m;
+        if (EPI == EPI_EXPERT_DOWN) of_row[i] = (own_e == g.E ? g.top : g.plane[(size_t)t * g.E + own_e]) * g.T + t;
+        else of_row[i] = __float_as_int(own_e == g.E && !g.shared_gate ? 1.0f : g.gates[(size_t)t * g.ld_gates + own_e]);
+    }
+    EpiArgs ep{out, nullptr, EPI == EPI_EXPERT_DOWN ? g.width : max(g.ff, g.shared), EPI == EPI_EXPERT_DOWN ? g.width : cols, K, 0};
+    const ExpertRows<EPI != EPI_EXPERT_DOWN> rows{g, list, e, first, of_row};
     const elem_t* own = W + (size_t)e * g.ff * (EPI == EPI_EXPERT_DOWN ? 1 : PER * g.width);  // its columns, or its rows
     gemm_tile<BM, BN, WM, WN, BK, EPI, STAGES, false>(A, own, count, N, K, ep, m0, n0, 0, rows);
 }
 
-// Rows of a tile: a step of at most 64 rows has one tile an expert; above, the larger tile where the experts' lists can be expected to fill it.
-static int expert_tile_rows(int T, int E, int top) {
+// The tile of a product.  A step of at most 64 rows has one tile of 64 rows an expert, its weight's columns streamed by blocks with three
+// steps in flight; above, the tile of the least predicted time, every expert's last tile counted as half empty.
+// 2,048 rows, 2 of 8 experts of 2,816 and one of 2,816 for every row, width 2,048, gated (us up / down): 256x256 191 / 83, 256x192 211 / 120,
+// 256x128 197 / 97, 128x128 179 / 106, 64x64 279 / 156; 128x128 alone, in the order of the columns and with the epilogue reading row by row, was 228 / 120.
+// 1,750 rows, 2 of 8 experts of 2,816: 122 / 73, 128 / 62, 130 / 87, 120 / 72 and 178 / 101 against 170 / 113.
+static int plan_experts(const ExpertArgs& g, bool down, int per) {
 #ifdef MS_ELEM_HALF
-    return T <= 64 || (long)T * top < 96L * E ? 64 : 128;
+    if (g.T <= 64) return TILE_64x64_DEEP;
+    const long rows = (long)g.T * g.top, used = min((long)g.E, rows);
+    int best = TILE_64x64;
+    float least = INFINITY;
+    for (int i = 0; i < TILE_COUNT; ++i) {
+        const TileCost& t = kTiles[i];
+        if (i == TILE_256x256 && !down && per == 1) continue;  // every sum in its own activation: too many registers
+        const long routed = max(used, rows / t.bm + (used + 1) / 2), all = g.shared ? ceil_div(g.T, t.bm) : 0;
+        const long blocks = down ? (routed + all) * ceil_div(g.width, t.bn) : routed * ceil_div(per * g.ff, t.bn) + all * ceil_div(per * g.shared, t.bn);
+        const long depth = down ? (routed * g.ff + all * g.shared) / (routed + all) : g.width;
+        const float us = tile_time(t, blocks, (int)depth, down);
+        if (us < least) {
+            least = us;
+            best = i;
+        }
+    }
+    return best;
 #else
-    (void)T; (void)E; (void)top;
-    return 64;
+    (void)g; (void)down; (void)per;
+    return TILE_64x64_DEEP;
 #endif
 }
 
-static long expert_routed_tiles(int T, int E, int top) {
+static long expert_routed_tiles(int T, int E, int top, long bm) {
     if (T <= 64) return E;
-    const long bm = expert_tile_rows(T, E, top);
     return min((long)T * top / bm + min((long)E, (long)T * top), (long)E * ceil_div((long)T, bm));
 }
 
@@ -365,16 +440,32 @@ static int check_experts(const char* what, const ExpertArgs& g) {
 template <int EPI>
 static int launch_experts(const void* a, const void* w, void* out, ExpertArgs g, hipStream_t stream) {
     MS_REQUIRE((reinterpret_cast<uintptr_t>(a) & 15) == 0 && (reinterpret_cast<uintptr_t>(w) & 15) == 0, "experts: operands must be 16-byte aligned");
-    const int bm = expert_tile_rows(g.T, g.E, g.top);
-    g.routed_tiles = (int)expert_routed_tiles(g.T, g.E, g.top);
-    g.shared_tiles = g.shared ? ceil_div(g.T, bm) : 0;
-    const int N = EPI == EPI_EXPERT_DOWN ? g.width : (EPI == EPI_EXPERT_GATED ? 2 : 1) * max(g.ff, g.shared);
-#define MS_EXPERTS(BM_, BN_, WM_, WN_, BK_, ST_)                                                                                           do {                                                                                                                                       const long nb = (long)(g.routed_tiles + g.shared_tiles) * ceil_div(N, BN_);                                                            hipLaunchKernelGGL((expert_gemm_kernel<BM_, BN_, WM_, WN_, BK_, EPI, ST_>), dim3((unsigned)nb), dim3(64 * WM_ * WN_), 0, stream,                            (const elem_t*)a, (const elem_t*)w, out, g);                                                                        return check_launch("experts " #BM_ "x" #BN_ "x" #BK_);                                                                            } while (0)
+    constexpr bool DOWN = EPI == EPI_EXPERT_DOWN;
+    constexpr int PER = EPI == EPI_EXPERT_GATED ? 2 : 1;
+    const TileCost& tile = kTiles[plan_experts(g, DOWN, PER)];
+    g.routed_tiles = (int)expert_routed_tiles(g.T, g.E, g.top, tile.bm);
+    g.shared_tiles = g.shared ? ceil_div(g.T, tile.bm) : 0;
+    g.routed_slots = (int)expert_routed_tiles(g.T, g.E, g.top, 64) * 64;
+    const long cols_one = ceil_div(DOWN ? g.width : PER * g.ff, tile.bn), cols_all = ceil_div(DOWN ? g.width : PER * g.shared, tile.bn);
+    const long nb = g.rows ? 8 * (ceil_div(g.routed_tiles * cols_one, 8L) + ceil_div(g.shared_tiles * cols_all, 8L))
+                           : (long)(g.routed_tiles + g.shared_tiles) * max(cols_one, cols_all);
+#define MS_EXPERTS(BM_, BN_, WM_, WN_, BK_, ST_)                                                                                    \
+    do {                                                                                                                            \
+        hipLaunchKernelGGL((expert_gemm_kernel<BM_, BN_, WM_, WN_, BK_, EPI, ST_>), dim3((unsigned)nb), dim3(64 * WM_ * WN_), 0,    \
+                           stream, (const elem_t*)a, (const elem_t*)w, out, g);                                                     \
+        return check_launch("experts " #BM_ "x" #BN_ "x" #BK_);                                                                     \
+    } while (0)
 #ifdef MS_ELEM_HALF
-    if (bm == 128) MS_EXPERTS(128, 128, 2, 4, 64, GEMM_PIPED);
-    MS_EXPERTS(64, 64, 2, 2, 64, 4);
+    switch ((int)(&tile - kTiles)) {
+        case TILE_256x256:
+            if constexpr (EPI != EPI_EXPERT_PLAIN) MS_EXPERTS(256, 256, 2, 4, 64, GEMM_PIPED);
+        case TILE_256x192: MS_EXPERTS(256, 192, 4, 2, 64, GEMM_PIPED);
+        case TILE_256x128: MS_EXPERTS(256, 128, 4, 2, 64, GEMM_PIPED);
+        case TILE_128x128: MS_EXPERTS(128, 128, 2, 4, 64, GEMM_PIPED);
+        case TILE_64x64: MS_EXPERTS(64, 64, 2, 2, 64, GEMM_PIPED);
+        default: MS_EXPERTS(64, 64, 2, 2, 64, 4);
+    }
 #else
-    (void)bm;
     MS_EXPERTS(64, 64, 2, 2, 32, 3);
 #endif
 #undef MS_EXPERTS
@@ -427,11 +518,11 @@ extern "C" int ms_add_scaled_rows(float* x, const void* h, const float* weights,
     return check_launch("add_scaled_rows");
 }
 
-// Rows of the activations that ms_experts_up leaves and ms_experts_down reads (a tile's rows one behind the other, tile after tile).
+// Rows of the activations that ms_experts_up leaves and ms_experts_down reads: the experts' one behind the other, each from a multiple
+// of 64, then those of the expert that every row uses.
 extern "C" long ms_experts_slots(int T, int E, int top, int shared) {
     if (T <= 0 || E <= 0 || top <= 0) return 0;
-    const long bm = expert_tile_rows(T, E, top);
-    return (expert_routed_tiles(T, E, top) + (shared > 0 ? ceil_div((long)T, bm) : 0)) * bm;
+    return expert_routed_tiles(T, E, top, 64) * 64 + (shared > 0 ? T : 0);
 }
 
 // rows [E, T], counts [E]: the rows that use each expert, in ascending order.
@@ -446,7 +537,7 @@ extern "C" int ms_expert_rows(const int* plane, int* rows, int* counts, int T, i
 extern "C" int ms_experts_up(const void* x, const void* w, void* out, const int* plane, const float* gates, const int* rows, const int* counts,
                              int T, int E, int ld_gates, int top, int ff, int shared, int width, int gated, int shared_gate, int weigh_input,
                              int act, hipStream_t stream) {
-    const ExpertArgs g{plane, gates, rows, counts, T, E, ld_gates, top, 0, 0, ff, shared, width, shared_gate, weigh_input, act};
+    const ExpertArgs g{plane, gates, rows, counts, T, E, ld_gates, top, 0, 0, 0, ff, shared, width, shared_gate, weigh_input, act};
     if (int rc = check_experts("experts up", g)) return rc;
     MS_REQUIRE(!weigh_input || gated, "experts up: weights inside experts that are not gated");
     return gated ? launch_experts<EPI_EXPERT_GATED>(x, w, out, g, stream) : launch_experts<EPI_EXPERT_PLAIN>(x, w, out, g, stream);
@@ -456,7 +547,7 @@ extern "C" int ms_experts_up(const void* x, const void* w, void* out, const int*
 // then the shared one's; sums [top (+ 1), T, width]: plane k of row t is the k-th expert that it uses, the last plane the shared one's.
 extern "C" int ms_experts_down(const void* a, const void* w, float* sums, const int* plane, const float* gates, const int* rows, const int* counts,
                                int T, int E, int ld_gates, int top, int ff, int shared, int width, hipStream_t stream) {
-    const ExpertArgs g{plane, gates, rows, counts, T, E, ld_gates, top, 0, 0, ff, shared, width, 0, 0, 0};
+    const ExpertArgs g{plane, gates, rows, counts, T, E, ld_gates, top, 0, 0, 0, ff, shared, width, 0, 0, 0};
     if (int rc = check_experts("experts down", g)) return rc;
     return launch_experts<EPI_EXPERT_DOWN>(a, w, sums, g, stream);
 }
