@@ -49,10 +49,11 @@ constexpr int KPAD = 4, VPAD = 4;
 constexpr int NT = BKV / 16;             // 16-key score tiles per key tile
 constexpr int NTP = (NT + 1) / 2;        // pairs of score tiles = K steps of the PV product
 constexpr int K_LD = HDT + KPAD, V_LD = BKV + VPAD;
-// Flat rows of a work item.  The kernel of 32-row tiles (two-byte elements, head size 64) takes 128 a block; the
-// general kernel takes 64, and where a library has both, two of its blocks share an item.
-#if defined(MS_ELEM_HALF) && MS_ATTN_ND == 4
+// Flat rows of a work item (two-byte elements and a head size of 64: two blocks of 64 rows share an item).
+#if defined(MS_ELEM_HALF) && (MS_ATTN_ND == 4 || MS_ATTN_ND == 8)
 #define MS_HAS_ROWS32 1
+#endif
+#if defined(MS_ELEM_HALF) && MS_ATTN_ND == 4
 constexpr int ROWS_PER_BLOCK = 128;
 #else
 constexpr int ROWS_PER_BLOCK = 64;
@@ -545,18 +546,24 @@ __global__ __launch_bounds__(256 * KG, attention_waves_per_simd<KG>()) void page
 
 // ---------------------------------------------------------------------------------------
 // The same attention in tiles of 32 query rows by 32 keys (`mfma_f32_32x32x16`), for the two-byte element
-// types and a head size of 64.  The counters of the kernel above say that it spends fifteen vector instructions
-// on every matrix instruction, and its blocks of 64 rows read the keys and values of a long prompt so often
-// (a block of 64 flat rows is nine tokens of seven heads) that the traffic from the L2 comes within sight of that
-// path's ceiling.  Here a block is 128 flat rows, four waves of 32 rows under each of four key groups (sixteen waves,
-// a whole CU), so a tile that was brought into LDS feeds twice the rows; a lane holds sixteen keys of one query row
-// (one step across lanes instead of two) and a fragment read from LDS feeds twice the arithmetic; the
-// accumulator is rescaled only when a row's maximum has risen by more than a factor of 2^8 (a probability then
-// reaches 256 at most, which neither the 32-bit sums nor the rounded probabilities mind); tiles go from memory
-// straight into one of four LDS stages, three rounds before they are multiplied (no staging registers, no
-// stores); and the block's share of the block table is copied into LDS once, so that no round waits for a page
-// number.  Key tiles start at absolute multiples of 32, tile t belongs to group t mod 4, and every decision is a
+// types and head sizes of 64 and 128.  The counters of the kernel above say that it spends fifteen vector instructions
+// on every matrix instruction.  Here a lane holds sixteen keys of one query row (one step across lanes instead of two) and a
+// fragment read from LDS feeds twice the arithmetic; the accumulator is rescaled only when a row's maximum has risen by more
+// than a factor of 2^8 (a probability then reaches 256 at most, which neither the 32-bit sums nor the rounded
+// probabilities mind); tiles go from memory straight into one of two LDS stages, a round before they are multiplied (no
+// staging registers, no stores); and the block's share of the block table is copied into LDS once, so that no round waits
+// for a page number.  A block is 64 flat rows, two waves of 32 rows under each of two key groups: three blocks (head size
+// 64; two with 128) share a CU, where one's exponentials overlap another's products and a causal prompt's long blocks lie beside its short
+// ones; what bounds it is that overlap (a tile is about as many cycles of vector as of matrix instructions) and, in one prompt, the longest block's
+// chain of rounds.  Key tiles start at absolute multiples of 32, tile t belongs to group t mod 2, and every decision is a
 // row's own, so a row's result depends neither on the step's cut nor on the rows beside it.
+//
+// Blocks measured (us; rows x key groups x stages, of 32 rows, 32 keys; general: the kernel above), prompts of 512, 2,048 and 4,096 tokens, eight of 200, 32 rows
+// behind 1,500 keys beside a prompt of 512:
+//   head size 64, 14 over 2 heads    general 14.1  42.5   111  12.5  31.9;  2x2x2 10.5  29.1  61  8.3  18.2;  2x2x4 11.1  30.4  73  8.7  -;
+//                                    2x4x2   12.5  32.8    83  12.8  -;     4x2x4 14.1  36.9  71  11.3  -;    4x4x4 14.8  32.9  66  12.8  -
+//   head size 128, 28 over 4 heads   general 17.5   101   318  28.7  34.1;  2x2x2 13.8  58   184  20.4  28.7; 2x4x2 14.5  75.6  218  30.2  -
+//   head size 128, 16 over 4 heads   general 16.4    57   181  19.5  33.6;  2x2x2 13.2  39   117  11.6  27.3; 2x4x2 13.4  40.3  124  19.9  -
 //
 // Operands (K = 16): A is 32 rows x 16, lane l holds row l % 32, elements (l / 32) * 8 .. + 8; B likewise by
 // column; the result has column l % 32 and, in register v, row 8 * (v / 4) + 4 * (l / 32) + v % 4.  With
@@ -564,16 +571,12 @@ __global__ __launch_bounds__(256 * KG, attention_waves_per_simd<KG>()) void page
 // tile: if row R of the tile holds key R with bits 2 and 3 exchanged, they are the eight consecutive keys
 // 16c + 8 * (l / 32) .., which is a B fragment of P^T as it stands and one 16-byte read of V^T.
 //
-// A tile that is loaded straight into LDS cannot be zeroed on its way: keys that are not there (beyond the
-// rows' positions, in pages given back behind a window, in tiles past the block's range) read the start of the
-// pool instead, and are masked in the scores; the pools hold finite values everywhere, so a value that meets a
-// zero probability adds nothing.
+// A tile that is loaded straight into LDS cannot be zeroed on its way: sixteen keys that are not there (beyond the
+// block's rows, in pages given back behind a window, in tiles past the block's range) read the start of the
+// pool instead, are masked in the scores, and their values are overwritten with zeros.
 #ifdef MS_HAS_ROWS32
 namespace r32 {
-constexpr int KG = 4, RW = 4, TK = 32;  // key groups, waves of rows, keys of a group's tile
-constexpr int GT = RW * 64;             // threads of a key group
-constexpr int ROUND = KG * TK;          // keys of a round of the block
-constexpr int NS = 4;                   // LDS stages: a tile is asked for NS - 1 rounds before it is multiplied
+constexpr int TK = 32;                  // keys of a group's tile
 constexpr int NC = HDT / 16;            // steps of the score product
 constexpr int NDT = HDT / 32;           // 32-row tiles of the output's head dimension
 // LDS rows are unpadded; 16-byte chunk q of row r sits at q ^ f(r), with f such that the rows a fragment read takes
@@ -581,11 +584,17 @@ constexpr int NDT = HDT / 32;           // 32-row tiles of the output's head dim
 constexpr int K_BYTES = TK * HDT * 2, V_BYTES = HDT * TK * 2;
 constexpr int STAGE = K_BYTES + V_BYTES;
 constexpr int PER_LANE = 16 * NDT + 2;  // what a group hands over per lane: the output, the reference, the sum
-constexpr int MERGE_BYTES = (KG - 1) * RW * 64 * PER_LANE * 4;
-constexpr int SMEM = NS * KG * STAGE > MERGE_BYTES ? NS * KG * STAGE : MERGE_BYTES;
 constexpr int MAX_TABLE = 2048;  // pages of a block's share of the block table (in LDS)
 constexpr float RISE = 8.0f;     // a row's reference maximum follows its maximum when that has risen by more (in powers of two)
-static_assert(ROWS_PER_BLOCK == RW * 32, "a work item is what one block of this kernel takes");
+constexpr int RW = 2, KG = 2, NS = 2;   // waves of rows, key groups, LDS stages: a tile is asked for a round before it is multiplied
+constexpr int GT = RW * 64;             // threads of a key group
+constexpr int ROUND = KG * TK;          // keys of a round of the block
+constexpr int MERGE_BYTES = (KG - 1) * RW * 64 * PER_LANE * 4;
+constexpr int SMEM = NS * KG * STAGE > MERGE_BYTES ? NS * KG * STAGE : MERGE_BYTES;
+constexpr int SUB = ROWS_PER_BLOCK / (RW * 32);  // blocks of a work item
+constexpr int LOADS = STAGE / 16 / GT;           // of a lane per tile
+constexpr int PER_CU = HDT == 64 ? 3 : 2;        // blocks that share a CU: by the registers
+static_assert(PER_CU * (SMEM + MAX_TABLE * 4 + 1024) <= 160 * 1024, "the tiles of a CU's blocks exceed its LDS");
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 __device__ __forceinline__ void mma_32x32x16(f32x16& acc, const Frag& a, const Frag& b) {
@@ -603,27 +612,34 @@ __device__ __forceinline__ float max3(float a, float b, float c) {
     return r;
 }
 __device__ __forceinline__ int swap_bits_2_3(int r) { return (r & ~12) | ((r & 4) << 1) | ((r & 8) >> 1); }
-__device__ __forceinline__ int k_swizzle(int r) { return ((r >> 1) & 3) | (((r >> 4) & 1) << 2); }  // rows of 8 chunks
+__device__ __forceinline__ int k_swizzle(int r) {
+    if constexpr (HDT == 64) return ((r >> 1) & 3) | (((r >> 4) & 1) << 2);  // rows of 8 chunks
+    else return (r & 7) | (((r >> 4) & 1) << 3);                             // rows of 16
+}
 __device__ __forceinline__ int v_swizzle(int d) { return ((d >> 2) & 1) | (((d >> 4) & 1) << 1); }  // rows of 4 chunks
 }  // namespace r32
 
-__global__ __launch_bounds__(r32::KG * r32::GT, 4) void paged_attention_rows32_kernel(AttnArgs a) {
+__global__ __launch_bounds__(r32::KG * r32::GT, r32::KG * r32::RW * r32::PER_CU / 4) void paged_attention_rows32_kernel(AttnArgs a) {
     using namespace r32;
-    static_assert(HDT == 64 && TK == 32 && RW == 4, "the swizzles and the tiles' split over a group's waves are written for this shape");
-    static_assert(SMEM + MAX_TABLE * 4 + 1024 <= 160 * 1024, "the tiles of a block exceed the LDS of a CU");
+    static_assert((HDT == 64 || HDT == 128) && TK == 32 && RW == 2 && NS == 2, "the swizzles, the tiles' split over a group's waves and the rounds are written for these shapes");
     __shared__ __attribute__((aligned(1024))) unsigned char smem[SMEM];
     __shared__ int tab[MAX_TABLE];
     __shared__ unsigned kofs[KG][NS][2], vofs[KG][NS][2];  // [group][round % NS][16-key group of the tile]
 
-    const int kg = threadIdx.x >> 8, tg = threadIdx.x & 255, lane = tg & 63, rw = tg >> 6;
+    const int kg = threadIdx.x / GT, tg = threadIdx.x % GT, lane = tg & 63, rw = tg >> 6;
     const int n32 = lane & 31, h = lane >> 5;
     auto stage = [&](int b) { return smem + (KG * b + kg) * STAGE; };
-    const int kvh = blockIdx.x % a.KV, item = blockIdx.x / a.KV;
-    const int s = a.work[item * 2], r0 = a.work[item * 2 + 1];
+    // the order of the blocks: as the general kernel's
+    const int kvh = blockIdx.x % a.KV, sub = blockIdx.x / a.KV % SUB, turn = blockIdx.x / (a.KV * SUB);
+    int item = turn;
+    if (a.pair_span > 0 && turn >= a.pair_span)
+        item = turn < 2 * a.pair_span ? a.n_work - 1 - (turn - a.pair_span) : turn - a.pair_span;
+    const int s = a.work[item * 2], r0 = a.work[item * 2 + 1] + RW * 32 * sub;
     if (s < 0) return;  // an item that only fills the list up (the same for the whole block)
     const int g = a.H / a.KV;
     const int q_start = a.seq_q_start[s], q_len = a.seq_q_len[s], pos0 = a.seq_pos0[s];
     const int R = q_len * g;
+    if (r0 >= R) return;  // the item's rows end in the block beside this one (the same for the whole block)
     constexpr int hd = HDT;
     const int ps = a.ps;
     const int* table = a.block_table + (size_t)s * a.table_stride;
@@ -636,7 +652,7 @@ __global__ __launch_bounds__(r32::KG * r32::GT, 4) void paged_attention_rows32_k
     const int pos = pos0 + tok;
     const bool wave_active = __builtin_amdgcn_readfirstlane((int)(r0 + rw * 32 < R)) != 0;  // the same for the whole wave
 
-    const int last_row = min(r0 + ROWS_PER_BLOCK, R) - 1;
+    const int last_row = min(r0 + RW * 32, R) - 1;
     int kv_hi = pos0 + last_row / g + 1;
     int kv_lo = 0;
     if (a.window > 0 || a.chunk > 0) kv_lo = max(0, first_visible_key(pos0 + r0 / g, a.window, a.chunk));
@@ -674,6 +690,7 @@ __global__ __launch_bounds__(r32::KG * r32::GT, 4) void paged_attention_rows32_k
         return;
     }
     // the pages of the block's keys, once: those of [kt_first, kv_hi), at most MAX_TABLE of them (the launcher sees to it)
+    kv_lo = __builtin_amdgcn_readfirstlane(kv_lo);
     kv_hi = __builtin_amdgcn_readfirstlane(kv_hi);
     const int kt_first = __builtin_amdgcn_readfirstlane((kv_lo / ROUND) * ROUND);
     const int page_first = kt_first / ps, n_tab = min(ceil_div(kv_hi, ps), a.table_stride) - page_first;
@@ -694,14 +711,21 @@ __global__ __launch_bounds__(r32::KG * r32::GT, 4) void paged_attention_rows32_k
     float m_ref = NEG_BIG, l_run = 0.f;
     const float sl = a.scale * 1.4426950408889634f;
 
-    // A group's four waves bring the group's tile, a quarter of K and a quarter of V^T each: a wave's load lands at the
-    // wave's LDS base + 16 * lane, so the chunk that belongs at place p = 64 * wave + lane of the K tile (row p / 8,
-    // chunk p % 8 ^ swizzle) is the one this lane asks for; likewise the V^T tile (row p / 4).  Which 16-key group of
+    // A group's waves bring the group's tile, an equal share of K and of V^T each: a wave's load lands at the
+    // wave's LDS base + 16 * lane, so the chunk that belongs at place p of the K tile (row p / (HDT / 8),
+    // chunk p % (HDT / 8) ^ swizzle) is the one this lane asks for; likewise the V^T tile (row p / 4).  Which 16-key group of
     // the tile a chunk lies in picks the page offset, which the group's first two threads leave in LDS a round before.
+    constexpr int KL = LOADS / 2;  // loads of K, and of V^T
     const int p_own = 64 * rw + lane;
-    const int Rk = p_own >> 3, kq = (p_own & 7) ^ k_swizzle(Rk), kl = swap_bits_2_3(Rk);  // row Rk of the tile holds key kl
-    const elem_t* k_src = a.kpool + (kl & 15) * hd + kq * 8;
-    const int k_grp = kl >> 4;
+    const elem_t* k_src[KL];
+    int k_grp[KL];
+#pragma unroll
+    for (int i = 0; i < KL; ++i) {
+        const int p = i * GT + p_own, Rk = p / (HDT / 8), kq = (p % (HDT / 8)) ^ k_swizzle(Rk), kl = swap_bits_2_3(Rk);  // row Rk of the tile holds key kl
+        k_src[i] = a.kpool + (kl & 15) * hd + kq * 8;
+        k_grp[i] = kl >> 4;
+    }
+    // (GT / 4 rows further on, the swizzle of a V^T row is the same)
     const int dv = p_own >> 2, vq = (p_own & 3) ^ v_swizzle(dv);  // keys 8 vq .. + 8 of row dv of V^T
     const elem_t* v_src = a.vpool + (size_t)dv * ps + (vq & 1) * 8;
     const int v_grp = vq >> 1;
@@ -732,11 +756,16 @@ __global__ __launch_bounds__(r32::KG * r32::GT, 4) void paged_attention_rows32_k
         (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const unsigned char*)(smem + kg * STAGE + 1024 * rw));
     auto load_direct = [&](int r) {
         const int b = r % NS;
-        const elem_t* gk = k_src + ((size_t)kofs[kg][b][k_grp] << 4);
-        const elem_t* gv = v_src + ((size_t)vofs[kg][b][v_grp] << 4);
         const uint32_t kb = lds_own + b * (KG * STAGE), vb = kb + K_BYTES;
-        asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(gk), "s"(kb) : "memory", "m0");
-        asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(gv), "s"(vb) : "memory", "m0");
+#pragma unroll
+        for (int i = 0; i < KL; ++i) {
+            const elem_t* gk = k_src[i] + ((size_t)kofs[kg][b][k_grp[i]] << 4);
+            asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(gk), "s"(kb + i * GT * 16) : "memory", "m0");
+        }
+        const elem_t* gv = v_src + ((size_t)vofs[kg][b][v_grp] << 4);
+#pragma unroll
+        for (int i = 0; i < KL; ++i)
+            asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(gv + i * (GT / 4) * ps), "s"(vb + i * GT * 16) : "memory", "m0");
     };
     // rows of this wave: the first and the last position decide which tiles need no mask at all
     const int pos_first = pos0 + (r0 + rw * 32) / g;
@@ -746,7 +775,7 @@ __global__ __launch_bounds__(r32::KG * r32::GT, 4) void paged_attention_rows32_k
     const int k_row = n32 * (HDT * 2), k_sw = k_swizzle(n32), v_row = K_BYTES + n32 * (TK * 2), v_sw = v_swizzle(n32);
 
     // Round r: group kg has the tile of absolute index (kt_first / 32) + r * KG + kg.  Its page offsets are written a
-    // round before its loads go out, its loads NS - 1 rounds before it is multiplied, and one barrier a round
+    // round before its loads go out, its loads a round before it is multiplied, and one barrier a round
     // separates the steps.
     // (the same for the whole block: kept in scalar registers, so that the rounds' branches are scalar ones)
     const int n_rounds = __builtin_amdgcn_readfirstlane(ceil_div(kv_hi - kt_first, ROUND));
@@ -756,24 +785,20 @@ __global__ __launch_bounds__(r32::KG * r32::GT, 4) void paged_attention_rows32_k
 #pragma unroll
     for (int c = 0; c < NC; ++c) asm volatile("" : "+v"(qf[c].v));
     __syncthreads();  // the table is in LDS
-    for (int r = 0; r < NS - 1; ++r) fill_offsets(r);
+    fill_offsets(0);
     __syncthreads();
-    for (int r = 0; r < NS - 1; ++r)
-        if (r < n_rounds) load_direct(r);
-    fill_offsets(NS - 1);
-    // End of a round: the tiles of all rounds but the youngest one asked for have landed (a wave's loads complete in
-    // order, two a round), and this wave's LDS accesses are done; then everybody's.
-    auto round_end = [&](bool one_behind) {
+    load_direct(0);
+    fill_offsets(1);
+    // End of a round: this wave's loads have landed and its LDS accesses are done; then everybody's.
+    auto round_end = [&]() {
         __builtin_amdgcn_sched_barrier(0);
-        if (one_behind) asm volatile("s_waitcnt vmcnt(2) lgkmcnt(0)" ::: "memory");
-        else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
         __builtin_amdgcn_s_barrier();
         __builtin_amdgcn_sched_barrier(0);
     };
-    round_end(n_rounds >= NS - 1);  // rounds 0 and 1 are here
+    round_end();
     // S^T = K Q^T of the group's tile of round r: register v of this lane is key kt0 + 16 (v / 8) + 8 h + v % 8 for query
-    // row n32.  The scores of round r + 1 are asked for at the end of round r, behind the products of round r: the
-    // matrix cores work on them while other waves take their exponentials.
+    // row n32.
     f32x16 sc;
     auto scores = [&](int r) {
         const unsigned char* st = stage(r % NS);
@@ -789,13 +814,26 @@ __global__ __launch_bounds__(r32::KG * r32::GT, 4) void paged_attention_rows32_k
     };
     const int kg_keys = __builtin_amdgcn_readfirstlane(kg * TK);
     auto busy_in = [&](int r) { return wave_active && kt_first + r * ROUND + kg_keys < kv_hi; };
-    if (busy_in(0)) scores(0);
     for (int r = 0; r < n_rounds; ++r) {
-        const int kt0 = kt_first + r * ROUND + kg * TK;
+        const int kt0 = kt_first + r * ROUND + kg_keys;
         const unsigned char* st = stage(r % NS);
-        const bool more = r + NS - 1 < n_rounds;
-        if (more) load_direct(r + NS - 1);  // into the stage that round r - 1 has left
+        if (r + 1 < n_rounds) load_direct(r + 1);  // into the stage that round r - 1 has left
+        if (kt_first + r * ROUND < kv_lo || kt_first + (r + 1) * ROUND > kv_hi) {
+            // (at most the first and the last round, the same for the whole block) values of sixteen keys that are not there: zero,
+            // for what was read in their place need not be finite
+            const int key = kt0 + 16 * v_grp;
+            if (key + 16 <= kv_lo || key >= kv_hi) {
+#pragma unroll
+                for (int i = 0; i < KL; ++i)
+                    *reinterpret_cast<u32x4*>(smem + (r % NS * KG + kg) * STAGE + K_BYTES + (i * GT + p_own) * 16) = (u32x4){0, 0, 0, 0};
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            __builtin_amdgcn_s_barrier();
+            __builtin_amdgcn_sched_barrier(0);
+        }
         if (busy_in(r)) {
+            scores(r);
             // the values of the first sixteen keys, which the step after next multiplies by: asked for before the exponentials
             auto v_frag = [&](int c, int dt) {
                 return frag_load(reinterpret_cast<const elem_t*>(st + v_row + dt * (32 * TK * 2) + (((2 * c + h) ^ v_sw) << 4)));
@@ -854,9 +892,8 @@ __global__ __launch_bounds__(r32::KG * r32::GT, 4) void paged_attention_rows32_k
                     if (c == 0) vf[dt] = v_frag(1, dt);
                 }
         }
-        if (r + 1 < n_rounds && busy_in(r + 1)) scores(r + 1);
-        if (r + NS < n_rounds) fill_offsets(r + NS);  // read when that round's loads go out, at the top of the next round
-        round_end(more);
+        if (r + 2 < n_rounds) fill_offsets(r + 2);  // read when that round's loads go out, at the top of the next round
+        round_end();
     }
 
     l_run += __shfl_xor(l_run, 32, WAVE);  // the row's two halves (they were scaled alike all along)
@@ -1405,22 +1442,22 @@ using namespace ms;
 
 // Attention of a mixed batch.  `work` lists (request index, first flat row) for every ROWS_PER_BLOCK
 // flat rows of a request (ms_attention_rows_per_block_nd<N>() tells the caller the number; the general kernel
-// takes an item as SUB_BLOCKS blocks of 64 rows, the kernel of 32-row tiles as one block); an item of
+// takes an item as SUB_BLOCKS blocks of 64 rows, the kernel of 32-row tiles as r32::SUB); an item of
 // request -1 only fills a list up and is skipped; see the file comment.  window = 0 means all keys.  max_key_groups = 0 lets the
 // launcher choose how many key groups share a block (1, 2 or 4) from the width of the block tables;
 // a positive value asks for that many (as far as this tile has them).  nsplit > 1 cuts every block's
 // keys over that many blocks (few blocks of rows over long contexts would leave most of the chip idle
 // and run as long as their chain of tiles); T is the number of rows, part_o [T, H, nsplit, hd] and
 // part_ml [T, H, nsplit, 2] are float workspaces.
-// Whether a launch with these sizes runs in the kernel of 32-row tiles: where the block tables allow contexts of
-// 2,048 keys and more (measured on one prompt of the 0.5B head shape: 512 tokens 13.9 against 11.9 us, 2,048 32.2
-// against 34.4, 4,096 60 against 83, 8,192 194 against 252), the head size is the tile's, and a block's share of the
-// block table fits its place in LDS (asked for by name with max_key_groups = 32).
+//
+// Whether a launch with these sizes runs in the kernel of 32-row tiles: where the head size is the tile's and a block's share of the
+// block table fits its place in LDS (asked for by name with max_key_groups = 32; 1, 2 and 4 ask for the general kernel).  It was
+// the faster one at every size measured (its comment has some): one prompt of 17 to 8,192 tokens, requests of 40 to 877, decode rows
+// behind 1,500 to 16,000 keys beside a prompt, windows of 512 and 1,024; with blocks of 128 rows, one a CU, it had been the slower one below 2,048 keys.
 static bool takes_rows32(int hd, int ps, int table_stride, int window, int max_key_groups) {
 #ifdef MS_HAS_ROWS32
-    const long span = window > 0 ? (long)window + BKV : (long)table_stride * ps;
     const long pages_of_span = window > 0 ? ((long)window + 2 * ROWS_PER_BLOCK + r32::ROUND) / ps + 2 : (long)table_stride;
-    return hd == HDT && pages_of_span <= r32::MAX_TABLE && (max_key_groups == 32 || (max_key_groups == 0 && span >= 2048));
+    return hd == HDT && pages_of_span <= r32::MAX_TABLE && (max_key_groups == 32 || max_key_groups == 0);
 #else
     (void)hd; (void)ps; (void)table_stride; (void)window; (void)max_key_groups;
     return false;
@@ -1455,7 +1492,7 @@ extern "C" int MS_CAT(ms_attention_splits_nd, MS_ATTN_ND)(int n_work, int KV, in
     if (window > 0 && span > (long)window + 64) span = (long)window + 64;
     if (span <= 2L * T) return 1;
     long n;
-    if (takes_rows32(hd, ps, table_stride, window, 0)) {
+    if (HDT == 64 && span >= 2048 && takes_rows32(hd, ps, table_stride, window, 0)) {
         n = std::min((long)attention_compute_units() / blocks, span / 1024);
     } else {
         if (blocks >= 192) return 1;
@@ -1515,11 +1552,9 @@ extern "C" int MS_CAT(ms_paged_attention_mask_nd, MS_ATTN_ND)(
     auto span_for = [&](int variant) { return resident[variant] == 2 ? (cus / (KV * SUB_BLOCKS) > 0 ? cus / (KV * SUB_BLOCKS) : 1) : 0; };
 #ifdef MS_HAS_ROWS32
     {
-        // tiles of 32 rows by 32 keys under four key groups, a block a CU (the list's order, longest contexts first, is
-        // the order the blocks start in)
         if (takes_rows32(hd, ps, table_stride, window, max_key_groups)) {
-            a.pair_span = 0;
-            const dim3 grid32((unsigned)(n_work * KV), (unsigned)nsplit);
+            a.pair_span = r32::PER_CU == 2 ? std::max(cus / (KV * r32::SUB), 1) : 0;
+            const dim3 grid32((unsigned)(n_work * KV * r32::SUB), (unsigned)nsplit);
             hipLaunchKernelGGL(paged_attention_rows32_kernel, grid32, dim3(r32::KG * r32::GT), 0, stream, a);
             int rc32 = check_launch("paged_attention (32-row tiles)");
             if (rc32 || nsplit == 1) return rc32;

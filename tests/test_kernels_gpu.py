@@ -449,6 +449,42 @@ def test_attention_in_tiles_of_32_rows(dtype, splits, dead_pages, H, KV, hd, ps,
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("splits,dead_pages", [(0, False), (3, False), (0, True)])
+@pytest.mark.parametrize("H,KV,ps,window", [(28, 4, 64, None), (6, 2, 16, 100), (20, 1, 128, None), (8, 8, 32, 333), (3, 1, 16, 31)])
+def test_attention_in_tiles_of_32_rows_by_a_head_of_128(dtype, splits, dead_pages, H, KV, ps, window):
+    """The same kernel for a head size of 128: blocks of 64 flat rows, two LDS stages."""
+    if dead_pages and window is None:
+        pytest.skip("pages are given back behind a window only")
+    seqs = [(0, 1), (0, 300), (517, 1), (3000, 37), (3, 2), (1023, 1), (128, 1), (127, 2), (31, 2), (95, 130), (2040, 19)]
+    got, ref = _attention_case(dtype, H, KV, 128, ps, window, seqs, 650 + ps + splits, peak=True, groups=32, splits=splits, dead_pages=dead_pages)
+    assert_close(got, ref, dtype, "attention in tiles of 32 rows, head size 128")
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("hd", [64, 128])
+def test_attention_reads_nothing_of_keys_that_are_not_there(dtype, hd):
+    """Keys beyond a request's rows and in pages given back are read from the start of the pool: what another request left there (an
+    overflow) stays out of the sums, in contexts that end in either half of a tile and windows that begin in either."""
+    ops, g, KV, ps, window = ops_for(dtype), 3, 2, 16, 40
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    for pos0, n in [(0, 1), (0, 16), (0, 17), (31, 1), (32, 5), (63, 1), (64, 16), (100, 30)]:
+        for w in (None, window):
+            first = 0 if w is None else max(0, pos0 - w + 1) // ps
+            pages = -(-(pos0 + n) // ps)
+            kp, vp = rnd((pages + 1, KV, ps, hd), dtype, pos0), rnd((pages + 1, KV, hd, ps), dtype, pos0 + 1)
+            q = rnd((n, KV * g * hd), dtype, pos0 + 2)
+            table = torch.arange(1, pages + 1, dtype=torch.int32)
+            table[:first] = -1
+            rows = ops.attention_rows_per_block(hd)
+            args = (table[None].to(DEV), i32([0]), i32([n]), i32([pos0]), i32([(0, r) for r in range(0, n * g, rows)]), KV * g, KV, hd, ps, w, hd ** -0.5)
+            kp[0], vp[0] = 0, 0
+            want = ops.paged_attention(q.to(DEV), kp.to(DEV), vp.to(DEV), *args)
+            kp[0], vp[0] = float("nan"), float("inf")
+            got = ops.paged_attention(q.to(DEV), kp.to(DEV), vp.to(DEV), *args)
+            assert torch.equal(got, want) and bool(torch.isfinite(got).all()), (pos0, n, w)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("splits", [2, 5, 64])
 @pytest.mark.parametrize("H,KV,hd,ps,window", [(4, 2, 16, 16, None), (14, 2, 64, 64, None), (6, 3, 128, 32, None),
                                                (6, 2, 64, 16, 100), (3, 1, 48, 32, 333)])
