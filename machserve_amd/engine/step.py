@@ -67,6 +67,7 @@ class LaunchedDecode:
 
 class StepFunction:
     TABLE_BUCKET = 8        # captured block tables are this many pages wide, or a multiple
+    SHORT_KEYS = 256        # ... or, of a decode step behind no more keys, as many pages as hold these, where its attention is then not cut
     MAX_GRAPHS = 256        # captured steps kept; the one unused longest goes first
     # ... and the most memory they may hold for good between them: each keeps its step buffer and its results (the
     # logits [rows, vocabulary] in 32-bit are nearly all of it, 39 MB at 64 rows of a 152k vocabulary, where the
@@ -90,6 +91,9 @@ class StepFunction:
         self.model, self.cache, self.rt = model, cache, rt
         self.rows_per_block = attention_rows_per_block
         self.heads_per_kv = model.attention_rows_per_token()
+        # pages of a short decode table (0: none): two-byte elements and heads of up to 128, where whole keys are the faster ones
+        whole = rt.dtype != torch.float32 and all(max(g.spec.head_dim, g.spec.v_head_dim) <= 128 for g in cache.groups.values())
+        self.short_pages = self.SHORT_KEYS // cache.page_size if whole and cache.page_size * self.TABLE_BUCKET > self.SHORT_KEYS else 0
         self.position_axes = model.position_axes() if hasattr(model, "position_axes") else 1
         # A step of few tokens is bound by its launches: it is captured into a HIP graph and replayed.
         # A decode step (one token a request), and any other step of few rows, when its shape
@@ -215,9 +219,11 @@ class StepFunction:
         decode step's time hardly depends on a few rows more."""
         slots, counts, tokens = checked[:3]
         pad = self._decode_bucket(len(slots)) - len(slots)
+        short = self.short_pages
+        fits = short > 0 and max(map(self.cache.length, slots)) < short * self.cache.page_size
         try:
             built = self.cache.build_step(slots, counts, tokens, list(range(len(slots) + pad)), self.heads_per_kv,
-                                          self.rows_per_block, self.TABLE_BUCKET, pad, self.position_axes)
+                                          self.rows_per_block, short if fits else self.TABLE_BUCKET, pad, self.position_axes)
         except CacheError as e:
             raise StepError(str(e)) from e
         return built, self._graph_key(counts + [1] * pad, len(slots) + pad, built[2], sampled), pad

@@ -517,9 +517,13 @@ class HipOps:
         with small heads and one with heads above 64 (measured at head sizes 64 and 128, 1 to 200 requests: a split more
         than that starts a second round of blocks, and every round has the kernel's whole chain of latencies in it: 7B
         heads, 48 requests of 512 keys, 22 us uncut, 31 in two; 0.5B heads, 200 requests, 19 against 25), at least
-        four key tiles each."""
+        four key tiles each.  Up to eight tiles in all stay whole: the merge takes longer than a block's second round of
+        tiles (one request behind 33, 120 and 250 keys: 0.5B heads 6.8, 6.8 and 7.8 us whole, 9.0 in two or four; 7B heads 9.8,
+        10.7 and 12.2 against 12.2), but not in 32-bit, whose tiles take longer (20.2 us whole, 15.6 in four), nor with larger heads."""
         span = table_width * page_size if not window else min(table_width * page_size, window + key_tile)
         tiles = max(1, -(-span // key_tile))
+        if tiles <= 8 and hd <= 128 and self.dtype != torch.float32:
+            return 1
         blocks = self._cus * (2 if hd <= 64 else 1)
         return max(1, min(blocks // (S * KV), -(-tiles // 4), 64))
 
