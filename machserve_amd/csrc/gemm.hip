@@ -109,8 +109,9 @@ static int launch_gemm(const elem_t* A, const elem_t* W, int M, int N, int K, Ep
     }
     if (forced == 8 && whole_steps) MS_GEMM_DEEP(64, 64, 2, 2, 64, 4);
     if (forced == 9) MS_GEMM(256, 256, 2, 4, 64);
-    // The largest tile that still gives every CU of the chip a block or two, with K steps of 64 (half
-    // the barriers of steps of 32).  Measured on M = 512..8192 of the 0.5B shapes; larger tiles under
+    // What is left are products of at most 64 rows, and those whose last K step is not a whole one, which run in the loop of one
+    // burst of loads a step: the largest tile that still gives every CU of the chip a block or two, with K steps of 64 (half
+    // the barriers of steps of 32).  The figures are that loop's with whole steps, which are planned above now; larger tiles under
     // four waves (256x128) lose: their accumulators no longer fit the registers of two blocks a CU.
     // two 128x128 blocks a CU are a round of the chip (512 on 256 CUs); a tile is taken when its blocks fill
     // six tenths of a round
