@@ -10,8 +10,8 @@ from .manager import CacheManager, KVBinding, StateBinding
 
 class DeviceCache:
     """Pools are zero-filled once: a page that is handed out again holds old but finite
-    values, which the attention kernel masks; uninitialised memory could hold NaNs that a
-    zero probability does not cancel."""
+    values (the kernels write no others: ``cache_value`` in ``csrc/common.cuh``), which the attention kernel
+    masks; uninitialised memory could hold NaNs that a zero probability does not cancel."""
 
     def __init__(self, manager: CacheManager, dtype: torch.dtype, device: torch.device):
         self.manager = manager

@@ -573,7 +573,9 @@ __global__ __launch_bounds__(256 * KG, attention_waves_per_simd<KG>()) void page
 //
 // A tile that is loaded straight into LDS cannot be zeroed on its way: sixteen keys that are not there (beyond the
 // block's rows, in pages given back behind a window, in tiles past the block's range) read the start of the
-// pool instead, are masked in the scores, and their values are overwritten with zeros.
+// pool instead, are masked in the scores, and their values are overwritten with zeros (a caller's pool may hold anything in a page
+// that no request of the step owns).  Of sixteen keys that are there in part the others' values are what the page's last owner left:
+// finite, as every writer of a page sees to (cache_value), and met by probabilities of zero.
 #ifdef MS_HAS_ROWS32
 namespace r32 {
 constexpr int TK = 32;                  // keys of a group's tile
@@ -731,7 +733,7 @@ __global__ __launch_bounds__(r32::KG * r32::GT, r32::KG * r32::RW * r32::PER_CU 
     const int v_grp = vq >> 1;
     // Offsets of the group's tile of the next round to be looked up, by the group's first two threads (one 16-key group of
     // the tile each), stepped from round to round rather than divided out.  Keys that are not there (past the
-    // block's range, in a page given back) get offset 0: the first rows of the pool, finite and masked.
+    // block's range, in a page given back) get offset 0: the first rows of the pool, masked.
     int key_next = kt_first + kg * TK + (tg & 1) * 16, lp_next = key_next / ps, off_next = key_next - lp_next * ps;
     const int round_pages = ROUND / ps, round_rem = ROUND % ps;
     auto fill_offsets = [&](int r) {
@@ -819,8 +821,7 @@ __global__ __launch_bounds__(r32::KG * r32::GT, r32::KG * r32::RW * r32::PER_CU 
         const unsigned char* st = stage(r % NS);
         if (r + 1 < n_rounds) load_direct(r + 1);  // into the stage that round r - 1 has left
         if (kt_first + r * ROUND < kv_lo || kt_first + (r + 1) * ROUND > kv_hi) {
-            // (at most the first and the last round, the same for the whole block) values of sixteen keys that are not there: zero,
-            // for what was read in their place need not be finite
+            // (at most the first and the last round, the same for the whole block) values of sixteen keys that are not there: zero
             const int key = kt0 + 16 * v_grp;
             if (key + 16 <= kv_lo || key >= kv_hi) {
 #pragma unroll
@@ -1024,7 +1025,7 @@ __global__ __launch_bounds__(256) void decode_attention_kernel(DecodeArgs a) {
     // Loads are unconditional and on one straight path, so that the compiler counts them and a wait
     // for one tile leaves the next in flight: a key that is not there (beyond the row, in a page
     // given back, in a tile past the split) is read from the start of the pool instead and masked in
-    // the scores.  The pools hold finite values everywhere, so a value that meets a zero probability
+    // the scores.  The pools hold finite values everywhere (cache_value), so a value that meets a zero probability
     // adds nothing.  The pages of a tile's 16-key groups are looked up one tile ahead.
     const float inv_gpp = 1.0f / (float)(ps >> 4);  // 1 / (16-key groups per page)
     // of this lane's groups: page as the table has it, -1 if the group is not to be read (else 0), offset in the page
@@ -1204,7 +1205,7 @@ __global__ __launch_bounds__(256) void decode_attention_kernel(DecodeArgs a) {
             }
             const float* vv_ = rowv + (g + 1) * hd;
             for (int d = tid; d < hd; d += 256) {
-                const elem_t ve = from_f32<elem_t>(vv_[d]);
+                const elem_t ve = cache_value(vv_[d]);
                 vnew[d] = to_f32(ve);
                 if (writes) vdst[(size_t)d * ps] = ve;
             }

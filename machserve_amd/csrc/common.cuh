@@ -82,6 +82,21 @@ __device__ __forceinline__ Frag frag_zero() {
 }
 
 // Load 8 consecutive elements (16-byte aligned for bf16, 32-byte for float).
+// A value as it is written into the pages: finite, the type's largest number in the place of an overflow (the lowest in that of a NaN).  The
+// attention kernels multiply whole groups of keys, and a value that is not the row's (in a page's places behind a request's last key, in the page
+// that is read where a request has none) meets a probability of zero: 0 * inf or 0 * NaN would carry one request's overflow into
+// another's rows.  Keys need no such care: scores of keys that are not the row's are replaced and not multiplied.
+__device__ __forceinline__ elem_t cache_value(float v) {
+#if defined(MS_ELEM_F16)
+    constexpr float most = 65504.0f;
+#elif defined(MS_ELEM_BF16)
+    constexpr float most = 0x1.fep127f;
+#else
+    constexpr float most = 0x1.fffffep127f;
+#endif
+    return from_f32<elem_t>(fminf(fmaxf(v, -most), most));
+}
+
 __device__ __forceinline__ Frag frag_load(const elem_t* p) {
     Frag f;
 #ifdef MS_ELEM_HALF

@@ -101,7 +101,7 @@ __global__ __launch_bounds__(256) void conv_row_kernel(ConvRowArgs a) {
             elem_t* vcol = a.vpool + ((size_t)page * a.KV + kh) * a.dp * a.ps + off;
             for (int e = lane; e < a.d; e += 64) {
                 krow[e] = from_f32<elem_t>(head[e] * inv);
-                if (a.values_are_keys) vcol[(size_t)e * a.ps] = from_f32<elem_t>(head[e]);
+                if (a.values_are_keys) vcol[(size_t)e * a.ps] = cache_value(head[e]);
             }
         }
     }
@@ -173,7 +173,7 @@ __device__ __forceinline__ void conv_head_first_row(const ConvRowArgs& a, int t,
             const int e = lane + 64 * ci;
             if (e < a.d) {
                 krow[e] = from_f32<elem_t>(y[ci] * inv);
-                if (a.values_are_keys) vcol[(size_t)e * a.ps] = from_f32<elem_t>(y[ci]);
+                if (a.values_are_keys) vcol[(size_t)e * a.ps] = cache_value(y[ci]);
             }
         }
     }
@@ -285,7 +285,7 @@ __global__ __launch_bounds__(256) void conv_head_kernel(ConvRowArgs a, int T) {
                 const int e = lane + 64 * ci;
                 if (e < a.d) {
                     krow[e] = from_f32<elem_t>(y[ci][i] * inv);
-                    if (a.values_are_keys) vcol[(size_t)e * a.ps] = from_f32<elem_t>(y[ci][i]);
+                    if (a.values_are_keys) vcol[(size_t)e * a.ps] = cache_value(y[ci][i]);
                 }
             }
         }
@@ -389,7 +389,7 @@ __global__ __launch_bounds__(256) void finish_rows_kernel(FinishArgs a) {
         a.q_out[((size_t)t * a.H + c / fill) * a.dp + a.d + c % fill] = from_f32<elem_t>(0.f);
     for (int c = threadIdx.x; c < nv; c += 256) {
         const int h = c / a.dv, e = c - h * a.dv;
-        if (slot >= 0) a.vpool[(((size_t)page * a.KV + h) * a.dp + e) * a.ps + off] = from_f32<elem_t>(row[nq + nk + c]);
+        if (slot >= 0) a.vpool[(((size_t)page * a.KV + h) * a.dp + e) * a.ps + off] = cache_value(row[nq + nk + c]);
     }
 }
 
@@ -470,7 +470,7 @@ __global__ __launch_bounds__(256) void head_row_kernel(HeadRowArgs a) {
     if (slot >= 0)
         for (int c = threadIdx.x; c < nv; c += 256) {
             const int h = c / a.dv, e = c - h * a.dv;
-            a.vpool[(((size_t)page * a.KV + h) * a.dp + e) * a.ps + off] = from_f32<elem_t>(row[nqk + c]);
+            a.vpool[(((size_t)page * a.KV + h) * a.dp + e) * a.ps + off] = cache_value(row[nqk + c]);
         }
     if (a.gate_out)
         for (int h = threadIdx.x; h < a.H; h += 256) a.gate_out[(size_t)t * a.H + h] = 1.0f / (1.0f + expf(-row[nqk + nv + h]));
@@ -575,7 +575,7 @@ __global__ __launch_bounds__(256) void head_row_quads_kernel(HeadRowArgs a, int 
             const f32x4 v = summed(nqk + h * a.dv + dd);
             elem_t* o = a.vpool + (((size_t)page * a.KV + h) * a.dp + dd) * a.ps + off;
 #pragma unroll
-            for (int e = 0; e < 4; ++e) o[(size_t)e * a.ps] = from_f32<elem_t>(v[e]);
+            for (int e = 0; e < 4; ++e) o[(size_t)e * a.ps] = cache_value(v[e]);
         } else {
             const int h = it - n_head - n_v;
             float v = 0.f;

@@ -558,7 +558,7 @@ __global__ __launch_bounds__(256) void rope_kv_write_kernel(RopeArgs a) {
     }
     for (int p = threadIdx.x; p < a.KV * a.hd; p += 256) {
         const int h = p / a.hd, dd = p % a.hd;
-        a.vpool[(((size_t)page * a.KV + h) * a.hd + dd) * a.ps + off] = from_f32<elem_t>(vrow[p]);
+        a.vpool[(((size_t)page * a.KV + h) * a.hd + dd) * a.ps + off] = cache_value(vrow[p]);
     }
 }
 
@@ -641,7 +641,7 @@ __global__ __launch_bounds__(256) void rope_kv_write_quads_kernel(RopeArgs a) {
             const f32x4 v = summed((a.H + a.KV + h) * a.hd + dd);
             elem_t* o = a.vpool + (((size_t)page * a.KV + h) * a.hd + dd) * a.ps + off;
 #pragma unroll
-            for (int e = 0; e < 4; ++e) o[(size_t)e * a.ps] = from_f32<elem_t>(v[e]);
+            for (int e = 0; e < 4; ++e) o[(size_t)e * a.ps] = cache_value(v[e]);
         }
     }
 }

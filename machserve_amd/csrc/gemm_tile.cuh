@@ -514,7 +514,7 @@ __device__ __forceinline__ void gemm_tile(const elem_t* __restrict__ A, const el
                         } else {
                             elem_t* o = ep.vpool + (((size_t)page * ep.KV + (head - ep.H - ep.KV)) * hd + r16) * ep.ps + off;
 #pragma unroll
-                            for (int j = 0; j < TN; ++j) o[(size_t)(j * 16) * ep.ps] = from_f32<elem_t>(x[j]);
+                            for (int j = 0; j < TN; ++j) o[(size_t)(j * 16) * ep.ps] = cache_value(x[j]);
                         }
                     }
                 }

@@ -81,9 +81,9 @@ __global__ __launch_bounds__(256) void latent_row_kernel(LatentRowArgs a) {
     elem_t* krow = a.kpool + ((size_t)page * a.ps + off) * a.hd;
     elem_t* vcol = a.vpool + (size_t)page * a.hd * a.ps + off;
     for (int c = threadIdx.x; c < a.rank; c += 256) {
-        const elem_t v = from_f32<elem_t>(row[a.q_rank + c] * inv_c * a.c_norm[c]);
-        krow[c] = v;
-        vcol[(size_t)c * a.ps] = v;
+        const float v = row[a.q_rank + c] * inv_c * a.c_norm[c];
+        krow[c] = from_f32<elem_t>(v);
+        vcol[(size_t)c * a.ps] = cache_value(v);
     }
     const float* kr = row + a.q_rank + a.rank;
     for (int i = threadIdx.x; i < a.rot / 2; i += 256) {

@@ -97,7 +97,7 @@ __global__ __launch_bounds__(256) void prepare_kernel(PrepareArgs a) {
         if (a.v_raw_out) a.v_raw_out[(size_t)t * nv + c] = v;
         if (a.v_other) v = (1.0f - lam) * v + lam * a.v_other[(size_t)t * nv + c];
         const int h = c / a.dv, e = c - h * a.dv;
-        if (slot >= 0) a.vpool[(((size_t)page * a.KV + h) * a.dv + e) * a.ps + off] = from_f32<elem_t>(v);
+        if (slot >= 0) a.vpool[(((size_t)page * a.KV + h) * a.dv + e) * a.ps + off] = cache_value(v);
     }
 }
 

@@ -463,8 +463,8 @@ def test_attention_in_tiles_of_32_rows_by_a_head_of_128(dtype, splits, dead_page
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("hd", [64, 128])
 def test_attention_reads_nothing_of_keys_that_are_not_there(dtype, hd):
-    """Keys beyond a request's rows and in pages given back are read from the start of the pool: what another request left there (an
-    overflow) stays out of the sums, in contexts that end in either half of a tile and windows that begin in either."""
+    """Sixteen keys wholly beyond a request's rows or in pages given back are read from the start of the pool: what lies there stays out
+    of the sums, in contexts that end in either half of a tile and windows that begin in either."""
     ops, g, KV, ps, window = ops_for(dtype), 3, 2, 16, 40
     i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
     for pos0, n in [(0, 1), (0, 16), (0, 17), (31, 1), (32, 5), (63, 1), (64, 16), (100, 30)]:
