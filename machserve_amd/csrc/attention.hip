@@ -95,6 +95,8 @@ struct AttnArgs {
     int chunk;
     // softcap > 0: the scaled score s becomes softcap * tanh(s / softcap) before the softmax
     float softcap;
+    // tiles of 32 rows: the reference of a row's exponentials follows its maximum when that has risen by more (in powers of two)
+    float rise;
 };
 
 // The first key a row at `pos` sees under a window and a chunked mask (either 0: none).
@@ -548,9 +550,7 @@ __global__ __launch_bounds__(256 * KG, attention_waves_per_simd<KG>()) void page
 // The same attention in tiles of 32 query rows by 32 keys (`mfma_f32_32x32x16`), for the two-byte element
 // types and head sizes of 64 and 128.  The counters of the kernel above say that it spends fifteen vector instructions
 // on every matrix instruction.  Here a lane holds sixteen keys of one query row (one step across lanes instead of two) and a
-// fragment read from LDS feeds twice the arithmetic; the accumulator is rescaled only when a row's maximum has risen by more
-// than a factor of 2^8 (a probability then reaches 256 at most, which neither the 32-bit sums nor the rounded
-// probabilities mind); tiles go from memory straight into one of two LDS stages, a round before they are multiplied (no
+// fragment read from LDS feeds twice the arithmetic; tiles go from memory straight into one of two LDS stages, a round before they are multiplied (no
 // staging registers, no stores); and the block's share of the block table is copied into LDS once, so that no round waits
 // for a page number.  A block is 64 flat rows, two waves of 32 rows under each of two key groups: three blocks (head size
 // 64; two with 128) share a CU, where one's exponentials overlap another's products and a causal prompt's long blocks lie beside its short
@@ -559,11 +559,19 @@ __global__ __launch_bounds__(256 * KG, attention_waves_per_simd<KG>()) void page
 // row's own, so a row's result depends neither on the step's cut nor on the rows beside it.
 //
 // Blocks measured (us; rows x key groups x stages, of 32 rows, 32 keys; general: the kernel above), prompts of 512, 2,048 and 4,096 tokens, eight of 200, 32 rows
-// behind 1,500 keys beside a prompt of 512:
+// behind 1,500 keys beside a prompt of 512, all with the reference left 2^8 behind (see below; 2x2x2 as it is now: 11.3, 30.6, 64, 8.7, 18.9; 15.3, 65, 200,
+// 20.6, 31.1; 14.3, 44, 124, 12.1, 29.4):
 //   head size 64, 14 over 2 heads    general 14.1  42.5   111  12.5  31.9;  2x2x2 10.5  29.1  61  8.3  18.2;  2x2x4 11.1  30.4  73  8.7  -;
 //                                    2x4x2   12.5  32.8    83  12.8  -;     4x2x4 14.1  36.9  71  11.3  -;    4x4x4 14.8  32.9  66  12.8  -
 //   head size 128, 28 over 4 heads   general 17.5   101   318  28.7  34.1;  2x2x2 13.8  58   184  20.4  28.7; 2x4x2 14.5  75.6  218  30.2  -
 //   head size 128, 16 over 4 heads   general 16.4    57   181  19.5  33.6;  2x2x2 13.2  39   117  11.6  27.3; 2x4x2 13.4  40.3  124  19.9  -
+//
+// How far a row's maximum may rise before the reference of its exponentials follows it, and its sums are rescaled (`rise`): not at all, as in
+// the kernel above, so that the largest probability is one, which rounds exactly.  Where it is left up to 2^8 behind this is 4 %
+// faster (up to 12 %: heads of 128, 1,024 rows behind 16,000 keys 232 us against 254), but every probability is rounded, and rows that few
+// keys decide are further off: 2.26e-3 of the result against 64 bits where following gives 1.78e-3 (bfloat16, scores of deviation
+// two; half precision alike).  Heads of 64 behind tables of 2,048 keys and more have always been left behind; 2^6 it is there: 2.13e-3,
+// where blocks of 128 rows under four key groups and 2^8 gave 2.22e-3 (128 rows behind 4,000 keys: 21.0 us; 2^8 20.2, not at all 22.3).
 //
 // Operands (K = 16): A is 32 rows x 16, lane l holds row l % 32, elements (l / 32) * 8 .. + 8; B likewise by
 // column; the result has column l % 32 and, in register v, row 8 * (v / 4) + 4 * (l / 32) + v % 4.  With
@@ -587,7 +595,6 @@ constexpr int K_BYTES = TK * HDT * 2, V_BYTES = HDT * TK * 2;
 constexpr int STAGE = K_BYTES + V_BYTES;
 constexpr int PER_LANE = 16 * NDT + 2;  // what a group hands over per lane: the output, the reference, the sum
 constexpr int MAX_TABLE = 2048;  // pages of a block's share of the block table (in LDS)
-constexpr float RISE = 8.0f;     // a row's reference maximum follows its maximum when that has risen by more (in powers of two)
 constexpr int RW = 2, KG = 2, NS = 2;   // waves of rows, key groups, LDS stages: a tile is asked for a round before it is multiplied
 constexpr int GT = RW * 64;             // threads of a key group
 constexpr int ROUND = KG * TK;          // keys of a round of the block
@@ -612,6 +619,11 @@ __device__ __forceinline__ float max3(float a, float b, float c) {
     float r;
     asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
     return r;
+}
+// The larger of a lane's number and its counterpart's in the wave's other half, in registers (`__shfl_xor` goes through LDS).
+__device__ __forceinline__ float max_of_halves(float v) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return max3(__uint_as_float(r[0]), __uint_as_float(r[1]), __uint_as_float(r[1]));
 }
 __device__ __forceinline__ int swap_bits_2_3(int r) { return (r & ~12) | ((r & 4) << 1) | ((r & 8) >> 1); }
 __device__ __forceinline__ int k_swizzle(int r) {
@@ -709,8 +721,7 @@ __global__ __launch_bounds__(r32::KG * r32::GT, r32::KG * r32::RW * r32::PER_CU 
     for (int dt = 0; dt < NDT; ++dt)
 #pragma unroll
         for (int i = 0; i < 16; ++i) acc[dt][i] = 0.f;
-    // m_ref: the maximum that the exponentials refer to (a row's own running maximum, followed lazily)
-    float m_ref = NEG_BIG, l_run = 0.f;
+    float m_run = NEG_BIG, l_run = 0.f;
     const float sl = a.scale * 1.4426950408889634f;
 
     // A group's waves bring the group's tile, an equal share of K and of V^T each: a wave's load lands at the
@@ -858,21 +869,19 @@ __global__ __launch_bounds__(r32::KG * r32::GT, r32::KG * r32::RW * r32::PER_CU 
             // this lane's half of the row's keys
             const float tmax = max3(max3(max3(sc[0], sc[1], sc[2]), max3(sc[3], sc[4], sc[5]), max3(sc[6], sc[7], sc[8])),
                                     max3(max3(sc[9], sc[10], sc[11]), sc[12], sc[13]), max3(sc[14], sc[15], sc[15]));
-            // A row's reference follows its maximum only when that has risen far (the two lanes of a row keep the same
-            // reference: where either's half has risen far they exchange their maxima); for every other row the factor
-            // is exactly one and nothing changes.  After a prompt's first tiles this is rare.
-            if (__any((tmax - m_ref) * sl > RISE)) {
-                const float row_max = max3(tmax, __shfl_xor(tmax, 32, WAVE), tmax);
-                const float m_new = (row_max - m_ref) * sl > RISE ? row_max : m_ref;
-                const float alpha = exp2_f((m_ref - m_new) * sl);
+            // (the two lanes of a row keep the same reference; for a row that stays the factor is exactly one)
+            if (__any((tmax - m_run) * sl > a.rise)) {
+                const float row_max = max_of_halves(tmax);
+                const float m_new = (row_max - m_run) * sl > a.rise ? row_max : m_run;
+                const float alpha = exp2_f((m_run - m_new) * sl);
                 l_run *= alpha;
 #pragma unroll
                 for (int dt = 0; dt < NDT; ++dt)
 #pragma unroll
                     for (int i = 0; i < 16; ++i) acc[dt][i] *= alpha;
-                m_ref = m_new;
+                m_run = m_new;
             }
-            const float mb = m_ref * sl;
+            const float mb = m_run * sl;
 #pragma unroll
             for (int i = 0; i < 16; ++i) sc[i] = exp2_f(fmaf(sc[i], sl, -mb));
             float t8[8];
@@ -906,7 +915,7 @@ __global__ __launch_bounds__(r32::KG * r32::GT, r32::KG * r32::RW * r32::PER_CU 
         for (int dt = 0; dt < NDT; ++dt)
 #pragma unroll
             for (int i = 0; i < 16; ++i) mine[(dt * 16 + i) * 64 + lane] = acc[dt][i];
-        mine[(16 * NDT) * 64 + lane] = m_ref;
+        mine[(16 * NDT) * 64 + lane] = m_run;
         mine[(16 * NDT + 1) * 64 + lane] = l_run;
     }
     __syncthreads();
@@ -914,19 +923,19 @@ __global__ __launch_bounds__(r32::KG * r32::GT, r32::KG * r32::RW * r32::PER_CU 
     for (int o = 0; o < KG - 1; ++o) {
         const float* other = mg + ((size_t)o * RW + rw) * 64 * PER_LANE;
         const float m_o = other[(16 * NDT) * 64 + lane], l_o = other[(16 * NDT + 1) * 64 + lane];
-        const float m_new = fmaxf(m_ref, m_o);
-        const float c0 = exp2_f((m_ref - m_new) * sl), c1 = exp2_f((m_o - m_new) * sl);
+        const float m_new = fmaxf(m_run, m_o);
+        const float c0 = exp2_f((m_run - m_new) * sl), c1 = exp2_f((m_o - m_new) * sl);
         l_run = l_run * c0 + l_o * c1;
-        m_ref = m_new;
+        m_run = m_new;
 #pragma unroll
         for (int dt = 0; dt < NDT; ++dt)
 #pragma unroll
             for (int i = 0; i < 16; ++i) acc[dt][i] = acc[dt][i] * c0 + other[(dt * 16 + i) * 64 + lane] * c1;
     }
     if (valid && a.nsplit > 1) {
-        write_partial(acc, m_ref, l_run);
+        write_partial(acc, m_run, l_run);
     } else if (valid) {
-        const float inv = softmax_norm(m_ref * a.scale, l_run, a.sinks, head, a.out_gate, (size_t)(q_start + tok) * a.H + head);
+        const float inv = softmax_norm(m_run * a.scale, l_run, a.sinks, head, a.out_gate, (size_t)(q_start + tok) * a.H + head);
         elem_t* orow = a.out + ((size_t)(q_start + tok) * a.H + head) * hd;
 #pragma unroll
         for (int dt = 0; dt < NDT; ++dt)
@@ -1555,6 +1564,7 @@ extern "C" int MS_CAT(ms_paged_attention_mask_nd, MS_ATTN_ND)(
     {
         if (takes_rows32(hd, ps, table_stride, window, max_key_groups)) {
             a.pair_span = r32::PER_CU == 2 ? std::max(cus / (KV * r32::SUB), 1) : 0;
+            a.rise = HDT == 64 && span >= 2048 ? 6.0f : 0.0f;  // see the kernel
             const dim3 grid32((unsigned)(n_work * KV * r32::SUB), (unsigned)nsplit);
             hipLaunchKernelGGL(paged_attention_rows32_kernel, grid32, dim3(r32::KG * r32::GT), 0, stream, a);
             int rc32 = check_launch("paged_attention (32-row tiles)");
