@@ -45,3 +45,25 @@ def test_tiles_of_32_rows_are_no_further_off_than_the_general_kernel(dtype, H, K
     # Heads of 64 behind tables of 2,048 keys and more are left up to 2^6 behind (17 to 20 %).
     behind = hd == 64 and pages * ps >= 2048
     assert tiles <= (1.21 if behind else 1.03) * general, (tiles, general)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("H,KV,hd", [(14, 2, 64), (28, 4, 128), (8, 2, 32)])
+@pytest.mark.parametrize("keys", [130, 200, 256])
+def test_uncut_decode_rows_are_as_exact_as_cut_ones(dtype, H, KV, hd, keys):
+    """A narrow table, whose keys one block takes, and the same table with absent pages behind, whose keys are cut over blocks: the same sums in
+    another order of 32-bit additions, so that few results round to another number."""
+    from machserve_amd.kernels import get_ops
+    ops, ps, S = get_ops(dtype, DEV), 64, 8
+    got = []
+    rows = [inputs(dtype, H, KV, hd, ps, keys - 1, 1, 7 * s + keys + hd) for s in range(S)]
+    q, kp, vp = (torch.cat([r[i] for r in rows]) for i in range(3))
+    pages = rows[0][3]
+    table = torch.arange(S * pages, dtype=torch.int32, device=DEV).view(S, pages)
+    for t in (table, torch.cat([table, table.new_full((S, 60), -1)], dim=1)):
+        got.append(ops.decode_attention(q, kp, vp, t.contiguous(), i32([keys - 1] * S), H, KV, hd, ps, None, hd ** -0.5))
+    tile = ops._attention_lib(hd)[4]
+    cuts = [ops._decode_splits(S, KV, n, ps, None, tile, hd) for n in (pages, pages + 60)]
+    assert cuts[0] == 1 and cuts[1] > 4, "the first is whole, a wave of the second has a tile at most"
+    assert (got[0] != got[1]).float().mean().item() < 0.01
+    assert error(got[0], torch.cat([r[4] for r in rows])) < {torch.bfloat16: 2.2e-3, torch.float16: 2.8e-4}[dtype]
