@@ -1498,10 +1498,19 @@ static int attention_compute_units() {
 // the price of the partial results' trip through memory and the merge's launch.  Block tables no wider than twice the
 // step's rows are (or may be) those of prompts that run whole, whose blocks walk half the keys on average and whose
 // longest block decides: cutting those only adds (0.5B heads, one prompt of 1,024 tokens 18.9 us uncut, 22.8 in two,
-// 31.9 in four; 1,536 tokens 24.4 / 32.3 / 36.8).  The kernel of 32-row tiles holds one block a CU: it is cut so that
-// blocks x splits stay within one round of the chip, at least 1,024 keys a split (256 rows behind 7,936 keys: 91 us
-// uncut, 25.8 in eight, 35.2 in sixteen; 512 rows behind 7,680: 90.6, 36.2 in four, 50.4 in six; 1,024 rows behind
-// 3,072: 49.4, 38.9 in two, 44.7 in four).  The cut depends on the batch, so results differ in rounding between batches.
+// 31.9 in four; 1,536 tokens 24.4 / 32.3 / 36.8).
+// Heads of 64 in the kernel of 32-row tiles, whose items are two blocks, three to a CU: two blocks a CU in all, at least 1,024 keys a split, and three
+// where that leaves 1,664 keys a split; where the items alone are more than that and yet no whole round of the chip, as many splits of 1,664 keys and
+// more as fill its rounds best.  us (0.5B heads unless said; splits by the first clause alone -> by all; in brackets the kernel of 128-row
+// blocks that the first clause was made for): 1,024 rows behind 4,000 keys 46.9 -> 43.5 (44.6), 16,000 keys 125 -> 108 (105); 2,048 rows behind
+// 16,000 keys 225 -> 208 (195); 512 rows behind 16,000 keys 66 -> 60 (62); 8 over 8 heads, 32 requests of two rows behind 8,000 keys 129 -> 109
+// (112).  Over 165 cases (17 to 2,048 rows behind 1,500 to 32,000 keys, 14 over 2, 8 over 8 and 4 over 2 heads) 0.91 of the time of those blocks, 1.06 at
+// most.  256 rows and fewer would gain by more and shorter splits (64 rows behind 4,000 keys: 19.8 in four, 13.5 in sixteen; those blocks 22.7).
+// Other heads, among them those of 128 in the kernel of 32-row tiles, go by the rule of the general kernel's 64-row blocks, two to a CU: three quarters of
+// a round and more stay whole, fewer are cut into a round and a half, at least 512 keys a split.  With heads of 128 all of 163 cases are faster by it
+// than in the general kernel (0.72 of its time), and 1.09 of the best cut; the furthest from it are 1,024 rows of 12 over 2 heads behind 32,000 keys (473
+// whole, 285 in eight).
+// The cut depends on the batch, so results differ in rounding between batches.
 extern "C" int MS_CAT(ms_attention_splits_nd, MS_ATTN_ND)(int n_work, int KV, int T, int hd, int ps, int table_stride, int window) {
     if (n_work < 1 || KV < 1 || ps < 1 || table_stride < 1) return 1;
     const long blocks = (long)n_work * KV;
@@ -1510,7 +1519,18 @@ extern "C" int MS_CAT(ms_attention_splits_nd, MS_ATTN_ND)(int n_work, int KV, in
     if (span <= 2L * T) return 1;
     long n;
     if (HDT == 64 && span >= 2048 && takes_rows32(hd, ps, table_stride, window, 0)) {
-        n = std::min((long)attention_compute_units() / blocks, span / 1024);
+        const long cus = attention_compute_units();
+        n = std::min(cus / blocks, span / 1024);
+#ifdef MS_HAS_ROWS32
+        const long places = cus * r32::PER_CU, small = blocks * r32::SUB, full = places / small;
+        if (n >= 2 && full > n && span / 1664 >= full) n = full;
+        if (n < 2) {
+            n = 1;
+            if (small < places)
+                for (long s = 2; s <= span / 1664; ++s)  // the chip's rounds times the length of a split
+                    if (ceil_div(small * s, places) * n < ceil_div(small * n, places) * s) n = s;
+        }
+#endif
     } else {
         if (blocks >= 192) return 1;
         n = std::min((384 + blocks - 1) / blocks, span / 512);
