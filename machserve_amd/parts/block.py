@@ -67,9 +67,10 @@ class ParallelBlock(Block):
 
 class _Branch:
     """What a branch of a sandwich block writes to in the stream's place: it keeps the branch's output, as the
-    operands of its last product or as a finished tensor, for the norm that follows."""
+    operands of its last product, as that product's sums or as a finished tensor, for the norm that follows.  Sums are taken only if
+    that norm (``post``, where it is the reader) has ``add_normed_sums``."""
 
-    def __init__(self, ops):
+    def __init__(self, ops, post=None):
         self.ops = ops
         self.product = None
         self.bias = None
@@ -78,6 +79,8 @@ class _Branch:
         self.weighted = None
         self.scaled = None
         self.sums = None
+        if post is not None and not hasattr(post, "add_normed_sums"):
+            self.add_sums = None
 
     def add_linear(self, a, w, bias=None) -> None:
         self.product, self.bias = (a, w), bias
@@ -191,7 +194,7 @@ class SandwichBlock(Block):
             self._branch(self.feed_forward_norm, self.feed_forward, self.feed_forward_post_norm, stream, ctx)
 
     def _branch(self, pre, part, post, stream, ctx):
-        out = _Branch(self.rt.ops)
+        out = _Branch(self.rt.ops, post)
         part.forward(PreNormBlock._input(pre, part, stream), out, ctx)
         stream.flush()  # a norm left pending has added what was pending by now; nothing else may be
         if out.weighted is not None:
@@ -232,7 +235,7 @@ class PostNormBlock(Block):
             self._branch(self.feed_forward, self.feed_forward_post_norm, stream, ctx)
 
     def _branch(self, part, post, stream, ctx):
-        out = _Branch(self.rt.ops)
+        out = _Branch(self.rt.ops, post)
         part.forward(stream.value() if getattr(part, "reads_stream", False) else stream.rows(), out, ctx)
         if out.branches is not None:
             post.add_normed_mean(stream, *out.branches)

@@ -7,7 +7,7 @@ matrix: the up product runs for every expert, one kernel applies the activation 
 (an exact zero for an expert the row did not choose, one for the expert that every row uses), and the down product
 sums the chosen experts' outputs.  A row's result depends on its own logits alone.  Where the kernels take the sizes
 (``routed_experts_takes``) the products run over the rows that chose each expert alone, and what the down product leaves are
-the chosen experts' outputs as sums that are still to be added.
+the chosen experts' outputs as sums that are still to be added (to a stream or collector with ``add_sums``).
 
 Variants that the spec names: experts with a gate, ``W_down (act(W_gate h) * (W_up h))`` (all gates are the first half of
 the one up matrix); scores that are the softmax over every router output, a correction added for the choice only, and
@@ -101,17 +101,15 @@ class RoutedMlp(FeedForward):
 
     def forward(self, h, stream, ctx):
         s, ops = self.spec, self.rt.ops
-        if self.grouped and ops.routed_experts_runs(h.shape[0]):
+        add_sums = getattr(stream, "add_sums", None)  # None: a collector of last products alone, which the products over every expert serve
+        if self.grouped and add_sums is not None and ops.routed_experts_runs(h.shape[0]):
             scoring = {"correction": self.w_correction, "softmax_all": True} if self.scoring == "softmax_all" else {"sigmoid": self.scoring == "sigmoid"}
             sums, gates = ops.routed_experts(h, self.w_router, self.b_router, s.top, self.w_up, self.w_down, s.experts, s.intermediate, s.shared,
                                              s.activation, gated=self.gated, weigh_input=self.weigh == "input", shared_gate=self.shared_gate,
                                              **scoring)
             if self.identity:
                 ops.add_scaled_rows(sums[0], h, gates, s.experts, self.identity)
-            if hasattr(stream, "add_sums"):
-                stream.add_sums(sums)
-            else:  # a block's own collector that knows finished tensors
-                stream.add(sums.sum(0))
+            add_sums(sums)
             return
         if self.scoring == "softmax_all":
             gates = ops.route(h, self.w_router, self.b_router, s.top, correction=self.w_correction, softmax_all=True)
