@@ -1359,6 +1359,15 @@ class HipOps:
             self._want(bias, torch.float32, "route bias", E)
         if correction is not None:
             self._want(correction, torch.float32, "route correction", E)
+        if (plane is None) != (sums is None):
+            raise KernelError("route: numbers of the experts that a row uses go with sums")
+        if plane is not None:
+            if plane.dim() != 2 or not 1 <= plane.shape[1] <= E:
+                raise KernelError(f"route numbers: expected {T} rows of 1 to {E} outputs, got {tuple(plane.shape)}")
+            self._want(plane, torch.int32, "route numbers", T, plane.shape[1])
+            if sums.dim() != 3 or sums.shape[0] < top:
+                raise KernelError(f"route sums: expected {top} planes of {T} rows of {d} or more, got {tuple(sums.shape)}")
+            self._want(sums, torch.float32, "route sums", sums.shape[0], T, d)
         gates = torch.empty((T, E + extra_gates), dtype=torch.float32, device=h.device)
         self._check(lib, lib.ms_route(_ptr(h), _ptr(w), _ptr(bias), _ptr(gates), _c_int(T), _c_int(d), _c_int(E), _c_int(top),
                                       _c_int(1 if softmax_all else (2 if sigmoid else 0)), _ptr(correction), _c_int(extra_gates), _ptr(plane),

@@ -85,3 +85,19 @@ def test_the_part_gives_what_it_gives_over_every_expert(dtype, T, spec, monkeypa
         part.forward(h, stream, None)
         got.append(stream.value())
     assert_close(got[0], got[1], dtype, str(spec))
+
+
+def test_the_router_refuses_numbers_and_sums_that_its_kernel_does_not_assume():
+    from machserve_amd.kernels import KernelError, get_ops
+    ops, new = get_ops(torch.bfloat16, DEV), lambda shape, dt: torch.zeros(shape, dtype=dt, device=DEV)  # noqa: E731
+    T, d, E, top = 5, 64, 6, 3
+    h, w = new((T, d), torch.bfloat16), new((E, d), torch.float32)
+    plane, sums = new((T, E), torch.int32), new((top, T, d), torch.float32)
+    for p, s in [(plane, None), (None, sums), (plane, sums[:top - 1]), (plane, sums[:, :T - 1].contiguous()), (plane, sums[..., :d // 2].contiguous()),
+                 (plane, sums.transpose(1, 2).contiguous().transpose(1, 2)), (plane, sums.double()), (plane, sums.cpu()), (plane, sums[0]),
+                 (plane[:T - 1], sums), (plane[0], sums), (plane.long(), sums), (plane.t().contiguous().t(), sums), (plane.cpu(), sums),
+                 (new((T, E + 1), torch.int32), sums), (new((T, 0), torch.int32), sums)]:
+        with pytest.raises(KernelError):
+            ops.route(h, w, None, top, plane=p, sums=s)
+    ops.route(h, w, None, top, plane=plane, sums=sums)
+    assert plane.tolist() == [[0, 1, 2, -1, -1, -1]] * T  # equal logits: the lower index wins
