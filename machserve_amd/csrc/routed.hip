@@ -299,7 +299,7 @@ __global__ __launch_bounds__(64 * WM * WN) void expert_gemm_kernel(const elem_t*
         col = blockIdx.x / tiles;
         if (tile < g.routed_tiles) {
             e = tile;
-            first = tile * 64;
+            first = tile * g.T;
             const bool mine = lane < g.T && g.plane[(size_t)min(lane, g.T - 1) * g.E + e] >= 0;
             const unsigned long long all = __ballot(mine);
             count = __popcll(all);
@@ -427,6 +427,10 @@ static long expert_routed_tiles(int T, int E, int top, long bm) {
     return min((long)T * top / bm + min((long)E, (long)T * top), (long)E * ceil_div((long)T, bm));
 }
 
+// Rows of the activations before those of the expert that every row uses: with lists every expert's begin at a multiple of 64; without, as
+// many as the step has rows are set aside for each (of one row and 1,024 experts of 2,048 columns 4 MB in two bytes, where 64 an expert were 268).
+static long expert_routed_slots(int T, int E, int top) { return T <= 64 ? (long)E * T : expert_routed_tiles(T, E, top, 64) * 64; }
+
 static int check_experts(const char* what, const ExpertArgs& g) {
     MS_REQUIRE(g.T > 0 && g.E > 0 && g.E <= MAX_EXPERTS && g.top >= 1 && g.top <= 64, "%s: %d rows, %d of %d experts", what, g.T, g.top, g.E);
     MS_REQUIRE(g.width > 0 && g.width % 64 == 0 && g.ff > 0 && g.ff % 64 == 0 && g.shared >= 0 && g.shared % 64 == 0,
@@ -445,7 +449,7 @@ static int launch_experts(const void* a, const void* w, void* out, ExpertArgs g,
     const TileCost& tile = kTiles[plan_experts(g, DOWN, PER)];
     g.routed_tiles = (int)expert_routed_tiles(g.T, g.E, g.top, tile.bm);
     g.shared_tiles = g.shared ? ceil_div(g.T, tile.bm) : 0;
-    g.routed_slots = (int)expert_routed_tiles(g.T, g.E, g.top, 64) * 64;
+    g.routed_slots = (int)expert_routed_slots(g.T, g.E, g.top);
     const long cols_one = ceil_div(DOWN ? g.width : PER * g.ff, tile.bn), cols_all = ceil_div(DOWN ? g.width : PER * g.shared, tile.bn);
     const long nb = g.rows ? 8 * (ceil_div(g.routed_tiles * cols_one, 8L) + ceil_div(g.shared_tiles * cols_all, 8L))
                            : (long)(g.routed_tiles + g.shared_tiles) * max(cols_one, cols_all);
@@ -518,11 +522,11 @@ extern "C" int ms_add_scaled_rows(float* x, const void* h, const float* weights,
     return check_launch("add_scaled_rows");
 }
 
-// Rows of the activations that ms_experts_up leaves and ms_experts_down reads: the experts' one behind the other, each from a multiple
-// of 64, then those of the expert that every row uses.
+// Rows of the activations that ms_experts_up leaves and ms_experts_down reads: the experts' one behind the other, then those of the expert
+// that every row uses.
 extern "C" long ms_experts_slots(int T, int E, int top, int shared) {
     if (T <= 0 || E <= 0 || top <= 0) return 0;
-    return expert_routed_tiles(T, E, top, 64) * 64 + (shared > 0 ? T : 0);
+    return expert_routed_slots(T, E, top) + (shared > 0 ? T : 0);
 }
 
 // rows [E, T], counts [E]: the rows that use each expert, in ascending order.

@@ -87,6 +87,27 @@ def test_the_part_gives_what_it_gives_over_every_expert(dtype, T, spec, monkeypa
     assert_close(got[0], got[1], dtype, str(spec))
 
 
+@pytest.mark.parametrize("T", [1, 2, 63, 64])
+@pytest.mark.parametrize("shared", [0, 64])
+def test_a_step_of_few_rows_sets_no_more_activations_aside_than_its_rows_could_fill(T, shared):
+    """... for every expert, and for the one that every row uses: what the whole call holds at its most is that and what it returns."""
+    from machserve_amd.kernels import get_ops
+    ops, E, top, ff, width = get_ops(torch.bfloat16, DEV), 200, 2, 64, 64
+    g = torch.Generator().manual_seed(T)
+    h, router = torch.randn(T, width, generator=g).to(DEV, torch.bfloat16), torch.randn(E, width, generator=g).to(DEV)
+    w_up, w_down = (torch.zeros(s, dtype=torch.bfloat16, device=DEV) for s in ((E * ff + shared, width), (width, E * ff + shared)))
+    call = lambda: ops.routed_experts(h, router, None, top, w_up, w_down, E, ff, shared, "silu")  # noqa: E731
+    call()
+    torch.cuda.synchronize()
+    before = torch.cuda.memory_allocated()
+    torch.cuda.reset_peak_memory_stats()
+    call()
+    torch.cuda.synchronize()
+    rows = E * T + (T if shared else 0)
+    # the activations; numbers and weights; the planes; a tensor is rounded up to 512 bytes
+    assert torch.cuda.max_memory_allocated() - before <= rows * ff * 2 + 2 * T * E * 4 + (top + 1) * T * width * 4 + 4 * 512
+
+
 def test_the_router_refuses_numbers_and_sums_that_its_kernel_does_not_assume():
     from machserve_amd.kernels import KernelError, get_ops
     ops, new = get_ops(torch.bfloat16, DEV), lambda shape, dt: torch.zeros(shape, dtype=dt, device=DEV)  # noqa: E731
