@@ -435,9 +435,9 @@ def test_attention_key_groups(dtype, groups, H, KV, hd, ps, window):
 @pytest.mark.parametrize("H,KV,hd,ps,window", [(14, 2, 64, 64, None), (6, 2, 64, 16, 100), (20, 1, 64, 128, None), (8, 8, 64, 32, 333),
                                                (3, 1, 64, 16, 31)])
 def test_attention_in_tiles_of_32_rows(dtype, splits, dead_pages, H, KV, hd, ps, window):
-    """The kernel of 32-row tiles that the two-byte libraries have for a head size of 64 (blocks of 128 flat rows, four
-    key groups, tiles loaded straight into four LDS stages, the block table in LDS, a reference maximum that follows
-    lazily), asked for by name: requests that end inside a tile, inside a round of four tiles and inside a block of
+    """The kernel of 32-row tiles that the two-byte libraries have for a head size of 64 (blocks of 64 flat rows, two to a work
+    item, two key groups, tiles loaded straight into two LDS stages, the block table in LDS; behind tables of 2,048 keys and more the
+    reference maximum follows lazily), asked for by name: requests that end inside a tile, inside a round of two tiles and inside a block of
     rows, contexts of a few thousand keys, a window with the pages behind it given back, the keys cut over blocks, and
     a far key that must not be missed.  (The 32-bit library has no such kernel and answers with its general one.)"""
     if dead_pages and window is None:
@@ -452,7 +452,7 @@ def test_attention_in_tiles_of_32_rows(dtype, splits, dead_pages, H, KV, hd, ps,
 @pytest.mark.parametrize("splits,dead_pages", [(0, False), (3, False), (0, True)])
 @pytest.mark.parametrize("H,KV,ps,window", [(28, 4, 64, None), (6, 2, 16, 100), (20, 1, 128, None), (8, 8, 32, 333), (3, 1, 16, 31)])
 def test_attention_in_tiles_of_32_rows_by_a_head_of_128(dtype, splits, dead_pages, H, KV, ps, window):
-    """The same kernel for a head size of 128: blocks of 64 flat rows, two LDS stages."""
+    """The same kernel for a head size of 128: one block to a work item, two blocks a CU, the reference always a row's maximum."""
     if dead_pages and window is None:
         pytest.skip("pages are given back behind a window only")
     seqs = [(0, 1), (0, 300), (517, 1), (3000, 37), (3, 2), (1023, 1), (128, 1), (127, 2), (31, 2), (95, 130), (2040, 19)]

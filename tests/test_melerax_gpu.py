@@ -364,7 +364,7 @@ def _attention_case(dtype, H, KV, hd, ps, before, now, seed, chunk, softcap, spi
 
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("chunk,softcap", [(16, 0.0), (7, 5.0), (64, 50.0), (100, 0.0), (0, 2.0), (1, 0.0)])
-@pytest.mark.parametrize("H,KV,hd", [(8, 2, 96), (6, 1, 32), (4, 4, 80), (17, 1, 32)])
+@pytest.mark.parametrize("H,KV,hd", [(8, 2, 96), (6, 1, 32), (4, 4, 80), (17, 1, 32), (14, 2, 64), (6, 2, 128), (3, 1, 64)])
 def test_attention_over_chunks_with_capped_scores(dtype, chunk, softcap, H, KV, hd):
     _attention_case(dtype, H, KV, hd, 16, [0, 5, 130], [150, 1, 9], 1, chunk, softcap)
     _attention_case(dtype, H, KV, hd, 16, [0, 5, 130], [40, 1, 9], 2, chunk, softcap, key_splits=3)

@@ -87,6 +87,42 @@ def test_the_part_gives_what_it_gives_over_every_expert(dtype, T, spec, monkeypa
     assert_close(got[0], got[1], dtype, str(spec))
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("T", [3, 200])
+@pytest.mark.parametrize("block", ["postnorm", "sandwich"])
+@pytest.mark.parametrize("top,shared", [(1, 0), (2, 64), (6, 64)])
+def test_the_norm_behind_the_experts(dtype, T, block, top, shared, monkeypatch):
+    """The feed-forward of a block whose norm stands behind it: the experts' planes (up to four, which that norm adds together with the
+    next one, and more) against the operands of one product."""
+    from machserve_amd.config import NormSpec, RoutedMlpSpec
+    from machserve_amd.kernels import get_ops
+    from machserve_amd.parts import FEED_FORWARDS, NORMS, Runtime
+    from machserve_amd.parts.base import ResidualStream
+    from machserve_amd.parts.block import PostNormBlock, SandwichBlock
+    ops, width, E, ff = get_ops(dtype, DEV), 128, 7, 64
+    g, rt = torch.Generator().manual_seed(T + top), Runtime(torch.device(DEV), dtype, ops)
+    rnd = lambda *s: torch.randn(*s, generator=g)  # noqa: E731
+    x, tensors, got = rnd(T, width).to(DEV), {}, []
+    pre, post, after = (NORMS.build(NormSpec("rmsnorm", width, 1e-5, {}), rt) for _ in range(3))
+    for norm in (pre, post, after):
+        norm.load({"weight": (1 + 0.1 * rnd(width)).to(DEV)})
+    for takes in (True, False):
+        monkeypatch.setattr(ops, "routed_experts_takes", lambda *a, takes=takes: takes)
+        part = FEED_FORWARDS.build(RoutedMlpSpec("routed_mlp", width, E, top, ff, "silu", shared, False, {}, gated=True), rt)
+        for d in part.tensor_decls():
+            if d.name not in tensors:
+                tensors[d.name] = (rnd(*d.shape) * 0.1).to(DEV, torch.float32 if d.role == "vector" else dtype)
+        part.load(tensors)
+        assert part.grouped == takes
+        kind = {"postnorm": PostNormBlock, "sandwich": SandwichBlock}[block]
+        own, stream = kind.__new__(kind), ResidualStream(x.clone(), ops)
+        own.rt = rt
+        own._branch(*([part, post] if block == "postnorm" else [pre, part, post]), stream, None)
+        got.append((after.forward(stream), stream.value()))
+    assert_close(got[0][0], got[1][0], dtype, "the next norm's rows")
+    assert_close(got[0][1], got[1][1], dtype, "the stream")
+
+
 @pytest.mark.parametrize("T", [1, 2, 63, 64])
 @pytest.mark.parametrize("shared", [0, 64])
 def test_a_step_of_few_rows_sets_no_more_activations_aside_than_its_rows_could_fill(T, shared):
