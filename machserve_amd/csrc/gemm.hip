@@ -111,23 +111,20 @@ static int launch_gemm(const elem_t* A, const elem_t* W, int M, int N, int K, Ep
     if (forced == 9) MS_GEMM(256, 256, 2, 4, 64);
     // What is left are products of at most 64 rows, and those whose last K step is not a whole one, which run in the loop of one
     // burst of loads a step: the largest tile that still gives every CU of the chip a block or two, with K steps of 64 (half
-    // the barriers of steps of 32).  The figures are that loop's with whole steps, which are planned above now; larger tiles under
-    // four waves (256x128) lose: their accumulators no longer fit the registers of two blocks a CU.
+    // the barriers of steps of 32).  The borders were found with whole steps in this loop, which are planned above now, and hold for
+    // partial ones: over 92 products (130 to 4,096 rows, 1,160 to 18,952 columns, K of 904, 1,544, 3,592, 4,872 and 9,000) the choice takes 1.03 times
+    // the best of 256x256, 128x128, 128x64 and 64x64 (1.26 at most: 130 rows of 9,736 columns, 17.6 us against 14.0 in 64x64), and each of these
+    // and 128x160 is the best somewhere.
     // two 128x128 blocks a CU are a round of the chip (512 on 256 CUs); a tile is taken when its blocks fill
     // six tenths of a round
     const long round_blocks = 2L * compute_units(), enough = round_blocks * 300 / 512;
     if (M > 64 && (ns == 1 || K >= 16384) && ep.k_per_split >= 128 && forced == 0) {
         // Tiles of 256x256 under eight waves (each 128 rows by 64 columns: 128 accumulator registers, 220 in all, two
         // waves a SIMD; 128 KB of LDS: one block a CU) bring half the bytes of two 128x128 tiles from the L2 into the CUs,
-        // which is what bounds the large products (every variant of the 128x128 loop pulls 13 to 15 TB/s).  They pay
-        // where the last of their rounds of one block a CU is well filled: measured against the choice below at the
-        // 0.5B, 1.5B and 7B layer sizes with 1,024 to 8,192 rows, +4 to +18 % from 0.72 of the rounds' blocks upwards
-        // (7B gate/up at 2,048 rows 604 -> 511 us, at 8,192 rows 2,167 -> 1,818 us = 1.22 PFLOP/s; 7B down at 4,096
-        // rows 588 -> 496), -15 to -44 % below 0.63; a short K (the 0.5B model's 896: fourteen steps between a tile's
-        // start and its 256x256 stores) wants the rounds fuller (0.95: +16 %; 0.89 - 1,536 and 3,072 rows of the 0.5B
-        // gate/up product - +24 and +7 %; 0.79: -5 to +6 %; 0.59: -20 %).  Three LDS stages
-        // (256x128, 128x256), four of K = 32 (256x256: 1.13 against 1.22 PFLOP/s) and four waves of 128x128 each with
-        // their sums in the accumulation registers (1.06) were slower than this.
+        // which is what bounds the large products.  They pay where the last of their rounds of one block a CU is well filled; a short K
+        // (few steps between a tile's start and its 256x256 stores) wants the rounds fuller.  us, 256x256 against 128x128: 4,096 x 18,952 x 1,544
+        // (1,200 tiles, 0.94 of five rounds) 275 and 354; 4,096 x 9,736 x 4,872 (0.81 of three) 418 and 488; 2,048 x 9,736 x 4,872
+        // (0.61 of two) 294 and 288; 1,024 x 4,616 x 4,872 (0.30 of one) 140 and 122.
         // (with K cut over `ns` blocks - a very long K under few tiles, see plan_tiled_splits - the slices fill the round)
         const long t256 = (long)ceil_div(M, 256) * ceil_div(N, 256) * ns, cus = compute_units();
         const long rounds = ceil_div(t256, cus);
@@ -137,9 +134,8 @@ static int launch_gemm(const elem_t* A, const elem_t* W, int M, int N, int K, Ep
         const long b128 = (long)ceil_div(M, 128) * ceil_div(N, 128), b12864 = (long)ceil_div(M, 128) * ceil_div(N, 64);
         // The chip holds a round of such blocks at a time and a round that is nearly empty takes as long as a full one:
         // the time is rounds times the tile's width.  Where tiles a quarter wider save more in rounds than they
-        // cost, they are taken (0.5B gate/up product at 2,048 rows: 1,216 tiles of 128x128 are two rounds and three
-        // eighths, 976 of 128x160 two rounds less a twentieth: 55 -> 45 us).  Tiles of 128x96 save rounds by the
-        // same count but lose more in themselves (8,192 rows: 16.3 against 15.7 ms for the whole prompt).
+        // cost, they are taken (2,048 x 9,736 x 4,872: 1,232 tiles of 128x128 are two rounds and four tenths, 976 of 128x160 two rounds less
+        // a twentieth: 288 -> 245 us; 2,048 x 4,616 x 4,872, one round and an eighth: 189 -> 128).
         if (ns == 1 && ep.k_per_split >= 128 && b128 >= enough) {
             const long rounds128 = ceil_div(b128, round_blocks), rounds160 = ceil_div((long)ceil_div(M, 128) * ceil_div(N, 160), round_blocks);
             if (rounds160 * 160 < rounds128 * 128) MS_GEMM(128, 160, 4, 1, 64);

@@ -2,7 +2,8 @@
 // (gemm.hip) and the products over the rows of routed experts (routed.hip) share.
 //
 // Both operands are contiguous along K, so a 16x32 MFMA fragment of either is "row
-// l % 16, elements (l / 16) * 8 .. + 8".  Two LDS buffers, one barrier per K step.  LDS has 64 banks
+// l % 16, elements (l / 16) * 8 .. + 8".  Two LDS buffers and one barrier a K step, three or four buffers with as many steps less one in
+// flight, or two buffers and two barriers in phases (GEMM_PIPED).  LDS has 64 banks
 // of 4 bytes; the 16-byte fragment reads of a wave are free of bank conflicts when the row pitch is
 // 32 modulo 64 bytes (measured: pitches of 80 or 144 bytes take twice as long), or, with unpadded
 // rows of 128 bytes, when chunk c of row r lies at position c ^ (r & 7).
