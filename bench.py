@@ -443,7 +443,8 @@ def compare_designs(args) -> int:
             slots = [lm.cache.admit() for _ in range(z["batch"])]
             for sl in slots:
                 lm.step([StepEntry(sl, toks(z["context"]), [])])
-            step = lambda: lm.step([StepEntry(sl, [1], [0]) for sl in slots], borrow_logits=True)
+            next_of = toks(z["batch"])  # unequal ones: equal tokens would share their choice of experts
+            step = lambda: lm.step([StepEntry(sl, [t], [0]) for sl, t in zip(slots, next_of)], borrow_logits=True)
             for _ in range(args.warmup + 2):
                 step()
             torch.cuda.synchronize()
