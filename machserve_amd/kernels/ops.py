@@ -1540,16 +1540,31 @@ class HipOps:
         self._want(state, torch.float32, "ssd state", state.shape[0], H, N, P)
         S = self._seq_operands("ssd", seq_q_start, seq_q_len, seq_slot)
         y = torch.empty((T, H * P), dtype=torch.float32, device=xbc.device)
-        seg, n_segs = self._walk_segments(T, S, self.SSD_SEGMENT, H * N * P)
-        carry = torch.empty((S, n_segs, H, N, P), dtype=torch.float32, device=xbc.device) if seg else None
-        cdec = torch.empty((S, n_segs, H), dtype=torch.float32, device=xbc.device) if seg else None
+        chunk = self._ssd_chunk(T, S, H, N)
+        work = None
+        if chunk:
+            lib.ms_ssd_chunk_floats.restype = ctypes.c_long
+            work = torch.empty(lib.ms_ssd_chunk_floats(_c_int(T), _c_int(S), _c_int(H), _c_int(P), _c_int(N), _c_int(G), _c_int(chunk)),
+                               dtype=torch.float32, device=xbc.device)
         self._check(lib, lib.ms_ssd_scan(_ptr(xbc), _c_int(xbc.shape[1]), _ptr(proj), _c_int(proj.shape[1]), _c_int(dt_col), _ptr(dt_bias),
                                          _ptr(a_log), _ptr(d_skip), _ptr(state), _ptr(seq_q_start), _ptr(seq_q_len), _ptr(seq_slot), _c_int(S),
-                                         _ptr(y), _c_int(T), _c_int(H), _c_int(P), _c_int(N), _c_int(G), _c_int(seg), _c_int(n_segs),
-                                         _ptr(carry), _ptr(cdec), self._stream()))
+                                         _ptr(y), _c_int(T), _c_int(H), _c_int(P), _c_int(N), _c_int(G), _c_int(chunk), _ptr(work),
+                                         self._stream()))
         return y
 
-    SSD_SEGMENT = 64  # rows of a segment of the state-space recurrence
+    SSD_SEGMENT = 128  # tokens of a chunk of the state-space recurrence
+    SSD_CHUNK_MIN_ROWS = 48  # steps with this many rows a request on average are cut into chunks
+
+    def _ssd_chunk(self, T: int, S: int, H: int, N: int) -> int:
+        """Tokens of a chunk for a step of ``T`` rows in ``S`` requests, 0: its requests are walked token by token.  A walk takes 2 us a
+        token and state of 128 whatever runs beside it, chunks 25 to 50 us a request that has the chip for itself: heads of 64 with 128
+        states, walked / in chunks, us: 64 heads, one request of 16 rows 51 / 27, of 128 264 / 46; sixteen requests of 32 rows 102 / 99,
+        of 48 140 / 120; 8 heads of 32 with 16 states, 32 rows 22 / 22, 48 rows 31 / 25.  The chunks' workspace is a state for every chunk:
+        with portions this long no more than a few times the layer's output."""
+        rows = T // S
+        least = min(self.SSD_CHUNK_MIN_ROWS, self.SCAN_CHUNK_MIN_ROWS // 2)
+        few = rows >= 16 and N >= 64 and S * H <= 256
+        return min(self.SSD_SEGMENT, T) if rows >= least or few else 0
 
     def gated_group_norm(self, y: torch.Tensor, proj: torch.Tensor, z_col: int, weight: torch.Tensor, eps: float, groups: int,
                          out_cols: int) -> torch.Tensor:

@@ -184,6 +184,36 @@ def test_state_space_recurrence_walked_in_segments(monkeypatch, dtype, H, P_, N,
     _ssd_case(dtype, H, P_, N, G, 1, lens, ([1000, 1000, 1000], [3 * seg - 1, 2, 4 * seg + 2], [2 * seg, 1, 2 * seg]))
 
 
+@pytest.mark.parametrize("H,P_,N,G,lens", [(2, 64, 128, 1, [128, 129, 127]), (6, 64, 64, 2, [1, 33, 257]), (5, 33, 65, 1, [96, 31, 160]), (2, 128, 256, 2, [130, 64])])
+def test_state_space_recurrence_in_chunks_at_their_edges(H, P_, N, G, lens):
+    """Chunks of 128 tokens in tiles of 32 by 32: requests that end on an edge of either, one short or one long of it; channels and states
+    that fill their tiles or do not."""
+    _ssd_case(torch.float32, H, P_, N, G, 1, lens, [lens, [max(n - 65, 1) for n in lens]])
+
+
+def test_a_later_token_s_overflow_stays_out_of_earlier_ones():
+    """x, B, C and the step size of a later token may be anything: the tokens before it in its chunk and the other requests keep their bits."""
+    ops = ops_of(torch.float32)
+    torch.manual_seed(3)
+    H, P_, N, lens, bad = 2, 64, 64, [100, 60], 37
+    inner, T = H * P_, sum(lens)
+    C = inner + 2 * N
+    proj, xbc = torch.randn(T, 2 * inner + 2 * N + H), torch.randn(T, C)
+    dt_bias, a_log, d_skip = torch.randn(H), torch.randn(H) * 0.5, torch.randn(H)
+    assert ops._ssd_chunk(T, 2, H, N)
+
+    def run(xbc, proj):
+        state = torch.zeros(2, H, N, P_, device=DEV)
+        return ops.ssd_scan(dev(xbc), dev(proj), inner + C, dev(dt_bias), dev(a_log), dev(d_skip), state, i32([0, 100]), i32(lens), i32([0, 1]), H, P_, N, 1).cpu()
+
+    want = run(xbc, proj)
+    for v in (float("inf"), float("nan"), 3e38):
+        x2, p2 = xbc.clone(), proj.clone()
+        x2[bad], p2[bad, inner + C:] = v, v
+        got = run(x2, p2)
+        assert torch.equal(got[:bad], want[:bad]) and torch.equal(got[100:], want[100:])
+
+
 def test_sizes_the_state_space_kernels_do_not_take_are_refused_when_the_part_is_built():
     from machserve_amd.config import StateSpaceDualSpec
     from machserve_amd.parts import MIXERS, Runtime
