@@ -5,6 +5,7 @@
 // kernels (crates/mach-model/src/kernels.rs:5772-5798, 6416-6455, 131-160).
 //
 // A block's loop over K and its epilogues are in gemm_tile.cuh; here are the choice of the tile and the entry points.
+#include "few_rows.cuh"
 #include "gemm_plan.h"
 #include "gemm_tile.cuh"
 
@@ -36,6 +37,8 @@ static int g_gemm_config = 0;  // 0: chosen by shape; else a fixed tile
 static constexpr int g_gemm_config = 0;
 #endif
 
+static int tiled_slices(int M, int N, int K);
+
 #ifdef MS_ELEM_HALF
 struct GemmPlan {
     int tile, splits;
@@ -58,6 +61,55 @@ static GemmPlan plan_gemm(int M, int N, int K, int splits, bool store32) {
         }
     }
     return best;
+}
+template <int MT, int NT, int STAGES, int EPI, bool SCALED>
+__global__ __launch_bounds__(64 * FEW_WAVES) void gemm_few_kernel(const elem_t* __restrict__ A, const elem_t* __restrict__ W, int M, int N, int K, EpiArgs ep) {
+    arguments_now(A, W, M, N, K, ep.out, ep.bias, ep.ldo, ep.n_out, ep.k_per_split, ep.split_stride);
+    if constexpr (SCALED) arguments_now(ep.row_ss, ep.ss_parts, ep.ss_eps);
+    if constexpr (EPI == EPI_PRENORM) arguments_now(ep.norm_w, ep.hn, ep.ss_part);
+    few_rows_tile<MT, NT, FEW_WAVES, STAGES, EPI, SCALED>(A, W, M, N, K, ep, 0, blockIdx.x * 16 * NT, blockIdx.y, NoExperts{});
+}
+
+template <int EPI, bool SCALED = false>
+static int launch_few(const elem_t* A, const elem_t* W, int M, int N, int K, const EpiArgs& ep, hipStream_t stream, int ns) {
+    constexpr bool PAIRS = EPI == EPI_SWIGLU;
+    const int rows = few_row_tiles(M), tile = plan_few(M, N, K, ns, PAIRS).tile;
+#define MS_FEW(ROWS_, TILE_)                                                                                                                          \
+    do {                                                                                                                                              \
+        constexpr FewCost t = kFew[ROWS_][TILE_];                                                                                                     \
+        if constexpr (!(PAIRS && t.nt == 1) && !(EPI == EPI_PRENORM && ROWS_ > 0)) {                                                                   \
+            hipLaunchKernelGGL((gemm_few_kernel<1 << ROWS_, t.nt, t.stages, EPI, SCALED>), dim3((unsigned)ceil_div(N, 16 * t.nt), (unsigned)ns),      \
+                               dim3(64 * FEW_WAVES), 0, stream, A, W, M, N, K, ep);                                                                   \
+            return check_launch("gemm, few rows");                                                                                                    \
+        }                                                                                                                                             \
+    } while (0)
+    if (rows == 0) {
+        if (tile == 0) MS_FEW(0, 0);
+        if (tile == 1) MS_FEW(0, 1);
+        MS_FEW(0, 2);
+    }
+    if (rows == 1) {
+        if (tile == 0) MS_FEW(1, 0);
+        if (tile == 1) MS_FEW(1, 1);
+        MS_FEW(1, 2);
+    }
+    if (tile == 0) MS_FEW(2, 0);
+    if (tile == 1) MS_FEW(2, 1);
+    MS_FEW(2, 2);
+#undef MS_FEW
+    MS_REQUIRE(false, "few-rows product: M=%d N=%d K=%d is not taken", M, N, K);
+}
+
+// Whether a product runs in few_rows.cuh, with K cut over several blocks (`slices`) or not: whole K steps, at least one for every wave, up to 16 rows; up to
+// 64 where it is predicted not to be slower than 64x64 tiles.  Their prediction (made for more rows) is an eighth short there: over 240
+// products of 32, 48 and 64 rows, cut and uncut, the choice takes 1.00 to 1.02 times the better of the two, which is 1.08 to 1.6 times as fast as the tiles.
+static bool few_rows(int M, int N, int K, bool slices, bool pairs) {
+    if (M > 64 || K % 64 != 0 || K < 64 * FEW_WAVES || g_gemm_config != 0) return false;
+    if (M <= 16) return true;
+    const int ns = slices ? tiled_slices(M, N, K) : 1, per = ceil_div(ceil_div(K, ns), 64) * 64;
+    const float tiled = fmaxf(tile_time(kTiles[TILE_64x64_DEEP], (long)ceil_div(N, 64) * ns, per, true), 2.5f + (float)N * (float)K * 4e-7f) +
+                        (float)(ns - 1) * (float)M * (float)N * (8.0f / 4.5e6f);
+    return plan_few(M, N, K, slices ? 0 : 1, pairs).us < 1.12f * tiled;
 }
 // products of more than 64 rows over whole K steps: what is planned as above
 static bool planned(int M, int K) { return M > 64 && K % 64 == 0 && g_gemm_config == 0; }
@@ -92,6 +144,7 @@ static int launch_gemm(const elem_t* A, const elem_t* W, int M, int N, int K, Ep
     } while (0)
 #ifdef MS_ELEM_HALF
     const int forced = g_gemm_config;
+    if (few_rows(M, N, K, ns > 1, EPI == EPI_SWIGLU)) return launch_few<EPI>(A, W, M, N, K, ep, stream, (int)ns);
     if (forced == 1) MS_GEMM(128, 128, 2, 2, 32);
     if (forced == 2) MS_GEMM(128, 128, 2, 2, 64);
     if (forced == 5) MS_GEMM(128, 64, 2, 2, 64);
@@ -181,7 +234,8 @@ static int g_force_splits = 0;
 static constexpr int g_force_splits = 0;
 #endif
 
-static int plan_tiled_splits(int M, int N, int K) {
+// K slices of a product in tiles.
+static int tiled_slices(int M, int N, int K) {
 #ifdef MS_ELEM_HALF
     const long b128 = (long)ceil_div(M, 128) * ceil_div(N, 128);
     const long round_blocks = 2L * compute_units();  // two 128x128 blocks a CU
@@ -237,6 +291,13 @@ static int plan_tiled_splits(int M, int N, int K) {
     (void)M; (void)N; (void)K;
     return 1;
 #endif
+}
+
+static int plan_tiled_splits(int M, int N, int K) {
+#ifdef MS_ELEM_HALF
+    if (g_force_splits == 0 && few_rows(M, N, K, true, false)) return plan_few(M, N, K, 0, false).splits;
+#endif
+    return tiled_slices(M, N, K);
 }
 
 }  // namespace ms
@@ -296,12 +357,44 @@ extern "C" int ms_linear_swiglu_scaled(const void* a, const float* row_ss, int s
     MS_REQUIRE((reinterpret_cast<uintptr_t>(a) & 15) == 0 && (reinterpret_cast<uintptr_t>(w) & 15) == 0, "gemm: operands must be 16-byte aligned");
     const int n = 2 * ceil_div(I, 16) * 16;
     EpiArgs ep{out, nullptr, I, I, K, 0, row_ss, ss_parts, eps, act};
+    if (few_rows(M, n, K, false, true)) return launch_few<EPI_SWIGLU, true>((const elem_t*)a, (const elem_t*)w, M, n, K, ep, stream, 1);
     hipLaunchKernelGGL((gemm_kernel<64, 64, 2, 2, 64, EPI_SWIGLU, 4, true>), dim3((unsigned)ceil_div(n, 64), 1), dim3(256), 0, stream,
                        (const elem_t*)a, (const elem_t*)w, M, n, K, ep);
     return check_launch("gemm 64x64x64 deep, row factors");
 #else
     (void)a; (void)row_ss; (void)ss_parts; (void)eps; (void)w; (void)out; (void)M; (void)I; (void)K; (void)act; (void)stream;
     MS_REQUIRE(false, "gated product with row factors: built for bfloat16 only");
+#endif
+}
+
+// Column tiles of ms_linear_residual_prenorm for this shape (the first size of its ss_part), or 0 if it is not taken: up to 16 rows over whole K steps,
+// uncut, where that takes no longer than the slices and the norm that would add them up (3 us: a launch and a trip to memory).
+extern "C" int ms_prenorm_parts(int M, int N, int K) {
+#ifdef MS_ELEM_HALF
+    if (!kRoundsBeforeTheNormIsSafe || M < 1 || M > 16 || !few_rows(M, N, K, false, false)) return 0;
+    return plan_few(16, N, K, 1, false).us < plan_few(16, N, K, 0, false).us + 2.5f ? ceil_div(N, 16) : 0;
+#else
+    (void)M; (void)N; (void)K;
+    return 0;
+#endif
+}
+
+// x[M, N] += a w^T, and beside it hn[M, N] = x * norm_w in the element type and ss_part[parts, M], whose sum over parts is the rows' sums of
+// squares of x (parts = ms_prenorm_parts).
+extern "C" int ms_linear_residual_prenorm(const void* a, const void* w, float* x, const float* norm_w, void* hn, float* ss_part, int M, int N, int K,
+                                          hipStream_t stream) {
+#ifdef MS_ELEM_HALF
+    MS_REQUIRE(ms_prenorm_parts(M, N, K) > 0, "product that prepares the norm: M=%d N=%d K=%d is not taken", M, N, K);
+    MS_REQUIRE(norm_w && hn && ss_part, "product that prepares the norm: its outputs are missing");
+    MS_REQUIRE((reinterpret_cast<uintptr_t>(a) & 15) == 0 && (reinterpret_cast<uintptr_t>(w) & 15) == 0, "gemm: operands must be 16-byte aligned");
+    EpiArgs ep{x, nullptr, N, N, K, 0};
+    ep.norm_w = norm_w;
+    ep.hn = (elem_t*)hn;
+    ep.ss_part = ss_part;
+    return launch_few<EPI_PRENORM>((const elem_t*)a, (const elem_t*)w, M, N, K, ep, stream, 1);
+#else
+    (void)a; (void)w; (void)x; (void)norm_w; (void)hn; (void)ss_part; (void)M; (void)N; (void)K; (void)stream;
+    MS_REQUIRE(false, "product that prepares the norm: built for bfloat16 only");
 #endif
 }
 
@@ -385,7 +478,19 @@ extern "C" int ms_tiled_tile(int M, int N, int K, int splits, int store32) {
 #endif
 }
 
-// Whether a product of M rows is better served by the tiled kernel than by the few-rows kernel (which
+// Whether the entry points of the tiled products run this product in few_rows.cuh (then they are the ones to call): `slices` if its reader adds up
+// K slices, `pairs` for the gated product.
+extern "C" int ms_few_rows_takes(int M, int N, int K, int slices, int pairs) {
+#ifdef MS_ELEM_HALF
+    return M >= 1 && N >= 1 && few_rows(M, N, K, slices != 0, pairs != 0);
+#else
+    (void)M; (void)N; (void)K; (void)slices; (void)pairs;
+    return 0;
+#endif
+}
+
+// Of the products that few_rows.cuh does not take (a K that is no whole number of steps, 17 to 64 rows of some shapes, 32-bit), and of norms that could be
+// folded in: whether a product of M rows is better served by the tiled kernel than by the one of skinny.hip (which
 // takes at most 64 rows).  The few-rows kernel reads its rows again for every 32 or 64 columns; with
 // many rows and a large weight that traffic outweighs the weight itself, and the tiled kernel, which
 // shares the rows of a block through LDS, streams the weight faster (measured at the 0.5B, 1.5B and 7B

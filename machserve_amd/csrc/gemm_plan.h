@@ -38,4 +38,48 @@ static inline float tile_time(const TileCost& t, long blocks, int k_per_split, b
     return us;
 }
 
+// Products of few rows (few_rows.cuh: four waves that share out K).  A block of `nt` tiles of 16 columns takes `step[n]` us for each of a wave's K steps
+// where n + 1 such blocks share a CU, `slope` more of it in proportion as the chip is full; the product takes `start` and `per_mb` for each MB of the weight.
+// A fit (non-negative least squares, 6 to 9 % off) to 672 products of 1 to 16 rows and 224 each of 32 and 64: 40 weights of 160 to 151,936 columns and
+// K of 320 to 18,944, cold, in one to eight slices.  The choice of tiles and slices takes 1.01 (uncut) and 1.025 times the best measured.
+struct FewCost {
+    int nt, stages, per_cu;
+    float step[3], slope, start, per_mb;
+};
+constexpr int FEW_WAVES = 4, FEW_TILES = 3;
+static constexpr FewCost kFew[3][FEW_TILES] = {  // up to 16, 32 and 64 rows
+    {{1, 3, 3, {0.148f, 0.239f, 0.280f}, 0.254f, 2.32f, 0.141f}, {2, 3, 2, {0.212f, 0.374f}, 0.354f, 2.34f, 0.144f}, {4, 2, 2, {0.440f, 0.797f}, 0.344f, 2.28f, 0.136f}},
+    {{1, 3, 2, {0.261f, 0.436f}, 0.557f, 2.21f, 0.149f}, {2, 2, 2, {0.358f, 0.620f}, 0.483f, 2.34f, 0.143f}, {4, 2, 1, {0.646f}, 1.792f, 2.50f, 0.118f}},
+    {{1, 2, 2, {0.406f, 0.717f}, 0.604f, 2.26f, 0.167f}, {2, 2, 1, {0.595f}, 1.792f, 2.52f, 0.114f}, {4, 2, 1, {0.935f}, 3.220f, 3.42f, 0.101f}},
+};
+static inline int few_row_tiles(int M) { return M <= 16 ? 0 : M <= 32 ? 1 : 2; }
+static inline float few_time(const FewCost& t, long blocks, int k_per_split, long N, long K) {
+    const long cus = compute_units(), round = cus * t.per_cu, full = blocks / round, rest = blocks % round;
+    const float steps = (float)ceil_div(k_per_split, 64 * FEW_WAVES);
+    float us = t.start + (float)(N * K) * 2e-6f * t.per_mb + (float)full * steps * (t.step[t.per_cu - 1] + t.slope);
+    if (rest) us += steps * (t.step[ceil_div(rest, cus) - 1] + t.slope * (float)rest / (float)round);
+    return us;
+}
+struct FewPlan {
+    int tile, splits;
+    float us;
+};
+// The best tile for `splits` slices, or, with splits == 0, the best tile and number of slices (a plane of sums more is written and read again, and
+// no slice is shorter than a step for every wave).  `pairs`: gate and up columns lie side by side.  Up to 32 rows the slices are those of 16, so that a row's
+// sums do not depend on how many rows come with it.
+static inline FewPlan plan_few(int M, int N, int K, int splits, bool pairs) {
+    if (splits == 0 && M <= 32 && M != 16) return plan_few(M, N, K, plan_few(16, N, K, 0, pairs).splits, pairs);
+    FewPlan best{0, 1, INFINITY};
+    for (int s = splits ? splits : 1; s <= (splits ? splits : 8); ++s) {
+        const int per = ceil_div(ceil_div(K, s), 64) * 64;
+        if (splits == 0 && s > 1 && (ceil_div(K, per) != s || per < 64 * FEW_WAVES)) continue;
+        for (int i = pairs ? 1 : 0; i < FEW_TILES; ++i) {
+            const FewCost& t = kFew[few_row_tiles(M)][i];
+            const float us = few_time(t, (long)ceil_div(N, 16 * t.nt) * s, per, N, K) + (float)(s - 1) * (float)M * (float)N * (8.0f / 4.5e6f);
+            if (us < best.us) best = {i, s, us};
+        }
+    }
+    return best;
+}
+
 }  // namespace ms

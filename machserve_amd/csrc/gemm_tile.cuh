@@ -35,6 +35,7 @@ constexpr int GEMM_PIPED = 1;  // in the place of a number of LDS buffers: two o
 enum EpiKind {
     EPI_STORE_F32 = 0, EPI_STORE_ELEM = 1, EPI_RESIDUAL = 2, EPI_SWIGLU = 3, EPI_QKV_ROPE = 4, EPI_ACT = 5,
     EPI_EXPERT_GATED = 6, EPI_EXPERT_PLAIN = 7, EPI_EXPERT_DOWN = 8,  // over the rows that chose an expert (routed.hip)
+    EPI_PRENORM = 9,  // few rows only (few_rows.cuh): into the residual stream, and what the norm that follows needs
 };
 
 struct NoExperts {
@@ -65,6 +66,11 @@ struct EpiArgs {
     elem_t* kpool;         // [pages, KV, ps, hd]
     elem_t* vpool;         // [pages, KV, hd, ps]
     int H, KV, ps;
+    // PRENORM: the new values of the stream times the norm's weight, not yet divided by the rows' root mean square, and each tile's 16 columns' share of
+    // the rows' sums of squares
+    const float* norm_w;  // [N]
+    elem_t* hn;           // [M, N]
+    float* ss_part;       // [N / 16, M]
 };
 
 // The block of rows m0 .. m0 + BM and columns n0 .. n0 + BN.  `rows` says which row of A the block's row i is and, for the

@@ -632,6 +632,7 @@ extern "C" int ms_linear_act_skinny(const void* a, const void* w, void* out, int
 // its own instructions, not by memory.)
 extern "C" int ms_swiglu_scaled_skinny_takes(int M, int I, int K) {
     if (!kHalf || !kRoundsBeforeTheNormIsSafe || M < 1 || M > 16 || K % 8) return 0;
+    if (K % 64 == 0 && K >= 256) return 0;  // few_rows.cuh
     const int n = 2 * ceil_div(I, 16) * 16;
     const SkinnyPlan p = plan_skinny(M, n, K, false, true);
     return ceil_div(n, 32 * p.wn) * p.wn * p.ksi <= 16 * compute_units();  // sixteen waves a CU

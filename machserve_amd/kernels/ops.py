@@ -271,18 +271,23 @@ class HipOps:
         return v
 
     def _tiled(self, M: int, N: int, K: int) -> bool:
-        """Whether the tiled kernel takes this product: always above SKINNY_ROWS rows; below, where it was
-        measured faster (in bfloat16 every large weight from one row on, because its blocks stream the
+        """Whether the tiled kernel is before the weight-streaming ones of ``skinny.hip`` for this product: always above SKINNY_ROWS
+        rows; below, where it was measured faster (in bfloat16 every large weight from one row on, because its blocks stream the
         weight with several K steps in flight, and smaller ones from 8 to 32 rows on; never in 32-bit)."""
         return M > self.SKINNY_ROWS or bool(self._plan("ms_prefers_tiled", M, N, K))
+
+    def _few(self, M: int, N: int, K: int, slices: bool, pairs: bool = False) -> bool:
+        """Whether this product of at most 64 rows runs in ``few_rows.cuh``, through the entry points of the tiled products
+        (two-byte elements, whole K steps, up to 16 rows always)."""
+        return M <= self.SKINNY_ROWS and bool(self._plan("ms_few_rows_takes", M, N, K, int(slices), int(pairs)))
 
     def linear_split(self, a: torch.Tensor, w: torch.Tensor, allow_partials: bool = True) -> torch.Tensor:
         """Float32 ``[P, M, N]`` whose sum over P is ``a @ w.T``.  Within one kernel family the cut
         of K depends on N and K only, so the consumer that adds the parts sees the same sums for a row
         whatever else is in the batch; which family runs depends on the number of rows (see
-        :meth:`_tiled`), and the two differ in rounding."""
+        :meth:`_few` and :meth:`_tiled`), and they differ in rounding."""
         M, N, K = self._mm_operands(a, w, "linear_split")
-        if self._tiled(M, N, K):
+        if self._few(M, N, K, allow_partials) or self._tiled(M, N, K):
             P = self._plan("ms_tiled_partials", M, N, K) if allow_partials else 1
             if P == 1:
                 return self.linear(a, w, None, out_f32=True).unsqueeze(0)
@@ -300,7 +305,7 @@ class HipOps:
                out_f32: bool = False) -> torch.Tensor:
         """``a @ w.T (+ bias)``; 32-bit output on request (logits)."""
         M, N, K = self._mm_operands(a, w, "linear")
-        if not self._tiled(M, N, K) and out_f32 and bias is None:
+        if not self._few(M, N, K, False) and not self._tiled(M, N, K) and out_f32 and bias is None:
             return self.linear_split(a, w, allow_partials=False)[0]
         if bias is not None:
             self._want(bias, torch.float32, "linear bias", N)
@@ -316,7 +321,7 @@ class HipOps:
         in; otherwise None."""
         M, N, K = self._mm_operands(a, w, "linear_residual")
         self._want(x, torch.float32, "residual stream", M, N)
-        if not self._tiled(M, N, K):
+        if not self._few(M, N, K, True) and not self._tiled(M, N, K):
             if M > 32 or self._plan("ms_skinny_partials", M, N, K, 1) > 1:
                 return self.linear_split(a, w)
             # all of K inside one block: one writer an element, added in the epilogue (up to 32 rows the
@@ -335,7 +340,7 @@ class HipOps:
         interleaved weight of ``n_gate_up`` rows can run as two kernels without a norm between them: the
         first leaves ``x * norm_w`` and the rows' sums of squares beside the sum, the second divides its
         finished sums by the root mean square (:meth:`linear_residual_prenorm`, :meth:`linear_swiglu_scaled`)."""
-        return (not self._tiled(M, N, K) and self._plan("ms_skinny_prenorm_parts", M, N, K) > 0
+        return ((self._plan("ms_prenorm_parts", M, N, K) > 0 or (not self._tiled(M, N, K) and self._plan("ms_skinny_prenorm_parts", M, N, K) > 0))
                 and bool(self._plan("ms_swiglu_scaled_takes", M, n_gate_up // 2, N)
                          or self._plan("ms_swiglu_scaled_skinny_takes", M, n_gate_up // 2, N)))
 
@@ -345,13 +350,14 @@ class HipOps:
         M, N, K = self._mm_operands(a, w, "linear_residual_prenorm")
         self._want(x, torch.float32, "residual stream", M, N)
         self._want(norm_w, torch.float32, "norm weight", N)
-        parts = self._plan("ms_skinny_prenorm_parts", M, N, K)
+        parts, fn = self._plan("ms_prenorm_parts", M, N, K), self._core.ms_linear_residual_prenorm
+        if parts < 1:
+            parts, fn = self._plan("ms_skinny_prenorm_parts", M, N, K), self._core.ms_linear_residual_prenorm_skinny
         if parts < 1:
             raise KernelError(f"linear_residual_prenorm: M={M} N={N} K={K} is not taken")
         hn = torch.empty((M, N), dtype=self.dtype, device=a.device)
         ss = torch.empty((parts, M), dtype=torch.float32, device=a.device)
-        self._check(self._core, self._core.ms_linear_residual_prenorm_skinny(
-            _ptr(a), _ptr(w), _ptr(x), _ptr(norm_w), _ptr(hn), _ptr(ss), _c_int(M), _c_int(N), _c_int(K), self._stream()))
+        self._check(self._core, fn(_ptr(a), _ptr(w), _ptr(x), _ptr(norm_w), _ptr(hn), _ptr(ss), _c_int(M), _c_int(N), _c_int(K), self._stream()))
         return hn, ss
 
     def linear_swiglu_scaled(self, hn: torch.Tensor, row_ss: torch.Tensor, eps: float, w_gate_up: torch.Tensor,
@@ -379,7 +385,8 @@ class HipOps:
         if N != 2 * ((intermediate + 15) // 16) * 16:
             raise KernelError(f"linear_swiglu: interleaved weight has {N} rows for intermediate size {intermediate}")
         out = torch.empty((M, intermediate), dtype=self.dtype, device=a.device)
-        fn = self._core.ms_linear_swiglu if self._tiled(M, N, K) else self._core.ms_linear_swiglu_skinny
+        tiled = self._few(M, N, K, False, True) or self._tiled(M, N, K)
+        fn = self._core.ms_linear_swiglu if tiled else self._core.ms_linear_swiglu_skinny
         self._check(self._core, fn(_ptr(a), _ptr(w_gate_up), _ptr(out), _c_int(M), _c_int(intermediate), _c_int(K),
                                    _c_int(act), self._stream()))
         return out
@@ -390,7 +397,7 @@ class HipOps:
             raise KernelError(f"linear_act: activation {activation!r} is not built (built: {', '.join(sorted(UNARY_ACTIVATIONS))})")
         M, N, K = self._mm_operands(a, w, "linear_act")
         out = torch.empty((M, N), dtype=self.dtype, device=a.device)
-        fn = self._core.ms_linear_act if self._tiled(M, N, K) else self._core.ms_linear_act_skinny
+        fn = self._core.ms_linear_act if self._few(M, N, K, False) or self._tiled(M, N, K) else self._core.ms_linear_act_skinny
         self._check(self._core, fn(_ptr(a), _ptr(w), _ptr(out), _c_int(M), _c_int(N), _c_int(K), _c_int(UNARY_ACTIVATIONS[activation]),
                                    self._stream()))
         return out

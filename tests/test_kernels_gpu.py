@@ -904,3 +904,44 @@ def test_qkv_product_that_rotates_and_writes_the_cache(dtype, M, H, KV, hd, K, p
     keep = (~written).view(pages, ps)
     assert torch.equal(kp2.cpu().permute(0, 2, 1, 3)[keep], kp0.permute(0, 2, 1, 3)[keep])
     assert torch.equal(vp2.cpu().permute(0, 3, 1, 2)[keep], vp0.permute(0, 3, 1, 2)[keep])
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("M", [1, 8, 9, 16, 17, 32, 33, 64])
+@pytest.mark.parametrize("N,K", [(16, 256), (1000, 320), (200, 4160), (5632, 1024), (40, 16384), (20000, 576)])
+def test_products_whose_waves_share_out_k(dtype, M, N, K):
+    """Few rows over whole K steps: one step a wave, waves with unequal numbers of steps, outputs that end inside a tile, one to many blocks a
+    CU, with and without slices of K; every epilogue.  The sums are 32-bit: what differs from 64 bits is the order (1e-6 of the terms' size)."""
+    from machserve_amd.kernels import interleave_gate_up
+    ops = ops_for(dtype)
+    a, w, bias = rnd((M, K), dtype, 71), rnd((N, K), dtype, 72, K ** -0.5), rnd((N,), torch.float32, 73)
+    ref = P.linear(a.double(), w.double())
+    ad, wd = a.to(DEV), w.to(DEV)
+    if M <= 16:
+        assert ops._few(M, N, K, True) and ops._few(M, N, K, False)
+    parts = ops.linear_split(ad, wd)
+    assert_close(parts.sum(0), ref, dtype, "slices")
+    assert_close(ops.linear(ad, wd, None, out_f32=True), ref, dtype, "whole")
+    assert_close(ops.linear(ad, wd, bias.to(DEV)), ref + bias.double(), dtype, "with a bias, in the element type")
+    assert_close(ops.linear_act(ad, wd, "relu2"), torch.relu(ref) ** 2, dtype, "activation")
+    x0 = rnd((M, N), torch.float32, 74)
+    x = x0.to(DEV)
+    pend = ops.linear_residual(ad, wd, x)
+    assert_close(x.cpu() - x0 if pend is None else pend.sum(0), ref, dtype, "into the stream")
+    g, u = rnd((N // 2 + 3, K), dtype, 75, 2 * K ** -0.5), rnd((N // 2 + 3, K), dtype, 76, K ** -0.5)
+    gated = P.silu(P.linear(a.double(), g.double())) * P.linear(a.double(), u.double())
+    gu = interleave_gate_up(g, u).to(DEV)
+    assert_close(ops.linear_swiglu(ad, gu, N // 2 + 3), gated, dtype, "gated")
+    if M <= 16 and ops._few(M, N, K, True) and parts.shape[0] == ops.linear_split(ad[:1].contiguous(), wd).shape[0]:
+        assert torch.equal(parts[:, :1], ops.linear_split(ad[:1].contiguous(), wd)), "a row's sums do not depend on the other rows"
+    if dtype == torch.bfloat16 and ops._plan("ms_prenorm_parts", M, N, K):
+        xd, nw = x0.to(DEV).clone(), 1 + rnd((N,), torch.float32, 77, 0.1)
+        hn, ss = ops.linear_residual_prenorm(ad, wd, xd, nw.to(DEV))
+        assert_close(xd, x0.double() + ref, dtype, "stream")
+        assert_close(hn, xd.cpu().double() * nw.double(), dtype, "stream times the norm's weight")
+        assert_close(ss.sum(0), (xd.cpu().double() ** 2).sum(1), torch.float32, "sums of squares")
+    if dtype == torch.bfloat16 and ops._plan("ms_swiglu_scaled_takes", M, N // 2 + 3, K):
+        share = rnd((5, M), torch.float32, 78).abs() * K
+        f = 1.0 / torch.sqrt(share.double().sum(0) / K + 1e-5)[:, None]
+        scaled = P.silu(P.linear(a.double(), g.double()) * f) * (P.linear(a.double(), u.double()) * f)
+        assert_close(ops.linear_swiglu_scaled(ad, share.to(DEV), 1e-5, gu, N // 2 + 3), scaled, dtype, "gated with row factors")
