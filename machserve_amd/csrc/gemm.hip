@@ -45,13 +45,13 @@ struct GemmPlan {
 };
 // The best tile for `splits` slices, or, with splits == 0, the best tile and number of slices: a slice more is a plane of sums more to
 // write and to read again (4.5 TB/s), and never less than three K steps.
-static GemmPlan plan_gemm(int M, int N, int K, int splits, bool store32) {
+static GemmPlan plan_gemm(int M, int N, int K, int splits, bool store32, bool gated = false) {
     GemmPlan best{0, max(1, splits)};
     float best_us = INFINITY;
     for (int s = splits ? splits : 1; s <= (splits ? splits : 6); ++s) {
         const int per = ceil_div(ceil_div(K, s), 64) * 64;
         if (splits == 0 && s > 1 && (ceil_div(K, per) != s || per < 192)) continue;
-        for (int i = 0; i < TILE_COUNT; ++i) {
+        for (int i = 0; i < (gated ? TILE_COUNT_GATED : TILE_COUNT); ++i) {
             const long blocks = (long)ceil_div(M, kTiles[i].bm) * ceil_div(N, kTiles[i].bn) * s;
             const float us = tile_time(kTiles[i], blocks, per, store32) + (float)(s - 1) * (float)M * (float)N * (8.0f / 4.5e6f);
             if (us < best_us) {
@@ -151,7 +151,9 @@ static int launch_gemm(const elem_t* A, const elem_t* W, int M, int N, int K, Ep
     if (forced == 6) MS_GEMM(64, 64, 2, 2, 64);
     const bool whole_steps = ep.k_per_split % 64 == 0 && K % 64 == 0;
     if (planned(M, K)) {
-        switch (plan_gemm(M, N, K, (int)ns, EPI == EPI_STORE_F32 || EPI == EPI_RESIDUAL).tile) {
+        switch (plan_gemm(M, N, K, (int)ns, EPI == EPI_STORE_F32 || EPI == EPI_RESIDUAL, EPI == EPI_SWIGLU).tile) {
+            case TILE_256x320:
+                if constexpr (EPI == EPI_SWIGLU) MS_GEMM_DEEP(256, 320, 2, 4, 64, GEMM_PIPED);
             case TILE_256x256: MS_GEMM_DEEP(256, 256, 2, 4, 64, GEMM_PIPED);
             case TILE_256x192: MS_GEMM_DEEP(256, 192, 4, 2, 64, GEMM_PIPED);
             case TILE_256x128: MS_GEMM_DEEP(256, 128, 4, 2, 64, GEMM_PIPED);
@@ -474,6 +476,16 @@ extern "C" int ms_tiled_tile(int M, int N, int K, int splits, int store32) {
     return planned(M, K) ? plan_gemm(M, N, K, max(1, splits), store32 != 0).tile : -1;
 #else
     (void)M; (void)N; (void)K; (void)splits; (void)store32;
+    return -1;
+#endif
+}
+
+// The same of a gated product of `N` columns, gate and up.
+extern "C" int ms_gated_tile(int M, int N, int K) {
+#ifdef MS_ELEM_HALF
+    return planned(M, K) ? plan_gemm(M, N, K, 1, false, true).tile : -1;
+#else
+    (void)M; (void)N; (void)K;
     return -1;
 #endif
 }

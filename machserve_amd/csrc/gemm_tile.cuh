@@ -88,6 +88,10 @@ __device__ __forceinline__ void gemm_tile(const elem_t* __restrict__ A, const el
 #endif
     constexpr bool PIPED = STAGES == GEMM_PIPED;
     constexpr int BUFS = PIPED ? 2 : STAGES;
+    // Tiles of more than 256 columns (256x320 under eight waves of 128x80: 160 registers of sums and 72 of fragments) have no register to spare for a lane's
+    // offsets into the operands: rows of W go in eights with a scalar base (N is a multiple of 8), those of A are worked out at each load.
+    constexpr bool WIDE = BN > 256;
+    static_assert(!WIDE || (PIPED && !Rows::GATHERS), "wide tiles: in phases, rows as they come");
     constexpr int LDS_LD = DIRECT ? BK : BK + KPAD;
     constexpr int CPR = BK / EPC;  // chunks per tile row
     // where chunk `chunk` of tile row `row` lies in a buffer
@@ -184,17 +188,26 @@ __device__ __forceinline__ void gemm_tile(const elem_t* __restrict__ A, const el
     const elem_t* base_a = A + (size_t)rows.source(m0) * rows.pitch(K);
     const elem_t* base_w = W + (size_t)n0 * rows.w_pitch(K);
     uint32_t oa[A_CHUNKS], ow[W_CHUNKS];
+    // (a product of 32 bits is made in 64, and its upper half would keep a register)
+    auto alone = [](uint32_t x) {
+        uint32_t y;
+        asm("v_mov_b32 %0, %1" : "=v"(y) : "v"(x));
+        return y;
+    };
+    auto a_offset = [&](int row) {  // of row m0 + `row`, or the last one
+        return ((uint32_t)min(row, M - 1 - m0) * (uint32_t)rows.pitch(K) + my_chunk * EPC) * (uint32_t)sizeof(elem_t);
+    };
     const elem_t* ga[Rows::GATHERS ? A_CHUNKS : 1];
     if constexpr (DIRECT) {
 #pragma unroll
         for (int i = 0; i < A_CHUNKS; ++i) {
-            const int m = min(m0 + a_row(i) + lane / 8, M - 1);
-            if constexpr (Rows::GATHERS) ga[i] = A + (size_t)rows.source(m) * rows.pitch(K) + my_chunk * EPC;
-            else oa[i] = ((uint32_t)(m - m0) * (uint32_t)rows.pitch(K) + my_chunk * EPC) * (uint32_t)sizeof(elem_t);
+            if constexpr (Rows::GATHERS) ga[i] = A + (size_t)rows.source(min(m0 + a_row(i) + lane / 8, M - 1)) * rows.pitch(K) + my_chunk * EPC;
+            else oa[i] = alone(a_offset(a_row(i) + lane / 8));
         }
 #pragma unroll
         for (int i = 0; i < W_CHUNKS; ++i)
-            ow[i] = ((uint32_t)(min(n0 + (tid + i * NT) / CPR, N - 1) - n0) * (uint32_t)rows.w_pitch(K) + my_chunk * EPC) * (uint32_t)sizeof(elem_t);
+            ow[i] = alone(((uint32_t)(WIDE ? lane / 8 : min(n0 + (tid + i * NT) / CPR, N - 1) - n0) * (uint32_t)rows.w_pitch(K) + my_chunk * EPC) *
+                          (uint32_t)sizeof(elem_t));
     }
     // load l of a step: A's rounds, then W's
     auto load_one = [&](int k0, int buf, int l) {
@@ -203,11 +216,12 @@ __device__ __forceinline__ void gemm_tile(const elem_t* __restrict__ A, const el
             if constexpr (Rows::GATHERS)
                 asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(ga[l] + k0), "s"(to) : "memory", "m0");
             else
-                asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(oa[l]), "s"(base_a + k0), "s"(to) : "memory", "m0");
+                asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(WIDE ? a_offset(a_row(l) + opaque(lane) / 8) : oa[l]), "s"(base_a + k0), "s"(to) : "memory", "m0");
         } else {
             const int i = l - A_CHUNKS;
             const uint32_t to = lds_w + buf * (BN * LDS_LD * (int)sizeof(elem_t)) + (i * (NT / 8) + swave * 8) * (LDS_LD * (int)sizeof(elem_t));
-            asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(ow[i]), "s"(base_w + k0), "s"(to) : "memory", "m0");
+            const elem_t* from = WIDE ? W + (size_t)min(n0 + i * (NT / 8) + swave * 8, N - 8) * rows.w_pitch(K) : base_w;
+            asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(ow[WIDE ? 0 : i]), "s"(from + k0), "s"(to) : "memory", "m0");
         }
     };
     auto load_direct = [&](int k0, int buf) {
@@ -225,6 +239,14 @@ __device__ __forceinline__ void gemm_tile(const elem_t* __restrict__ A, const el
             __syncthreads();
         }
     };
+
+    // The first column of a wave's tile j.  Gate and up tiles alternate; where a wave has an odd number of them, the last is an even wave's
+    // gate tile and the next wave's up tile to it.
+    constexpr bool SPLIT_PAIR = EPI == EPI_SWIGLU && TN % 2 != 0;
+    static_assert(!SPLIT_PAIR || (PIPED && WN % 2 == 0), "a pair between two waves: in phases");
+    const bool second = SPLIT_PAIR && (swave & 1);
+    const int col_first = wn * (BN / WN) + (second ? 16 : 0), col_last = wn * (BN / WN) + (second ? 0 : (TN - 1) * 16);
+    auto tile_col = [&](int j) { return SPLIT_PAIR && j == TN - 1 ? col_last : col_first + j * 16; };
 
     f32x4 acc[TM][TN];
 #pragma unroll
@@ -286,11 +308,20 @@ __device__ __forceinline__ void gemm_tile(const elem_t* __restrict__ A, const el
         static_assert(TM % 2 == 0 && A_CHUNKS % 2 == 0, "a wave's rows in two halves");
         constexpr int TH = TM / 2;
         Frag fa[2][TH], fb[2][TN];
-        auto fetch_a = [&](int buf, int p, int i) {
-            fa[p & 1][i] = frag_load(&As[buf][at(wm * (BM / WM) + (p / 2 * TH + i) * 16 + r16, (p & 1) * (32 / EPC) + grp)]);
+        // A lane's places in the tiles' first rows, for both K chunks: the others are constants further (rows 16 apart are swizzled alike).
+        int lane_a[2], lane_b[2];
+#pragma unroll
+        for (int kk = 0; kk < 2; ++kk) {
+            lane_a[kk] = (int)opaque((uint32_t)at(wm * (BM / WM) + r16, kk * (32 / EPC) + grp));
+            lane_b[kk] = (int)opaque((uint32_t)at(col_first + r16, kk * (32 / EPC) + grp));
+        }
+        const int last_b = col_last - col_first;
+        auto fetch_a = [&](int buf, int half, int kk, int to, int i) {
+            fa[to][i] = frag_load(&As[0][lane_a[kk] + (WIDE ? 0 : buf * BM * LDS_LD) + (half * TH + i) * 16 * LDS_LD]);
         };
         auto fetch_b = [&](int buf, int kk, int j) {
-            fb[kk][j] = frag_load(&Ws[buf][at(wn * (BN / WN) + j * 16 + r16, kk * (32 / EPC) + grp)]);
+            const int at_j = SPLIT_PAIR && j == TN - 1 ? last_b * LDS_LD : j * 16 * LDS_LD;
+            fb[kk][j] = frag_load(&Ws[0][lane_b[kk] + (WIDE ? 0 : buf * BN * LDS_LD) + at_j]);
         };
         constexpr int PER_STEP = A_CHUNKS + W_CHUNKS, EARLY = W_CHUNKS + A_CHUNKS / 2;
         static_assert(PER_STEP <= 63, "the wait count is a 6-bit field");
@@ -309,7 +340,7 @@ __device__ __forceinline__ void gemm_tile(const elem_t* __restrict__ A, const el
             for (int l = 0; l < PER_STEP; ++l) load_nth(k_begin + BK, 1, l);
         arrive(nk > 1);
 #pragma unroll
-        for (int i = 0; i < TH; ++i) fetch_a(0, 0, i);
+        for (int i = 0; i < TH; ++i) fetch_a(0, 0, 0, 0, i);
 #pragma unroll
         for (int j = 0; j < TN; ++j) fetch_b(0, 0, j);
         constexpr int GR = TH * TN % 4 == 0 ? 4 : 2, GROUPS = TH * TN / GR;  // matrix instructions in groups, each with its share of reads and loads ahead
@@ -320,6 +351,14 @@ __device__ __forceinline__ void gemm_tile(const elem_t* __restrict__ A, const el
             for (int p = 0; p < 4; ++p) {
                 const int np = (p + 1) & 3, nbuf = p == 3 ? buf ^ 1 : buf;  // (behind the last step: what is left there, and not used)
                 const int reads = TH + (np < 2 ? TN : 0);
+                if (WIDE && p == 3) {  // to the other buffer
+                    const int turn = buf ? -1 : 1;
+#pragma unroll
+                    for (int kk = 0; kk < 2; ++kk) {
+                        lane_a[kk] += turn * BM * LDS_LD;
+                        lane_b[kk] += turn * BN * LDS_LD;
+                    }
+                }
                 // phase 1: the second half's rows of this step have come; phase 3: W and the first half's rows of the next one
                 if (p == 1) arrive(kt + 1 < nk);
                 if (p == 3) arrive(more);
@@ -329,7 +368,7 @@ __device__ __forceinline__ void gemm_tile(const elem_t* __restrict__ A, const el
 #pragma unroll
                     for (int r = 0; r < TH + TN; ++r) {
                         if (r >= reads || r * GROUPS / reads != g) continue;
-                        if (r < TH) fetch_a(nbuf, np, r);
+                        if (r < TH) fetch_a(nbuf, np / 2, np & 1, np & 1, r);
                         else fetch_b(nbuf, np, r - TH);
                     }
 #pragma unroll
@@ -342,11 +381,16 @@ __device__ __forceinline__ void gemm_tile(const elem_t* __restrict__ A, const el
             }
         };
         int kt = 0;
-        for (; kt + 1 < nk; kt += 2) {
-            step(kt, 0);
-            step(kt + 1, 1);
+        if constexpr (WIDE) {  // one body for both buffers
+#pragma unroll 1
+            for (; kt < nk; ++kt) step(kt, kt & 1);
+        } else {
+            for (; kt + 1 < nk; kt += 2) {
+                step(kt, 0);
+                step(kt + 1, 1);
+            }
+            if (kt < nk) step(kt, 0);
         }
-        if (kt < nk) step(kt, 0);
 #endif
     } else if constexpr (DIRECT && STAGES > 2) {
         // A block that is alone on its CU (few tiles: one tile of rows under a weight of a few hundred column
@@ -439,13 +483,23 @@ __device__ __forceinline__ void gemm_tile(const elem_t* __restrict__ A, const el
     const int row_base = m0 + wm * (BM / WM) + grp * 4;
     const int col_base = n0 + wn * (BN / WN) + r16;
     const bool whole = m0 + BM <= M && n0 + BN <= N && (EPI != EPI_SWIGLU || (n0 + BN) / 2 <= ep.n_out);
+    f32x4* over = nullptr;
+    f32x4 last_up;
+    if constexpr (SPLIT_PAIR) {  // the up tiles go over through LDS, when everybody's last fragments have been read
+        static_assert(sizeof(As) >= (size_t)NT / 2 * TM * sizeof(f32x4), "room for the tiles that go over");
+        over = reinterpret_cast<f32x4*>(&As[0][0]) + (size_t)(wave / 2) * TM * 64 + lane;
+        __syncthreads();
+        if (second)
+#pragma unroll
+            for (int i = 0; i < TM; ++i) over[i * 64] = acc[i][TN - 1];
+        __syncthreads();
+    }
     // A tile at the lower edge of an output whose rows come in whole groups of sixteen (a decode step
     // of 48 requests in a 64-row tile) skips the groups beyond the last row and stores the others
     // without checks as well.
     auto emit = [&](auto checked, auto row_groups) {
         constexpr bool CHECKED = decltype(checked)::value, ROW_GROUPS = decltype(row_groups)::value;
         if constexpr (EPI == EPI_SWIGLU) {
-            static_assert(TN % 2 == 0, "gate and up tiles come in pairs");
             elem_t* out = reinterpret_cast<elem_t*>(ep.out);
 #pragma unroll
             for (int i = 0; i < TM; ++i) {
@@ -461,14 +515,19 @@ __device__ __forceinline__ void gemm_tile(const elem_t* __restrict__ A, const el
                         f[e] = 1.0f / sqrtf(ssum / (float)K + ep.ss_eps);
                     }
                 }
+                if constexpr (SPLIT_PAIR) {
+                    __builtin_amdgcn_sched_barrier(0);
+                    if (!second) last_up = over[i * 64];
+                }
 #pragma unroll
                 for (int j = 0; j < TN; j += 2) {
-                    const int col = (col_base + j * 16 - r16) / 2 + r16;  // tiles 2t, 2t+1 -> output tile t
+                    if (SPLIT_PAIR && j == TN - 1 && second) continue;
+                    const int col = (n0 + tile_col(j)) / 2 + r16;  // tiles 2t, 2t+1 -> output tile t
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
                         const int row = row_base + i * 16 + e;
                         if (CHECKED && !(row < M && col < ep.n_out)) continue;
-                        float gv = acc[i][j][e], uv = acc[i][j + 1][e];
+                        float gv = acc[i][j][e], uv = SPLIT_PAIR && j == TN - 1 ? last_up[e] : acc[i][min(j + 1, TN - 1)][e];
                         if constexpr (SCALED) {
                             gv *= f[e];
                             uv *= f[e];

@@ -47,6 +47,22 @@ def test_products_in_every_tile(dtype, M, N, K, tile):
     assert torch.equal(some, out[:65])
 
 
+# Gated products in 256x320 tiles, a pair of gate and up tiles in every two waves: whole tiles, ragged at both edges, a single row in the last tile; K steps even and odd
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("act", ["silu", "gelu_tanh"])
+@pytest.mark.parametrize("M,I,K", [(2048, 4800, 896), (1990, 4850, 960), (1985, 4850, 1024), (3001, 2811, 1024), (1793, 4864, 896)])
+def test_gated_products_in_the_widest_tiles(dtype, act, M, I, K):
+    from machserve_amd.kernels.ops import interleave_gate_up
+    ops = ops_for(dtype)
+    a, gate, up = rnd((M, K), dtype, 8), rnd((I, K), dtype, 9, 2 * K ** -0.5), rnd((I, K), dtype, 10, K ** -0.5)
+    w = interleave_gate_up(gate, up)
+    assert ops._plan("ms_gated_tile", M, w.shape[0], K) == 6, "the sizes are those of another tile"
+    z, u = a.float() @ gate.float().T, a.float() @ up.float().T
+    got = ops.linear_swiglu(a, w, I, act)
+    assert_close(got, (torch.nn.functional.silu(z) if act == "silu" else torch.nn.functional.gelu(z, approximate="tanh")) * u, dtype, "gated product")
+    assert torch.equal(ops.linear_swiglu(a[:300].contiguous(), w, I, act), got[:300]), "a row does not depend on its batch"
+
+
 # 32-bit: tiles of 32x32 (gated products 32x64) and 64x64 with whole K steps, one to many of them, and a partial last step
 @pytest.mark.parametrize("M,N,K", [(65, 40, 32), (97, 130, 64), (130, 200, 96), (501, 896, 160), (1025, 2056, 32), (1100, 2050, 352), (200, 136, 104)])
 def test_32_bit_products_in_every_tile(M, N, K):
