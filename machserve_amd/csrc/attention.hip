@@ -559,7 +559,7 @@ __global__ __launch_bounds__(256 * KG, attention_waves_per_simd<KG>()) void page
 // row's own, so a row's result depends neither on the step's cut nor on the rows beside it.
 //
 // Blocks measured (us; rows x key groups x stages, of 32 rows, 32 keys; general: the kernel above), prompts of 512, 2,048 and 4,096 tokens, eight of 200, 32 rows
-// behind 1,500 keys beside a prompt of 512, all with the reference left 2^8 behind (see below; 2x2x2 as it is now: 11.3, 30.6, 64, 8.7, 18.9; 15.3, 65, 200,
+// behind 1,500 keys beside a prompt of 512, all with the reference left 2^8 behind (see below; 2x2x2 then: 11.3, 30.6, 64, 8.7, 18.9; 15.3, 65, 200,
 // 20.6, 31.1; 14.3, 44, 124, 12.1, 29.4):
 //   head size 64, 14 over 2 heads    general 14.1  42.5   111  12.5  31.9;  2x2x2 10.5  29.1  61  8.3  18.2;  2x2x4 11.1  30.4  73  8.7  -;
 //                                    2x4x2   12.5  32.8    83  12.8  -;     4x2x4 14.1  36.9  71  11.3  -;    4x4x4 14.8  32.9  66  12.8  -
@@ -580,7 +580,7 @@ __global__ __launch_bounds__(256 * KG, attention_waves_per_simd<KG>()) void page
 // 16c + 8 * (l / 32) .., which is a B fragment of P^T as it stands and one 16-byte read of V^T.
 //
 // A tile that is loaded straight into LDS cannot be zeroed on its way: sixteen keys that are not there (beyond the
-// block's rows, in pages given back behind a window, in tiles past the block's range) read the start of the
+// block's rows, in pages given back behind a window, in tiles past the block's range) read the block's last page or the start of the
 // pool instead, are masked in the scores, and their values are overwritten with zeros (a caller's pool may hold anything in a page
 // that no request of the step owns).  Of sixteen keys that are there in part the others' values are what the page's last owner left:
 // finite, as every writer of a page sees to (cache_value), and met by probabilities of zero.
@@ -633,16 +633,16 @@ __device__ __forceinline__ int k_swizzle(int r) {
 __device__ __forceinline__ int v_swizzle(int d) { return ((d >> 2) & 1) | (((d >> 4) & 1) << 1); }  // rows of 4 chunks
 }  // namespace r32
 
+// ONE_PAGE: the page size is a multiple of a tile's 32 keys
+template <bool ONE_PAGE>
 __global__ __launch_bounds__(r32::KG * r32::GT, r32::KG * r32::RW * r32::PER_CU / 4) void paged_attention_rows32_kernel(AttnArgs a) {
     using namespace r32;
     static_assert((HDT == 64 || HDT == 128) && TK == 32 && RW == 2 && NS == 2, "the swizzles, the tiles' split over a group's waves and the rounds are written for these shapes");
     __shared__ __attribute__((aligned(1024))) unsigned char smem[SMEM];
-    __shared__ int tab[MAX_TABLE];
-    __shared__ unsigned kofs[KG][NS][2], vofs[KG][NS][2];  // [group][round % NS][16-key group of the tile]
+    __shared__ uint32_t tab[MAX_TABLE];
 
     const int kg = threadIdx.x / GT, tg = threadIdx.x % GT, lane = tg & 63, rw = tg >> 6;
     const int n32 = lane & 31, h = lane >> 5;
-    auto stage = [&](int b) { return smem + (KG * b + kg) * STAGE; };
     // the order of the blocks: as the general kernel's
     const int kvh = blockIdx.x % a.KV, sub = blockIdx.x / a.KV % SUB, turn = blockIdx.x / (a.KV * SUB);
     int item = turn;
@@ -708,7 +708,12 @@ __global__ __launch_bounds__(r32::KG * r32::GT, r32::KG * r32::RW * r32::PER_CU 
     kv_hi = __builtin_amdgcn_readfirstlane(kv_hi);
     const int kt_first = __builtin_amdgcn_readfirstlane((kv_lo / ROUND) * ROUND);
     const int page_first = kt_first / ps, n_tab = min(ceil_div(kv_hi, ps), a.table_stride) - page_first;
-    for (int i = threadIdx.x; i < n_tab; i += KG * GT) tab[i] = table[page_first + i];
+    // (as where the head's keys, and values, of a page begin in the pool, in units of sixteen numbers; a page that was given back: the pool's start)
+    const uint32_t page_units = (uint32_t)(a.KV * ps * HDT) >> 4, head_units = (uint32_t)(kvh * ps * HDT) >> 4;
+    for (int i = threadIdx.x; i < n_tab; i += KG * GT) {
+        const int page = table[page_first + i];
+        tab[i] = page >= 0 ? (uint32_t)page * page_units + head_units : 0u;
+    }
 
     Frag qf[NC];
     {
@@ -726,82 +731,116 @@ __global__ __launch_bounds__(r32::KG * r32::GT, r32::KG * r32::RW * r32::PER_CU 
 
     // A group's waves bring the group's tile, an equal share of K and of V^T each: a wave's load lands at the
     // wave's LDS base + 16 * lane, so the chunk that belongs at place p of the K tile (row p / (HDT / 8),
-    // chunk p % (HDT / 8) ^ swizzle) is the one this lane asks for; likewise the V^T tile (row p / 4).  Which 16-key group of
-    // the tile a chunk lies in picks the page offset, which the group's first two threads leave in LDS a round before.
+    // chunk p % (HDT / 8) ^ swizzle) is the one this lane asks for; likewise the V^T tile (row p / 4; GT / 4 rows further on its
+    // swizzle is the same).  Where a tile lies in one page its addresses are a scalar each for K and V^T and a lane's constant offsets;
+    // else a load of K has the scalar of its rows' 16-key group, and a lane of V^T that of its chunk's.
     constexpr int KL = LOADS / 2;  // loads of K, and of V^T
     const int p_own = 64 * rw + lane;
-    const elem_t* k_src[KL];
-    int k_grp[KL];
+    uint32_t k_off[KL], v_off[KL];
+    auto k_group = [](int i) { return i * GT / (HDT / 8) / 16; };
+    const int dv = p_own >> 2, vq = (p_own & 3) ^ v_swizzle(dv);  // keys 8 vq .. + 8 of row dv of V^T
+    const int v_grp = vq >> 1;
 #pragma unroll
     for (int i = 0; i < KL; ++i) {
         const int p = i * GT + p_own, Rk = p / (HDT / 8), kq = (p % (HDT / 8)) ^ k_swizzle(Rk), kl = swap_bits_2_3(Rk);  // row Rk of the tile holds key kl
-        k_src[i] = a.kpool + (kl & 15) * hd + kq * 8;
-        k_grp[i] = kl >> 4;
+        k_off[i] = ((ONE_PAGE ? kl : kl & 15) * hd + kq * 8) * (uint32_t)sizeof(elem_t);
+        v_off[i] = ((dv + i * (GT / 4)) * ps + (ONE_PAGE ? vq : vq & 1) * 8) * (uint32_t)sizeof(elem_t);
     }
-    // (GT / 4 rows further on, the swizzle of a V^T row is the same)
-    const int dv = p_own >> 2, vq = (p_own & 3) ^ v_swizzle(dv);  // keys 8 vq .. + 8 of row dv of V^T
-    const elem_t* v_src = a.vpool + (size_t)dv * ps + (vq & 1) * 8;
-    const int v_grp = vq >> 1;
-    // Offsets of the group's tile of the next round to be looked up, by the group's first two threads (one 16-key group of
-    // the tile each), stepped from round to round rather than divided out.  Keys that are not there (past the
-    // block's range, in a page given back) get offset 0: the first rows of the pool, masked.
-    int key_next = kt_first + kg * TK + (tg & 1) * 16, lp_next = key_next / ps, off_next = key_next - lp_next * ps;
+    // Where the tiles lie: every wave looks its group's tile up for itself, in scalars.  `look_up` asks LDS for the next tile's page (or its two 16-key groups'
+    // pages), stepped from tile to tile rather than divided out; `resolve`, a round later, makes addresses of it.  (Two threads that did it for their group
+    // through LDS were a chain in every round.)  Behind the block's keys it is the last page's, as keys that are not there.
+    const int kg_keys = __builtin_amdgcn_readfirstlane(kg * TK);
+    int lp_next = (kt_first + kg_keys) / ps - page_first, off_next = (kt_first + kg_keys) % ps;
     const int round_pages = ROUND / ps, round_rem = ROUND % ps;
-    auto fill_offsets = [&](int r) {
-        if (tg < 2) {
-            const bool there = key_next < kv_hi && lp_next < a.table_stride;
-            const int page = there ? tab[min(lp_next - page_first, n_tab - 1)] : -1;
-            const size_t pk = (size_t)max(page, 0) * a.KV + kvh;
-            kofs[kg][r % NS][tg] = page >= 0 ? (unsigned)(((pk * ps + off_next) * hd) >> 4) : 0u;
-            vofs[kg][r % NS][tg] = page >= 0 ? (unsigned)((pk * hd * ps + off_next) >> 4) : 0u;
-            key_next += ROUND;
-            lp_next += round_pages;
-            off_next += round_rem;
-            if (off_next >= ps) {
-                off_next -= ps;
-                ++lp_next;
-            }
+    constexpr int NG = ONE_PAGE ? 1 : 2;
+    uint32_t entry[NG];
+    int entry_off[NG];
+    auto look_up = [&]() {
+        entry[0] = tab[min(lp_next, n_tab - 1)];
+        entry_off[0] = off_next;
+        if constexpr (!ONE_PAGE) {
+            const bool over = off_next + 16 >= ps;
+            entry[1] = tab[min(lp_next + (over ? 1 : 0), n_tab - 1)];
+            entry_off[1] = off_next + 16 - (over ? ps : 0);
+        }
+        lp_next += round_pages;
+        off_next += round_rem;
+        if (off_next >= ps) {
+            off_next -= ps;
+            ++lp_next;
         }
     };
-    // the group's tile of round r straight into stage r % NS (in assembly: of a load that it knows to write LDS the
+    const char *keys_at[NG], *values_at[NG], *next_values_at[NG];  // of the tile whose loads go out next
+    auto resolve = [&]() {
+#pragma unroll
+        for (int u = 0; u < NG; ++u) {
+            const size_t page = (size_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)entry[u]) * (16 * sizeof(elem_t));
+            values_at[u] = next_values_at[u];
+            keys_at[u] = reinterpret_cast<const char*>(a.kpool) + page + (uint32_t)entry_off[u] * (uint32_t)(HDT * sizeof(elem_t));
+            next_values_at[u] = reinterpret_cast<const char*>(a.vpool) + page + (uint32_t)entry_off[u] * (uint32_t)sizeof(elem_t);
+        }
+    };
+    // a tile straight into stage `B` (in assembly: of a load that it knows to write LDS the
     // compiler would make every later LDS read wait; the waits are written by hand at the rounds' ends)
     const uint32_t lds_own = __builtin_amdgcn_readfirstlane(
         (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const unsigned char*)(smem + kg * STAGE + 1024 * rw));
-    auto load_direct = [&](int r) {
-        const int b = r % NS;
-        const uint32_t kb = lds_own + b * (KG * STAGE), vb = kb + K_BYTES;
+    auto load_keys = [&](auto stage_of, const char* const (&from)[NG]) {
 #pragma unroll
         for (int i = 0; i < KL; ++i) {
-            const elem_t* gk = k_src[i] + ((size_t)kofs[kg][b][k_grp[i]] << 4);
-            asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(gk), "s"(kb + i * GT * 16) : "memory", "m0");
+            const uint32_t off = k_off[i], to = lds_own;
+            const char* base = from[ONE_PAGE ? 0 : k_group(i)];
+            asm volatile("s_add_i32 m0, %2, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(to),
+                         "n"(decltype(stage_of)::value * (KG * STAGE) + i * GT * 16) : "memory", "m0", "scc");
         }
-        const elem_t* gv = v_src + ((size_t)vofs[kg][b][v_grp] << 4);
+    };
+    auto load_values = [&](auto stage_of, const char* const (&from)[NG]) {
 #pragma unroll
-        for (int i = 0; i < KL; ++i)
-            asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(gv + i * (GT / 4) * ps), "s"(vb + i * GT * 16) : "memory", "m0");
+        for (int i = 0; i < KL; ++i) {
+            constexpr int at = decltype(stage_of)::value * (KG * STAGE) + K_BYTES;
+            const uint32_t off = v_off[i], to = lds_own;
+            const char* base = v_grp && !ONE_PAGE ? from[NG - 1] : from[0];
+            if constexpr (ONE_PAGE)
+                asm volatile("s_add_i32 m0, %2, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(to), "n"(at + i * GT * 16)
+                             : "memory", "m0", "scc");
+            else
+                asm volatile("s_add_i32 m0, %1, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(base + off), "s"(to), "n"(at + i * GT * 16)
+                             : "memory", "m0", "scc");
+        }
     };
     // rows of this wave: the first and the last position decide which tiles need no mask at all
-    const int pos_first = pos0 + (r0 + rw * 32) / g;
-    const int pos_last = pos0 + min(r0 + rw * 32 + 31, max(R - 1, 0)) / g;
+    const int first_row = __builtin_amdgcn_readfirstlane(r0 + rw * 32);
+    const int pos_first = pos0 + first_row / g;
+    const int pos_last = pos0 + min(first_row + 31, max(R - 1, 0)) / g;
     const int lo_last = first_visible_key(pos_last, a.window, a.chunk);
     // where this lane reads its fragments in a stage: row n32 of the K tile, row 32 dt + n32 of V^T, chunk 2c + h
     const int k_row = n32 * (HDT * 2), k_sw = k_swizzle(n32), v_row = K_BYTES + n32 * (TK * 2), v_sw = v_swizzle(n32);
 
-    // Round r: group kg has the tile of absolute index (kt_first / 32) + r * KG + kg.  Its page offsets are written a
-    // round before its loads go out, its loads a round before it is multiplied, and one barrier a round
-    // separates the steps.
+    // Round r: group kg has the tile of absolute index (kt_first / 32) + r * KG + kg.  Its scores are multiplied a round ahead, between round r - 1's
+    // exponentials, so that a wave's matrix and vector instructions run beside each other and not in turn; so its keys run a round ahead of its values and
+    // take the place of the last round's but one, whose scores are done.  Pages are looked up a round before the keys' loads go out, loads go out a round
+    // before what they bring is multiplied, and one barrier a round separates the steps.  A round is bound by what a wave does one after the other, scalar
+    // instructions included (a prompt of 2,048, 14 heads of 64, 31.0 us: with the scores ahead and two lookups in scalars 29.1, with
+    // one page a tile and a table of offsets in place of pages 28.0, and with two rounds in the loop's body, so that stages are constants and the scores
+    // change places without moves, 22.9; 4,096 tokens 61 -> 47; heads of 128, 28 over 4, 60 -> 54; loads two or three rounds ahead, tiles of 64 keys,
+    // and two blocks a CU in place of three gain nothing).
     // (the same for the whole block: kept in scalar registers, so that the rounds' branches are scalar ones)
     const int n_rounds = __builtin_amdgcn_readfirstlane(ceil_div(kv_hi - kt_first, ROUND));
+    using Stage0 = std::integral_constant<int, 0>;
+    using Stage1 = std::integral_constant<int, 1>;
     // the queries and the table are here before the first tile is asked for, so that no later wait of the compiler's
     // for them takes the tiles' loads with it
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 #pragma unroll
     for (int c = 0; c < NC; ++c) asm volatile("" : "+v"(qf[c].v));
     __syncthreads();  // the table is in LDS
-    fill_offsets(0);
-    __syncthreads();
-    load_direct(0);
-    fill_offsets(1);
+    look_up();
+    resolve();
+    load_keys(Stage0{}, keys_at);
+    load_values(Stage0{}, next_values_at);
+    look_up();
+    resolve();
+    load_keys(Stage1{}, keys_at);
+    look_up();
     // End of a round: this wave's loads have landed and its LDS accesses are done; then everybody's.
     auto round_end = [&]() {
         __builtin_amdgcn_sched_barrier(0);
@@ -810,49 +849,48 @@ __global__ __launch_bounds__(r32::KG * r32::GT, r32::KG * r32::RW * r32::PER_CU 
         __builtin_amdgcn_sched_barrier(0);
     };
     round_end();
-    // S^T = K Q^T of the group's tile of round r: register v of this lane is key kt0 + 16 (v / 8) + 8 h + v % 8 for query
-    // row n32.
-    f32x16 sc;
-    auto scores = [&](int r) {
-        const unsigned char* st = stage(r % NS);
+    // S^T = K Q^T of the group's tile: register v of this lane is key kt0 + 16 (v / 8) + 8 h + v % 8 for query row n32.
+    f32x16 sc0, sc1;
+    const unsigned char* own = smem + kg * STAGE;
+    auto k_frag = [&](int b, int c) { return frag_load(reinterpret_cast<const elem_t*>(own + b * (KG * STAGE) + k_row + (((2 * c + h) ^ k_sw) << 4))); };
 #pragma unroll
-        for (int i = 0; i < 16; ++i) sc[i] = 0.f;
-        auto k_frag = [&](int c) { return frag_load(reinterpret_cast<const elem_t*>(st + k_row + (((2 * c + h) ^ k_sw) << 4))); };
-        Frag kf[2] = {k_frag(0), k_frag(1)};  // two fragments in flight
+    for (int i = 0; i < 16; ++i) sc0[i] = 0.f;
 #pragma unroll
-        for (int c = 0; c < NC; ++c) {
-            mma_32x32x16(sc, kf[c & 1], qf[c]);
-            if (c + 2 < NC) kf[c & 1] = k_frag(c + 2);
-        }
-    };
-    const int kg_keys = __builtin_amdgcn_readfirstlane(kg * TK);
-    auto busy_in = [&](int r) { return wave_active && kt_first + r * ROUND + kg_keys < kv_hi; };
-    for (int r = 0; r < n_rounds; ++r) {
-        const int kt0 = kt_first + r * ROUND + kg_keys;
-        const unsigned char* st = stage(r % NS);
-        if (r + 1 < n_rounds) load_direct(r + 1);  // into the stage that round r - 1 has left
-        if (kt_first + r * ROUND < kv_lo || kt_first + (r + 1) * ROUND > kv_hi) {
-            // (at most the first and the last round, the same for the whole block) values of sixteen keys that are not there: zero
+    for (int c = 0; c < NC; ++c) mma_32x32x16(sc0, k_frag(0, c), qf[c]);
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();  // everybody has round 0's keys
+    __builtin_amdgcn_sched_barrier(0);
+    int kt0 = kt_first + kg_keys;
+    // the round with its scores in `sc` and its tile's values in stage B, which leaves the next round's scores in `next`
+    auto round_of = [&](int r, auto stage_of, f32x16& sc, f32x16& next) {
+        constexpr int B = decltype(stage_of)::value;
+        resolve();
+        if (r + 2 < n_rounds) load_keys(std::integral_constant<int, B>{}, keys_at);  // into the places that the last round has left
+        if (r + 1 < n_rounds) load_values(std::integral_constant<int, B ^ 1>{}, values_at);
+        look_up();
+        if (r == 0 || r + 1 == n_rounds) {
+            // (the same for the whole block) values of sixteen keys that are not there: zero
             const int key = kt0 + 16 * v_grp;
             if (key + 16 <= kv_lo || key >= kv_hi) {
 #pragma unroll
                 for (int i = 0; i < KL; ++i)
-                    *reinterpret_cast<u32x4*>(smem + (r % NS * KG + kg) * STAGE + K_BYTES + (i * GT + p_own) * 16) = (u32x4){0, 0, 0, 0};
+                    *reinterpret_cast<u32x4*>(smem + (B * KG + kg) * STAGE + K_BYTES + (i * GT + p_own) * 16) = (u32x4){0, 0, 0, 0};
             }
             __builtin_amdgcn_sched_barrier(0);
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
             __builtin_amdgcn_s_barrier();
             __builtin_amdgcn_sched_barrier(0);
         }
-        if (busy_in(r)) {
-            scores(r);
+        if (wave_active && kt0 < kv_hi) {
             // the values of the first sixteen keys, which the step after next multiplies by: asked for before the exponentials
             auto v_frag = [&](int c, int dt) {
-                return frag_load(reinterpret_cast<const elem_t*>(st + v_row + dt * (32 * TK * 2) + (((2 * c + h) ^ v_sw) << 4)));
+                return frag_load(reinterpret_cast<const elem_t*>(own + B * (KG * STAGE) + v_row + dt * (32 * TK * 2) + (((2 * c + h) ^ v_sw) << 4)));
             };
             Frag vf[NDT];
 #pragma unroll
             for (int dt = 0; dt < NDT; ++dt) vf[dt] = v_frag(0, dt);
+            Frag kf[2] = {k_frag(B ^ 1, 0), k_frag(B ^ 1, 1)};  // two fragments in flight
             if (a.softcap > 0.f) {
 #pragma unroll
                 for (int i = 0; i < 16; ++i) sc[i] = capped_raw(sc[i], a.scale, a.softcap);
@@ -882,8 +920,17 @@ __global__ __launch_bounds__(r32::KG * r32::GT, r32::KG * r32::RW * r32::PER_CU 
                 m_run = m_new;
             }
             const float mb = m_run * sl;
+            // the exponentials, and between them the next tile's scores (behind the last tile of what the places hold, and not used)
 #pragma unroll
-            for (int i = 0; i < 16; ++i) sc[i] = exp2_f(fmaf(sc[i], sl, -mb));
+            for (int i = 0; i < 16; ++i) next[i] = 0.f;
+#pragma unroll
+            for (int c = 0; c < NC; ++c) {
+                mma_32x32x16(next, kf[c & 1], qf[c]);
+                if (c + 2 < NC) kf[c & 1] = k_frag(B ^ 1, c + 2);
+#pragma unroll
+                for (int i = 16 / NC * c; i < 16 / NC * (c + 1); ++i) sc[i] = exp2_f(fmaf(sc[i], sl, -mb));
+                __builtin_amdgcn_sched_barrier(0);
+            }
             float t8[8];
 #pragma unroll
             for (int i = 0; i < 8; ++i) t8[i] = sc[i] + sc[i + 8];
@@ -902,8 +949,12 @@ __global__ __launch_bounds__(r32::KG * r32::GT, r32::KG * r32::RW * r32::PER_CU 
                     if (c == 0) vf[dt] = v_frag(1, dt);
                 }
         }
-        if (r + 2 < n_rounds) fill_offsets(r + 2);  // read when that round's loads go out, at the top of the next round
+        kt0 += ROUND;
         round_end();
+    };
+    for (int r = 0; r < n_rounds; r += 2) {
+        round_of(r, Stage0{}, sc0, sc1);
+        if (r + 1 < n_rounds) round_of(r + 1, Stage1{}, sc1, sc0);
     }
 
     l_run += __shfl_xor(l_run, 32, WAVE);  // the row's two halves (they were scaled alike all along)
@@ -1593,7 +1644,8 @@ extern "C" int MS_CAT(ms_paged_attention_mask_nd, MS_ATTN_ND)(
             a.pair_span = r32::PER_CU == 2 ? std::max(cus / (KV * r32::SUB), 1) : 0;
             a.rise = HDT == 64 && span >= 2048 ? 6.0f : 0.0f;  // see the kernel
             const dim3 grid32((unsigned)(n_work * KV * r32::SUB), (unsigned)nsplit);
-            hipLaunchKernelGGL(paged_attention_rows32_kernel, grid32, dim3(r32::KG * r32::GT), 0, stream, a);
+            if (ps % r32::TK == 0) hipLaunchKernelGGL(paged_attention_rows32_kernel<true>, grid32, dim3(r32::KG * r32::GT), 0, stream, a);
+            else hipLaunchKernelGGL(paged_attention_rows32_kernel<false>, grid32, dim3(r32::KG * r32::GT), 0, stream, a);
             int rc32 = check_launch("paged_attention (32-row tiles)");
             if (rc32 || nsplit == 1) return rc32;
             hipLaunchKernelGGL(decode_merge_kernel, dim3((unsigned)((size_t)T * H)), dim3(64), 0, stream, part_o, part_ml, (elem_t*)out, hd, nsplit, a.sinks, H, a.out_gate);

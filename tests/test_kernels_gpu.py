@@ -484,6 +484,16 @@ def test_attention_reads_nothing_of_keys_that_are_not_there(dtype, hd):
             assert torch.equal(got, want) and bool(torch.isfinite(got).all()), (pos0, n, w)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("ps", [16, 32, 48, 64, 96])
+def test_prompts_of_any_page_size(dtype, hd, ps):
+    """Prompts whose keys end before, at and behind a tile of 32 and a round of 64 keys, in pages that hold whole tiles and in pages that do not."""
+    for window, seqs in ((None, [(0, 1), (0, 32), (0, 33), (31, 34), (60, 70), (100, 97)]), (50, [(0, 130), (90, 40), (64, 64)])):
+        got, ref = _attention_case(dtype, 4, 2, hd, ps, window, seqs, 300 + ps, groups=32)
+        assert_close(got, ref, dtype, f"window {window}")
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("splits", [2, 5, 64])
 @pytest.mark.parametrize("H,KV,hd,ps,window", [(4, 2, 16, 16, None), (14, 2, 64, 64, None), (6, 3, 128, 32, None),
