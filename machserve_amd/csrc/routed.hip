@@ -17,8 +17,8 @@
 // beyond the outputs to choose from (`extra`) are gates that every row has, the sigmoids of their own logits, left behind
 // the experts' weights; the first of them can stand for the expert that every row uses.  A weight may also multiply a gated
 // expert's input instead of its output: act(w gate) * (w up).
+#include "few_rows.cuh"
 #include "gemm_plan.h"
-#include "gemm_tile.cuh"
 
 namespace ms {
 
@@ -392,8 +392,46 @@ __global__ __launch_bounds__(64 * WM * WN) void expert_gemm_kernel(const elem_t*
     gemm_tile<BM, BN, WM, WN, BK, EPI, STAGES, false>(A, own, count, N, K, ep, m0, n0, 0, rows);
 }
 
-// The tile of a product.  A step of at most 64 rows has one tile of 64 rows an expert, its weight's columns streamed by blocks with three
-// steps in flight; above, the tile of the least predicted time, every expert's last tile counted as half empty.
+#ifdef MS_ELEM_HALF
+// A step of at most 32 rows, a step of K or more for every wave: four waves share out K (few_rows.cuh), a block an expert and 16 NT of its columns.  The rows
+// that chose the expert, and what the epilogue needs of them, are one trip: every wave reads all rows' planes, lane t row t's.
+// Bound by the chosen experts' weights.  32 columns a block (72 and 64 KB of LDS, two blocks a CU) are better than 64: four rows that use 5 of 8 experts of 2,816
+// and one for every row, width 2,048 (us up + down): 64x64 tiles 44.5 + 21.6, 64 columns 38.3 + 21.8, 32 columns 34.4 + 17.1; sixteen rows 49.3 + 25.4,
+// 47.2 + 25.5, 39.2 + 21.1; 24 rows 49.8 + 26, 50.4 + 27, 41.0 + 22.3; eight rows, 6 of 64 experts of 1,408, 94 + 49 and 79 + 42.  Above 32 rows the tiles are
+// the better ones (48 rows 52.1 + 28.3; as two or three row tiles here 58.8 + 30.5 and 44 + 25, but 64 rows 44 + 18 against 54 + 26 and 84 + 40).
+template <int MT, int NT, int STAGES, int EPI>
+__global__ __launch_bounds__(64 * FEW_WAVES) void expert_few_kernel(const elem_t* __restrict__ A, const elem_t* __restrict__ W, void* out, ExpertArgs g) {
+    constexpr bool DOWN = EPI == EPI_EXPERT_DOWN;
+    constexpr int PER = EPI == EPI_EXPERT_GATED ? 2 : 1;
+    __shared__ int few[16 * MT], of_row[16 * MT];
+    const int lane = threadIdx.x & 63, tiles = g.routed_tiles + g.shared_tiles, tile = blockIdx.x % tiles, n0 = blockIdx.x / tiles * (16 * NT);
+    const bool shared = tile >= g.routed_tiles;
+    const int e = shared ? g.E : tile, cols = shared ? g.shared : g.ff;
+    const int N = DOWN ? g.width : PER * cols, K = DOWN ? cols : g.width;
+    if (n0 >= N) return;
+    const int t = min(lane, g.T - 1);
+    const int plane = shared ? g.top : g.plane[(size_t)t * g.E + e];
+    const float gate = DOWN || (shared && !g.shared_gate) ? 1.0f : g.gates[(size_t)t * g.ld_gates + e];
+    const bool mine = lane < g.T && plane >= 0;
+    const unsigned long long all = __ballot(mine);
+    const int count = __builtin_amdgcn_readfirstlane(__popcll(all));
+    if (count == 0) return;  // the whole block
+    if (threadIdx.x < 64 && mine) {
+        const int at = __popcll(all & ((1ull << lane) - 1));
+        few[at] = lane;
+        of_row[at] = DOWN ? plane * g.T + lane : __float_as_int(gate);
+    }
+    __syncthreads();
+    EpiArgs ep{out, nullptr, DOWN ? g.width : max(g.ff, g.shared), DOWN ? g.width : cols, K, 0};
+    ep.k_per_split = K;
+    const ExpertRows<!DOWN> rows{g, shared ? nullptr : few, e, shared ? g.routed_slots : tile * g.T, of_row};
+    const elem_t* own = W + (size_t)e * g.ff * (DOWN ? 1 : PER * g.width);  // its columns, or its rows
+    few_rows_tile<MT, NT, FEW_WAVES, STAGES, EPI, false>(A, own, count, N, K, ep, 0, n0, 0, rows);
+}
+#endif
+
+// The tile of a product.  A step of 33 to 64 rows (and of any number up to 64 in 32-bit) has one tile of 64 rows an expert, its weight's columns streamed by blocks with
+// three steps in flight; above, the tile of the least predicted time, every expert's last tile counted as half empty.
 // 2,048 rows, 2 of 8 experts of 2,816 and one of 2,816 for every row, width 2,048, gated (us up / down): 256x256 191 / 83, 256x192 211 / 120,
 // 256x128 197 / 97, 128x128 179 / 106, 64x64 279 / 156; 128x128 alone, in the order of the columns and with the epilogue reading row by row, was 228 / 120.
 // 1,750 rows, 2 of 8 experts of 2,816: 122 / 73, 128 / 62, 130 / 87, 120 / 72 and 178 / 101 against 170 / 113.
@@ -460,6 +498,18 @@ static int launch_experts(const void* a, const void* w, void* out, ExpertArgs g,
         return check_launch("experts " #BM_ "x" #BN_ "x" #BK_);                                                                     \
     } while (0)
 #ifdef MS_ELEM_HALF
+    if (g.T <= 32 && (DOWN ? min(g.ff, g.shared ? g.shared : g.ff) : g.width) >= 64 * FEW_WAVES) {
+#define MS_EXPERTS_FEW(MT_, NT_, ST_)                                                                                                       \
+    do {                                                                                                                                    \
+        const long blocks = (long)(g.routed_tiles + g.shared_tiles) * ceil_div(DOWN ? g.width : PER * max(g.ff, g.shared), 16 * NT_);        \
+        hipLaunchKernelGGL((expert_few_kernel<MT_, NT_, ST_, EPI>), dim3((unsigned)blocks), dim3(64 * FEW_WAVES), 0, stream, (const elem_t*)a, \
+                           (const elem_t*)w, out, g);                                                                                        \
+        return check_launch("experts, few rows");                                                                                            \
+    } while (0)
+        if (g.T <= 16) MS_EXPERTS_FEW(1, 2, 3);
+        MS_EXPERTS_FEW(2, 2, 2);
+#undef MS_EXPERTS_FEW
+    }
     switch ((int)(&tile - kTiles)) {
         case TILE_256x256:
             if constexpr (EPI != EPI_EXPERT_PLAIN) MS_EXPERTS(256, 256, 2, 4, 64, GEMM_PIPED);

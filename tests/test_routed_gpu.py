@@ -11,7 +11,10 @@ pytestmark = pytest.mark.gpu
 # rows, router outputs, of them experts, used a row, columns of an expert, columns of the expert for every row, width
 SIZES = [(1, 8, 8, 2, 64, 0, 128), (4, 9, 8, 2, 128, 64, 192), (64, 5, 5, 3, 64, 128, 64), (65, 5, 5, 3, 64, 64, 64), (129, 8, 6, 2, 192, 0, 256),
          (300, 70, 68, 1, 64, 0, 128), (700, 4, 3, 2, 128, 64, 320), (1025, 2, 2, 2, 64, 64, 64),
-         (3100, 4, 4, 2, 1472, 64, 832), (4300, 2, 2, 1, 1984, 1024, 832), (40, 130, 130, 12, 64, 64, 64)]
+         (3100, 4, 4, 2, 1472, 64, 832), (4300, 2, 2, 1, 1984, 1024, 832), (40, 130, 130, 12, 64, 64, 64),
+         # products of few rows: whole and partial rounds of the waves' K steps, 16, 17, 32 and 33 rows, most of an expert's rows and hardly any
+         (1, 8, 8, 2, 256, 256, 256), (16, 9, 8, 2, 320, 256, 448), (17, 5, 5, 3, 256, 320, 576), (32, 2, 2, 2, 704, 0, 320), (33, 8, 8, 2, 256, 256, 256),
+         (30, 40, 40, 1, 256, 0, 256)]
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
