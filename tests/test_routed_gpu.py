@@ -147,6 +147,25 @@ def test_a_step_of_few_rows_sets_no_more_activations_aside_than_its_rows_could_f
     assert torch.cuda.max_memory_allocated() - before <= rows * ff * 2 + 2 * T * E * 4 + (top + 1) * T * width * 4 + 4 * 512
 
 
+# one row a block and four, a ragged last block; few outputs (one lane each), more than 64; columns that come in fours and that do not
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("T,E,top,d", [(1, 8, 2, 256), (5, 13, 13, 1030), (1023, 9, 2, 128), (1030, 64, 6, 192), (1025, 65, 5, 130), (3, 200, 64, 2048)])
+@pytest.mark.parametrize("scoring", [{}, {"softmax_all": True}, {"sigmoid": True, "extra_gates": 3}])
+def test_the_router_in_its_forms(dtype, T, E, top, d, scoring):
+    from machserve_amd.kernels import get_ops
+    g = torch.Generator().manual_seed(T + E)
+    x, w = torch.randn(T, d, generator=g).to(dtype), torch.randn(E + scoring.get("extra_gates", 0), d, generator=g) * d ** -0.5
+    w[E // 2] = w[0]  # two outputs that tie in every row: the first is chosen
+    got = get_ops(dtype, DEV).route(x.to(DEV), w.to(DEV), None, top, **scoring).cpu()
+    want = EmulatedOps(torch.float32).route(x.float(), w, None, top, **scoring)
+    z = (x.double() @ w[:E].double().T).sort(1, descending=True).values
+    # logits are 32-bit sums of d products: off by about sqrt(d) 2^-24 of their size; rows whose last chosen logit has a near equal may differ
+    clear = torch.ones(T, dtype=torch.bool) if top == E else ((z[:, top - 1] - z[:, top]).abs() > 1e-5)
+    assert clear.float().mean() > 0.5
+    assert not bool(((got[:, E // 2] > 0) & (got[:, 0] == 0)).any()), "of equals the first"
+    assert (got - want)[clear].abs().max().item() <= 1e-5
+
+
 def test_the_router_refuses_numbers_and_sums_that_its_kernel_does_not_assume():
     from machserve_amd.kernels import KernelError, get_ops
     ops, new = get_ops(torch.bfloat16, DEV), lambda shape, dt: torch.zeros(shape, dtype=dt, device=DEV)  # noqa: E731
