@@ -100,6 +100,25 @@ def test_convolution_over_sums_in_one_step_and_in_many(C, taps, biases):
         close(got, want, torch.float32, f"steps of {cuts}")
 
 
+@pytest.mark.parametrize("C,taps,biases", [(1020, 2, True), (1024, 3, False), (1020, 4, True), (1022, 4, True)])
+def test_convolution_over_many_rows(C, taps, biases):
+    """Runs of eight rows of four columns a thread, and columns that do not come in fours: requests that begin and end anywhere in a run, behind older inputs."""
+    ops = ops_of(torch.float32)
+    torch.manual_seed(C + taps)
+    lens = [1, 2, 3, 700, 5, 394]
+    q0 = [sum(lens[:i]) for i in range(len(lens))]
+    sums, old = torch.randn(2, sum(lens), C + 16), torch.randn(8, taps - 1, C)
+    w, b_in, b_out = torch.randn(C, taps) * 0.5, (torch.randn(C) if biases else None), (torch.randn(C) if biases else None)
+    slots, state = [3, 0, 7, 1, 2, 5], dev(old.clone())
+    got = ops.conv_sums(dev(sums), 8, C, dev(b_in), dev(w), dev(b_out), state, i32(q0), i32(lens), i32(slots))
+    u = sums.sum(0)[:, 8:8 + C].double() + (b_in.double() if biases else 0.0)
+    for s, n, slot in zip(q0, lens, slots):
+        own = torch.cat([old[slot].double(), u[s:s + n]])
+        want = sum(own[k:k + n] * w[:, k].double() for k in range(taps)) + (b_out.double() if biases else 0.0)
+        close(got[s:s + n].cpu(), want, torch.float32, f"rows {s} to {s + n}")
+        close(state[slot].cpu(), own[n:], torch.float32, "the state")
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("C,blocks", [(48, 3), (40, 5), (256, 1), (320, 4), (24, 24)])
 def test_gated_recurrence_in_one_step_and_in_many(dtype, C, blocks):
