@@ -229,7 +229,13 @@ __global__ __launch_bounds__(256) void route_kernel(const elem_t* __restrict__ x
 __device__ __forceinline__ float expert_activation(float z, int act) {
     if (act == 0) return 0.5f * z * (1.0f + erff(z * 0.7071067811865476f));
     if (act == 1) return 0.5f * z * (1.0f + tanhf(0.7978845608028654f * (z + 0.044715f * z * z * z)));
+#ifdef MS_ELEM_HALF
+    // as gate_activation: exponential and reciprocal of the hardware, a unit or two in the last place of 32 bits ahead of a rounding to the element type.
+    // The up product's epilogue is all vector instructions: 2,048 rows, 2 of 8 experts of 2,816 and one for every row 173 -> 162 us.
+    return z * __builtin_amdgcn_rcpf(1.0f + __expf(-z));
+#else
     return z / (1.0f + expf(-z));
+#endif
 }
 
 // a[t, c] = act(up[t, c]) * gates[t, c / ff] for c < E * ff, act(up[t, c]) beyond (experts that every row uses, whose weight is
@@ -520,20 +526,33 @@ __global__ __launch_bounds__(64 * FEW_WAVES) void expert_few_kernel(const elem_t
 #endif
 
 // The tile of a product.  A step of 33 to 64 rows (and of any number up to 64 in 32-bit) has one tile of 64 rows an expert, its weight's columns streamed by blocks with
-// three steps in flight; above, the tile of the least predicted time, every expert's last tile counted as half empty.
+// three steps in flight; above, the tile of the least predicted time, its tiles counted from how many rows
+// an expert can be expected to have.
+// us up, the choice of half an expert's last tile empty -> this one (2 of 8 experts of 2,816, width 2,048): 1,900 rows 120 -> 98, 1,200 102 -> 92, 700 and
+// an expert for every row 88 -> 63, 2,048 of experts of 1,408 and width 1,024 61 -> 50.
 // 2,048 rows, 2 of 8 experts of 2,816 and one of 2,816 for every row, width 2,048, gated (us up / down): 256x256 191 / 83, 256x192 211 / 120,
 // 256x128 197 / 97, 128x128 179 / 106, 64x64 279 / 156; 128x128 alone, in the order of the columns and with the epilogue reading row by row, was 228 / 120.
 // 1,750 rows, 2 of 8 experts of 2,816: 122 / 73, 128 / 62, 130 / 87, 120 / 72 and 178 / 101 against 170 / 113.
 static int plan_experts(const ExpertArgs& g, bool down, int per) {
 #ifdef MS_ELEM_HALF
     if (g.T <= 64) return TILE_64x64_DEEP;
-    const long rows = (long)g.T * g.top, used = min((long)g.E, rows);
+    // Rows fall to the router's outputs (of which some may be no experts) as if at random: an expert has `mean` rows, give or take `spread`, and
+    // its tiles are counted as the chances that it has more rows than each of them begins with.
+    const int outputs = max(g.E, g.ld_gates - (g.shared ? 1 : 0));  // (a gate of the expert for every row is none of them)
+    const double mean = (double)g.T * g.top / outputs, spread = sqrt(mean * (1.0 - 1.0 / outputs)) + 1e-3;
     int best = TILE_64x64;
     float least = INFINITY;
     for (int i = 0; i < TILE_COUNT; ++i) {
         const TileCost& t = kTiles[i];
         if (i == TILE_256x256 && !down && per == 1) continue;  // every sum in its own activation: too many registers
-        const long routed = max(used, rows / t.bm + (used + 1) / 2), all = g.shared ? ceil_div(g.T, t.bm) : 0;
+        // (and their deviation with them: blocks that come to just a round in the mean are often a round and one)
+        double tiles = 0.0, variance = 0.0;
+        for (long at = 0; at < g.T && at < mean + 4.0 * spread; at += t.bm) {
+            const double p = 0.5 * erfc((at + 0.5 - mean) / (spread * 1.4142135623730951));
+            tiles += p * g.E;
+            variance += p * (1.0 - p) * g.E;
+        }
+        const long routed = max(1L, lround(tiles + sqrt(variance))), all = g.shared ? ceil_div(g.T, t.bm) : 0;
         const long blocks = down ? (routed + all) * ceil_div(g.width, t.bn) : routed * ceil_div(per * g.ff, t.bn) + all * ceil_div(per * g.shared, t.bn);
         const long depth = down ? (routed * g.ff + all * g.shared) / (routed + all) : g.width;
         const float us = tile_time(t, blocks, (int)depth, down);
