@@ -1454,51 +1454,63 @@ __global__ __launch_bounds__(256) void decode_attention_kernel(DecodeArgs a) {
 }
 
 // out[row, :] = sum_sp o_sp exp(m_sp - m) / sum_sp l_sp exp(m_sp - m), splits in order.
-// One wave per (request, head); lane = element of the head (in chunks of 64).  The splits' outputs are
-// asked for eight at a time, the first eight together with the (max, sum) pairs and before anything
-// is computed from those, so that the kernel waits for memory once.
-__global__ __launch_bounds__(64) void decode_merge_kernel(const float* __restrict__ part_o, const float* __restrict__ part_ml,
-                                                          elem_t* __restrict__ out, int hd, int nsplit,
-                                                          const float* __restrict__ sinks, int H,
-                                                          const float* __restrict__ out_gate) {
-    arguments_now(part_o, part_ml, out, hd, nsplit, sinks, H, out_gate);
-    constexpr int BATCH = 8;
+// One wave per (request, head); lane = element of the head (in chunks of 64).  The splits' outputs of all chunks are
+// asked for BATCH at a time, the first together with the (max, sum) pairs and before anything
+// is computed from those: with as many as there are splits the kernel waits for memory once.  A split's coefficient is read
+// from its lane into a scalar.
+constexpr int MERGE_CHUNKS = (HDT + 63) / 64;
+template <int BATCH>
+__device__ __forceinline__ void merge_row(const float* __restrict__ part_o, const float* __restrict__ part_ml, elem_t* __restrict__ out, int hd, int nsplit,
+                                          const float* __restrict__ sinks, int H, const float* __restrict__ out_gate) {
     const size_t row = blockIdx.x;  // (request, head)
     const int lane = threadIdx.x;
     const float* ml = part_ml + row * nsplit * 2;
     const float* po = part_o + row * nsplit * hd;
-    auto fetch = [&](int d, int sp0, float (&v)[BATCH]) {
+    float v[BATCH][MERGE_CHUNKS];
+    auto fetch = [&](int sp0) {
 #pragma unroll
-        for (int u = 0; u < BATCH; ++u) v[u] = po[(size_t)min(sp0 + u, nsplit - 1) * hd + min(d, hd - 1)];
+        for (int u = 0; u < BATCH; ++u)
+#pragma unroll
+            for (int c = 0; c < MERGE_CHUNKS; ++c) v[u][c] = po[(size_t)min(sp0 + u, nsplit - 1) * hd + min(lane + 64 * c, hd - 1)];
     };
-    float first[BATCH];
-    fetch(lane, 0, first);
+    fetch(0);
     // every lane holds one split's (max, sum); nsplit <= 64
     const int own = min(lane, nsplit - 1);
     const float m_ld = ml[own * 2], l_ld = ml[own * 2 + 1];
     const float m_own = lane < nsplit ? m_ld : NEG_BIG;
     const float l_own = lane < nsplit ? l_ld : 0.f;
     const float m = wave_max(m_own);
-    const float c = lane < nsplit ? exp_f(m_own - m) : 0.f;
+    const float c_own = lane < nsplit ? exp_f(m_own - m) : 0.f;
+    auto of_lane = [](float x, int from) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), from)); };
     float l = 0.f;
-    for (int sp = 0; sp < nsplit; ++sp) l += __shfl(l_own * c, sp, WAVE);  // in split order
+    for (int sp = 0; sp < nsplit; ++sp) l += of_lane(l_own * c_own, sp);  // in split order
     const float inv = softmax_norm(m, l, sinks, sinks ? (int)(row % (size_t)H) : 0, out_gate, row);
-    const float coef = c * inv;  // of split `lane`; zero beyond the last split
-    for (int d = lane; d - lane < hd; d += 64) {
-        float o = 0.f;
-        for (int sp0 = 0; sp0 < nsplit; sp0 += BATCH) {
-            float v[BATCH];
-            if (d == lane && sp0 == 0) {
+    const float coef = c_own * inv;  // of split `lane`; zero beyond the last split
+    float o[MERGE_CHUNKS] = {};
+    for (int sp0 = 0; sp0 < nsplit; sp0 += BATCH) {
+        if (sp0) fetch(sp0);
 #pragma unroll
-                for (int u = 0; u < BATCH; ++u) v[u] = first[u];
-            } else {
-                fetch(d, sp0, v);
-            }
+        for (int u = 0; u < BATCH; ++u) {
+            const float of = of_lane(coef, min(sp0 + u, 63));  // zero beyond the last split
 #pragma unroll
-            for (int u = 0; u < BATCH; ++u) o += v[u] * __shfl(coef, min(sp0 + u, 63), WAVE);  // zero beyond the last split
+            for (int c = 0; c < MERGE_CHUNKS; ++c) o[c] += v[u][c] * of;
         }
-        if (d < hd) out[row * hd + d] = from_f32<elem_t>(o);
     }
+#pragma unroll
+    for (int c = 0; c < MERGE_CHUNKS; ++c)
+        if (lane + 64 * c < hd) out[row * hd + lane + 64 * c] = from_f32<elem_t>(o[c]);
+}
+__global__ __launch_bounds__(64) void decode_merge_kernel(const float* __restrict__ part_o, const float* __restrict__ part_ml,
+                                                          elem_t* __restrict__ out, int hd, int nsplit,
+                                                          const float* __restrict__ sinks, int H,
+                                                          const float* __restrict__ out_gate) {
+    arguments_now(part_o, part_ml, out, hd, nsplit, sinks, H, out_gate);
+    constexpr int MOST = 64 / MERGE_CHUNKS / 16 * 16;  // splits whose outputs fit the registers at once: 64, 32 or 16
+    if (nsplit <= 4) merge_row<4>(part_o, part_ml, out, hd, nsplit, sinks, H, out_gate);
+    else if (nsplit <= 8) merge_row<8>(part_o, part_ml, out, hd, nsplit, sinks, H, out_gate);
+    else if (nsplit <= 16 || MOST == 16) merge_row<16>(part_o, part_ml, out, hd, nsplit, sinks, H, out_gate);
+    else if (nsplit <= 24 || MOST < 64) merge_row<MOST == 64 ? 24 : MOST>(part_o, part_ml, out, hd, nsplit, sinks, H, out_gate);
+    else merge_row<32>(part_o, part_ml, out, hd, nsplit, sinks, H, out_gate);
 }
 
 }  // namespace ms
