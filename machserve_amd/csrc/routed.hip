@@ -528,18 +528,20 @@ __global__ __launch_bounds__(64 * FEW_WAVES) void expert_few_kernel(const elem_t
 // The tile of a product.  A step of 33 to 64 rows (and of any number up to 64 in 32-bit) has one tile of 64 rows an expert, its weight's columns streamed by blocks with
 // three steps in flight; above, the tile of the least predicted time, its tiles counted from how many rows
 // an expert can be expected to have.
-// us up, the choice of half an expert's last tile empty -> this one (2 of 8 experts of 2,816, width 2,048): 1,900 rows 120 -> 98, 1,200 102 -> 92, 700 and
-// an expert for every row 88 -> 63, 2,048 of experts of 1,408 and width 1,024 61 -> 50.
+// us up, the choice of half an expert's last tile empty -> this one (2 of 8 experts of 2,816, width 2,048): 1,900 rows 121 -> 111, 1,200 100 -> 88, 700 and
+// an expert for every row 88 -> 62, 2,048 of experts of 1,408 and width 1,024 60 -> 50.
 // 2,048 rows, 2 of 8 experts of 2,816 and one of 2,816 for every row, width 2,048, gated (us up / down): 256x256 191 / 83, 256x192 211 / 120,
 // 256x128 197 / 97, 128x128 179 / 106, 64x64 279 / 156; 128x128 alone, in the order of the columns and with the epilogue reading row by row, was 228 / 120.
 // 1,750 rows, 2 of 8 experts of 2,816: 122 / 73, 128 / 62, 130 / 87, 120 / 72 and 178 / 101 against 170 / 113.
 static int plan_experts(const ExpertArgs& g, bool down, int per) {
 #ifdef MS_ELEM_HALF
     if (g.T <= 64) return TILE_64x64_DEEP;
-    // Rows fall to the router's outputs (of which some may be no experts) as if at random: an expert has `mean` rows, give or take `spread`, and
+    // Rows fall to the router's outputs (of which some may be no experts) nearly as if at random: an expert has `mean` rows, give or take `spread` (a little more
+    // than chance gives: with chance alone the down product of 2,048 rows over nine outputs, eight of them experts, took 256x128 tiles, a round if no expert had more than 512
+    // rows, and ran two: 86 us; 256x192 59), and
     // its tiles are counted as the chances that it has more rows than each of them begins with.
     const int outputs = max(g.E, g.ld_gates - (g.shared ? 1 : 0));  // (a gate of the expert for every row is none of them)
-    const double mean = (double)g.T * g.top / outputs, spread = sqrt(mean * (1.0 - 1.0 / outputs)) + 1e-3;
+    const double mean = (double)g.T * g.top / outputs, spread = sqrt(mean * (1.0 - 1.0 / outputs)) + 0.03 * mean + 1e-3;
     int best = TILE_64x64;
     float least = INFINITY;
     for (int i = 0; i < TILE_COUNT; ++i) {
