@@ -154,7 +154,7 @@ __device__ __forceinline__ void few_rows_tile(const elem_t* __restrict__ A, cons
         const int u = u0 + wave;
         if (UNITS % KW != 0 && u >= UNITS) break;
         const int i = u / ACROSS, j = u % ACROSS * PAIR;
-        if (m0 + i * 16 >= M) continue;
+        if (m0 + i * 16 >= M || n0 + j * 16 >= N) continue;  // the same for the whole wave; beyond the last column there is no share of ss_part either
         float v[PAIR][4];
 #pragma unroll
         for (int p = 0; p < PAIR; ++p)

@@ -70,7 +70,7 @@ struct EpiArgs {
     // the rows' sums of squares
     const float* norm_w;  // [N]
     elem_t* hn;           // [M, N]
-    float* ss_part;       // [N / 16, M]
+    float* ss_part;       // [N / 16 rounded up, M]
 };
 
 // The block of rows m0 .. m0 + BM and columns n0 .. n0 + BN.  `rows` says which row of A the block's row i is and, for the

@@ -955,3 +955,22 @@ def test_products_whose_waves_share_out_k(dtype, M, N, K):
         f = 1.0 / torch.sqrt(share.double().sum(0) / K + 1e-5)[:, None]
         scaled = P.silu(P.linear(a.double(), g.double()) * f) * (P.linear(a.double(), u.double()) * f)
         assert_close(ops.linear_swiglu_scaled(ad, share.to(DEV), 1e-5, gu, N // 2 + 3), scaled, dtype, "gated with row factors")
+
+
+@pytest.mark.parametrize("M", [13, 16])
+@pytest.mark.parametrize("N,K", [(4240, 1024), (9456, 256), (4104, 320)])
+def test_sums_of_squares_of_a_last_block_that_is_part_full(M, N, K):
+    """Widths whose blocks take two or four tiles of 16 columns and whose last block has fewer: nothing is written behind the parts that the plan
+    states, and the parts add up to the rows' squares."""
+    ops = ops_for(torch.bfloat16)
+    a, w = rnd((M, K), torch.bfloat16, 81).to(DEV), rnd((N, K), torch.bfloat16, 82, K ** -0.5).to(DEV)
+    x0, nw = rnd((M, N), torch.float32, 83), (1 + rnd((N,), torch.float32, 84, 0.1)).to(DEV)
+    parts = ops._plan("ms_prenorm_parts", M, N, K)
+    assert parts == -(-N // 16)
+    x, hn, room = x0.to(DEV), torch.empty((M, N), dtype=torch.bfloat16, device=DEV), torch.full(((parts + 4) * M,), -7.0, device=DEV)
+    from machserve_amd.kernels.ops import _c_int, _ptr
+    ops._check(ops._core, ops._core.ms_linear_residual_prenorm(_ptr(a), _ptr(w), _ptr(x), _ptr(nw), _ptr(hn), _ptr(room), _c_int(M), _c_int(N),
+                                                               _c_int(K), ops._stream()))
+    assert bool((room[parts * M:] == -7.0).all())
+    assert_close(x, x0.double() + P.linear(a.cpu().double(), w.cpu().double()), torch.bfloat16, "stream")
+    assert_close(room[:parts * M].view(parts, M).sum(0), (x.cpu().double() ** 2).sum(1), torch.float32, "sums of squares")
