@@ -580,7 +580,7 @@ __global__ __launch_bounds__(256 * KG, attention_waves_per_simd<KG>()) void page
 // 16c + 8 * (l / 32) .., which is a B fragment of P^T as it stands and one 16-byte read of V^T.
 //
 // A tile that is loaded straight into LDS cannot be zeroed on its way: sixteen keys that are not there (beyond the
-// block's rows, in pages given back behind a window, in tiles past the block's range) read the block's last page or the start of the
+// block's rows, in pages given back behind a window, in tiles past the block's range) read the rest of the block's last page or the start of the
 // pool instead, are masked in the scores, and their values are overwritten with zeros (a caller's pool may hold anything in a page
 // that no request of the step owns).  Of sixteen keys that are there in part the others' values are what the page's last owner left:
 // finite, as every writer of a page sees to (cache_value), and met by probabilities of zero.
@@ -639,7 +639,7 @@ __global__ __launch_bounds__(r32::KG * r32::GT, r32::KG * r32::RW * r32::PER_CU 
     using namespace r32;
     static_assert((HDT == 64 || HDT == 128) && TK == 32 && RW == 2 && NS == 2, "the swizzles, the tiles' split over a group's waves and the rounds are written for these shapes");
     __shared__ __attribute__((aligned(1024))) unsigned char smem[SMEM];
-    __shared__ uint32_t tab[MAX_TABLE];
+    __shared__ uint32_t tab[MAX_TABLE + 1];
 
     const int kg = threadIdx.x / GT, tg = threadIdx.x % GT, lane = tg & 63, rw = tg >> 6;
     const int n32 = lane & 31, h = lane >> 5;
@@ -707,13 +707,15 @@ __global__ __launch_bounds__(r32::KG * r32::GT, r32::KG * r32::RW * r32::PER_CU 
     kv_lo = __builtin_amdgcn_readfirstlane(kv_lo);
     kv_hi = __builtin_amdgcn_readfirstlane(kv_hi);
     const int kt_first = __builtin_amdgcn_readfirstlane((kv_lo / ROUND) * ROUND);
-    const int page_first = kt_first / ps, n_tab = min(ceil_div(kv_hi, ps), a.table_stride) - page_first;
-    // (as where the head's keys, and values, of a page begin in the pool, in units of sixteen numbers; a page that was given back: the pool's start)
+    const int page_first = kt_first / ps, n_tab = max(min(ceil_div(kv_hi, ps), a.table_stride) - page_first, 0);
+    // (as where the head's keys, and values, of a page begin in the pool, in units of sixteen numbers; a page that was given back, and the place behind the
+    // last one, which stands for all that are not in the table: the pool's start)
     const uint32_t page_units = (uint32_t)(a.KV * ps * HDT) >> 4, head_units = (uint32_t)(kvh * ps * HDT) >> 4;
     for (int i = threadIdx.x; i < n_tab; i += KG * GT) {
         const int page = table[page_first + i];
         tab[i] = page >= 0 ? (uint32_t)page * page_units + head_units : 0u;
     }
+    if (threadIdx.x == 0) tab[n_tab] = 0u;
 
     Frag qf[NC];
     {
@@ -748,7 +750,7 @@ __global__ __launch_bounds__(r32::KG * r32::GT, r32::KG * r32::RW * r32::PER_CU 
     }
     // Where the tiles lie: every wave looks its group's tile up for itself, in scalars.  `look_up` asks LDS for the next tile's page (or its two 16-key groups'
     // pages), stepped from tile to tile rather than divided out; `resolve`, a round later, makes addresses of it.  (Two threads that did it for their group
-    // through LDS were a chain in every round.)  Behind the block's keys it is the last page's, as keys that are not there.
+    // through LDS were a chain in every round.)  Behind the block's pages it is the pool's start, as for keys that are not there.
     const int kg_keys = __builtin_amdgcn_readfirstlane(kg * TK);
     int lp_next = (kt_first + kg_keys) / ps - page_first, off_next = (kt_first + kg_keys) % ps;
     const int round_pages = ROUND / ps, round_rem = ROUND % ps;
@@ -756,11 +758,11 @@ __global__ __launch_bounds__(r32::KG * r32::GT, r32::KG * r32::RW * r32::PER_CU 
     uint32_t entry[NG];
     int entry_off[NG];
     auto look_up = [&]() {
-        entry[0] = tab[min(lp_next, n_tab - 1)];
+        entry[0] = tab[min(lp_next, n_tab)];
         entry_off[0] = off_next;
         if constexpr (!ONE_PAGE) {
             const bool over = off_next + 16 >= ps;
-            entry[1] = tab[min(lp_next + (over ? 1 : 0), n_tab - 1)];
+            entry[1] = tab[min(lp_next + (over ? 1 : 0), n_tab)];
             entry_off[1] = off_next + 16 - (over ? ps : 0);
         }
         lp_next += round_pages;

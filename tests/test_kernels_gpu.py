@@ -486,6 +486,25 @@ def test_attention_reads_nothing_of_keys_that_are_not_there(dtype, hd):
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("ps,window,splits", [(64, None, 1), (64, 50, 1), (64, None, 3), (16, 50, 1), (48, 50, 2)])
+def test_keys_behind_a_narrow_block_table_are_read_from_the_pool(dtype, hd, ps, window, splits):
+    """A table that holds none of the pages that a request's rows see: its keys are the pool's first page, and the requests beside it keep their results."""
+    ops, g, KV = ops_for(dtype), 3, 2
+    kp, vp = rnd((3, KV, ps, hd), dtype, 91).to(DEV), rnd((3, KV, hd, ps), dtype, 92).to(DEV)
+    n0, n1 = ps - 3, 33
+    q = rnd((n0 + n1, KV * g * hd), dtype, 93).to(DEV)
+    rows = ops.attention_rows_per_block(hd)
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)  # noqa: E731
+    work = [[(i, r) for r in range(0, n * g, rows)] for i, n in ((0, n0), (1, n1))]
+    tail = (KV * g, KV, hd, ps, window, hd ** -0.5, 32, splits)
+    alone = ops.paged_attention(q[:n0].contiguous(), kp, vp, i32([[1]]), i32([0]), i32([n0]), i32([0]), i32(work[0]), *tail)
+    both = ops.paged_attention(q, kp, vp, i32([[1], [2]]), i32([0, n0]), i32([n0, n1]), i32([0, 3000]), i32(work[0] + work[1]), *tail)
+    assert torch.equal(both[:n0], alone)
+    assert bool(torch.isfinite(both).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("hd", [64, 128])
 @pytest.mark.parametrize("ps", [16, 32, 48, 64, 96])
 def test_prompts_of_any_page_size(dtype, hd, ps):
     """Prompts whose keys end before, at and behind a tile of 32 and a round of 64 keys, in pages that hold whole tiles and in pages that do not."""
