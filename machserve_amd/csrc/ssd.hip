@@ -133,17 +133,18 @@ __global__ __launch_bounds__(256) void ssd_scan_kernel(SsdArgs a) {
 // Rows of 64 numbers in LDS, unpadded: lanes 32 .. 63 read the row four below that of lanes 0 .. 31, so column p of row r
 // lies at p ^ 32 where bit 2 of r is set, and the two halves of a wave read different banks.
 
-// e^x for x <= 80 (what lies below -150 counts as -150): the hardware's 2^p, and the part of x log2(e) that p lost to first order.
+// e^x for x <= 87 (what lies below -150 counts as -150): the hardware's 2^p, and the part of x log2(e) that p lost to first order.
 __device__ __forceinline__ float exp_near(float x) {
     x = fmaxf(x, -150.0f);
     const float p = x * 0x1.715476p+0f, rest = __builtin_fmaf(x, 0x1.4ae0bep-26f, __builtin_fmaf(x, 0x1.715476p+0f, -p));
     const float e = __builtin_amdgcn_exp2f(p);
     return __builtin_fmaf(e, rest * 0x1.62e430p-1f, e);
 }
-// z / (1 + e^-z) with the reciprocal refined once: within a unit of the last place, in half of the division's instructions
+// z / (1 + e^-z) with the reciprocal refined once: within a unit of the last place, in half of the division's instructions.  Below -87, where
+// 1 + e^-z leaves the numbers whose reciprocal is normal, the factor is zero: the result is less than 2e-36 there (-inf: NaN, as the division has it).
 __device__ __forceinline__ float silu_near(float z) {
-    const float d = 1.0f + exp_near(fminf(-z, 80.0f)), r = __builtin_amdgcn_rcpf(d);
-    return z * __builtin_fmaf(__builtin_fmaf(-d, r, 1.0f), r, r);
+    const float d = 1.0f + exp_near(fminf(-z, 87.0f)), r = __builtin_amdgcn_rcpf(d);
+    return z * (z < -87.0f ? 0.0f : __builtin_fmaf(__builtin_fmaf(-d, r, 1.0f), r, r));
 }
 
 // Per (chunk, head) in LDS, tokens in order.

@@ -214,6 +214,33 @@ def test_a_later_token_s_overflow_stays_out_of_earlier_ones():
         assert torch.equal(got[:bad], want[:bad]) and torch.equal(got[100:], want[100:])
 
 
+def _walked_and_in_chunks(monkeypatch, xbc, proj, lens, H, P_, N):
+    """y and the state of the same rows token by token and in chunks, on the CPU."""
+    ops, out = ops_of(torch.float32), []
+    torch.manual_seed(5)
+    dt_bias, a_log, d_skip = torch.randn(H), torch.randn(H) * 0.5, torch.randn(H)
+    q0 = [sum(lens[:i]) for i in range(len(lens))]
+    for chunk in (0, 128):
+        monkeypatch.setattr(type(ops), "_ssd_chunk", lambda self, *a, **k: chunk)
+        state = torch.zeros(len(lens), H, N, P_, device=DEV)
+        y = ops.ssd_scan(dev(xbc), dev(proj), 0, dev(dt_bias), dev(a_log), dev(d_skip), state, i32(q0), i32(lens), i32(range(len(lens))), H, P_, N, 1)
+        out.append((y.cpu(), state.cpu()))
+    return out
+
+
+def test_very_negative_inputs_of_the_state_space_recurrence(monkeypatch):
+    """SiLU goes to zero there: x, B and C of -80 to -3e38, walked token by token and in chunks."""
+    torch.manual_seed(4)
+    H, P_, N, T = 2, 64, 64, 300
+    xbc, proj = torch.randn(T, H * P_ + 2 * N), torch.randn(T, H)
+    for i, v in enumerate((-79.0, -84.0, -86.9, -87.1, -100.0, -1e10, -1e30, -3e38)):
+        xbc[7 + 31 * i, i::9] = v
+    (y0, s0), (y1, s1) = _walked_and_in_chunks(monkeypatch, xbc, proj, [T], H, P_, N)
+    assert bool(torch.isfinite(y0).all())
+    close(y1, y0, torch.float32, "the outputs")
+    close(s1, s0, torch.float32, "the state")
+
+
 def test_sizes_the_state_space_kernels_do_not_take_are_refused_when_the_part_is_built():
     from machserve_amd.config import StateSpaceDualSpec
     from machserve_amd.parts import MIXERS, Runtime
