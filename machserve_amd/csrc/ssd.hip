@@ -16,6 +16,7 @@ constexpr int SSD_TOK = 8;      // tokens whose B, C, dt and decay a walking blo
 constexpr int SSD_CHUNK = 128;  // most tokens of a chunk
 constexpr int SSD_HEADS = 4;    // most heads that a block takes one after the other
 constexpr int SSD_PT = 2;       // tiles of 32 value channels that a block takes
+constexpr float SSD_NOT_FINITE = 0x1.fffffep127f, SSD_LARGEST = 0x1.fffffcp127f;
 
 struct SsdArgs {
     const float* xbc;      // [T, ld_xbc]: x [H, P], B [G, N], C [G, N] before their SiLU
@@ -37,7 +38,8 @@ struct SsdArgs {
     int np, pz;            // states filled up to 64, 128 or 256; blocks of 64 value channels
     // what the chunks' kernels pass on, piece by piece (see ssd_work)
     float* states;         // [pieces, H, pz, np, 64]: what a chunk adds from zero, then the state that comes into it
-    float* x;              // [pieces, H, pz, 128, 64]: x behind its SiLU
+    float* x;              // [pieces, H, pz, 128, 64]: x behind its SiLU; what is not finite as SSD_NOT_FINITE, nothing else as large
+    float* odd;            // [pieces, H, pz, 4]: whether a quarter of those tokens (a wave's) has any such
     float* scores;         // [pieces, G, 10, 4, 64, 4]: tiles of B C^T on and below the diagonal, as the lanes hold them
     float* c;              // [pieces, G, 4, np / 8, 64, 4]: C behind its SiLU, as the lanes hold it
     float* cdec;           // [pieces, H]: the product of a chunk's decays
@@ -153,6 +155,7 @@ struct SsdGates {
     float hi[SSD_HEADS][SSD_CHUNK], lo[SSD_HEADS][SSD_CHUNK];
     float out[SSD_HEADS][SSD_CHUNK];  // dt times the decays behind the token
     float skip[SSD_HEADS];
+    __align__(16) float odd[SSD_HEADS][4];  // of the outputs' kernel: SsdArgs::odd
 };
 
 // The request's rows that a block of chunk kernels has: false if there are none.
@@ -327,6 +330,7 @@ __global__ __launch_bounds__(256, 2) void ssd_chunk_add_kernel(SsdArgs a) {
         const int h = r.h0 + hh;
         float* keep = a.x + (((size_t)r.piece * a.H + h) * a.pz + pz) * SSD_CHUNK * 64;
         const int lane = opaque(l);  // places are worked out for each head anew: kept over the loop they would fill the registers
+        bool odd = false;
         __syncthreads();  // the head before has been read
 #pragma unroll
         for (int k0 = 0; k0 < SSD_CHUNK / 4; k0 += 8)
@@ -337,11 +341,17 @@ __global__ __launch_bounds__(256, 2) void ssd_chunk_add_kernel(SsdArgs a) {
                     x[k] = silu_near(x[k]);
                     xs[(w + 4 * k) * 64 + (lane ^ (k % 2 * 32))] = x[k] * gates.out[hh][w + 4 * k];
                 }
-                if (n0 == 0) {  // in the outputs a later token meets a factor of zero: finite, so that its overflow stays its own
+                if (n0 == 0) {  // in the outputs a later token meets a factor of zero: finite, so that its overflow stays out of earlier ones
 #pragma unroll
-                    for (int k = k0; k < k0 + 8; ++k) keep[(w + 4 * k) * 64 + (lane ^ (k % 2 * 32))] = fminf(fmaxf(x[k], -0x1.fffffep127f), 0x1.fffffep127f);
+                    for (int k = k0; k < k0 + 8; ++k) {
+                        const bool finite = fabsf(x[k]) < INFINITY;
+                        odd |= !finite;
+                        keep[(w + 4 * k) * 64 + (lane ^ (k % 2 * 32))] = finite ? __builtin_amdgcn_fmed3f(x[k], -SSD_LARGEST, SSD_LARGEST) : SSD_NOT_FINITE;
+                    }
                 }
             }
+        const float any_odd = __ballot(odd) ? 1.f : 0.f;
+        if (n0 == 0 && l == 0) a.odd[(((size_t)r.piece * a.H + h) * a.pz + pz) * 4 + w] = any_odd;
         ask(min(h + 1, r.h0 + r.heads - 1));
         __syncthreads();
         if (!busy) continue;
@@ -462,6 +472,8 @@ __global__ __launch_bounds__(256, NT <= 4 ? 2 : 1) void ssd_chunk_out_kernel(Ssd
             }
         }
     }
+    if ((int)threadIdx.x < 4 * r.heads)
+        gates.odd[threadIdx.x / 4][threadIdx.x % 4] = a.odd[(first + (size_t)(r.h0 + threadIdx.x / 4) * a.pz) * 4 + threadIdx.x % 4];
     ssd_gates(a, r, gates);
     // C and the scores have arrived: a wait of the compiler's for them inside the loop would be one for the loads into LDS as well
 #pragma unroll
@@ -534,6 +546,15 @@ __global__ __launch_bounds__(256, NT <= 4 ? 2 : 1) void ssd_chunk_out_kernel(Ssd
 #pragma unroll
                         for (int i = 0; i < 16; ++i) y[pt][i] += acc[pt][i];
                 }
+            const f32x4 odd = *reinterpret_cast<const f32x4*>(gates.odd[hh]);
+            if (__builtin_amdgcn_readfirstlane((int)(odd[0] + odd[1] + odd[2] + odd[3])) != 0) {  // a channel is not finite from such an x on, as in a walk
+                for (int s = 0; s <= min(t, r.n - 1); ++s)
+#pragma unroll
+                    for (int pt = 0; pt < SSD_PT; ++pt)
+#pragma unroll
+                        for (int i = 0; i < 16; ++i)
+                            if (xs[s * 64 + ((32 * pt + row_of(i, half)) ^ ((s & 4) * 8))] == SSD_NOT_FINITE) y[pt][i] = NAN;
+            }
             if (t < r.n) {
                 float* out = a.y + (size_t)(r.row0 + t) * inner + h * a.P;
 #pragma unroll
@@ -617,7 +638,7 @@ static int launch_chunks(const SsdArgs& a, int pieces, hipStream_t stream) {
 
 // Places of the chunks' parts in their workspace, in floats; every part is a multiple of four.
 struct SsdWork {
-    size_t states, x, scores, c, cdec, end;
+    size_t states, x, scores, c, odd, cdec, end;
 };
 static int ssd_states(int N) { return N <= 64 ? 64 : N <= 128 ? 128 : 256; }
 static SsdWork ssd_work(int T, int S, int H, int P, int N, int G, int chunk) {
@@ -626,7 +647,8 @@ static SsdWork ssd_work(int T, int S, int H, int P, int N, int G, int chunk) {
     w.x = pieces * H * pz * np * 64;
     w.scores = w.x + pieces * H * pz * SSD_CHUNK * 64;
     w.c = w.scores + pieces * G * SSD_TILES * 1024;
-    w.cdec = w.c + pieces * G * 4 * (np / 8) * 256;
+    w.odd = w.c + pieces * G * 4 * (np / 8) * 256;
+    w.cdec = w.odd + pieces * H * pz * 4;
     w.end = w.cdec + pieces * H;
     return w;
 }
@@ -665,6 +687,7 @@ extern "C" int ms_ssd_scan(const float* xbc, int ld_xbc, const float* proj, int 
     a.x = work + at.x;
     a.scores = work + at.scores;
     a.c = work + at.c;
+    a.odd = work + at.odd;
     a.cdec = work + at.cdec;
     // a block's heads share its B, C and scores: as many heads as leave two blocks for every CU
     a.heads = 1;

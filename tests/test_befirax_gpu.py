@@ -241,6 +241,26 @@ def test_very_negative_inputs_of_the_state_space_recurrence(monkeypatch):
     close(s1, s0, torch.float32, "the state")
 
 
+@pytest.mark.parametrize("value", [float("nan"), float("inf"), -3.4e38, 1e37])
+@pytest.mark.parametrize("lens,bad", [([300, 60], 37), ([300, 60], 127), ([33, 290], 160), ([100, 31], 130)])
+def test_what_is_not_finite_stays_so_in_its_channel(monkeypatch, value, lens, bad):
+    """An x that is NaN or infinite: its channel of that head is not finite from that token to the request's end, in the outputs and in the
+    state, and everything else is as without it.  Large finite numbers are no such x."""
+    torch.manual_seed(6)
+    H, P_, N, T, where = 3, 80, 64, sum(lens), [5, 70, 80 + 33]  # channels of the first and the second block of a head, and of another head
+    xbc, proj = torch.randn(T, H * P_ + 2 * N), torch.randn(T, H) - 3.0
+    clean = _walked_and_in_chunks(monkeypatch, xbc, proj, lens, H, P_, N)[1]
+    xbc[bad, where] = value
+    (y0, s0), (y1, s1) = _walked_and_in_chunks(monkeypatch, xbc, proj, lens, H, P_, N)
+    assert torch.equal(torch.isfinite(y1), torch.isfinite(y0)) and torch.equal(torch.isfinite(s1), torch.isfinite(s0))
+    if not torch.isfinite(torch.tensor(value)):
+        end = lens[0] if bad < lens[0] else T
+        assert not bool(torch.isfinite(y1[bad:end, where]).any())
+        other = torch.ones_like(y1, dtype=torch.bool)
+        other[bad:end, where] = False
+        assert torch.equal(y1[other], clean[0][other])
+
+
 def test_sizes_the_state_space_kernels_do_not_take_are_refused_when_the_part_is_built():
     from machserve_amd.config import StateSpaceDualSpec
     from machserve_amd.parts import MIXERS, Runtime
