@@ -229,13 +229,7 @@ __global__ __launch_bounds__(256) void route_kernel(const elem_t* __restrict__ x
 __device__ __forceinline__ float expert_activation(float z, int act) {
     if (act == 0) return 0.5f * z * (1.0f + erff(z * 0.7071067811865476f));
     if (act == 1) return 0.5f * z * (1.0f + tanhf(0.7978845608028654f * (z + 0.044715f * z * z * z)));
-#ifdef MS_ELEM_HALF
-    // as gate_activation: exponential and reciprocal of the hardware, a unit or two in the last place of 32 bits ahead of a rounding to the element type.
-    // The up product's epilogue is all vector instructions: 2,048 rows, 2 of 8 experts of 2,816 and one for every row 173 -> 162 us.
-    return z * __builtin_amdgcn_rcpf(1.0f + __expf(-z));
-#else
     return z / (1.0f + expf(-z));
-#endif
 }
 
 // a[t, c] = act(up[t, c]) * gates[t, c / ff] for c < E * ff, act(up[t, c]) beyond (experts that every row uses, whose weight is

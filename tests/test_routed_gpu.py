@@ -180,3 +180,15 @@ def test_the_router_refuses_numbers_and_sums_that_its_kernel_does_not_assume():
             ops.route(h, w, None, top, plane=p, sums=s)
     ops.route(h, w, None, top, plane=plane, sums=sums)
     assert plane.tolist() == [[0, 1, 2, -1, -1, -1]] * T  # equal logits: the lower index wins
+
+
+@pytest.mark.parametrize("z0,z1", [(-60.0, -30.0), (-8.0, 8.0)])
+def test_the_experts_silu_is_as_exact_as_32_bits_allow(z0, z1):
+    """e^-z, the sum and the division are each right to about a unit of 32 bits, 2^-22 of the result together: it is rounded to another
+    bfloat16 than the exact result where that lies so near to the middle of two of them (2^-8 apart or more), which is one number in 8,192."""
+    from machserve_amd.kernels import get_ops
+    n = 1 << 18
+    z = torch.rand(1, n, generator=torch.Generator().manual_seed(11)) * (z1 - z0) + z0
+    got = get_ops(torch.bfloat16, DEV).expert_act(z.to(DEV), torch.ones(1, 1, device=DEV), n, "silu").cpu()
+    want = (z.double() / (1.0 + torch.exp(-z.double()))).to(torch.bfloat16)
+    assert int((got != want).sum()) <= n // 8192
