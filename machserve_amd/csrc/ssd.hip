@@ -135,18 +135,12 @@ __global__ __launch_bounds__(256) void ssd_scan_kernel(SsdArgs a) {
 // Rows of 64 numbers in LDS, unpadded: lanes 32 .. 63 read the row four below that of lanes 0 .. 31, so column p of row r
 // lies at p ^ 32 where bit 2 of r is set, and the two halves of a wave read different banks.
 
-// e^x for x <= 87 (what lies below -150 counts as -150): the hardware's 2^p, and the part of x log2(e) that p lost to first order.
+// e^x for x <= 0 (what lies below -150 counts as -150): the hardware's 2^p, and the part of x log2(e) that p lost to first order.
 __device__ __forceinline__ float exp_near(float x) {
     x = fmaxf(x, -150.0f);
     const float p = x * 0x1.715476p+0f, rest = __builtin_fmaf(x, 0x1.4ae0bep-26f, __builtin_fmaf(x, 0x1.715476p+0f, -p));
     const float e = __builtin_amdgcn_exp2f(p);
     return __builtin_fmaf(e, rest * 0x1.62e430p-1f, e);
-}
-// z / (1 + e^-z) with the reciprocal refined once: within a unit of the last place, in half of the division's instructions.  Below -87, where
-// 1 + e^-z leaves the numbers whose reciprocal is normal, the factor is zero: the result is less than 2e-36 there (-inf: NaN, as the division has it).
-__device__ __forceinline__ float silu_near(float z) {
-    const float d = 1.0f + exp_near(fminf(-z, 87.0f)), r = __builtin_amdgcn_rcpf(d);
-    return z * (z < -87.0f ? 0.0f : __builtin_fmaf(__builtin_fmaf(-d, r, 1.0f), r, r));
 }
 
 // Per (chunk, head) in LDS, tokens in order.
@@ -269,7 +263,7 @@ __device__ __forceinline__ void ssd_scores(const SsdArgs& a, int g, int tile, co
 #pragma unroll
         for (int e = 0; e < PARTS; ++e) {
 #pragma unroll
-            for (int i = 0; i < 16; ++i) C[e][i] = 32 * (part0 + e) + row_of(i, half) < a.N ? silu_near(C[e][i]) : 0.f;
+            for (int i = 0; i < 16; ++i) C[e][i] = 32 * (part0 + e) + row_of(i, half) < a.N ? silu_f(C[e][i]) : 0.f;
             if (st == w) {
 #pragma unroll
                 for (int q = 0; q < 4; ++q)
@@ -277,7 +271,7 @@ __device__ __forceinline__ void ssd_scores(const SsdArgs& a, int g, int tile, co
             }
             f32x16 acc = zero16();
 #pragma unroll
-            for (int i = 0; i < 16; ++i) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(silu_near(B[e][i]), C[e][i], acc, 0, 0, 0);
+            for (int i = 0; i < 16; ++i) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(silu_f(B[e][i]), C[e][i], acc, 0, 0, 0);
 #pragma unroll
             for (int i = 0; i < 16; ++i) sum[i] += acc[i];
         }
@@ -324,7 +318,7 @@ __global__ __launch_bounds__(256, 2) void ssd_chunk_add_kernel(SsdArgs a) {
 #pragma unroll
     for (int j = 0; j < SSD_CHUNK / 2; ++j) {
         if (j % 8 == 0) __builtin_amdgcn_sched_barrier(0);
-        B[j] = silu_near(B[j]);
+        B[j] = silu_f(B[j]);
     }
     for (int hh = 0; hh < r.heads; ++hh) {
         const int h = r.h0 + hh;
@@ -338,7 +332,7 @@ __global__ __launch_bounds__(256, 2) void ssd_chunk_add_kernel(SsdArgs a) {
                 __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
                 for (int k = k0; k < k0 + 8; ++k) {
-                    x[k] = silu_near(x[k]);
+                    x[k] = silu_f(x[k]);
                     xs[(w + 4 * k) * 64 + (lane ^ (k % 2 * 32))] = x[k] * gates.out[hh][w + 4 * k];
                 }
                 if (n0 == 0) {  // in the outputs a later token meets a factor of zero: finite, so that its overflow stays out of earlier ones

@@ -241,6 +241,16 @@ def test_very_negative_inputs_of_the_state_space_recurrence(monkeypatch):
     close(s1, s0, torch.float32, "the state")
 
 
+def test_walks_and_chunks_have_the_same_silu(monkeypatch):
+    """With B of zero the outputs are D times SiLU of x: bit for bit the same, whichever way the rows go."""
+    torch.manual_seed(8)
+    H, P_, N, T = 2, 64, 64, 300
+    xbc = torch.randn(T, H * P_ + 2 * N) * 12.0
+    xbc[:, H * P_:H * P_ + N] = 0.0
+    (y0, _), (y1, _) = _walked_and_in_chunks(monkeypatch, xbc, torch.randn(T, H), [T], H, P_, N)
+    assert torch.equal(y0, y1)
+
+
 @pytest.mark.parametrize("value", [float("nan"), float("inf"), -3.4e38, 1e37])
 @pytest.mark.parametrize("lens,bad", [([300, 60], 37), ([300, 60], 127), ([33, 290], 160), ([100, 31], 130)])
 def test_what_is_not_finite_stays_so_in_its_channel(monkeypatch, value, lens, bad):
