@@ -35,14 +35,15 @@ struct SsdArgs {
     int H, P, N, G;
     int chunk;             // tokens of a chunk (0: requests are walked)
     int heads;             // heads of a block, all of one group
+    int h0, hw, g0, gw;    // the heads h0 .. h0 + hw that a launch takes, whole groups or part of one, and their groups
     int np, pz;            // states filled up to 64, 128 or 256; blocks of 64 value channels
-    // what the chunks' kernels pass on, piece by piece (see ssd_work)
-    float* states;         // [pieces, H, pz, np, 64]: what a chunk adds from zero, then the state that comes into it
-    float* x;              // [pieces, H, pz, 128, 64]: x behind its SiLU; what is not finite as SSD_NOT_FINITE, nothing else as large
-    float* odd;            // [pieces, H, pz, 4]: whether a quarter of those tokens (a wave's) has any such
-    float* scores;         // [pieces, G, 10, 4, 64, 4]: tiles of B C^T on and below the diagonal, as the lanes hold them
-    float* c;              // [pieces, G, 4, np / 8, 64, 4]: C behind its SiLU, as the lanes hold it
-    float* cdec;           // [pieces, H]: the product of a chunk's decays
+    // what the chunks' kernels pass on, piece by piece, of the launch's hw heads and gw groups (see ssd_work)
+    float* states;         // [pieces, hw, pz, np, 64]: what a chunk adds from zero, then the state that comes into it
+    float* x;              // [pieces, hw, pz, 128, 64]: x behind its SiLU; what is not finite as SSD_NOT_FINITE, nothing else as large
+    float* odd;            // [pieces, hw, pz, 4]: whether a quarter of those tokens (a wave's) has any such
+    float* scores;         // [pieces, gw, 10, 4, 64, 4]: tiles of B C^T on and below the diagonal, as the lanes hold them
+    float* c;              // [pieces, gw, 4, np / 8, 64, 4]: C behind its SiLU, as the lanes hold it
+    float* cdec;           // [pieces, hw]: the product of a chunk's decays
 };
 
 // One request and head, token by token: a thread owns one value channel and keeps its column of the state in registers;
@@ -164,10 +165,10 @@ __device__ __forceinline__ bool ssd_rows_of(const SsdArgs& a, int head_block, Ss
     if (left <= 0) return false;
     r.n = min(left, a.chunk);
     r.row0 = a.seq_q_start[pc.s] + pc.first;
-    const int per = a.H / a.G, blocks = ceil_div(per, a.heads);
-    r.g = head_block / blocks;
-    const int first = (head_block - r.g * blocks) * a.heads;
-    r.h0 = r.g * per + first;
+    const int per = a.hw / a.gw, blocks = ceil_div(per, a.heads), group = head_block / blocks;  // (of the launch)
+    const int first = (head_block - group * blocks) * a.heads;
+    r.g = a.g0 + group;
+    r.h0 = a.h0 + group * per + first;
     r.heads = min(a.heads, per - first);
     return true;
 }
@@ -244,8 +245,8 @@ __device__ __forceinline__ void ssd_scores(const SsdArgs& a, int g, int tile, co
     if (tile >= SSD_TILES || 32 * w >= r.n) return;
     const float* rows = a.xbc + (size_t)r.row0 * a.ld_xbc + a.H * a.P + g * a.N;
     const unsigned mine = min(32 * w + col, r.n - 1) * a.ld_xbc + a.G * a.N, row = min(32 * st + col, r.n - 1) * a.ld_xbc;
-    float* c_out = a.c + (((size_t)r.piece * a.G + g) * 4 + w) * (a.np / 8) * 256 + 4 * l;
-    float* s_out = a.scores + (((size_t)r.piece * a.G + g) * SSD_TILES + tile) * 1024 + 4 * l;
+    float* c_out = a.c + (((size_t)r.piece * a.gw + g - a.g0) * 4 + w) * (a.np / 8) * 256 + 4 * l;
+    float* s_out = a.scores + (((size_t)r.piece * a.gw + g - a.g0) * SSD_TILES + tile) * 1024 + 4 * l;
     f32x16 sum = zero16();
     constexpr int PARTS = NT < 4 ? NT : 4;  // 32 states each, asked for at once
 #pragma unroll 1
@@ -288,10 +289,10 @@ __global__ __launch_bounds__(256, 2) void ssd_chunk_add_kernel(SsdArgs a) {
     __shared__ SsdGates gates;
     __shared__ __align__(16) float xs[SSD_CHUNK * 64];
     SsdRows r;
-    const int head_block = (int)blockIdx.y - a.G * SSD_SCORE_BLOCKS;
+    const int head_block = (int)blockIdx.y - a.gw * SSD_SCORE_BLOCKS;
     if (!ssd_rows_of(a, max(head_block, 0), r)) return;
     if (head_block < 0) {
-        if (blockIdx.z == 0) ssd_scores<NT>(a, blockIdx.y / SSD_SCORE_BLOCKS, __builtin_amdgcn_readfirstlane(blockIdx.y % SSD_SCORE_BLOCKS * 4 + threadIdx.x / WAVE), r);
+        if (blockIdx.z == 0) ssd_scores<NT>(a, a.g0 + blockIdx.y / SSD_SCORE_BLOCKS, __builtin_amdgcn_readfirstlane(blockIdx.y % SSD_SCORE_BLOCKS * 4 + threadIdx.x / WAVE), r);
         return;
     }
     const int pz = blockIdx.z % a.pz, n0 = blockIdx.z / a.pz * 128;
@@ -314,7 +315,7 @@ __global__ __launch_bounds__(256, 2) void ssd_chunk_add_kernel(SsdArgs a) {
     ask(r.h0);
     ssd_gates(a, r, gates);
     if ((int)threadIdx.x < r.heads && blockIdx.z == 0)
-        a.cdec[(size_t)r.piece * a.H + r.h0 + threadIdx.x] = expf(gates.hi[threadIdx.x][SSD_CHUNK - 1] + gates.lo[threadIdx.x][SSD_CHUNK - 1]);
+        a.cdec[(size_t)r.piece * a.hw + r.h0 - a.h0 + threadIdx.x] = expf(gates.hi[threadIdx.x][SSD_CHUNK - 1] + gates.lo[threadIdx.x][SSD_CHUNK - 1]);
 #pragma unroll
     for (int j = 0; j < SSD_CHUNK / 2; ++j) {
         if (j % 8 == 0) __builtin_amdgcn_sched_barrier(0);
@@ -322,7 +323,8 @@ __global__ __launch_bounds__(256, 2) void ssd_chunk_add_kernel(SsdArgs a) {
     }
     for (int hh = 0; hh < r.heads; ++hh) {
         const int h = r.h0 + hh;
-        float* keep = a.x + (((size_t)r.piece * a.H + h) * a.pz + pz) * SSD_CHUNK * 64;
+        const size_t at_head = ((size_t)r.piece * a.hw + h - a.h0) * a.pz + pz;
+        float* keep = a.x + at_head * SSD_CHUNK * 64;
         const int lane = opaque(l);  // places are worked out for each head anew: kept over the loop they would fill the registers
         bool odd = false;
         __syncthreads();  // the head before has been read
@@ -345,7 +347,7 @@ __global__ __launch_bounds__(256, 2) void ssd_chunk_add_kernel(SsdArgs a) {
                 }
             }
         const float any_odd = __ballot(odd) ? 1.f : 0.f;
-        if (n0 == 0 && l == 0) a.odd[(((size_t)r.piece * a.H + h) * a.pz + pz) * 4 + w] = any_odd;
+        if (n0 == 0 && l == 0) a.odd[at_head * 4 + w] = any_odd;
         ask(min(h + 1, r.h0 + r.heads - 1));
         __syncthreads();
         if (!busy) continue;
@@ -363,7 +365,7 @@ __global__ __launch_bounds__(256, 2) void ssd_chunk_add_kernel(SsdArgs a) {
                     for (int pt = 0; pt < SSD_PT; ++pt)
                         acc[pt] = __builtin_amdgcn_mfma_f32_32x32x2f32(B[16 * st + i], xs[(32 * st + row_of(i, half)) * 64 + 32 * (pt ^ half) + c], acc[pt], 0, 0, 0);
             }
-        float* out = a.states + ((((size_t)r.piece * a.H + h) * a.pz + pz) * a.np + n0 + w * 32) * 64;
+        float* out = a.states + (at_head * a.np + n0 + w * 32) * 64;
 #pragma unroll
         for (int pt = 0; pt < SSD_PT; ++pt)
 #pragma unroll
@@ -374,14 +376,14 @@ __global__ __launch_bounds__(256, 2) void ssd_chunk_add_kernel(SsdArgs a) {
 // S_in(chunk + 1) = (product of the chunk's decays) * S_in(chunk) + what the chunk adds, from the slot's state, which takes
 // what comes out of the request's last chunk; zeros in the places of states and channels that are not there.
 __global__ __launch_bounds__(256) void ssd_carry_kernel(SsdArgs a) {
-    const int s = blockIdx.x, h = blockIdx.y, i = (blockIdx.z * 256 + threadIdx.x) * 4;
+    const int s = blockIdx.x, h = a.h0 + blockIdx.y, i = (blockIdx.z * 256 + threadIdx.x) * 4;
     const int n_pieces = ceil_div(a.seq_q_len[s], a.chunk), size = a.pz * a.np * 64;
     if (i >= size || n_pieces <= 0) return;
-    const size_t piece0 = piece_base(s, a.chunk, a.seq_q_start), hop = (size_t)a.H * size;
+    const size_t piece0 = piece_base(s, a.chunk, a.seq_q_start), hop = (size_t)a.hw * size;
     const int n = i / 64 % a.np, p = i / (64 * a.np) * 64 + (i % 64 ^ (n & 4) * 8);
     float* slot = a.state + (((size_t)a.seq_slot[s] * a.H + h) * a.N + n) * a.P + p;
-    float* at = a.states + (piece0 * a.H + h) * size + i;
-    const float* cd = a.cdec + piece0 * a.H + h;
+    float* at = a.states + (piece0 * a.hw + blockIdx.y) * size + i;
+    const float* cd = a.cdec + piece0 * a.hw + blockIdx.y;
     f32x4 Sin;
     bool there[4];
 #pragma unroll
@@ -397,7 +399,7 @@ __global__ __launch_bounds__(256) void ssd_carry_kernel(SsdArgs a) {
         for (int k = 0; k < BATCH; ++k) {
             const int piece = min(k0 + k, n_pieces - 1);
             add[k] = *reinterpret_cast<const f32x4*>(at + piece * hop);
-            dec[k] = cd[(size_t)piece * a.H];
+            dec[k] = cd[(size_t)piece * a.hw];
         }
 #pragma unroll
         for (int k = 0; k < BATCH; ++k)
@@ -426,14 +428,14 @@ __global__ __launch_bounds__(256, NT <= 4 ? 2 : 1) void ssd_chunk_out_kernel(Ssd
     // wave 3's tokens have four tiles of scores, wave 0's one: every other block the other way round, so that a SIMD with waves of two blocks has both
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), w = (blockIdx.y & 1) ? 3 - wave : wave;
     const unsigned xs_at = (unsigned)(uintptr_t)(__attribute__((address_space(3))) float*)xs, ss_at = (unsigned)(uintptr_t)(__attribute__((address_space(3))) float*)ss;
-    const size_t first = (size_t)r.piece * a.H * a.pz + blockIdx.z;
+    const size_t first = (size_t)r.piece * a.hw * a.pz + blockIdx.z;
     auto ask_state = [&](int h) {
-        const float* from = a.states + (first + (size_t)h * a.pz) * NP * 64 + threadIdx.x * 4;
+        const float* from = a.states + (first + (size_t)(h - a.h0) * a.pz) * NP * 64 + threadIdx.x * 4;
 #pragma unroll
         for (int i = 0; i < NP / 16; ++i) to_lds(from + i * 1024, ss_at + i * 4096 + wave * 1024);
     };
     auto ask_x = [&](int h) {
-        const float* from = a.x + (first + (size_t)h * a.pz) * SSD_CHUNK * 64 + threadIdx.x * 4;
+        const float* from = a.x + (first + (size_t)(h - a.h0) * a.pz) * SSD_CHUNK * 64 + threadIdx.x * 4;
 #pragma unroll
         for (int i = 0; i < SSD_CHUNK / 16; ++i) to_lds(from + i * 1024, xs_at + i * 4096 + wave * 1024);
     };
@@ -443,8 +445,8 @@ __global__ __launch_bounds__(256, NT <= 4 ? 2 : 1) void ssd_chunk_out_kernel(Ssd
 #pragma unroll
     for (int j = 0; j < NT * 16; ++j) C[j] = 0.f;
     {
-        const float* c_in = a.c + (((size_t)r.piece * a.G + r.g) * 4 + w) * (NP / 8) * 256 + 4 * l;
-        const float* s_in = a.scores + (((size_t)r.piece * a.G + r.g) * SSD_TILES + w * (w + 1) / 2) * 1024 + 4 * l;
+        const float* c_in = a.c + (((size_t)r.piece * a.gw + r.g - a.g0) * 4 + w) * (NP / 8) * 256 + 4 * l;
+        const float* s_in = a.scores + (((size_t)r.piece * a.gw + r.g - a.g0) * SSD_TILES + w * (w + 1) / 2) * 1024 + 4 * l;
         if (busy) {
 #pragma unroll
             for (int q = 0; q < NT * 4; ++q) {
@@ -467,7 +469,7 @@ __global__ __launch_bounds__(256, NT <= 4 ? 2 : 1) void ssd_chunk_out_kernel(Ssd
         }
     }
     if ((int)threadIdx.x < 4 * r.heads)
-        gates.odd[threadIdx.x / 4][threadIdx.x % 4] = a.odd[(first + (size_t)(r.h0 + threadIdx.x / 4) * a.pz) * 4 + threadIdx.x % 4];
+        gates.odd[threadIdx.x / 4][threadIdx.x % 4] = a.odd[(first + (size_t)(r.h0 - a.h0 + threadIdx.x / 4) * a.pz) * 4 + threadIdx.x % 4];
     ssd_gates(a, r, gates);
     // C and the scores have arrived: a wait of the compiler's for them inside the loop would be one for the loads into LDS as well
 #pragma unroll
@@ -618,10 +620,10 @@ static void launch_walk(const SsdArgs& a, hipStream_t stream) {
 
 template <int NT>
 static int launch_chunks(const SsdArgs& a, int pieces, hipStream_t stream) {
-    const int head_blocks = a.G * ceil_div(a.H / a.G, a.heads);
-    hipLaunchKernelGGL(ssd_chunk_add_kernel<NT>, dim3(pieces, a.G * SSD_SCORE_BLOCKS + head_blocks, a.pz * ceil_div(a.N, 128)), dim3(256), 0, stream, a);
+    const int head_blocks = a.gw * ceil_div(a.hw / a.gw, a.heads);
+    hipLaunchKernelGGL(ssd_chunk_add_kernel<NT>, dim3(pieces, a.gw * SSD_SCORE_BLOCKS + head_blocks, a.pz * ceil_div(a.N, 128)), dim3(256), 0, stream, a);
     if (int rc = check_launch("ssd_scan, chunks from zero")) return rc;
-    hipLaunchKernelGGL(ssd_carry_kernel, dim3(a.S, a.H, ceil_div(a.pz * a.np * 16, 256)), dim3(256), 0, stream, a);
+    hipLaunchKernelGGL(ssd_carry_kernel, dim3(a.S, a.hw, ceil_div(a.pz * a.np * 16, 256)), dim3(256), 0, stream, a);
     if (int rc = check_launch("ssd_scan, states between chunks")) return rc;
     const dim3 grid(pieces, head_blocks, a.pz);
     // four numbers a store where every head's channels start at a multiple of four
@@ -647,17 +649,32 @@ static SsdWork ssd_work(int T, int S, int H, int P, int N, int G, int chunk) {
     return w;
 }
 
-// floats of the workspace of ms_ssd_scan in chunks
-extern "C" long ms_ssd_chunk_floats(int T, int S, int H, int P, int N, int G, int chunk) {
-    if (T <= 0 || S <= 0 || H <= 0 || P <= 0 || N <= 0 || G <= 0 || chunk <= 0) return 0;
-    return (long)ssd_work(T, S, H, P, N, G, chunk).end;
+// Heads that go through the chunks' kernels at a time (heads are independent, and their groups' scores are worked out by every launch that has heads of
+// them): all, or as many whole groups, or of one group as many heads, as a workspace of `floats` and a grid hold, and at least one.
+static int ssd_heads_at_a_time(int T, int S, int H, int P, int N, int G, int chunk, size_t floats) {
+    constexpr int MOST = 65535;
+    const int per = H / G;
+    if (ssd_work(T, S, H, P, N, G, chunk).end <= floats && H + SSD_SCORE_BLOCKS * G <= MOST) return H;
+    const size_t group = ssd_work(T, S, per, P, N, 1, chunk).end, head = ssd_work(T, S, 2, P, N, 1, chunk).end - ssd_work(T, S, 1, P, N, 1, chunk).end;
+    const size_t groups = min(floats / group, (size_t)(MOST / (per + SSD_SCORE_BLOCKS)));
+    const auto evenly = [](int all, int most) { return ceil_div(all, ceil_div(all, most)); };
+    if (groups >= 1) return evenly(G, (int)min(groups, (size_t)G)) * per;
+    const size_t scores = ssd_work(T, S, 1, P, N, 1, chunk).end - head, left = floats > scores ? floats - scores : 0;
+    return evenly(per, (int)max(min(left / head, (size_t)min(per, MOST - SSD_SCORE_BLOCKS)), (size_t)1));
+}
+
+// floats of a workspace of ms_ssd_scan in chunks: what all heads take, or if that is more than `most`, what as many of them take as need no more (one at least).
+extern "C" long ms_ssd_chunk_floats(int T, int S, int H, int P, int N, int G, int chunk, long most) {
+    if (T <= 0 || S <= 0 || H <= 0 || P <= 0 || N <= 0 || G <= 0 || H % G || chunk <= 0 || most <= 0) return 0;
+    const int heads = ssd_heads_at_a_time(T, S, H, P, N, G, chunk, (size_t)most);
+    return (long)ssd_work(T, S, heads, P, N, max(1, heads / (H / G)), chunk).end;
 }
 
 // chunk 0: every request's rows in one walk.  Else chunks of that many tokens, numbered as pieces of a step are (T / chunk + S of
-// them); `work` is float [ms_ssd_chunk_floats], 16-byte aligned.
+// them); `work` is float [work_floats], 16-byte aligned: what ms_ssd_chunk_floats says for any limit.
 extern "C" int ms_ssd_scan(const float* xbc, int ld_xbc, const float* proj, int ld_proj, int dt_col, const float* dt_bias, const float* a_log,
                            const float* d_skip, float* state, const int* seq_q_start, const int* seq_q_len, const int* seq_slot, int S, float* y,
-                           int T, int H, int P, int N, int G, int chunk, float* work, hipStream_t stream) {
+                           int T, int H, int P, int N, int G, int chunk, float* work, long work_floats, hipStream_t stream) {
     MS_REQUIRE(T > 0 && S > 0 && H > 0 && G > 0 && H % G == 0, "ssd_scan: %d rows of %d requests, %d heads in %d groups", T, S, H, G);
     MS_REQUIRE(P >= 1 && P <= SSD_MAX_HEAD && N >= 1 && N <= SSD_MAX_STATES, "ssd_scan: heads of %d (at most %d) with %d states (at most %d)", P,
                SSD_MAX_HEAD, N, SSD_MAX_STATES);
@@ -672,7 +689,9 @@ extern "C" int ms_ssd_scan(const float* xbc, int ld_xbc, const float* proj, int 
     MS_REQUIRE(chunk > 0 && chunk <= SSD_CHUNK && work && (uintptr_t)work % 16 == 0, "ssd_scan: chunks of %d rows (at most %d) or without their workspace",
                chunk, SSD_CHUNK);
     MS_REQUIRE((long)ld_xbc * SSD_CHUNK < (1L << 30), "ssd_scan: rows of %d numbers", ld_xbc);
-    const SsdWork at = ssd_work(T, S, H, P, N, G, chunk);
+    const int per = H / G, together = ssd_heads_at_a_time(T, S, H, P, N, G, chunk, (size_t)max(work_floats, 0L));
+    const SsdWork at = ssd_work(T, S, together, P, N, max(1, together / per), chunk);
+    MS_REQUIRE((size_t)work_floats >= at.end, "ssd_scan: a workspace of %ld numbers, %zu are needed", work_floats, at.end);
     const int pieces = T / chunk + S;
     a.chunk = chunk;
     a.np = ssd_states(N);
@@ -683,12 +702,18 @@ extern "C" int ms_ssd_scan(const float* xbc, int ld_xbc, const float* proj, int 
     a.c = work + at.c;
     a.odd = work + at.odd;
     a.cdec = work + at.cdec;
-    // a block's heads share its B, C and scores: as many heads as leave two blocks for every CU
-    a.heads = 1;
-    while (a.heads < SSD_HEADS && (long)pieces * H * a.pz / (2 * a.heads) >= 2 * compute_units()) a.heads *= 2;
-    if (a.np == 64) return launch_chunks<2>(a, pieces, stream);
-    if (a.np == 128) return launch_chunks<4>(a, pieces, stream);
-    return launch_chunks<8>(a, pieces, stream);
+    for (int h = 0; h < H; h += a.hw) {
+        a.h0 = h;
+        a.hw = min(together, together >= per ? H - h : per - h % per);
+        a.g0 = h / per;
+        a.gw = max(1, a.hw / per);
+        // a block's heads share its B, C and scores: as many heads as leave two blocks for every CU
+        a.heads = 1;
+        while (a.heads < SSD_HEADS && (long)pieces * a.hw * a.pz / (2 * a.heads) >= 2 * compute_units()) a.heads *= 2;
+        if (int rc = a.np == 64 ? launch_chunks<2>(a, pieces, stream) : a.np == 128 ? launch_chunks<4>(a, pieces, stream) : launch_chunks<8>(a, pieces, stream))
+            return rc;
+    }
+    return 0;
 }
 
 extern "C" int ms_gated_group_norm(const float* y, const float* z, int ld_z, const float* w, void* out, int ld_out, int T, int n, int parts,

@@ -1551,23 +1551,25 @@ class HipOps:
         work = None
         if chunk:
             lib.ms_ssd_chunk_floats.restype = ctypes.c_long
-            work = torch.empty(lib.ms_ssd_chunk_floats(_c_int(T), _c_int(S), _c_int(H), _c_int(P), _c_int(N), _c_int(G), _c_int(chunk)),
-                               dtype=torch.float32, device=xbc.device)
+            work = torch.empty(lib.ms_ssd_chunk_floats(_c_int(T), _c_int(S), _c_int(H), _c_int(P), _c_int(N), _c_int(G), _c_int(chunk),
+                                                       ctypes.c_long(self.SSD_WORK_BYTES // 4)), dtype=torch.float32, device=xbc.device)
         self._check(lib, lib.ms_ssd_scan(_ptr(xbc), _c_int(xbc.shape[1]), _ptr(proj), _c_int(proj.shape[1]), _c_int(dt_col), _ptr(dt_bias),
                                          _ptr(a_log), _ptr(d_skip), _ptr(state), _ptr(seq_q_start), _ptr(seq_q_len), _ptr(seq_slot), _c_int(S),
                                          _ptr(y), _c_int(T), _c_int(H), _c_int(P), _c_int(N), _c_int(G), _c_int(chunk), _ptr(work),
-                                         self._stream()))
+                                         ctypes.c_long(work.numel() if work is not None else 0), self._stream()))
         return y
 
     SSD_SEGMENT = 128  # tokens of a chunk of the state-space recurrence
     SSD_CHUNK_MIN_ROWS = 48  # steps with this many rows a request on average are cut into chunks
+    SSD_WORK_BYTES = 256 << 20  # most of the chunks' workspace: heads go in turn where all of them would need more (one at a time takes what it needs)
 
     def _ssd_chunk(self, T: int, S: int, H: int, N: int) -> int:
         """Tokens of a chunk for a step of ``T`` rows in ``S`` requests, 0: its requests are walked token by token.  A walk takes 2 us a
         token and state of 128 whatever runs beside it, chunks 25 to 50 us a request that has the chip for itself: heads of 64 with 128
         states, walked / in chunks, us: 64 heads, one request of 16 rows 51 / 27, of 128 264 / 46; sixteen requests of 32 rows 102 / 99,
-        of 48 140 / 120; 8 heads of 32 with 16 states, 32 rows 22 / 22, 48 rows 31 / 25.  The chunks' workspace is a state for every chunk:
-        with portions this long no more than a few times the layer's output."""
+        of 48 140 / 120; 8 heads of 32 with 16 states, 32 rows 22 / 22, 48 rows 31 / 25.  The chunks' workspace is
+        a state and x for every chunk and head, states and channels filled up: (T / 128 + S) ceil(P / 64) 64 (states + 128) numbers a head, up to
+        :attr:`SSD_WORK_BYTES` (2,048 rows of 64 heads of 64 with 128 states: 73 MB)."""
         rows = T // S
         least = min(self.SSD_CHUNK_MIN_ROWS, self.SCAN_CHUNK_MIN_ROWS // 2)
         few = rows >= 16 and N >= 64 and S * H <= 256

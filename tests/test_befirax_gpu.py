@@ -271,6 +271,49 @@ def test_what_is_not_finite_stays_so_in_its_channel(monkeypatch, value, lens, ba
         assert torch.equal(y1[other], clean[0][other])
 
 
+@pytest.mark.parametrize("H,G,P_,N", [(6, 2, 64, 64), (5, 1, 33, 100), (6, 6, 80, 16), (12, 4, 64, 200)])
+def test_heads_that_go_through_the_chunks_in_turn(monkeypatch, H, G, P_, N):
+    """A smaller workspace: several groups at a time, one, part of one, a single head; the bits are those of all heads together."""
+    ops = ops_of(torch.float32)
+    torch.manual_seed(9)
+    lens = [200, 129, 70]
+    T, q0 = sum(lens), [0, 200, 329]
+    xbc, proj, vec = torch.randn(T, H * P_ + 2 * G * N), torch.randn(T, H), torch.randn(3, H) * 0.5
+    asked = []
+
+    def run(most):
+        monkeypatch.setattr(type(ops), "SSD_WORK_BYTES", most)
+        state = torch.zeros(3, H, N, P_, device=DEV)
+        args = [dev(xbc), dev(proj), 0, dev(vec[0]), dev(vec[1]), dev(vec[2]), state, i32(q0), i32(lens), i32([0, 1, 2]), H, P_, N, G]
+        torch.cuda.synchronize()
+        torch.cuda.reset_peak_memory_stats()
+        before = torch.cuda.memory_allocated()
+        y = ops.ssd_scan(*args)
+        asked.append(torch.cuda.max_memory_allocated() - before - y.numel() * 4)
+        return y.cpu(), state.cpu()
+
+    want = run(1 << 40)
+    one = run(4)  # a head at a time, whatever it takes
+    assert torch.equal(one[0], want[0]) and torch.equal(one[1], want[1]) and asked[1] <= asked[0] / H * 2 + 1024
+    for part in (0.2, 0.35, 0.6, 0.9):
+        most = int(asked[0] * part)
+        got = run(most)
+        assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+        assert asked[-1] <= max(most, asked[1]) + 1024
+
+
+def test_the_workspace_of_a_long_step_of_many_heads_is_bounded():
+    ops = ops_of(torch.float32)
+    T, H, P_, N = 8192, 64, 64, 256
+    xbc, proj, vec = torch.randn(T, H * P_ + 2 * N, device=DEV), torch.randn(T, H, device=DEV), torch.zeros(H, device=DEV)
+    state, at = torch.zeros(1, H, N, P_, device=DEV), (i32([0]), i32([T]), i32([0]))
+    torch.cuda.synchronize()
+    torch.cuda.reset_peak_memory_stats()
+    before = torch.cuda.memory_allocated()
+    y = ops.ssd_scan(xbc, proj, 0, vec, vec, vec, state, *at, H, P_, N, 1)
+    assert torch.cuda.max_memory_allocated() - before <= y.numel() * 4 + (256 << 20) + 4096
+
+
 def test_sizes_the_state_space_kernels_do_not_take_are_refused_when_the_part_is_built():
     from machserve_amd.config import StateSpaceDualSpec
     from machserve_amd.parts import MIXERS, Runtime
