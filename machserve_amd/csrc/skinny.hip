@@ -628,14 +628,13 @@ extern "C" int ms_linear_act_skinny(const void* a, const void* w, void* out, int
     return launch_skinny<SK_ACT>(args, plan_skinny(M, N, K, false), stream);
 }
 
-// Whether ms_linear_swiglu_scaled_skinny takes this shape, and is the faster of the two forms for it: one
+// Whether ms_linear_swiglu_scaled_skinny takes this shape, and is the faster form for it where few_rows.cuh does not take it: one
 // tile of rows, and so few waves that all of them are on the chip at once (sixteen a CU), each
 // waiting for its one trip to memory.  (0.5B gate/up, 304 blocks: 9.9 us tiled with three K steps in flight,
 // which multiplies 64-row tiles of padding and ends in a long epilogue; the walk over K there is bound by
 // its own instructions, not by memory.)
 extern "C" int ms_swiglu_scaled_skinny_takes(int M, int I, int K) {
     if (!kHalf || !kRoundsBeforeTheNormIsSafe || M < 1 || M > 16 || K % 8) return 0;
-    if (K % 64 == 0 && K >= 256) return 0;  // few_rows.cuh
     const int n = 2 * ceil_div(I, 16) * 16;
     const SkinnyPlan p = plan_skinny(M, n, K, false, true);
     return ceil_div(n, 32 * p.wn) * p.wn * p.ksi <= 16 * compute_units();  // sixteen waves a CU

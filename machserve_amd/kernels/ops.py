@@ -281,13 +281,24 @@ class HipOps:
         (two-byte elements, whole K steps, up to 16 rows always)."""
         return M <= self.SKINNY_ROWS and bool(self._plan("ms_few_rows_takes", M, N, K, int(slices), int(pairs)))
 
+    @staticmethod
+    def _aligned(a: torch.Tensor, w: torch.Tensor) -> bool:
+        """Whether both operands begin where 16 bytes do, as the tiled entry points want it.  Products that no tile is the choice for are taken at
+        any address, by the kernels of ``skinny.hip``."""
+        return (a.data_ptr() | w.data_ptr()) % 16 == 0
+
+    def _through_tiles(self, a: torch.Tensor, w: torch.Tensor, slices: bool, pairs: bool = False) -> bool:
+        """Whether this product goes to the entry points of the tiled products."""
+        (M, K), N = a.shape, w.shape[0]
+        return (self._few(M, N, K, slices, pairs) and self._aligned(a, w)) or self._tiled(M, N, K)
+
     def linear_split(self, a: torch.Tensor, w: torch.Tensor, allow_partials: bool = True) -> torch.Tensor:
         """Float32 ``[P, M, N]`` whose sum over P is ``a @ w.T``.  Within one kernel family the cut
         of K depends on N and K only, so the consumer that adds the parts sees the same sums for a row
         whatever else is in the batch; which family runs depends on the number of rows (see
         :meth:`_few` and :meth:`_tiled`), and they differ in rounding."""
         M, N, K = self._mm_operands(a, w, "linear_split")
-        if self._few(M, N, K, allow_partials) or self._tiled(M, N, K):
+        if self._through_tiles(a, w, allow_partials):
             P = self._plan("ms_tiled_partials", M, N, K) if allow_partials else 1
             if P == 1:
                 return self.linear(a, w, None, out_f32=True).unsqueeze(0)
@@ -305,7 +316,7 @@ class HipOps:
                out_f32: bool = False) -> torch.Tensor:
         """``a @ w.T (+ bias)``; 32-bit output on request (logits)."""
         M, N, K = self._mm_operands(a, w, "linear")
-        if not self._few(M, N, K, False) and not self._tiled(M, N, K) and out_f32 and bias is None:
+        if out_f32 and bias is None and not self._through_tiles(a, w, False):
             return self.linear_split(a, w, allow_partials=False)[0]
         if bias is not None:
             self._want(bias, torch.float32, "linear bias", N)
@@ -321,7 +332,7 @@ class HipOps:
         in; otherwise None."""
         M, N, K = self._mm_operands(a, w, "linear_residual")
         self._want(x, torch.float32, "residual stream", M, N)
-        if not self._few(M, N, K, True) and not self._tiled(M, N, K):
+        if not self._through_tiles(a, w, True):
             if M > 32 or self._plan("ms_skinny_partials", M, N, K, 1) > 1:
                 return self.linear_split(a, w)
             # all of K inside one block: one writer an element, added in the epilogue (up to 32 rows the
@@ -350,7 +361,7 @@ class HipOps:
         M, N, K = self._mm_operands(a, w, "linear_residual_prenorm")
         self._want(x, torch.float32, "residual stream", M, N)
         self._want(norm_w, torch.float32, "norm weight", N)
-        parts, fn = self._plan("ms_prenorm_parts", M, N, K), self._core.ms_linear_residual_prenorm
+        parts, fn = self._plan("ms_prenorm_parts", M, N, K) if self._aligned(a, w) else 0, self._core.ms_linear_residual_prenorm
         if parts < 1:
             parts, fn = self._plan("ms_skinny_prenorm_parts", M, N, K), self._core.ms_linear_residual_prenorm_skinny
         if parts < 1:
@@ -370,8 +381,9 @@ class HipOps:
             raise KernelError(f"linear_swiglu_scaled: interleaved weight has {N} rows for intermediate size {intermediate}")
         self._want(row_ss, torch.float32, "linear_swiglu_scaled sums of squares", row_ss.shape[0], M)
         out = torch.empty((M, intermediate), dtype=self.dtype, device=hn.device)
-        few_rows = bool(self._plan("ms_swiglu_scaled_skinny_takes", M, intermediate, K))
-        fn = self._core.ms_linear_swiglu_scaled_skinny if few_rows else self._core.ms_linear_swiglu_scaled
+        few_rows = self._few(M, N, K, False, True) and self._aligned(hn, w_gate_up)
+        skinny = not few_rows and bool(self._plan("ms_swiglu_scaled_skinny_takes", M, intermediate, K))
+        fn = self._core.ms_linear_swiglu_scaled_skinny if skinny else self._core.ms_linear_swiglu_scaled
         self._check(self._core, fn(_ptr(hn), _ptr(row_ss), _c_int(row_ss.shape[0]), _c_float(eps), _ptr(w_gate_up), _ptr(out),
                                    _c_int(M), _c_int(intermediate), _c_int(K), _c_int(act), self._stream()))
         return out
@@ -385,8 +397,7 @@ class HipOps:
         if N != 2 * ((intermediate + 15) // 16) * 16:
             raise KernelError(f"linear_swiglu: interleaved weight has {N} rows for intermediate size {intermediate}")
         out = torch.empty((M, intermediate), dtype=self.dtype, device=a.device)
-        tiled = self._few(M, N, K, False, True) or self._tiled(M, N, K)
-        fn = self._core.ms_linear_swiglu if tiled else self._core.ms_linear_swiglu_skinny
+        fn = self._core.ms_linear_swiglu if self._through_tiles(a, w_gate_up, False, True) else self._core.ms_linear_swiglu_skinny
         self._check(self._core, fn(_ptr(a), _ptr(w_gate_up), _ptr(out), _c_int(M), _c_int(intermediate), _c_int(K),
                                    _c_int(act), self._stream()))
         return out
@@ -397,7 +408,7 @@ class HipOps:
             raise KernelError(f"linear_act: activation {activation!r} is not built (built: {', '.join(sorted(UNARY_ACTIVATIONS))})")
         M, N, K = self._mm_operands(a, w, "linear_act")
         out = torch.empty((M, N), dtype=self.dtype, device=a.device)
-        fn = self._core.ms_linear_act if self._few(M, N, K, False) or self._tiled(M, N, K) else self._core.ms_linear_act_skinny
+        fn = self._core.ms_linear_act if self._through_tiles(a, w, False) else self._core.ms_linear_act_skinny
         self._check(self._core, fn(_ptr(a), _ptr(w), _ptr(out), _c_int(M), _c_int(N), _c_int(K), _c_int(UNARY_ACTIVATIONS[activation]),
                                    self._stream()))
         return out

@@ -993,3 +993,41 @@ def test_sums_of_squares_of_a_last_block_that_is_part_full(M, N, K):
     assert bool((room[parts * M:] == -7.0).all())
     assert_close(x, x0.double() + P.linear(a.cpu().double(), w.cpu().double()), torch.bfloat16, "stream")
     assert_close(room[:parts * M].view(parts, M).sum(0), (x.cpu().double() ** 2).sum(1), torch.float32, "sums of squares")
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M,N,K", [(1, 896, 896), (3, 1000, 320), (6, 448, 1024), (4, 72, 2048)])
+def test_few_rows_whose_operands_begin_at_any_multiple_of_eight_bytes(dtype, M, N, K):
+    """Operands that are views into a buffer: products that no tile is the choice for are taken as they lie, whole K steps or not."""
+    from machserve_amd.kernels import interleave_gate_up
+    ops = ops_for(dtype)
+    if ops._tiled(M, N, K):
+        pytest.skip("a tile is the choice for this one, whose operands are aligned")
+
+    def off(t):  # the same numbers eight bytes behind a multiple of sixteen
+        room = torch.empty(t.numel() + 12, dtype=t.dtype, device=DEV)
+        at = 4 if room.data_ptr() % 16 == 0 else 0
+        room[at:at + t.numel()] = t.flatten().to(DEV)
+        return room[at:at + t.numel()].view(t.shape)
+
+    a, w, x0, nw = rnd((M, K), dtype, 91), rnd((N, K), dtype, 92, K ** -0.5), rnd((M, N), torch.float32, 93), 1 + rnd((N,), torch.float32, 94, 0.1)
+    g, u = rnd((N, K), dtype, 95, K ** -0.5), rnd((N, K), dtype, 96, K ** -0.5)
+    ref, ad, wd, gu = P.linear(a.double(), w.double()), off(a), off(w), off(interleave_gate_up(g, u))
+    assert ad.data_ptr() % 16 == 8 and wd.data_ptr() % 16 == 8 and ad.is_contiguous()
+    assert_close(ops.linear_split(ad, wd).sum(0), ref, dtype, "slices")
+    assert_close(ops.linear(ad, wd, None, out_f32=True), ref, dtype, "whole")
+    assert_close(ops.linear_act(ad, wd, "relu2"), torch.relu(ref) ** 2, dtype, "activation")
+    x = x0.to(DEV)
+    pend = ops.linear_residual(ad, wd, x)
+    assert_close(x.cpu() - x0 if pend is None else pend.sum(0), ref, dtype, "into the stream")
+    pg, pu = P.linear(a.double(), g.double()), P.linear(a.double(), u.double())
+    assert_close(ops.linear_swiglu(ad, gu, N), P.silu(pg) * pu, dtype, "gated")
+    if ops._plan("ms_skinny_prenorm_parts", M, N, K):
+        xd = x0.to(DEV)
+        hn, ss = ops.linear_residual_prenorm(ad, wd, xd, nw.to(DEV))
+        assert_close(xd, x0.double() + ref, dtype, "stream")
+        assert_close(ss.sum(0), (xd.cpu().double() ** 2).sum(1), torch.float32, "sums of squares")
+    if ops._plan("ms_swiglu_scaled_skinny_takes", M, N, K):
+        share = rnd((5, M), torch.float32, 97).abs() * K
+        f = 1.0 / torch.sqrt(share.double().sum(0) / K + 1e-5)[:, None]
+        assert_close(ops.linear_swiglu_scaled(ad, share.to(DEV), 1e-5, gu, N), P.silu(pg * f) * (pu * f), dtype, "gated with row factors")
