@@ -1558,7 +1558,7 @@ class HipOps:
         self._want(state, torch.float32, "ssd state", state.shape[0], H, N, P)
         S = self._seq_operands("ssd", seq_q_start, seq_q_len, seq_slot)
         y = torch.empty((T, H * P), dtype=torch.float32, device=xbc.device)
-        chunk = self._ssd_chunk(T, S, H, N)
+        chunk = self._ssd_chunk(T, S, H, N, xbc.shape[1])
         work = None
         if chunk:
             lib.ms_ssd_chunk_floats.restype = ctypes.c_long
@@ -1574,7 +1574,7 @@ class HipOps:
     SSD_CHUNK_MIN_ROWS = 48  # steps with this many rows a request on average are cut into chunks
     SSD_WORK_BYTES = 256 << 20  # most of the chunks' workspace: heads go in turn where all of them would need more (one at a time takes what it needs)
 
-    def _ssd_chunk(self, T: int, S: int, H: int, N: int) -> int:
+    def _ssd_chunk(self, T: int, S: int, H: int, N: int, row: int = 0) -> int:
         """Tokens of a chunk for a step of ``T`` rows in ``S`` requests, 0: its requests are walked token by token.  A walk takes 2 us a
         token and state of 128 whatever runs beside it, chunks 25 to 50 us a request that has the chip for itself: heads of 64 with 128
         states, walked / in chunks, us: 64 heads, one request of 16 rows 51 / 27, of 128 264 / 46; sixteen requests of 32 rows 102 / 99,
@@ -1584,7 +1584,8 @@ class HipOps:
         rows = T // S
         least = min(self.SSD_CHUNK_MIN_ROWS, self.SCAN_CHUNK_MIN_ROWS // 2)
         few = rows >= 16 and N >= 64 and S * H <= 256
-        return min(self.SSD_SEGMENT, T) if rows >= least or few else 0
+        near = row < 1 << 23  # numbers of a row of x, B and C: the chunks' kernels count a chunk's bytes in 32 bits
+        return min(self.SSD_SEGMENT, T) if near and (rows >= least or few) else 0
 
     def gated_group_norm(self, y: torch.Tensor, proj: torch.Tensor, z_col: int, weight: torch.Tensor, eps: float, groups: int,
                          out_cols: int) -> torch.Tensor:

@@ -285,3 +285,10 @@ def test_a_layer_without_feed_forward_may_bring_its_unused_tensors(tmp_path):
     save_file(w, path)
     with pytest.raises(WeightsError, match="l2.mlp.router"):
         loaded(d)
+
+
+def test_rows_that_the_recurrence_in_chunks_does_not_reach_are_walked():
+    """Its kernels count the bytes of a chunk's 128 rows in 32 bits; wider rows go token by token, as they did before there were chunks."""
+    from machserve_amd.kernels.ops import HipOps
+    assert HipOps._ssd_chunk(HipOps, 300, 1, 64, 128, (1 << 23) - 1) == 128
+    assert HipOps._ssd_chunk(HipOps, 300, 1, 64, 128, 1 << 23) == 0
