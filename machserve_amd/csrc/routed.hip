@@ -34,15 +34,14 @@ struct RouteSums {
     int real, width, T;
 };
 
-// gates[t, e] = the row's weight for expert e, 0 where it was not chosen.  A block takes R rows, a wave three outputs at a time, whose weights it asks
-// for together, V columns a lane; a logit is the sum of a lane's columns, then of the lanes, whatever R.  The choice and all that follows are a wave's a row.
+// gates[t, e] = the row's weight for expert e, 0 where it was not chosen.  A block takes R rows, a wave EW outputs at a time, whose weights it asks
+// for together, V columns a lane; a logit is the sum of a lane's columns, then of the lanes, whatever R and EW.  The choice and all that follows are a wave's a row.
 // An output at a time was a trip to memory for every fourth, and with one row a block every row brought the weights from the L2 again
 // (us, warm: four rows of 2,048 over 9 outputs 7.1 -> 5.1, 2,048 rows 14.7 -> 8.5; 64 rows over 64 outputs 25.2 -> 17.6, 2,048 72.8 -> 33.2).
-template <int R, int V>
+template <int R, int V, int EW>
 __global__ __launch_bounds__(256) void route_kernel(const elem_t* __restrict__ x, const float* __restrict__ w,
                                                     const float* __restrict__ bias, float* __restrict__ gates, int d, int E, int top,
                                                     int scoring, const float* __restrict__ correction, int extra, RouteSums rs) {
-    constexpr int EW = 3;
     static_assert(R == 1 || R == 4, "sums over the lanes of four rows at a time; a wave a row");
     const bool softmax_all = scoring == SOFTMAX_ALL;
     __shared__ float zs[R][MAX_EXPERTS];
@@ -647,16 +646,23 @@ extern "C" int ms_route(const void* x, const float* w, const float* bias, float*
     MS_REQUIRE(top >= 1 && top <= E && top <= 64, "route: %d of %d experts a row (at most 64)", top, E);
     MS_REQUIRE((plane == nullptr) == (sums == nullptr) && (!plane || (real > 0 && real <= E)), "route: %d of %d outputs are experts", real, E);
     const RouteSums rs{plane, sums, real, d, T};
-#define MS_ROUTE(R_, V_)                                                                                                                         \
-    hipLaunchKernelGGL((route_kernel<R_, V_>), dim3(ceil_div(T, R_)), dim3(256), 0, stream, (const elem_t*)x, w, bias, gates, d, E, top, scoring, \
+#define MS_ROUTE(R_, V_, EW_)                                                                                                                         \
+    hipLaunchKernelGGL((route_kernel<R_, V_, EW_>), dim3(ceil_div(T, R_)), dim3(256), 0, stream, (const elem_t*)x, w, bias, gates, d, E, top, scoring, \
                        correction, extra, rs)
     // four columns a load where every row begins at a multiple of them; four rows a block where that leaves every CU a block
     const bool fours = d % 4 == 0 && (reinterpret_cast<uintptr_t>(w) & 15) == 0 && (reinterpret_cast<uintptr_t>(x) & (4 * sizeof(elem_t) - 1)) == 0;
     const bool many = T >= 4 * compute_units();
-    if (fours && many) MS_ROUTE(4, 4);
-    else if (fours) MS_ROUTE(1, 4);
-    else if (many) MS_ROUTE(4, 1);
-    else MS_ROUTE(1, 1);
+    // up to four outputs: one a wave, which asks for nothing twice (four outputs of 2,048, three a wave / one / an output in turn: 16 rows 5.0 / 4.2 / 4.9 us,
+    // 1,000 rows 7.8 / 5.6 / 6.6; five outputs, three a wave / in turn: 5.0 / 5.7 and 7.9 / 7.5)
+    const bool one = E + extra <= 4;
+    if (one && fours && many) MS_ROUTE(4, 4, 1);
+    else if (one && fours) MS_ROUTE(1, 4, 1);
+    else if (one && many) MS_ROUTE(4, 1, 1);
+    else if (one) MS_ROUTE(1, 1, 1);
+    else if (fours && many) MS_ROUTE(4, 4, 3);
+    else if (fours) MS_ROUTE(1, 4, 3);
+    else if (many) MS_ROUTE(4, 1, 3);
+    else MS_ROUTE(1, 1, 3);
 #undef MS_ROUTE
     return check_launch("route");
 }

@@ -166,6 +166,21 @@ def test_the_router_in_its_forms(dtype, T, E, top, d, scoring):
     assert (got - want)[clear].abs().max().item() <= 1e-5
 
 
+# at most four outputs, extra gates among them: a wave has one and not three; one row a block and four, columns in fours and not.  (With two outputs
+# that tie, two thirds of the rows of three have no tie at the second place, and none matters where all are chosen.)
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("T,E,top,d", [(1, 4, 2, 256), (1023, 3, 2, 130), (1030, 4, 4, 192), (1030, 2, 2, 1030)])
+def test_the_router_of_few_outputs(dtype, T, E, top, d):
+    from machserve_amd.kernels import get_ops
+    test_the_router_in_its_forms(dtype, T, E, top, d, {"softmax_all": True})
+    if E < 4:
+        test_the_router_in_its_forms(dtype, T, E, top, d, {"sigmoid": True, "extra_gates": 4 - E})
+    g = torch.Generator().manual_seed(E)
+    x, w, bias = torch.randn(T, d, generator=g).to(dtype), torch.randn(5, d, generator=g) * d ** -0.5, torch.tensor([0.0] * E + [-1e4] * (5 - E))
+    few, more = (get_ops(dtype, DEV).route(x.to(DEV), w[:n].contiguous().to(DEV), bias[:n].to(DEV), top) for n in (E, 5))
+    assert torch.equal(few, more[:, :E]), "a logit does not depend on how many there are"
+
+
 def test_the_router_refuses_numbers_and_sums_that_its_kernel_does_not_assume():
     from machserve_amd.kernels import KernelError, get_ops
     ops, new = get_ops(torch.bfloat16, DEV), lambda shape, dt: torch.zeros(shape, dtype=dt, device=DEV)  # noqa: E731
