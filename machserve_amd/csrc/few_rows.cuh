@@ -2,8 +2,9 @@
 // and nothing of it is reused, so the block's waves share out K and not the columns.  Wave w of KW takes the steps w, w + KW, ... of 16 NT
 // columns and 16 MT rows, through a ring of its own in LDS that loads straight from memory fill (global_load_lds_dwordx4: eight
 // lanes bring 128 contiguous bytes of a row, swizzled as in gemm_tile.cuh): there is no barrier before the waves' sums are added, in
-// wave order, and a wave waits for its own oldest step only.  How K falls to the waves depends on KW and the slice alone, so a row's sums
-// do not depend on what else is in the step.
+// wave order, and a wave waits for its own oldest step only.  How K falls to the waves depends on KW and the slice alone.  The slices are those of 16 rows
+// up to 32 (plan_few), and up to 16 rows every product comes here, so that a row's sums do not depend on what else is in such a step; between 17 and 64
+// rows it goes by their number whether a product comes here or goes in tiles, above 32 in how many slices.
 //
 // What bounds it: the weight's bytes (5 TB/s) behind 2.3 us of launch, first trip and end, and the rows, which every block reads again.  The kernel that
 // this replaces for large weights shares 64 rows and 64 columns out over its waves, with a barrier a step of 0.36 us, so a wide output

@@ -370,7 +370,7 @@ extern "C" int ms_linear_swiglu_scaled(const void* a, const float* row_ss, int s
 }
 
 // Column tiles of ms_linear_residual_prenorm for this shape (the first size of its ss_part), or 0 if it is not taken: up to 16 rows over whole K steps,
-// uncut, where that takes no longer than the slices and the norm that would add them up (3 us: a launch and a trip to memory).
+// uncut, where that is predicted to take no longer than the slices and the norm that would add them up (2.5 us: a launch and a trip to memory).
 extern "C" int ms_prenorm_parts(int M, int N, int K) {
 #ifdef MS_ELEM_HALF
     if (!kRoundsBeforeTheNormIsSafe || M < 1 || M > 16 || !few_rows(M, N, K, false, false)) return 0;

@@ -529,10 +529,12 @@ __global__ __launch_bounds__(64 * FEW_WAVES) void expert_few_kernel(const elem_t
 static int plan_experts(const ExpertArgs& g, bool down, int per) {
 #ifdef MS_ELEM_HALF
     if (g.T <= 64) return TILE_64x64_DEEP;
-    // Rows fall to the router's outputs (of which some may be no experts) nearly as if at random: an expert has `mean` rows, give or take `spread` (a little more
-    // than chance gives: with chance alone the down product of 2,048 rows over nine outputs, eight of them experts, took 256x128 tiles, a round if no expert had more than 512
-    // rows, and ran two: 86 us; 256x192 59), and
-    // its tiles are counted as the chances that it has more rows than each of them begins with.
+    // Rows fall to the router's outputs (of which some may be no experts) nearly as if at random: an expert has `mean` rows, give or take `spread`, and
+    // its tiles are counted as the chances that it has more rows than each of them begins with.  `spread` is chance's and 3 % of the mean: routers do not share
+    // out their rows quite as evenly as chance.  Over 220 products a line (110 sizes, 65 to 4,096 rows, 1 to 6 of 4 to 64 experts), the chosen tile's time
+    // over the best one's on average, with 0, 3 and 10 %: loads as chance has them 1.025 1.026 1.030 and 1.033 1.041 1.049, wider by 2 to 3 % of the mean
+    // 1.035 1.031 1.031 and 1.037 1.036 1.038, by 9 % 1.038 1.032 1.028.  (The down product of 2,048 rows over nine outputs, eight of them experts: 256x128 tiles are a round if
+    // no expert has more than 512 rows and two if one has, 43 and 86 us; 256x192 53 to 59.)
     const int outputs = max(g.E, g.ld_gates - (g.shared ? 1 : 0));  // (a gate of the expert for every row is none of them)
     const double mean = (double)g.T * g.top / outputs, spread = sqrt(mean * (1.0 - 1.0 / outputs)) + 0.03 * mean + 1e-3;
     int best = TILE_64x64;

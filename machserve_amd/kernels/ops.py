@@ -293,10 +293,11 @@ class HipOps:
         return (self._few(M, N, K, slices, pairs) and self._aligned(a, w)) or self._tiled(M, N, K)
 
     def linear_split(self, a: torch.Tensor, w: torch.Tensor, allow_partials: bool = True) -> torch.Tensor:
-        """Float32 ``[P, M, N]`` whose sum over P is ``a @ w.T``.  Within one kernel family the cut
-        of K depends on N and K only, so the consumer that adds the parts sees the same sums for a row
-        whatever else is in the batch; which family runs depends on the number of rows (see
-        :meth:`_few` and :meth:`_tiled`), and they differ in rounding."""
+        """Float32 ``[P, M, N]`` whose sum over P is ``a @ w.T``.  The cut of K depends on N and K only in
+        the weight-streaming kernels and, up to 32 rows, in those whose waves share K, so the consumer
+        that adds the parts sees the same sums for a row whatever else is in such a batch; above, and in
+        tiles, it depends on the number of rows as well.  Which family runs does too (see :meth:`_few`
+        and :meth:`_tiled`), and they differ in rounding."""
         M, N, K = self._mm_operands(a, w, "linear_split")
         if self._through_tiles(a, w, allow_partials):
             P = self._plan("ms_tiled_partials", M, N, K) if allow_partials else 1
@@ -1578,7 +1579,9 @@ class HipOps:
         """Tokens of a chunk for a step of ``T`` rows in ``S`` requests, 0: its requests are walked token by token.  A walk takes 2 us a
         token and state of 128 whatever runs beside it, chunks 25 to 50 us a request that has the chip for itself: heads of 64 with 128
         states, walked / in chunks, us: 64 heads, one request of 16 rows 51 / 27, of 128 264 / 46; sixteen requests of 32 rows 102 / 99,
-        of 48 140 / 120; 8 heads of 32 with 16 states, 32 rows 22 / 22, 48 rows 31 / 25.  The chunks' workspace is
+        of 48 140 / 120; 8 heads of 32 with 16 states, 32 rows 22 / 22, 48 rows 31 / 25.  It goes by the rows of a request on average, all that a
+        captured step's shape says of them: a long portion beside many decoding requests is walked (2,000 rows beside 60 single ones 4,550 us, in
+        chunks it would be 540; 200 beside 16 477 and 128).  The chunks' workspace is
         a state and x for every chunk and head, states and channels filled up: (T / 128 + S) ceil(P / 64) 64 (states + 128) numbers a head, up to
         :attr:`SSD_WORK_BYTES` (2,048 rows of 64 heads of 64 with 128 states: 73 MB)."""
         rows = T // S
