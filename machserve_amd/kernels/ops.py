@@ -1585,10 +1585,9 @@ class HipOps:
         a state and x for every chunk and head, states and channels filled up: (T / 128 + S) ceil(P / 64) 64 (states + 128) numbers a head, up to
         :attr:`SSD_WORK_BYTES` (2,048 rows of 64 heads of 64 with 128 states: 73 MB)."""
         rows = T // S
-        least = min(self.SSD_CHUNK_MIN_ROWS, self.SCAN_CHUNK_MIN_ROWS // 2)
         few = rows >= 16 and N >= 64 and S * H <= 256
         near = row < 1 << 23  # numbers of a row of x, B and C: the chunks' kernels count a chunk's bytes in 32 bits
-        return min(self.SSD_SEGMENT, T) if near and (rows >= least or few) else 0
+        return min(self.SSD_SEGMENT, T) if near and (rows >= self.SSD_CHUNK_MIN_ROWS or few) else 0
 
     def gated_group_norm(self, y: torch.Tensor, proj: torch.Tensor, z_col: int, weight: torch.Tensor, eps: float, groups: int,
                          out_cols: int) -> torch.Tensor:

@@ -180,6 +180,8 @@ def test_state_space_recurrence_walked_in_segments(monkeypatch, dtype, H, P_, N,
     ops = ops_of(dtype)
     monkeypatch.setattr(type(ops), "SCAN_CHUNK_MIN_ROWS", 2 * seg)
     monkeypatch.setattr(type(ops), "SSD_SEGMENT", seg)
+    monkeypatch.setattr(type(ops), "SSD_CHUNK_MIN_ROWS", seg)
+    assert ops._ssd_chunk(13 * seg + 4, 3, H, N) == seg, "the rows go in chunks of this length"
     lens = [4 * seg, 3, 9 * seg + 1]
     _ssd_case(dtype, H, P_, N, G, 1, lens, ([1000, 1000, 1000], [3 * seg - 1, 2, 4 * seg + 2], [2 * seg, 1, 2 * seg]))
 

@@ -961,6 +961,8 @@ def test_products_whose_waves_share_out_k(dtype, M, N, K):
     gated = P.silu(P.linear(a.double(), g.double())) * P.linear(a.double(), u.double())
     gu = interleave_gate_up(g, u).to(DEV)
     assert_close(ops.linear_swiglu(ad, gu, N // 2 + 3), gated, dtype, "gated")
+    if M <= 16:
+        assert parts.shape[0] == ops.linear_split(ad[:1].contiguous(), wd).shape[0], "as many slices as for one row"
     if M <= 16 and ops._few(M, N, K, True) and parts.shape[0] == ops.linear_split(ad[:1].contiguous(), wd).shape[0]:
         assert torch.equal(parts[:, :1], ops.linear_split(ad[:1].contiguous(), wd)), "a row's sums do not depend on the other rows"
     if dtype == torch.bfloat16 and ops._plan("ms_prenorm_parts", M, N, K):
