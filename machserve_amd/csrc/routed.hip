@@ -521,8 +521,9 @@ __global__ __launch_bounds__(64 * FEW_WAVES) void expert_few_kernel(const elem_t
 // The tile of a product.  A step of 33 to 64 rows (and of any number up to 64 in 32-bit) has one tile of 64 rows an expert, its weight's columns streamed by blocks with
 // three steps in flight; above, the tile of the least predicted time, its tiles counted from how many rows
 // an expert can be expected to have.
-// us up, the choice of half an expert's last tile empty -> this one (2 of 8 experts of 2,816, width 2,048): 1,900 rows 121 -> 111, 1,200 100 -> 88, 700 and
-// an expert for every row 88 -> 62, 2,048 of experts of 1,408 and width 1,024 60 -> 50.
+// With half of every expert's last tile counted as empty instead, the chosen tiles take 1.039 times the best ones' time where these take 1.025 (220 products,
+// the worst 1.65 and 1.28), with uneven loads 1.044 and 1.034; us up (2 of 8 experts of 2,816, width 2,048): 700 rows and an expert for every row 68 -> 59,
+// 2,048 over nine outputs 110 -> 103, 1,200 87 -> 92.
 // 2,048 rows, 2 of 8 experts of 2,816 and one of 2,816 for every row, width 2,048, gated (us up / down): 256x256 191 / 83, 256x192 211 / 120,
 // 256x128 197 / 97, 128x128 179 / 106, 64x64 279 / 156; 128x128 alone, in the order of the columns and with the epilogue reading row by row, was 228 / 120.
 // 1,750 rows, 2 of 8 experts of 2,816: 122 / 73, 128 / 62, 130 / 87, 120 / 72 and 178 / 101 against 170 / 113.

@@ -128,8 +128,8 @@ __global__ __launch_bounds__(256) void ssd_scan_kernel(SsdArgs a) {
 // added up in 64 bits and kept as the sum of two 32-bit numbers, so that L_t - L_s is as exact as one decay is.
 //
 // A walk is a serial chain of tokens in vector arithmetic (2 us a token with 128 states of 64 channels).  64 such heads, walked in segments
-// of 64 tokens side by side before / in chunks: a prompt of 2,048 358 / 150 us (71 + 17 + 74 in the three kernels), of 256 246 / 53, of 877,
-// 585 and 293 at once 351 / 124.  The matrix instructions are 53,000 cycles of a SIMD's 120,000 in the last kernel; what is left is
+// of 64 tokens side by side before / in chunks: a prompt of 2,048 358 / 150 us, of 256 246 / 53, of 877,
+// 585 and 293 at once 351 / 124 (inside the model, operands cold: 71 + 17 + 74 in the three kernels).  The matrix instructions are 53,000 cycles of a SIMD's 120,000 in the last kernel; what is left is
 // a block's start (gates, C, scores: 5 us of 18 for a single head), vector instructions (25,000) and memory: 250 MB pass between the kernels.
 // Tried: operands straight from memory into registers, every wave with its own SiLU 237 us; one or four heads a block 147 and 162.
 //
