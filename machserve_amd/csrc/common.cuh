@@ -4,7 +4,7 @@
 // One library is built per element type: MS_ELEM_BF16 or MS_ELEM_F16 (bfloat16 or half-precision
 // storage, 32-bit accumulation; MS_ELEM_HALF is defined for both: they share every tile and
 // schedule) or MS_ELEM_F32 (everything in true 32-bit; its matrix products use the
-// full-precision v_mfma_f32_16x16x4_f32, never a reduced-precision mode).
+// full-precision v_mfma_f32_16x16x4_f32, or all bits of the numbers in three parts of 16, see gemm_tile.cuh).
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -23,6 +23,7 @@ constexpr int WAVE = 64;
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 // ---- element type ---------------------------------------------------------------
 #if defined(MS_ELEM_BF16)
@@ -58,6 +59,15 @@ template <typename T> __device__ __forceinline__ T from_f32(float v);
 template <> __device__ __forceinline__ float from_f32<float>(float v) { return v; }
 template <> __device__ __forceinline__ __bf16 from_f32<__bf16>(float v) { return (__bf16)v; }
 template <> __device__ __forceinline__ _Float16 from_f32<_Float16>(float v) { return (_Float16)v; }
+
+// Two numbers rounded to bfloat16, the first in the lower half.
+__device__ __forceinline__ uint32_t round_pair(float x, float y) {
+    typedef float f32x2 __attribute__((ext_vector_type(2)));
+    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+    union { bf16x2 v; uint32_t u; } pair;
+    pair.v = __builtin_convertvector((f32x2){x, y}, bf16x2);
+    return pair.u;
+}
 
 // A fragment is 8 consecutive elements along the reduction dimension of one row of an
 // operand: for lane l of a wave, row l % 16 and elements (l / 16) * 8 .. + 8 of a chunk of

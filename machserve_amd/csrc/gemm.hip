@@ -115,6 +115,21 @@ static bool few_rows(int M, int N, int K, bool slices, bool pairs) {
 static bool planned(int M, int K) { return M > 64 && K % 64 == 0 && g_gemm_config == 0; }
 #endif
 
+#ifndef MS_ELEM_HALF
+// Whether a 32-bit product runs in parts of 16 bits (GEMM_SPLIT): whole K steps, an output of at least 4,096 columns whose 64x64 tiles are one and a half a CU, or
+// K in slices.  us, 32-bit instructions and parts: 192 x 9,728 x 896 (1.8 a CU) 33.8 and 30.4, 128 rows (1.2) 27.7 and 28.1, 65 rows 20.7 and 27.7; 512 x 4,096 x 1,024 37.7
+// and 35.3.  Narrower outputs gain no more (1,024 x 2,048 x 2,048 69 and 63) and keep sums that are the same in every batch of more than 64 rows.
+static bool parted(int M, int N, int K, int slices) {
+    return K % 32 == 0 && M > 64 && (slices > 1 || (N >= 4096 && 2L * ceil_div(M, 64) * ceil_div(N, 64) >= 3L * compute_units()));
+}
+// ... in tiles of 128x128, a block a CU, which take 1.45 us a K step and round, or of 64x64, 0.5 us for each that a CU has: 768 x 9,728 x 896 (two rounds, 7.1 a CU) 84 and
+// 98 us, 512 rows (two rounds, 4.8) 75 and 67, 512 x 2,048 x 5,632 in four slices (one round, 4) 69 and 85.
+static bool parted_wide(int M, int N, int slices) {
+    const long cus = compute_units(), wide = (long)ceil_div(M, 128) * ceil_div(N, 128) * slices, narrow = (long)ceil_div(M, 64) * ceil_div(N, 64) * slices;
+    return 1.45 * (double)ceil_div(wide, cus) < 0.5 * (double)narrow / (double)cus;
+}
+#endif
+
 template <int EPI>
 static int launch_gemm(const elem_t* A, const elem_t* W, int M, int N, int K, EpiArgs ep, hipStream_t stream,
                        int nsplit = 1) {
@@ -213,6 +228,10 @@ static int launch_gemm(const elem_t* A, const elem_t* W, int M, int N, int K, Ep
     // Whole K steps straight to LDS, three or two of them in flight (the loop through registers waits for a trip to memory every step:
     // 1,024 x 2,048 x 2,048 in 512 tiles of 64x64 90 -> 69 us); where the 64x64 tiles are less than two a CU, four times as many of
     // 32x32 (512 x 896 x 4,864 118 -> 50 us, 512 x 896 x 896 25 -> 12; at two a CU 69 against 75).  The sums keep their order.
+    if (parted(M, N, K, (int)ns)) {
+        if (parted_wide(M, N, (int)ns)) MS_GEMM_DEEP(128, 128, 2, 4, 32, GEMM_SPLIT);
+        MS_GEMM_DEEP(64, 64, 2, 2, 32, GEMM_SPLIT);
+    }
     if (K % 32 == 0) {
         const bool few = (long)ceil_div(M, 64) * ceil_div(N, 64) < 2L * compute_units();
         if constexpr (EPI == EPI_SWIGLU) {  // gate and up columns lie side by side: 32 columns a wave
@@ -229,7 +248,7 @@ static int launch_gemm(const elem_t* A, const elem_t* W, int M, int N, int K, Ep
 }
 
 // K slices for a product whose consumer adds partial sums: enough 128x128 blocks to fill the chip,
-// at least 512 of K each.  The 32-bit build never slices: its sums keep one order.
+// at least 512 of K each.  The 32-bit build does not slice here: its sums keep one order.
 #ifdef MS_MEASURE
 static int g_force_splits = 0;
 #else
@@ -480,6 +499,16 @@ extern "C" int ms_tiled_tile(int M, int N, int K, int splits, int store32) {
 #endif
 }
 
+// Whether a 32-bit product with that many K slices runs in parts of 16 bits: 1 in tiles of 64x64, 2 of 128x128, else 0 (the two-byte builds: 0).
+extern "C" int ms_parted(int M, int N, int K, int slices) {
+#ifdef MS_ELEM_HALF
+    (void)M; (void)N; (void)K; (void)slices;
+    return 0;
+#else
+    return parted(M, N, K, slices) ? 1 + parted_wide(M, N, slices) : 0;
+#endif
+}
+
 // The same of a gated product of `N` columns, gate and up.
 extern "C" int ms_gated_tile(int M, int N, int K) {
 #ifdef MS_ELEM_HALF
@@ -539,6 +568,25 @@ extern "C" int ms_prefers_tiled(int M, int N, int K) {
 #else
     return 0;
 #endif
+}
+
+// K slices of a product that is added to the residual stream, whose next norm adds them up: those of ms_tiled_partials, and in the 32-bit build those of a long K
+// under a narrow output, whose uncut 32x32 tiles are each a chain of all K steps: slices that fill the chip with 128x128 tiles, eight at most.  us, uncut and in slices:
+// 512 x 896 x 4,864 53.6 and 32.9 (eight), 192 rows 44 and 22.
+extern "C" int ms_residual_partials(int M, int N, int K) {
+#ifndef MS_ELEM_HALF
+    if (M > 64 && N < 4096 && K >= 4096 && K % 32 == 0) {
+        const int want = max(1, min(8, (int)(compute_units() / ((long)ceil_div(M, 128) * ceil_div(N, 128)))));
+        return ceil_div(K, ceil_div(ceil_div(K, want), 64) * 64);
+    }
+#endif
+    return plan_tiled_splits(M, N, K);
+}
+
+// out[slices, M, N] (float) = partial sums of a w^T over that many slices of K.
+extern "C" int ms_linear_slices(const void* a, const void* w, float* out, int M, int N, int K, int slices, hipStream_t stream) {
+    EpiArgs ep{out, nullptr, N, N, 0, 0};
+    return launch_gemm<EPI_STORE_F32>((const elem_t*)a, (const elem_t*)w, M, N, K, ep, stream, slices);
 }
 
 // out[ks, M, N] (float) = partial sums of a w^T over ms_tiled_partials(M, N, K) slices of K.

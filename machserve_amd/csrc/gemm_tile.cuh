@@ -14,7 +14,8 @@
 // two-byte elements, and in 32-bit whatever has a partial last step, go global -> registers -> LDS (padded rows); the other
 // products of the 32-bit build go straight to LDS as well (its K steps of 32 are rows of 128 bytes too).
 // Every output element is the sum over K in steps of 32 in ascending order whatever the
-// tile shape or the number of rows, so a row's result does not depend on its batch.
+// tile shape or the number of rows, so a row's result does not depend on its batch (of the 32-bit products with wide outputs
+// those of large batches are worked out in parts, with sums of their own: GEMM_SPLIT).
 #pragma once
 #include <type_traits>
 
@@ -31,6 +32,7 @@ constexpr int KPAD = 8;  // rows of 160 bytes (BK 32)
 #endif
 
 constexpr int GEMM_PIPED = 1;  // in the place of a number of LDS buffers: two of them, in phases (see gemm_tile)
+constexpr int GEMM_SPLIT = 8;  // 32-bit: two buffers, and every number in three parts of 16 bits (see gemm_tile)
 
 enum EpiKind {
     EPI_STORE_F32 = 0, EPI_STORE_ELEM = 1, EPI_RESIDUAL = 2, EPI_SWIGLU = 3, EPI_QKV_ROPE = 4, EPI_ACT = 5,
@@ -84,15 +86,15 @@ __device__ __forceinline__ void gemm_tile(const elem_t* __restrict__ A, const el
 #ifdef MS_ELEM_HALF
     constexpr bool DIRECT = BK == 64;
 #else
-    constexpr bool DIRECT = STAGES > 2;
+    constexpr bool DIRECT = STAGES > 2 && STAGES != GEMM_SPLIT;
 #endif
-    constexpr bool PIPED = STAGES == GEMM_PIPED;
-    constexpr int BUFS = PIPED ? 2 : STAGES;
+    constexpr bool PIPED = STAGES == GEMM_PIPED, SPLIT = STAGES == GEMM_SPLIT;
+    constexpr int BUFS = PIPED || SPLIT ? 2 : STAGES;
     // Tiles of more than 256 columns (256x320 under eight waves of 128x80: 160 registers of sums and 72 of fragments) have no register to spare for a lane's
     // offsets into the operands: rows of W go in eights with a scalar base (N is a multiple of 8), those of A are worked out at each load.
     constexpr bool WIDE = BN > 256;
     static_assert(!WIDE || (PIPED && !Rows::GATHERS), "wide tiles: in phases, rows as they come");
-    constexpr int LDS_LD = DIRECT ? BK : BK + KPAD;
+    constexpr int LDS_LD = SPLIT ? BK * 3 / 2 : DIRECT ? BK : BK + KPAD;
     constexpr int CPR = BK / EPC;  // chunks per tile row
     // where chunk `chunk` of tile row `row` lies in a buffer
     auto at = [](int row, int chunk) { return row * LDS_LD + (DIRECT ? (chunk ^ (row & 7)) : chunk) * EPC; };
@@ -100,7 +102,7 @@ __device__ __forceinline__ void gemm_tile(const elem_t* __restrict__ A, const el
     constexpr int A_CHUNKS = BM * CPR / NT, W_CHUNKS = BN * CPR / NT;
     static_assert(BM * CPR % NT == 0 && BN * CPR % NT == 0, "tile loads divide over the block");
     static_assert(NT == 256 || !SCALED, "the row factors' shares are dealt to four waves");
-    static_assert(STAGES == 2 || DIRECT, "more than two LDS buffers, and phases, only with direct loads");
+    static_assert(STAGES == 2 || DIRECT || SPLIT, "more than two LDS buffers, and phases, only with direct loads");
     static_assert(!SCALED || (STAGES > 2 && EPI == EPI_SWIGLU), "row factors: built for the gated product with several steps in flight");
     static_assert(256 % BM == 0 || !SCALED, "threads are dealt to the rows");
     __shared__ float ss_q[SCALED ? 256 / BM : 1][SCALED ? BM : 1];  // the rows' sums of squares, in 256 / BM interleaved shares
@@ -291,7 +293,127 @@ __device__ __forceinline__ void gemm_tile(const elem_t* __restrict__ A, const el
                 for (int j = 0; j < TN; ++j) mma_16x16x32(acc[i][j], fa[i], fb[j]);
         }
     };
-    if constexpr (PIPED) {
+    if constexpr (SPLIT) {
+#ifndef MS_ELEM_HALF
+        // Numbers of 32 bits in three parts of 16 (bfloat16, which has their exponents): x = x1 + x2 + x3, each the rounding of what the ones before it
+        // leave, so that nothing is lost, and the product's terms x1 y1, x1 y2, x2 y1, x2 y2, x1 y3 and x3 y1 on the 16-bit matrix instructions with their sums in 32
+        // bits; what is left out is below 2^-26 of a product, a quarter of its rounding in 32 bits.  The six take 96 cycles where the 32-bit instructions take 256.  Error
+        // against 64 bits (relative, normal inputs), in those and here: K = 896 5.4e-7 and 4.5e-7, 2,048 8.1e-7 and 7.0e-7, 4,864 in eight slices 4.5e-7 and
+        // 3.8e-7.  (Of numbers below 2^-110 the lowest part falls among the subnormal ones.)
+        // The threads hold a step's numbers for two steps, part them two at a time between the matrix instructions, and store each part's rows of 64 bytes for
+        // the next step; two buffers, one barrier a step.  What bounds it (parts left out, 128x128 of K = 4,864, one block a CU, 166 us): parting and storing alone
+        // 115, the matrix instructions and LDS reads 110: a matrix instruction leaves the issue of two others free, and LDS takes stores at a third of the rate of
+        // reads.  Three buffers with the fragments a step ahead, loads of four steps ahead, other groupings: the same.  us, 32-bit instructions and here: 512 x 9,728 x 896 91.6
+        // and 66.6 (64x64), 1,024 x 17,920 x 1,536 460 and 344 (128x128); with K in slices 512 x 896 x 4,864 53.6 (uncut) and 32.9.
+        static_assert(BK == 32 && BM * 4 % NT == 0 && BN * 4 % NT == 0, "four threads a row");
+        constexpr int A_ROUNDS = BM * 4 / NT, W_ROUNDS = BN * 4 / NT, ROUNDS = A_ROUNDS + W_ROUNDS;
+        // thread t has the eight numbers t % 4 of row t / 4 of every round
+        const int t_row = tid / 4, t_chunk = tid % 4;
+        const float* from[ROUNDS];
+#pragma unroll
+        for (int i = 0; i < ROUNDS; ++i) {
+            const int row = (i < A_ROUNDS ? i : i - A_ROUNDS) * (NT / 4) + t_row;
+            from[i] = (i < A_ROUNDS ? A + (size_t)rows.source(min(m0 + row, M - 1)) * rows.pitch(K) : W + (size_t)min(n0 + row, N - 1) * rows.w_pitch(K)) + k_begin + t_chunk * 8;
+        }
+        f32x4 held[2][ROUNDS][2];  // of two steps
+        auto ask = [&](int kt, int set) {
+#pragma unroll
+            for (int i = 0; i < ROUNDS; ++i)
+#pragma unroll
+                for (int h = 0; h < 2; ++h) held[set][i][h] = *reinterpret_cast<const f32x4*>(from[i] + kt * 32 + h * 4);
+        };
+        auto place = [](int row, int chunk) { return row * LDS_LD + (chunk ^ ((row >> 1) & 2)) * 4; };  // in floats; a part's rows are 64 bytes, 192 apart
+        u32x4 part[3];
+        auto put = [&](int set, int buf, int unit) {  // two numbers of round unit / 4, and the round's stores behind its last
+            const int i = unit / 4, e = unit % 4;
+            float x = held[set][i][e / 2][e % 2 * 2], y = held[set][i][e / 2][e % 2 * 2 + 1];
+#pragma unroll
+            for (int q = 0; q < 3; ++q) {
+                const uint32_t xy = round_pair(x, y);
+                part[q][e] = xy;
+                if (q < 2) {
+                    x -= __uint_as_float(xy << 16);
+                    y -= __uint_as_float(xy & 0xffff0000u);
+                }
+            }
+            if (e == 3) {
+                float* to = (i < A_ROUNDS ? &As[buf][0] : &Ws[buf][0]) + place((i < A_ROUNDS ? i : i - A_ROUNDS) * (NT / 4) + t_row, t_chunk);
+#pragma unroll
+                for (int q = 0; q < 3; ++q) *reinterpret_cast<u32x4*>(to + q * 16) = part[q];
+            }
+        };
+        constexpr int UNITS = ROUNDS * 4, FIRST = UNITS / 4;
+        ask(0, 0);
+        ask(min(1, nk - 1), 1);
+#pragma unroll
+        for (int u = 0; u < UNITS; ++u) put(0, 0, u);
+        __syncthreads();
+        auto step = [&](int kt, int buf) {
+            ask(min(kt + 2, nk - 1), buf);
+            bf16x8 fa[TM][3], fb[TN][3];
+#pragma unroll
+            for (int q = 2; q >= 0; --q) {
+#pragma unroll
+                for (int i = 0; i < TM; ++i) fa[i][2 - q] = *reinterpret_cast<const bf16x8*>(&As[buf][place(wm * (BM / WM) + i * 16 + r16, grp) + (2 - q) * 16]);
+#pragma unroll
+                for (int j = 0; j < TN; ++j) fb[j][q] = *reinterpret_cast<const bf16x8*>(&Ws[buf][place(wn * (BN / WN) + j * 16 + r16, grp) + q * 16]);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int u = 0; u < FIRST; ++u) put(buf ^ 1, buf ^ 1, u);  // (behind the last step: a place that nobody reads)
+            __builtin_amdgcn_sched_barrier(0);
+            constexpr int GR = TM * TN >= 4 ? 4 : TM * TN, GROUPS = 6 * TM * TN / GR;
+#pragma unroll
+            for (int g = 0; g < GROUPS; ++g) {  // the smallest products first
+                constexpr int qa[6] = {0, 2, 1, 0, 1, 0}, qb[6] = {2, 0, 1, 1, 0, 0};
+#pragma unroll
+                for (int u = FIRST; u < UNITS; ++u)
+                    if ((u - FIRST) * GROUPS / (UNITS - FIRST) == g) put(buf ^ 1, buf ^ 1, u);
+#pragma unroll
+                for (int m = g * GR; m < (g + 1) * GR; ++m) {
+                    const int t = m / (TM * TN), i = m / TN % TM, j = m % TN;
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[i][qa[t]], fb[j][qb[t]], acc[i][j], 0, 0, 0);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            __syncthreads();
+        };
+        int kt = 0;
+        for (; kt + 1 < nk; kt += 2) {
+            step(kt, 0);
+            step(kt + 1, 1);
+        }
+        if (kt < nk) step(kt, 0);
+        // An infinity or a NaN among the numbers (an infinity's second part is NaN), numbers whose first part is rounded up to infinity, and sums beyond the
+        // largest number leave sums that are not finite: such a block is worked out again on the 32-bit matrix instructions.
+        bool finite = true;
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) finite &= __builtin_isfinite(acc[i][j][e]);
+        if (__syncthreads_or(!finite)) {
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+                for (int j = 0; j < TN; ++j) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+            for (int k = k_begin; k < k_end; k += 32) {
+                Frag ra_[TM];
+#pragma unroll
+                for (int i = 0; i < TM; ++i)
+                    ra_[i] = frag_load(A + (size_t)rows.source(min(m0 + wm * (BM / WM) + i * 16 + r16, M - 1)) * rows.pitch(K) + k + grp * 8);
+#pragma unroll
+                for (int j = 0; j < TN; ++j) {
+                    const Frag rb = frag_load(W + (size_t)min(n0 + wn * (BN / WN) + j * 16 + r16, N - 1) * rows.w_pitch(K) + k + grp * 8);
+#pragma unroll
+                    for (int i = 0; i < TM; ++i) mma_16x16x32(acc[i][j], ra_[i], rb);
+                }
+            }
+        }
+#endif
+    } else if constexpr (PIPED) {
 #ifdef MS_ELEM_HALF
         // Two LDS buffers, whole K steps.  What bounds the loop with one burst of loads a step and all of a K chunk's fragments read before they are
         // multiplied (measured with parts of it left out, 256x256 tiles, 2,048 x 37,888 x 3,584: 493 us; without the loads

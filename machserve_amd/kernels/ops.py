@@ -341,8 +341,11 @@ class HipOps:
             self._check(self._core, self._core.ms_linear_residual_skinny(_ptr(a), _ptr(w), _ptr(x), _c_int(M), _c_int(N),
                                                                          _c_int(K), self._stream()))
             return None
-        if self._plan("ms_tiled_partials", M, N, K) > 1:
-            return self.linear_split(a, w)
+        P = self._plan("ms_residual_partials", M, N, K)
+        if P > 1:
+            out = torch.empty((P, M, N), dtype=torch.float32, device=a.device)
+            self._check(self._core, self._core.ms_linear_slices(_ptr(a), _ptr(w), _ptr(out), _c_int(M), _c_int(N), _c_int(K), _c_int(P), self._stream()))
+            return out
         self._check(self._core, self._core.ms_linear_residual(_ptr(a), _ptr(w), _ptr(x), _c_int(M), _c_int(N), _c_int(K),
                                                               self._stream()))
         return None

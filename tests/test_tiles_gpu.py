@@ -79,3 +79,44 @@ def test_32_bit_products_in_every_tile(M, N, K):
     z, u = a.double() @ gate.double().T, a.double() @ up.double().T
     assert_close(ops.linear_swiglu(a, interleave_gate_up(gate, up), N // 2), z * torch.sigmoid(z) * u, torch.float32, "gated product")
     assert torch.equal(ops.linear(a[:65].contiguous(), w, None, out_f32=True), out[:65]), "a row's sums do not depend on its batch"
+
+
+# 32-bit products whose numbers are taken in parts of 16 bits: 64x64 and 128x128 tiles, one to many K steps, even and odd, ragged edges; K in slices, the last one short.
+# The sums of many normal terms in 32 bits are off by sqrt(K) 2^-25 of their size, a slice's by less: within assert_close's 32-bit limit with room.
+@pytest.mark.parametrize("M,N,K", [(193, 8200, 32), (200, 8202, 96), (321, 9000, 64), (330, 9008, 160), (65, 40, 4128), (130, 200, 4096), (900, 1030, 4160), (513, 896, 4864)])
+def test_32_bit_products_in_parts(M, N, K):
+    from machserve_amd.kernels.ops import interleave_gate_up
+    ops = ops_for(torch.float32)
+    a, w, x = rnd((M, K), torch.float32, 5), rnd((N, K), torch.float32, 6, K ** -0.5), rnd((M, N), torch.float32, 7)
+    if N >= 4096:
+        assert ops._plan("ms_parted", M, N, K, 1) == (2 if M > 300 else 1), "the sizes are those of another tile"
+    else:
+        slices = ops._plan("ms_residual_partials", M, N, K)
+        assert slices > 1 and ops._plan("ms_parted", M, N, K, slices) > 0, "the sizes are those of an uncut product"
+    ref = (a.double() @ w.double().T).float()
+    def product():
+        if N >= 4096:
+            return ops.linear(a, w, None, out_f32=True)
+        return ops.linear_residual(a, w, x).sum(0)
+
+    out = product()
+    assert_close(out, ref, torch.float32, "sums")
+    if N >= 4096:
+        x1 = x.clone()
+        assert ops.linear_residual(a, w, x1) is None
+        assert_close(x1, x + ref, torch.float32, "added to the stream")
+    gate, up = w[:N // 2].contiguous(), w[N // 2:N // 2 * 2].contiguous()
+    z, u = a.double() @ gate.double().T, a.double() @ up.double().T
+    assert_close(ops.linear_swiglu(a, interleave_gate_up(gate, up), N // 2), z * torch.sigmoid(z) * u, torch.float32, "gated product")
+    if M > 300 and N >= 4096:
+        assert torch.equal(ops.linear(a[:193].contiguous(), w, None, out_f32=True), out[:193]), "a row's sums do not depend on the tile"
+    # what is not finite, and a number whose first part is not, come out as in the 32-bit products
+    a[3, 5], a[64, 7], w[9, 11] = float("inf"), float("nan"), float("-inf")
+    w[:, 1] *= 1e-3  # (no sum of these is beyond 3.4e38 * 5e-3, in whatever order)
+    a[:, 2] *= 1e-3
+    a[20, 1], w[21, 2] = 3.4e38, 3.4e38
+    got, ref = product(), a.double() @ w.double().T
+    assert torch.equal(torch.isnan(got), torch.isnan(ref)) and torch.equal(got[~torch.isfinite(got)].nan_to_num(0.5), ref[~torch.isfinite(ref)].float().nan_to_num(0.5))
+    fine = torch.isfinite(ref)
+    err = (got.double() - ref).abs()[fine] / (a.abs().double().nan_to_num(0, 0, 0) @ w.abs().double().nan_to_num(0, 0, 0).T)[fine]
+    assert float(err.max()) < 2e-6
