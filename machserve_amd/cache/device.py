@@ -29,6 +29,14 @@ class DeviceCache:
         for key, req in manager.states.items():
             self._states[key] = {k: torch.zeros((manager.max_requests + 1, *shape), dtype=req.dtype, device=device)
                                  for k, shape in req.shapes.items()}
+        # the states' arrays stay where they are as long as this object has them: one launch zeroes a slot of them all
+        self._zero = None
+        arrays = [t for tensors in self._states.values() for t in tensors.values() if t.numel()]
+        if arrays and torch.device(device).type == "cuda":
+            from ..kernels import get_ops
+            ops = get_ops(dtype, str(device))
+            places = ops.places_of(arrays)
+            self._zero = lambda slot: ops.zero_places(places, slot)
         # the one-request view
         self.kpools = {i: t for (i, j), t in self._kpools.items() if not manager.layer_requests[i][0]}
         self.vpools = {i: t for (i, j), t in self._vpools.items() if not manager.layer_requests[i][0]}
@@ -53,6 +61,9 @@ class DeviceCache:
         return out if several else out[0]
 
     def zero_state(self, slot: int) -> None:
+        if self._zero is not None:
+            self._zero(slot)
+            return
         for tensors in self._states.values():
             for t in tensors.values():
                 t[slot].zero_()

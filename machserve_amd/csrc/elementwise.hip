@@ -457,6 +457,19 @@ __global__ __launch_bounds__(256) void round_rows_kernel(const float* __restrict
     if (i < n) out[i] = from_f32<elem_t>(x[i]);
 }
 
+// Zeros in place `slot` of every listed array: `arrays` holds (first address, bytes of a place) for each.  One launch for all of them; a launch an array took the host 6
+// and the device 3.3 us each, which the first prompts
+// of a batch waited for (16 requests of the delta rule and linear attention in bench sizes: a pass of 11.09 ms 0.11 shorter).
+__global__ __launch_bounds__(256) void zero_places_kernel(const uint64_t* __restrict__ arrays, int slot) {
+    const uint64_t bytes = arrays[2 * blockIdx.y + 1];
+    char* to = reinterpret_cast<char*>(arrays[2 * blockIdx.y]) + bytes * (uint64_t)slot;
+    const size_t first = (size_t)blockIdx.x * 256 + threadIdx.x, all = (size_t)gridDim.x * 256;
+    if (((reinterpret_cast<uintptr_t>(to) | bytes) & 15) == 0)
+        for (size_t i = first; i < bytes / 16; i += all) reinterpret_cast<u32x4*>(to)[i] = (u32x4){0u, 0u, 0u, 0u};
+    else
+        for (size_t i = first; i < bytes; i += all) to[i] = 0;
+}
+
 // x[t, :] = float(table[tokens[t], :]) + float(pairs[row(t), :]) with row(t) = (previous * mul_prev + tokens[t] * mul_cur) mod
 // buckets, and row `buckets` for a request's first token.  The previous token is the row before in the step, or, for the
 // first row of a request's portion, what the request's slot of `prev [slots]` holds.
@@ -875,6 +888,14 @@ extern "C" int ms_round_rows(const float* x, void* out, long n, hipStream_t stre
     MS_REQUIRE(n > 0 && x && out, "round_rows: empty problem");
     hipLaunchKernelGGL(round_rows_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream, x, (elem_t*)out, (size_t)n);
     return check_launch("round_rows");
+}
+
+// `arrays` on the device: n pairs (address, bytes of a place); `most` is the largest of those bytes.
+extern "C" int ms_zero_places(const void* arrays, int n, long most, int slot, hipStream_t stream) {
+    MS_REQUIRE(arrays && n > 0 && n <= 65535 && most > 0 && slot >= 0, "zero_places: %d arrays, place %d", n, slot);
+    const long blocks = (most + 256 * 32 - 1) / (256 * 32);  // two rounds of 16 bytes a thread in the largest
+    hipLaunchKernelGGL(zero_places_kernel, dim3((unsigned)(blocks < 1024 ? blocks : 1024), n), dim3(256), 0, stream, (const uint64_t*)arrays, slot);
+    return check_launch("zero_places");
 }
 
 extern "C" int ms_embed_pair(const int* tokens, const void* table, const void* pairs, int* prev, const int* seq_q_start,

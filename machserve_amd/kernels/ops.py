@@ -129,6 +129,23 @@ class HipOps:
                                                     self._stream()))
         return x
 
+    @staticmethod
+    def places_of(tensors) -> tuple:
+        """What :meth:`zero_places` takes for arrays ``[places, ...]`` that stay where they are: the device table of their addresses and the
+        bytes of a place, how many they are, the most bytes of a place, and the fewest places."""
+        if not tensors or any(not t.is_cuda or not t.is_contiguous() or t.shape[0] < 1 or t[0].numel() < 1 for t in tensors):
+            raise KernelError("places_of: contiguous arrays of at least one place on the device wanted")
+        sizes = [t[0].numel() * t.element_size() for t in tensors]
+        table = torch.tensor([v for t, b in zip(tensors, sizes) for v in (t.data_ptr(), b)], dtype=torch.int64).to(tensors[0].device)
+        return table, len(sizes), max(sizes), min(t.shape[0] for t in tensors)
+
+    def zero_places(self, places: tuple, slot: int) -> None:
+        """Zeros in place ``slot`` of every array of :meth:`places_of`, in one launch."""
+        table, n, most, count = places
+        if not 0 <= slot < count:
+            raise KernelError(f"zero_places: place {slot} of {count}")
+        self._check(self._core, self._core.ms_zero_places(_ptr(table), _c_int(n), ctypes.c_long(most), _c_int(slot), self._stream()))
+
     def feed_tokens(self, tokens: torch.Tensor, sampled: torch.Tensor, rows: torch.Tensor, src: torch.Tensor) -> None:
         """``tokens[rows[i]] = sampled[src[i]]`` where ``rows[i]`` is no negative number: the rows of a step whose
         input the step before it sampled take it on the device."""

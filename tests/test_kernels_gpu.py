@@ -1033,3 +1033,18 @@ def test_few_rows_whose_operands_begin_at_any_multiple_of_eight_bytes(dtype, M, 
         share = rnd((5, M), torch.float32, 97).abs() * K
         f = 1.0 / torch.sqrt(share.double().sum(0) / K + 1e-5)[:, None]
         assert_close(ops.linear_swiglu_scaled(ad, share.to(DEV), 1e-5, gu, N), P.silu(pg * f) * (pu * f), dtype, "gated with row factors")
+
+
+def test_zeroing_a_place_of_several_arrays():
+    """Arrays of unequal types and sizes, some no multiple of sixteen bytes: the place is zeros, its neighbours stay, a place that is not there is refused."""
+    from machserve_amd.kernels import KernelError
+    ops = ops_for(torch.bfloat16)
+    arrays = [torch.ones((4, *s), dtype=t, device=DEV) for s, t in [((3,), torch.float32), ((16, 128, 128), torch.float32), ((1,), torch.int32), ((5, 7), torch.bfloat16), ((2048,), torch.float32)]]
+    places = ops.places_of(arrays)
+    for place in (2, 0, 3):
+        ops.zero_places(places, place)
+        for a in arrays:
+            assert not bool(a[place].any()) and bool((a[1] == 1).all()) and bool((a[:place][[i not in (0, 2) for i in range(place)]] == 1).all())
+    for place in (4, -1):
+        with pytest.raises(KernelError):
+            ops.zero_places(places, place)
