@@ -8,14 +8,45 @@
 
 namespace ms {
 
-// x[t, :] = float(table[tokens[t], :]) * scale
+// x[t, :] = float(table[tokens[t], :]) * scale, and the same in the element type in `rounded` if it is given.
 __global__ __launch_bounds__(256) void embed_kernel(const int* __restrict__ tokens, const elem_t* __restrict__ table,
-                                                    float* __restrict__ x, int d, float scale) {
-    arguments_now(tokens, table, x, d, scale);
+                                                    float* __restrict__ x, elem_t* __restrict__ rounded, int d, float scale) {
+    arguments_now(tokens, table, x, rounded, d, scale);
     const int t = blockIdx.x;
     const elem_t* src = table + (size_t)tokens[t] * d;
-    float* dst = x + (size_t)t * d;
-    for (int c = threadIdx.x; c < d; c += 256) dst[c] = to_f32(src[c]) * scale;
+    for (int c = threadIdx.x; c < d; c += 256) {
+        const float v = to_f32(src[c]) * scale;
+        x[(size_t)t * d + c] = v;
+        if (rounded) rounded[(size_t)t * d + c] = from_f32<elem_t>(v);
+    }
+}
+// The same for widths of up to 1,024 GROUPS in whole fours, 8 or 16 bytes a load, all of a row's asked for at once: an element a load and one after the other the kernel
+// was a chain of trips to memory, eight at a width of 2,048.  us, back to back from a graph, before and
+// now: 4 x 2,048 2.7 and 2.3, 16 x 3,584 3.5 and 2.5, 2,048 x 3,584 14.9 and 10.3, 512 x 896 in 32-bit 3.5 and 2.8.
+template <int GROUPS>
+__global__ __launch_bounds__(256) void embed_wide_kernel(const int* __restrict__ tokens, const elem_t* __restrict__ table,
+                                                         float* __restrict__ x, elem_t* __restrict__ rounded, int d, float scale) {
+    arguments_now(tokens, table, x, rounded, d, scale);
+    typedef elem_t elem4_t __attribute__((ext_vector_type(4)));
+    const int t = blockIdx.x;
+    const elem_t* src = table + (size_t)tokens[t] * d;
+    elem4_t v[GROUPS];
+#pragma unroll
+    for (int g = 0; g < GROUPS; ++g) v[g] = *reinterpret_cast<const elem4_t*>(src + min((g * 256 + (int)threadIdx.x) * 4, d - 4));
+#pragma unroll
+    for (int g = 0; g < GROUPS; ++g) {
+        const int c = (g * 256 + threadIdx.x) * 4;
+        if (c >= d) continue;
+        f32x4 f;
+        elem4_t r;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            f[e] = to_f32(v[g][e]) * scale;
+            r[e] = from_f32<elem_t>(f[e]);
+        }
+        *reinterpret_cast<f32x4*>(x + (size_t)t * d + c) = f;
+        if (rounded) *reinterpret_cast<elem4_t*>(rounded + (size_t)t * d + c) = r;
+    }
 }
 
 // tokens[rows[i]] = sampled[src[i]] for the i with 0 <= rows[i] < n_tokens and 0 <= src[i] < n_sampled: the input of
@@ -678,10 +709,22 @@ extern "C" int ms_rope_table(const int* positions, const float* inv_freq, float*
     return check_launch("rope_table");
 }
 
-extern "C" int ms_embed(const int* tokens, const void* table, float* x, int T, int d, float scale, hipStream_t stream) {
+// `rounded` may be null.
+extern "C" int ms_embed_rounded(const int* tokens, const void* table, float* x, void* rounded, int T, int d, float scale, hipStream_t stream) {
     MS_REQUIRE(T > 0 && d > 0, "embed: empty problem T=%d d=%d", T, d);
-    hipLaunchKernelGGL(embed_kernel, dim3(T), dim3(256), 0, stream, tokens, (const elem_t*)table, x, d, scale);
+    const bool fours = d % 4 == 0 && ((reinterpret_cast<uintptr_t>(table) | reinterpret_cast<uintptr_t>(rounded)) & (4 * sizeof(elem_t) - 1)) == 0 &&
+                       (reinterpret_cast<uintptr_t>(x) & 15) == 0;
+#define MS_EMBED(KERNEL) hipLaunchKernelGGL(KERNEL, dim3(T), dim3(256), 0, stream, tokens, (const elem_t*)table, x, (elem_t*)rounded, d, scale)
+    if (fours && d <= 1024) MS_EMBED(embed_wide_kernel<1>);
+    else if (fours && d <= 2048) MS_EMBED(embed_wide_kernel<2>);
+    else if (fours && d <= 4096) MS_EMBED(embed_wide_kernel<4>);
+    else MS_EMBED(embed_kernel);
+#undef MS_EMBED
     return check_launch("embed");
+}
+
+extern "C" int ms_embed(const int* tokens, const void* table, float* x, int T, int d, float scale, hipStream_t stream) {
+    return ms_embed_rounded(tokens, table, x, nullptr, T, d, scale, stream);
 }
 
 extern "C" int ms_feed_tokens(int* tokens, const int* sampled, const int* rows, const int* src, int n, int n_tokens, int n_sampled,

@@ -129,6 +129,17 @@ class HipOps:
                                                     self._stream()))
         return x
 
+    def embed_rounded(self, tokens: torch.Tensor, table: torch.Tensor, scale: float = 1.0):
+        """:meth:`embed` and the same rows in the element type, ``(float32 [T, d], element type [T, d])``."""
+        T, (V, d) = tokens.numel(), table.shape
+        self._want(tokens, torch.int32, "embed tokens", T)
+        self._want(table, self.dtype, "embed table")
+        x = torch.empty((T, d), dtype=torch.float32, device=table.device)
+        rounded = torch.empty((T, d), dtype=self.dtype, device=table.device)
+        self._check(self._core, self._core.ms_embed_rounded(_ptr(tokens), _ptr(table), _ptr(x), _ptr(rounded), _c_int(T), _c_int(d), _c_float(scale),
+                                                            self._stream()))
+        return x, rounded
+
     @staticmethod
     def places_of(tensors) -> tuple:
         """What :meth:`zero_places` takes for arrays ``[places, ...]`` that stay where they are: the device table of their addresses and the

@@ -382,6 +382,7 @@ class Block:
     :meth:`mixers`, and :meth:`cache_request` / :meth:`bind_cache` deal the requests and bindings out in order."""
 
     mixer: Optional[Mixer] = None
+    reads_rows = False  # its first part reads the stream as it is, in the element type (``ResidualStream.rows``)
 
     def __init__(self, spec, rt: Runtime):
         self.spec, self.rt = spec, rt

@@ -214,6 +214,8 @@ class PostNormBlock(Block):
     themselves; what it leaves (a last product with or without bias, branches side by side, a finished tensor) is
     normed and added by the post norm's own kernel."""
 
+    reads_rows = True
+
     def __init__(self, spec, rt):
         super().__init__(spec, rt)
         self.mixer = MIXERS.build(spec.mixer, rt)
@@ -255,6 +257,8 @@ class SumNormBlock(Block):
     branch reads the stream's rows as they are (in the element type, or the 32-bit rows if it says ``reads_stream``); what
     it leaves is added to ``alpha`` times the stream and the sum is normed, by one kernel that leaves the rows for the
     next branch as well (a norm with ``normalise_sum``)."""
+
+    reads_rows = True
 
     def __init__(self, spec, rt):
         super().__init__(spec, rt)

@@ -27,6 +27,11 @@ class Embedding(Part):
     def forward(self, tokens: torch.Tensor) -> torch.Tensor:
         return self.rt.ops.embed(tokens, self.weight, getattr(self.spec, "scale", 1.0))
 
+    def forward_rounded(self, tokens: torch.Tensor):
+        """The rows, and the same in the element type or None where the kernels do not leave them."""
+        both = getattr(self.rt.ops, "embed_rounded", None)
+        return (self.forward(tokens), None) if both is None else both(tokens, self.weight, getattr(self.spec, "scale", 1.0))
+
 
 @register_embedding("pair_embedding")
 class PairEmbedding(Part):
@@ -200,9 +205,16 @@ class DecoderModel:
         # from the captured graph, which would then rotate every later step by the first step's positions.
         ctx.shared.clear()
         embedding = self.embedding
-        x = embedding.forward_step(ctx) if getattr(embedding, "reads_step", False) else embedding.forward(ctx.tokens)
         streams = getattr(self.spec, "streams", None)  # several residual streams that all start as the embedding
+        rounded = None
+        if getattr(embedding, "reads_step", False):
+            x = embedding.forward_step(ctx)
+        elif not streams and self.blocks[self.order[0]].reads_rows and hasattr(embedding, "forward_rounded"):
+            x, rounded = embedding.forward_rounded(ctx.tokens)
+        else:
+            x = embedding.forward(ctx.tokens)
         stream = MultiStream(x, streams, self.rt.ops) if streams else ResidualStream(x, self.rt.ops)
+        stream.rounded = rounded
         watch = self.observer
         if watch is not None:
             watch("embedding", stream.value())

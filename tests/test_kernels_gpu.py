@@ -1035,6 +1035,19 @@ def test_few_rows_whose_operands_begin_at_any_multiple_of_eight_bytes(dtype, M, 
         assert_close(ops.linear_swiglu_scaled(ad, share.to(DEV), 1e-5, gu, N), P.silu(pg * f) * (pu * f), dtype, "gated with row factors")
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("T,d", [(1, 8), (3, 896), (2, 1024), (5, 1032), (4, 2048), (1, 2052), (7, 4096), (2, 4100), (3, 6)])
+def test_embedding_rows_in_both_types(dtype, T, d):
+    """One, two and four groups of 1,024 columns, widths behind them and widths that are no whole fours: rows in 32 bits and in the element type."""
+    ops = ops_for(dtype)
+    table, tokens = rnd((50, d), dtype, 101).to(DEV), torch.tensor([49, 0, 7, 7, 31, 2, 48][:T], dtype=torch.int32, device=DEV)
+    for scale in (1.0, 3.0):
+        ref = table[tokens.long()].float() * scale
+        x, rounded = ops.embed_rounded(tokens, table, scale)
+        assert torch.equal(x, ref) and torch.equal(rounded, ref.to(dtype))
+        assert torch.equal(ops.embed(tokens, table, scale), ref)
+
+
 def test_zeroing_a_place_of_several_arrays():
     """Arrays of unequal types and sizes, some no multiple of sixteen bytes: the place is zeros, its neighbours stay, a place that is not there is refused."""
     from machserve_amd.kernels import KernelError
