@@ -45,8 +45,11 @@ __global__ __launch_bounds__(256) void key_decay_kernel(Sums in, int col, const 
 // WALK_BATCH at a time through LDS; the next batch's numbers are asked for before the current batch is walked.  seg_len 0: a
 // block walks all of a request's rows.  Else a request's rows are cut into segments (numbered by piece_of): LOCAL walks
 // each from zero and leaves what it adds (carry [numbers, H, d, dvp]) and the product of its decays (cdec [numbers, H, d]),
-// the carry kernel replaces what it adds by the state that comes into it, and the second walk makes the outputs.
-constexpr int WALK_BATCH = 8;
+// the carry kernel replaces what it adds by the state that comes into it, and the second walk makes the outputs.  A request of at most
+// WALK_WHOLE rows is walked by one block all the same, whatever comes with it: its rows take 1.25 us each, three kernels over segments 80 us and more (100 rows alone
+// 131 us walked, 79 in segments of 32; 64 rows 86 and 78; 64 requests of 17 rows 43 and 94), and 60 single rows beside a prompt of 2,000 took 2,468 us while
+// the rows a request had on average decided for all of a step (in segments 188).
+constexpr int WALK_BATCH = 8, WALK_WHOLE = 64;
 struct WalkArgs {
     StateArgs a;
     int seg_len;
@@ -65,17 +68,19 @@ __global__ __launch_bounds__(NT) void state_walk_kernel(WalkArgs w) {
     if (w.seg_len) pc = piece_of(blockIdx.x, w.seg_len, a.seq_q_start, a.S);
     const int left = a.seq_q_len[pc.s] - pc.first;
     if (left <= 0) return;  // the same for the whole block
-    const int n = w.seg_len ? min(left, w.seg_len) : left;
+    const bool whole = w.seg_len == 0 || a.seq_q_len[pc.s] <= WALK_WHOLE;
+    if (whole && pc.first > 0) return;  // its first number's block has all of its rows
+    const int n = whole ? left : min(left, w.seg_len);
     const bool last = n == left;
     if (LOCAL && last) return;  // nobody needs what the last segment passes on
     const int q0 = a.seq_q_start[pc.s] + pc.first, kh = h / (a.H / a.G);
     const bool live = j < a.dv;
     const size_t head = (size_t)d * a.dvp;
     float* st = a.state + ((size_t)a.seq_slot[pc.s] * a.H + h) * head + j;
-    float* pass = w.seg_len ? w.carry + ((size_t)blockIdx.x * a.H + h) * head + j : nullptr;
+    float* pass = whole ? nullptr : w.carry + ((size_t)blockIdx.x * a.H + h) * head + j;
     float S[DP];
     {
-        const float* from = w.seg_len ? pass : st;
+        const float* from = whole ? st : pass;
 #pragma unroll
         for (int i = 0; i < DP; ++i) S[i] = (!LOCAL && live && i < d) ? from[(size_t)i * a.dvp] : 0.f;
     }
@@ -214,21 +219,31 @@ __global__ __launch_bounds__(NT) void state_walk_kernel(WalkArgs w) {
     }
 }
 
-// Between the two walks: S_in(next) = diag(product of the segment's decays) S_in + what the segment adds, from the slot's state.
+// Between the two walks: S_in(next) = diag(product of the segment's decays) S_in + what the segment adds, from the slot's state.  A thread has four neighbouring
+// value channels of a row; what CARRY_AHEAD segments add is asked for together (one after the other each was a trip to memory: 64 segments 25 us, now 15).
+constexpr int CARRY_AHEAD = 8;
 __global__ __launch_bounds__(256) void state_carry_kernel(WalkArgs w) {
     const StateArgs& a = w.a;
-    const int s = blockIdx.x, h = blockIdx.y, idx = blockIdx.z * 256 + threadIdx.x, head = a.d * a.dvp;
-    if (idx >= head) return;
+    const int s = blockIdx.x, h = blockIdx.y, idx = (blockIdx.z * 256 + threadIdx.x) * 4, head = a.d * a.dvp;
+    if (idx >= head || a.seq_q_len[s] <= WALK_WHOLE) return;
     const int i = idx / a.dvp, base = piece_base(s, w.seg_len, a.seq_q_start);
     const int nseg = (a.seq_q_len[s] + w.seg_len - 1) / w.seg_len;
-    float Sin = a.state[((size_t)a.seq_slot[s] * a.H + h) * head + idx];
-    for (int seg = 0; seg < nseg; ++seg) {
-        const size_t at = (size_t)(base + seg) * a.H + h;
-        float* p = w.carry + at * head + idx;
-        const bool more = seg + 1 < nseg;
-        const float dec = more ? w.cdec[at * a.d + i] : 0.f, add = more ? *p : 0.f;
-        *p = Sin;
-        Sin = dec * Sin + add;
+    f32x4 Sin = *reinterpret_cast<const f32x4*>(a.state + ((size_t)a.seq_slot[s] * a.H + h) * head + idx);
+    for (int seg0 = 0; seg0 < nseg; seg0 += CARRY_AHEAD) {
+        f32x4 add[CARRY_AHEAD];
+        float dec[CARRY_AHEAD];
+#pragma unroll
+        for (int u = 0; u < CARRY_AHEAD; ++u) {  // (what the last segment would pass on is never written: the one before is read in its place, and not used)
+            const size_t at = (size_t)(base + max(min(seg0 + u, nseg - 2), 0)) * a.H + h;
+            dec[u] = w.cdec[at * a.d + i];
+            add[u] = *reinterpret_cast<const f32x4*>(w.carry + at * head + idx);
+        }
+#pragma unroll
+        for (int u = 0; u < CARRY_AHEAD; ++u) {
+            if (seg0 + u >= nseg) break;
+            *reinterpret_cast<f32x4*>(w.carry + ((size_t)(base + seg0 + u) * a.H + h) * head + idx) = Sin;
+            Sin = dec[u] * Sin + add[u];
+        }
     }
 }
 
@@ -290,7 +305,7 @@ extern "C" int ms_gated_linear(const float* rows, int n_partials, int ld, int q_
     const int numbers = T / seg_len + S;
     MS_WALK_D(true, numbers);
     if (int rc = check_launch("gated linear, segments from zero")) return rc;
-    hipLaunchKernelGGL(state_carry_kernel, dim3(S, H, ceil_div(d * dvp, 256)), dim3(256), 0, stream, w);
+    hipLaunchKernelGGL(state_carry_kernel, dim3(S, H, ceil_div(d * dvp, 1024)), dim3(256), 0, stream, w);
     if (int rc = check_launch("gated linear, states between segments")) return rc;
     MS_WALK_D(false, numbers);
 #undef MS_WALK_D

@@ -1327,6 +1327,11 @@ class HipOps:
         the step's rows and requests alone."""
         if T < self.SCAN_CHUNK_MIN_ROWS or T // S < self.SCAN_CHUNK_MIN_ROWS // 2:
             return 0, 0
+        return self._cut_rows(T, S, seg, floats_per_segment)
+
+    @staticmethod
+    def _cut_rows(T: int, S: int, seg: int, floats_per_segment: int) -> tuple:
+        """Segments of ``seg`` rows, longer ones where their workspace would pass 256 MiB."""
         n_segs = -(-T // seg)
         while S * n_segs * floats_per_segment * 4 > (256 << 20) and n_segs > 1:
             seg *= 2
@@ -1669,6 +1674,7 @@ class HipOps:
         return alpha
 
     STATE_SEGMENT = 32  # rows of a segment of gated linear attention
+    STATE_WHOLE = 64  # ... of requests of more rows than this (WALK_WHOLE in the kernels)
 
     def gated_linear(self, sums: torch.Tensor, alpha: torch.Tensor, norm_w: torch.Tensor, eps: float, q_scale: float, state: torch.Tensor,
                      seq_q_start: torch.Tensor, seq_q_len: torch.Tensor, seq_slot: torch.Tensor, H: int, d: int, dv: int, out_cols: int,
@@ -1687,7 +1693,8 @@ class HipOps:
         seg = n = 0
         carry = cdec = None
         if not single:
-            seg, n = self._walk_segments(T, 1, self.STATE_SEGMENT, H * d * dvp) if T // S >= self.SCAN_CHUNK_MIN_ROWS // 2 else (0, 0)
+            # a request may have T - S + 1 rows; those of at most 64 are walked whole by the kernels themselves, whatever comes with them
+            seg, n = self._cut_rows(T, 1, self.STATE_SEGMENT, H * d * dvp) if T - S >= self.STATE_WHOLE else (0, 0)
         if seg:
             n = T // seg + S
             carry = torch.empty((n, H, d, dvp), dtype=torch.float32, device=sums.device)
