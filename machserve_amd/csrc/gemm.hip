@@ -247,6 +247,37 @@ static int launch_gemm(const elem_t* A, const elem_t* W, int M, int N, int K, Ep
 #undef MS_GEMM_DEEP
 }
 
+#ifdef MS_ELEM_HALF
+// The columns of a wave in the tile that a product into the residual stream is planned in: those of a part of the rows' sums of squares (EPI_PRENORM).
+static int wave_columns(int tile) {
+    constexpr int cols[TILE_COUNT] = {256 / 4, 192 / 2, 128 / 2, 128 / 4, 64 / 2, 64 / 2};
+    return cols[tile];
+}
+// Steps of more than 64 rows: the product before a norm, which prepares it (EPI_PRENORM), and the gated product behind it, which applies the rows' factors (SCALED), in the
+// tiles that they are planned in without the norm.
+template <int EPI, bool SCALED>
+static int launch_around_norm(const elem_t* A, const elem_t* W, int M, int N, int K, EpiArgs ep, hipStream_t stream) {
+    ep.k_per_split = K;
+#define MS_AROUND(BM_, BN_, WM_, WN_, ST_)                                                                                                                 \
+    do {                                                                                                                                                   \
+        hipLaunchKernelGGL((gemm_kernel<BM_, BN_, WM_, WN_, 64, EPI, ST_, SCALED>), dim3((unsigned)((long)ceil_div(M, BM_) * ceil_div(N, BN_)), 1),       \
+                           dim3(64 * WM_ * WN_), 0, stream, A, W, M, N, K, ep);                                                                            \
+        return check_launch("gemm around a norm, " #BM_ "x" #BN_);                                                                                         \
+    } while (0)
+    switch (plan_gemm(M, N, K, 1, EPI == EPI_PRENORM, SCALED).tile) {
+        case TILE_256x320:
+            if constexpr (SCALED) MS_AROUND(256, 320, 2, 4, GEMM_PIPED);
+        case TILE_256x256: MS_AROUND(256, 256, 2, 4, GEMM_PIPED);
+        case TILE_256x192: MS_AROUND(256, 192, 4, 2, GEMM_PIPED);
+        case TILE_256x128: MS_AROUND(256, 128, 4, 2, GEMM_PIPED);
+        case TILE_128x128: MS_AROUND(128, 128, 2, 4, GEMM_PIPED);
+        case TILE_64x64: MS_AROUND(64, 64, 2, 2, GEMM_PIPED);
+        default: MS_AROUND(64, 64, 2, 2, 4);
+    }
+#undef MS_AROUND
+}
+#endif
+
 // K slices for a product whose consumer adds partial sums: enough 128x128 blocks to fill the chip,
 // at least 512 of K each.  The 32-bit build does not slice here: its sums keep one order.
 #ifdef MS_MEASURE
@@ -356,11 +387,11 @@ extern "C" int ms_linear_act(const void* a, const void* w, void* out, int M, int
     return launch_gemm<EPI_ACT>((const elem_t*)a, (const elem_t*)w, M, N, K, ep, stream);
 }
 
-// Whether ms_linear_swiglu_scaled takes this shape: bfloat16, one tile of rows, whole K steps of 64.
+// Whether ms_linear_swiglu_scaled takes this shape: bfloat16, whole K steps of 64.
 extern "C" int ms_swiglu_scaled_takes(int M, int I, int K) {
 #ifdef MS_ELEM_HALF
     (void)I;
-    return kRoundsBeforeTheNormIsSafe && M >= 1 && M <= 64 && K % 64 == 0 && K >= 256;
+    return kRoundsBeforeTheNormIsSafe && M >= 1 && K % 64 == 0 && K >= 256;
 #else
     (void)M; (void)I; (void)K;
     return 0;
@@ -378,6 +409,9 @@ extern "C" int ms_linear_swiglu_scaled(const void* a, const float* row_ss, int s
     MS_REQUIRE((reinterpret_cast<uintptr_t>(a) & 15) == 0 && (reinterpret_cast<uintptr_t>(w) & 15) == 0, "gemm: operands must be 16-byte aligned");
     const int n = 2 * ceil_div(I, 16) * 16;
     EpiArgs ep{out, nullptr, I, I, K, 0, row_ss, ss_parts, eps, act};
+    if (planned(M, K)) {
+        if constexpr (kRoundsBeforeTheNormIsSafe) return launch_around_norm<EPI_SWIGLU, true>((const elem_t*)a, (const elem_t*)w, M, n, K, ep, stream);
+    }
     if (few_rows(M, n, K, false, true)) return launch_few<EPI_SWIGLU, true>((const elem_t*)a, (const elem_t*)w, M, n, K, ep, stream, 1);
     hipLaunchKernelGGL((gemm_kernel<64, 64, 2, 2, 64, EPI_SWIGLU, 4, true>), dim3((unsigned)ceil_div(n, 64), 1), dim3(256), 0, stream,
                        (const elem_t*)a, (const elem_t*)w, M, n, K, ep);
@@ -389,9 +423,12 @@ extern "C" int ms_linear_swiglu_scaled(const void* a, const float* row_ss, int s
 }
 
 // Column tiles of ms_linear_residual_prenorm for this shape (the first size of its ss_part), or 0 if it is not taken: up to 16 rows over whole K steps,
-// uncut, where that is predicted to take no longer than the slices and the norm that would add them up (2.5 us: a launch and a trip to memory).
+// uncut, where that is predicted to take no longer than the slices and the norm that would add them up (2.5 us: a launch and a trip to memory); more than 64
+// rows where the product is not cut: of the norm's 5.1 us a layer of 2,048 rows of the 0.5B sizes 1 goes to this product's epilogue and 2.4 to the gated product's
+// start and end, and a prompt takes 3.14 ms for 3.17.
 extern "C" int ms_prenorm_parts(int M, int N, int K) {
 #ifdef MS_ELEM_HALF
+    if (kRoundsBeforeTheNormIsSafe && planned(M, K) && plan_tiled_splits(M, N, K) == 1) return ceil_div(N, wave_columns(plan_gemm(M, N, K, 1, true).tile));
     if (!kRoundsBeforeTheNormIsSafe || M < 1 || M > 16 || !few_rows(M, N, K, false, false)) return 0;
     return plan_few(16, N, K, 1, false).us < plan_few(16, N, K, 0, false).us + 2.5f ? ceil_div(N, 16) : 0;
 #else
@@ -412,6 +449,9 @@ extern "C" int ms_linear_residual_prenorm(const void* a, const void* w, float* x
     ep.norm_w = norm_w;
     ep.hn = (elem_t*)hn;
     ep.ss_part = ss_part;
+    if (planned(M, K)) {
+        if constexpr (kRoundsBeforeTheNormIsSafe) return launch_around_norm<EPI_PRENORM, false>((const elem_t*)a, (const elem_t*)w, M, N, K, ep, stream);
+    }
     return launch_few<EPI_PRENORM>((const elem_t*)a, (const elem_t*)w, M, N, K, ep, stream, 1);
 #else
     (void)a; (void)w; (void)x; (void)norm_w; (void)hn; (void)ss_part; (void)M; (void)N; (void)K; (void)stream;

@@ -37,7 +37,7 @@ constexpr int GEMM_SPLIT = 8;  // 32-bit: two buffers, and every number in three
 enum EpiKind {
     EPI_STORE_F32 = 0, EPI_STORE_ELEM = 1, EPI_RESIDUAL = 2, EPI_SWIGLU = 3, EPI_QKV_ROPE = 4, EPI_ACT = 5,
     EPI_EXPERT_GATED = 6, EPI_EXPERT_PLAIN = 7, EPI_EXPERT_DOWN = 8,  // over the rows that chose an expert (routed.hip)
-    EPI_PRENORM = 9,  // few rows only (few_rows.cuh): into the residual stream, and what the norm that follows needs
+    EPI_PRENORM = 9,  // into the residual stream, and what the norm that follows needs
 };
 
 struct NoExperts {
@@ -68,11 +68,11 @@ struct EpiArgs {
     elem_t* kpool;         // [pages, KV, ps, hd]
     elem_t* vpool;         // [pages, KV, hd, ps]
     int H, KV, ps;
-    // PRENORM: the new values of the stream times the norm's weight, not yet divided by the rows' root mean square, and each tile's 16 columns' share of
-    // the rows' sums of squares
+    // PRENORM: the new values of the stream times the norm's weight, not yet divided by the rows' root mean square, and each tile's (of 16 columns; in
+    // tiles of more than 64 rows each column of waves') share of the rows' sums of squares
     const float* norm_w;  // [N]
     elem_t* hn;           // [M, N]
-    float* ss_part;       // [N / 16 rounded up, M]
+    float* ss_part;       // [N / 16, or the columns of a wave, rounded up, M]
 };
 
 // The block of rows m0 .. m0 + BM and columns n0 .. n0 + BN.  `rows` says which row of A the block's row i is and, for the
@@ -101,11 +101,12 @@ __device__ __forceinline__ void gemm_tile(const elem_t* __restrict__ A, const el
     constexpr int TM = BM / WM / 16, TN = BN / WN / 16;
     constexpr int A_CHUNKS = BM * CPR / NT, W_CHUNKS = BN * CPR / NT;
     static_assert(BM * CPR % NT == 0 && BN * CPR % NT == 0, "tile loads divide over the block");
-    static_assert(NT == 256 || !SCALED, "the row factors' shares are dealt to four waves");
+    static_assert(NT == 256 || !SCALED || PIPED, "the row factors' shares are dealt to four waves");
     static_assert(STAGES == 2 || DIRECT || SPLIT, "more than two LDS buffers, and phases, only with direct loads");
-    static_assert(!SCALED || (STAGES > 2 && EPI == EPI_SWIGLU), "row factors: built for the gated product with several steps in flight");
+    static_assert(!SCALED || ((STAGES > 2 || PIPED) && EPI == EPI_SWIGLU), "row factors: built for the gated product with several steps in flight");
     static_assert(256 % BM == 0 || !SCALED, "threads are dealt to the rows");
-    __shared__ float ss_q[SCALED ? 256 / BM : 1][SCALED ? BM : 1];  // the rows' sums of squares, in 256 / BM interleaved shares
+    // the rows' sums of squares, in 256 / BM interleaved shares; in phases the rows' factors
+    __shared__ float ss_q[SCALED && !PIPED ? 256 / BM : 1][SCALED ? BM : 1];
     float ss_v[SCALED ? 8 : 1];
     int ss_r = 0;
     __shared__ __attribute__((aligned(16))) elem_t As[BUFS][BM * LDS_LD];
@@ -460,6 +461,22 @@ __device__ __forceinline__ void gemm_tile(const elem_t* __restrict__ A, const el
         if (nk > 1)
 #pragma unroll
             for (int l = 0; l < PER_STEP; ++l) load_nth(k_begin + BK, 1, l);
+        if constexpr (SCALED) {
+            // A row's factor is its thread's: the parts of its sum of squares, written by the kernel before this one, are asked for behind the first steps,
+            // thirty-two at a time, and come with them.
+            if (tid < BM) {
+                const int row = min(m0 + tid, M - 1);
+                float sum = 0.f;
+                for (int p0 = 0; p0 < ep.ss_parts; p0 += 32) {
+                    float v[32];
+#pragma unroll
+                    for (int u = 0; u < 32; ++u) v[u] = ep.row_ss[(size_t)min(p0 + u, ep.ss_parts - 1) * M + row];
+#pragma unroll
+                    for (int u = 0; u < 32; ++u) sum += p0 + u < ep.ss_parts ? v[u] : 0.f;
+                }
+                ss_q[0][tid] = 1.0f / sqrtf(sum / (float)K + ep.ss_eps);
+            }
+        }
         arrive(nk > 1);
 #pragma unroll
         for (int i = 0; i < TH; ++i) fetch_a(0, 0, 0, 0, i);
@@ -631,9 +648,13 @@ __device__ __forceinline__ void gemm_tile(const elem_t* __restrict__ A, const el
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
                         const int lr = wm * (BM / WM) + i * 16 + grp * 4 + e;
+                        if constexpr (PIPED) {
+                            f[e] = ss_q[0][lr];
+                            continue;
+                        }
                         float ssum = 0.f;
 #pragma unroll
-                        for (int qq = 0; qq < 256 / BM; ++qq) ssum += ss_q[qq][lr];
+                        for (int qq = 0; qq < 256 / BM; ++qq) ssum += ss_q[PIPED ? 0 : qq][lr];
                         f[e] = 1.0f / sqrtf(ssum / (float)K + ep.ss_eps);
                     }
                 }
@@ -711,8 +732,12 @@ __device__ __forceinline__ void gemm_tile(const elem_t* __restrict__ A, const el
             // RESIDUAL: what the stream holds is asked for a group of sixteen rows ahead of its stores.  Added to in place, every load stood behind the
             // stores before it, which may write the same address: 14.7 of 65 us in 256x128 tiles of 2,048 x 3,584 x 3,584.  Cold operands, before and
             // now: that product 69.6 -> 59.9 us, 2,048 x 1,536 x 1,536 (128x128) 24.2 -> 20.3, 2,048 x 896 x 896 (64x64) 10.0 -> 8.7.
-            constexpr int AHEAD = EPI == EPI_RESIDUAL ? 2 : 1;
-            float prior[AHEAD][EPI == EPI_RESIDUAL ? TN : 1][4];
+            constexpr bool ADDS = EPI == EPI_RESIDUAL || EPI == EPI_PRENORM;
+            constexpr int AHEAD = ADDS ? 2 : 1;
+            float prior[AHEAD][ADDS ? TN : 1][4], nw[EPI == EPI_PRENORM ? TN : 1];
+            if constexpr (EPI == EPI_PRENORM)
+#pragma unroll
+                for (int j = 0; j < TN; ++j) nw[j] = ep.norm_w[min(col_base + j * 16, N - 1)];
             auto ask = [&](int i) {
 #pragma unroll
                 for (int j = 0; j < TN; ++j)
@@ -722,14 +747,15 @@ __device__ __forceinline__ void gemm_tile(const elem_t* __restrict__ A, const el
                         prior[i % AHEAD][j][e] = reinterpret_cast<const float*>(ep.out)[(size_t)(CHECKED || ROW_GROUPS ? min(row, M - 1) : row) * ep.ldo + (CHECKED ? min(col, N - 1) : col)];
                     }
             };
-            if constexpr (EPI == EPI_RESIDUAL) ask(0);
+            if constexpr (ADDS) ask(0);
 #pragma unroll
             for (int i = 0; i < TM; ++i) {
-                if constexpr (EPI == EPI_RESIDUAL) {
+                if constexpr (ADDS) {
                     if (i + 1 < TM) ask(i + 1);
                     __builtin_amdgcn_sched_barrier(0);
                 }
                 if (ROW_GROUPS && m0 + wm * (BM / WM) + i * 16 >= M) continue;
+                float ss[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
                 for (int j = 0; j < TN; ++j) {
                     const int col = col_base + j * 16;
@@ -744,7 +770,21 @@ __device__ __forceinline__ void gemm_tile(const elem_t* __restrict__ A, const el
                         else if constexpr (EPI == EPI_STORE_ELEM) reinterpret_cast<elem_t*>(ep.out)[o] = from_f32<elem_t>(v);
                         else if constexpr (EPI == EPI_ACT) reinterpret_cast<elem_t*>(ep.out)[o] = from_f32<elem_t>(unary_activation(v, ep.act));
                         else reinterpret_cast<float*>(ep.out)[o] = prior[i % AHEAD][j][e] + v;  // residual stream, 32-bit
+                        if constexpr (EPI == EPI_PRENORM) {
+                            const float x = prior[i % AHEAD][j][e] + v;
+                            ep.hn[o] = from_f32<elem_t>(x * nw[j]);
+                            ss[e] = fmaf(x, x, ss[e]);
+                        }
                     }
+                }
+                if constexpr (EPI == EPI_PRENORM) {  // the sixteen lanes of a row, each of which then has the sum of one row of four to store
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+#pragma unroll
+                        for (int o = 1; o < 16; o <<= 1) ss[e] += __shfl_xor(ss[e], o, WAVE);
+                    const int row = row_base + i * 16 + r16;  // (of lanes 0 to 3 of the sixteen)
+                    if (r16 < 4 && row < M && n0 + wn * (BN / WN) < N)  // (a wave behind the last column has no share)
+                        ep.ss_part[(size_t)((n0 + wn * (BN / WN)) / (BN / WN)) * M + row] = r16 == 0 ? ss[0] : r16 == 1 ? ss[1] : r16 == 2 ? ss[2] : ss[3];
                 }
             }
         }

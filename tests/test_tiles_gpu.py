@@ -120,3 +120,41 @@ def test_32_bit_products_in_parts(M, N, K):
     fine = torch.isfinite(ref)
     err = (got.double() - ref).abs()[fine] / (a.abs().double().nan_to_num(0, 0, 0) @ w.abs().double().nan_to_num(0, 0, 0).T)[fine]
     assert float(err.max()) < 2e-6
+
+
+# Around a norm, more than 64 rows: the product that prepares it in every tile, ragged at both edges, a last column of waves that has no columns (widths of 20 and 1,030); what
+# the kernel leaves behind its last part stays untouched.
+@pytest.mark.parametrize("M,N,K,tile", SIZES + [(1030, 1030, 512, None), (65, 20, 64, None), (200, 24, 128, None), (2048, 896, 896, None)])
+def test_products_that_prepare_a_norm(M, N, K, tile):
+    from machserve_amd.kernels.ops import _c_int, _ptr
+    ops = ops_for(torch.bfloat16)
+    a, w, x0 = rnd((M, K), torch.bfloat16, 21), rnd((N, K), torch.bfloat16, 22, K ** -0.5), rnd((M, N), torch.float32, 23)
+    nw = 1 + rnd((N,), torch.float32, 24, 0.1)
+    parts = ops._plan("ms_prenorm_parts", M, N, K)
+    if ops._plan("ms_tiled_partials", M, N, K) > 1:
+        assert parts == 0 and ops.linear_residual(a, w, x0.clone()) is not None
+        return
+    assert parts > 0
+    want = x0.clone()
+    assert ops.linear_residual(a, w, want) is None
+    x, hn, room = x0.clone(), torch.empty((M, N), dtype=torch.bfloat16, device=DEV), torch.full(((parts + 4) * M,), -7.0, device=DEV)
+    ops._check(ops._core, ops._core.ms_linear_residual_prenorm(_ptr(a), _ptr(w), _ptr(x), _ptr(nw), _ptr(hn), _ptr(room), _c_int(M), _c_int(N), _c_int(K), ops._stream()))
+    assert torch.equal(x, want) and torch.equal(hn, (x * nw).bfloat16())
+    assert bool((room[parts * M:] == -7.0).all())
+    assert_close(room[:parts * M].view(parts, M).sum(0), (x.double() ** 2).sum(1), torch.float32, "sums of squares")
+
+
+# ... and the gated product that applies the rows' factors, in every tile: one part and more than sixteen
+@pytest.mark.parametrize("M,I,K,parts", [(2048, 4800, 896, 28), (1990, 4850, 960, 17), (1537, 4100, 1024, 1), (1000, 4100, 1024, 16), (700, 3076, 1024, 5), (1000, 2052, 320, 33),
+                                         (193, 2052, 256, 4), (65, 1028, 256, 40), (130, 20, 320, 3), (512, 4864, 896, 28)])
+def test_gated_products_with_row_factors_of_many_rows(M, I, K, parts):
+    from machserve_amd.kernels.ops import interleave_gate_up
+    ops = ops_for(torch.bfloat16)
+    a, gate, up = rnd((M, K), torch.bfloat16, 31), rnd((I, K), torch.bfloat16, 32, 2 * K ** -0.5), rnd((I, K), torch.bfloat16, 33, K ** -0.5)
+    w, share = interleave_gate_up(gate, up), rnd((parts, M), torch.float32, 34).abs() * K / parts
+    f = 1.0 / torch.sqrt(share.double().sum(0) / K + 1e-5)[:, None]
+    z, u = (a.double() @ gate.double().T) * f, (a.double() @ up.double().T) * f
+    got = ops.linear_swiglu_scaled(a, share, 1e-5, w, I)
+    assert_close(got, z * torch.sigmoid(z) * u, torch.bfloat16, "gated product with row factors")
+    if M > 300:
+        assert_close(ops.linear_swiglu_scaled(a[:200].contiguous(), share[:, :200].contiguous(), 1e-5, w, I), got[:200].double(), torch.bfloat16, "a row in another batch")
