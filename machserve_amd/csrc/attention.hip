@@ -1052,7 +1052,8 @@ struct DecodeTile {
     Frag vf[DNTP][ND];
 };
 
-template <bool FUSED>
+// MANY (fused): the q/k/v product left more than two partial sums, of which up to eight are then asked for first of all.
+template <bool FUSED, bool MANY = false>
 __global__ __launch_bounds__(256) void decode_attention_kernel(DecodeArgs a) {
     arguments_now(a.q, a.kpool, a.vpool, a.out, a.part_o, a.part_ml, a.block_table, a.seq_pos0, a.table_stride, a.H, a.KV, a.hd,
                   a.ps, a.window, a.nsplit, a.scale, a.qkv, a.bias, a.inv_freq, a.slot_map, a.n_partials, a.stride);
@@ -1147,9 +1148,10 @@ __global__ __launch_bounds__(256) void decode_attention_kernel(DecodeArgs a) {
         }
     };
     // The fused prologue stages this KV head's share of the step's row: its g query heads, its key, its
-    // value, (g + 2) * hd columns, four per thread at a time.  What the first four need from memory
-    // (the bias and the first two partial sums) is asked for here, before anything else: nothing of it
-    // depends on the row's position, and the row's query is what the block waits for in the end.
+    // value, (g + 2) * hd columns, four per thread at a time, with heads of more than 64 five (1,280: seven heads of 128 beside key and value are 1,152).  What the
+    // first of them need from memory (the bias and the first partial sums) is asked for here, before anything else: nothing of it
+    // depends on the row's position, and the row's query is what the block waits for in the end.  (Seven sums of 1,152 columns, 28 heads
+    // over 4 of 128, 16 requests: two first, five more and the last 128 columns behind them 13.8 us, all at once 11.5.)
     const int width = FUSED ? (g + 2) * hd : 0;
     const size_t pstride = FUSED ? (size_t)gridDim.x * a.stride : 0;
     const float* row0 = FUSED ? a.qkv + (size_t)s * a.stride : nullptr;
@@ -1160,17 +1162,21 @@ __global__ __launch_bounds__(256) void decode_attention_kernel(DecodeArgs a) {
         const int qcol = kvh * g * hd, kcol = a.H * hd + kvh * hd, vcol = (a.H + a.KV) * hd + kvh * hd;
         return c < g * hd ? qcol + c : (c < (g + 1) * hd ? kcol + c - g * hd : vcol + c - (g + 1) * hd);
     };
-    int col_e[4];
-    float bias_e[4], part_e[2][4], freq_e = 0.f;
+    constexpr int COLS = ND > 4 ? 5 : 4, EARLY = MANY ? 8 : 2;
+    int col_e[COLS];
+    float bias_e[COLS], part_e[EARLY][COLS], freq_e = 0.f;
     int slot = -1;
     if constexpr (FUSED) {
-        const size_t p1 = (size_t)min(1, a.n_partials - 1) * pstride;
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
+        for (int u = 0; u < COLS; ++u) {
             col_e[u] = column(tid + u * 256);
             bias_e[u] = bias[col_e[u]];
-            part_e[0][u] = row0[col_e[u]];
-            part_e[1][u] = row0[p1 + col_e[u]];
+        }
+#pragma unroll
+        for (int q = 0; q < EARLY; ++q) {
+            const size_t po = (size_t)min(q, a.n_partials - 1) * pstride;
+#pragma unroll
+            for (int u = 0; u < COLS; ++u) part_e[q][u] = row0[po + col_e[u]];
         }
         freq_e = (a.inv_freq ? a.inv_freq : row0)[min(tid, hd / 2 - 1)];
         slot = a.slot_map[s];
@@ -1200,44 +1206,48 @@ __global__ __launch_bounds__(256) void decode_attention_kernel(DecodeArgs a) {
         // Further partial sums, eight at a time, all of their loads asked for before the first is added: the
         // sums were written by the kernel before this one, and one load after the other would be as many trips
         // to them (beyond the last partial sum: the last one again, not added).
-        auto add_partials = [&](int first, const int (&col)[4], float (&v)[4]) {
+        auto add_partials = [&](int first, const int (&col)[COLS], float (&v)[COLS]) {
             constexpr int NB = 8;
             for (int p0 = first; p0 < a.n_partials; p0 += NB) {
-                float t[NB][4];
+                float t[NB][COLS];
 #pragma unroll
                 for (int q = 0; q < NB; ++q) {
                     const size_t po = (size_t)min(p0 + q, a.n_partials - 1) * pstride;
 #pragma unroll
-                    for (int u = 0; u < 4; ++u) t[q][u] = row0[po + col[u]];
+                    for (int u = 0; u < COLS; ++u) t[q][u] = row0[po + col[u]];
                 }
 #pragma unroll
                 for (int q = 0; q < NB; ++q)
                     if (p0 + q < a.n_partials) {
 #pragma unroll
-                        for (int u = 0; u < 4; ++u) v[u] += t[q][u];
+                        for (int u = 0; u < COLS; ++u) v[u] += t[q][u];
                     }
             }
         };
         {
-            float v[4];
+            float v[COLS];
 #pragma unroll
-            for (int u = 0; u < 4; ++u) v[u] = bias_e[u] * bias_on + part_e[0][u] + (a.n_partials > 1 ? part_e[1][u] : 0.f);
-            add_partials(2, col_e, v);
+            for (int u = 0; u < COLS; ++u) {
+                v[u] = bias_e[u] * bias_on + part_e[0][u];
 #pragma unroll
-            for (int u = 0; u < 4; ++u)
+                for (int q = 1; q < EARLY; ++q) v[u] += q < a.n_partials ? part_e[q][u] : 0.f;
+            }
+            add_partials(EARLY, col_e, v);
+#pragma unroll
+            for (int u = 0; u < COLS; ++u)
                 if (tid + u * 256 < width) rowv[tid + u * 256] = v[u];
         }
-        for (int c0 = tid + 4 * 256; c0 < width; c0 += 4 * 256) {  // more than 1,024 columns: many large heads
-            int col[4];
-            float v[4];
+        for (int c0 = tid + COLS * 256; c0 < width; c0 += COLS * 256) {  // more columns: many large heads
+            int col[COLS];
+            float v[COLS];
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
+            for (int u = 0; u < COLS; ++u) {
                 col[u] = column(c0 + u * 256);
                 v[u] = bias[col[u]] * bias_on;
             }
             add_partials(0, col, v);
 #pragma unroll
-            for (int u = 0; u < 4; ++u)
+            for (int u = 0; u < COLS; ++u)
                 if (c0 + u * 256 < width) rowv[c0 + u * 256] = v[u];
         }
         __syncthreads();
@@ -1831,7 +1841,8 @@ extern "C" int MS_CAT(ms_decode_attention_fused_nd, MS_ATTN_ND)(
     MS_REQUIRE(slot_map && kpool && vpool, "decode attention: the fused form writes the cache");
     DecodeArgs a{nullptr, (const elem_t*)kpool, (const elem_t*)vpool, (elem_t*)out, part_o, part_ml, block_table, seq_pos0,
                  table_stride, H, KV, hd, ps, window, nsplit, scale, qkv, bias, inv_freq, slot_map, n_partials, stride, nullptr, nullptr};
-    hipLaunchKernelGGL(decode_attention_kernel<true>, dim3((unsigned)S, (unsigned)KV, (unsigned)nsplit), dim3(256), 0, stream, a);
+    if (n_partials > 2) hipLaunchKernelGGL((decode_attention_kernel<true, true>), dim3((unsigned)S, (unsigned)KV, (unsigned)nsplit), dim3(256), 0, stream, a);
+    else hipLaunchKernelGGL((decode_attention_kernel<true>), dim3((unsigned)S, (unsigned)KV, (unsigned)nsplit), dim3(256), 0, stream, a);
     int rc = check_launch("decode_attention_fused");
     if (rc || nsplit == 1) return rc;
     hipLaunchKernelGGL(decode_merge_kernel, dim3((unsigned)(S * H)), dim3(64), 0, stream, part_o, part_ml, (elem_t*)out, hd, nsplit, a.sinks, H, a.out_gate);
