@@ -1061,3 +1061,24 @@ def test_zeroing_a_place_of_several_arrays():
     for place in (4, -1):
         with pytest.raises(KernelError):
             ops.zero_places(places, place)
+
+
+@pytest.mark.parametrize("d", [4, 896, 1024, 1028, 2048, 2052, 4096, 4100])
+@pytest.mark.parametrize("na,nb", [(1, 1), (2, 1), (3, 2), (8, 8), (9, 1)])
+def test_normed_branches_added_to_the_stream(d, na, nb):
+    """One, two and four groups of 1,024 columns and widths behind them; up to two, up to eight and more sums: a branch, a branch with a bias, two branches weighed."""
+    ops = ops_for(torch.bfloat16)
+    T, eps = 3, 1e-5
+    x0, pa, pb = rnd((T, d), torch.float32, 111), rnd((na, T, d), torch.float32, 112), rnd((nb, T, d), torch.float32, 113)
+    w, bias = 1 + rnd((d,), torch.float32, 114, 0.2), rnd((d,), torch.float32, 115)
+    norm = lambda y: y / torch.sqrt((y * y).mean(-1, keepdim=True) + eps) * w.double()  # noqa: E731
+    dev = lambda t: t.to(DEV)  # noqa: E731
+    x = dev(x0)
+    ops.norm_add(x, dev(pa), dev(w), eps)
+    assert_close(x, x0.double() + norm(pa.double().sum(0)), torch.float32, "a branch")
+    x = dev(x0)
+    ops.norm_add_bias(x, dev(pa), dev(bias), dev(w), eps)
+    assert_close(x, x0.double() + norm(pa.double().sum(0) + bias.double()), torch.float32, "a branch with a bias")
+    x = dev(x0)
+    ops.norm_add_weighted(x, dev(pa), 1.2, dev(pb), 0.7, dev(w), eps)
+    assert_close(x, x0.double() + norm(1.2 * pa.double().sum(0) + 0.7 * pb.double().sum(0)), torch.float32, "two branches")
