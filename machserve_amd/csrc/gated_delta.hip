@@ -177,21 +177,44 @@ constexpr int CH = 64;        // tokens of a chunk: one a lane where their decay
 constexpr int SL = 64;        // channels of q and k that a block holds in LDS at a time
 constexpr int LDP = SL + 4;   // their row stride
 
-// What the kernels hand on lies per (chunk's number, head) in whole tiles of 16, zeros beyond the chunk's tokens and the head's
-// channels, with the index that an operand's four steps run over innermost: every load of an operand is 16 bytes, without
-// conditions.
+// What the kernels hand on lies per (chunk's number, head) in whole tiles of 16 x 16, zeros beyond the chunk's tokens and the
+// head's channels, each as the operand that the next kernel wants of it: lane (grp, r16) has the four numbers from grp * 4 on
+// of the tile's line r16.  So every load of an operand is 1 KB in one piece, without conditions (in rows
+// of 64 bytes of whole matrices the pass took 86 us for a prompt of 2,048 tokens, 16 heads of 128, and 69 so).
 struct DeltaChunkArgs {
     StateArgs a;   // q and k already unit vectors and scaled: one partial sum, columns from 0
-    float* W;      // [numbers, H, CH, dk16]
-    float* Kt;     // [numbers, H, dk16, CH]: exp(L_n - L_j) k_j
-    float* U0;     // [numbers, H, dv16, CH]
-    float* U;      // [numbers, H, dv16, CH]
-    float* Sb;     // [numbers, H, dv16, dk16]: the state before each chunk
+    float* W;      // [numbers, H, dk16 / 16, CH / 16] tiles, a line a token
+    float* Kt;     // [numbers, H, dk16 / 16, CH / 16] tiles, a line a channel: exp(L_n - L_j) k_j
+    float* U0;     // [numbers, H, dv16 / 16, CH / 16] tiles, a line a channel
+    float* U;      // as U0
+    float* Sb;     // [numbers, H, dv16 / 16, dk16 / 16] tiles, a line a value channel: the state before each chunk
     float* total;  // [numbers, H]: exp(L_n)
     int dk16, dv16;
 };
 
 __device__ __forceinline__ f32x4 mfma_f32(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
+
+constexpr int CT16 = CH / 16, TILE = 256;
+
+// x[i] of lane q becomes x[q] of lane i among each four lanes
+__device__ __forceinline__ float from_lane_xor1(float v) { return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xB1, 0xF, 0xF, true)); }
+__device__ __forceinline__ float from_lane_xor2(float v) { return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x4E, 0xF, 0xF, true)); }
+__device__ __forceinline__ f32x4 turn_quads(f32x4 x, int lane) {
+    const bool q1 = lane & 1, q2 = lane & 2;
+#pragma unroll
+    for (int i = 0; i < 4; i += 2) {
+        const float got = from_lane_xor1(q1 ? x[i] : x[i + 1]);
+        x[i] = q1 ? got : x[i];
+        x[i + 1] = q1 ? x[i + 1] : got;
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const float got = from_lane_xor2(q2 ? x[i] : x[i + 2]);
+        x[i] = q2 ? got : x[i];
+        x[i + 2] = q2 ? x[i + 2] : got;
+    }
+    return x;
+}
 
 // lane i: the sum of v over lanes 0 .. i
 __device__ __forceinline__ float lane_sums(float v, int lane) {
@@ -237,7 +260,7 @@ __device__ __forceinline__ void lower_tile(int t, int& rt, int& ct) {
 __global__ __launch_bounds__(256) void delta_solve_kernel(DeltaChunkArgs p) {
     const StateArgs& a = p.a;
     __shared__ __align__(16) float Ks[CH * LDP], As[CH * LDP];
-    __shared__ float Ls[CH], bs[CH];
+    __shared__ __align__(16) float Ls[CH], bs[CH], es[CH];
     const Piece pc = piece_of(blockIdx.x, CH, a.seq_q_start, a.S);
     const int left = a.seq_q_len[pc.s] - pc.first;
     if (left <= 0) return;  // the same for the whole block
@@ -247,7 +270,9 @@ __global__ __launch_bounds__(256) void delta_solve_kernel(DeltaChunkArgs p) {
     const float* kp = a.k.p + (size_t)t0 * ldk + (size_t)kh * a.d;
     const size_t at = (size_t)blockIdx.x * a.H + h;
     if (wave == 0) {
-        Ls[lane] = decay_sums(a.decay, t0, n, a.H, h, lane);
+        const float L = decay_sums(a.decay, t0, n, a.H, h, lane);
+        Ls[lane] = L;
+        es[lane] = expf(__shfl(L, CH - 1, WAVE) - L);  // (the sums stay as they are beyond the chunk's end)
         bs[lane] = lane < n ? a.beta[(size_t)(t0 + lane) * a.H + h] : 0.f;
     }
     const int used = (n + 15) / 16, tiles = used * (used + 1) / 2;  // row tiles with tokens, and their lower triangle
@@ -283,8 +308,17 @@ __global__ __launch_bounds__(256) void delta_solve_kernel(DeltaChunkArgs p) {
         if (c0) __syncthreads();
         put_slice(Ks, ks, c0, n, a.d);
         __syncthreads();
-        const float e = expf(Ls[CH - 1] - Ls[lane]);  // (the sums stay as they are beyond the chunk's end)
-        for (int c = wave; c < min(SL, p.dk16 - c0); c += 4) p.Kt[(at * p.dk16 + c0 + c) * CH + lane] = e * Ks[lane * LDP + c];
+        static_assert(SL == 64, "a tile of channels a wave");
+        if (c0 + wave * 16 < p.dk16) {
+            float* dst = p.Kt + at * p.dk16 * CH + (size_t)(c0 / 16 + wave) * CT16 * TILE + lane * 4;
+#pragma unroll
+            for (int rt = 0; rt < CT16; ++rt) {
+                f32x4 e = *reinterpret_cast<const f32x4*>(&es[rt * 16 + grp * 4]);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) e[i] *= Ks[(rt * 16 + grp * 4 + i) * LDP + wave * 16 + r16];
+                *reinterpret_cast<f32x4*>(dst + rt * TILE) = e;
+            }
+        }
 #pragma unroll
         for (int u = 0; u < 3; ++u) {
             const int tile = wave + u * 4;
@@ -367,15 +401,14 @@ __global__ __launch_bounds__(256) void delta_solve_kernel(DeltaChunkArgs p) {
         for (int u = 0; u < 2; ++u) {
             if (ct0 + u * 4 >= cts) continue;
             if (is_k[u]) {
-                float* dst = p.W + at * CH * p.dk16 + c[u];
+                // lane (grp, r16) has rows grp * 4 + i of column r16 and leaves row grp * 4 + r16 % 4, columns from r16 / 4 * 4 on
+                float* dst = p.W + at * CH * p.dk16 + (size_t)(c[u] - r16) / 16 * CT16 * TILE + ((r16 / 4) * 16 + grp * 4 + r16 % 4) * 4;
 #pragma unroll
-                for (int b = 0; b < 4; ++b)
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) dst[(size_t)(b * 16 + grp * 4 + i) * p.dk16] = X[u][b][i];
+                for (int b = 0; b < CT16; ++b) *reinterpret_cast<f32x4*>(dst + b * TILE) = turn_quads(X[u][b], lane);
             } else {
-                float* dst = p.U0 + (at * p.dv16 + c[u]) * CH + grp * 4;
+                float* dst = p.U0 + at * CH * p.dv16 + (size_t)(c[u] - r16) / 16 * CT16 * TILE + lane * 4;
 #pragma unroll
-                for (int b = 0; b < 4; ++b) *reinterpret_cast<f32x4*>(dst + b * 16) = X[u][b];
+                for (int b = 0; b < CT16; ++b) *reinterpret_cast<f32x4*>(dst + b * TILE) = X[u][b];
             }
         }
     }
@@ -385,7 +418,10 @@ __global__ __launch_bounds__(256) void delta_solve_kernel(DeltaChunkArgs p) {
 // w * KT .. w * KT + KT - 1 as accumulators, which serve as operands as they are: lane (grp, r16) holds rows grp * 4 + i of
 // column r16, and supplies them as the four steps i of a product over those rows.
 // FULL: every wave's tiles lie within the head.  Operands are asked for a chunk ahead, into one of two sets of registers in
-// turn, and no load or store of the loop stands behind a condition.
+// turn, and no load or store of the loop stands behind a condition.  The 20 loads (80 KB a block) are spread among the products, a
+// group's loads before its products: all of them ahead of the first product kept it from starting for as long as half of a
+// chunk's products take.  A chunk: 2.6 us with the operands in matrices and the loads ahead of all, 2.1 with the operands in
+// tiles, 1.65 with the loads among the products (its products alone 1.0), 2,048 tokens 86, 69 and 54 us.
 template <int KT>
 struct PassOperands {
     f32x4 W[4][KT], K[KT][4], U[4];
@@ -419,51 +455,46 @@ __global__ __launch_bounds__(256) void delta_pass_kernel(DeltaChunkArgs p) {
     const int nch = (len + CH - 1) / CH;
     const size_t at0 = (size_t)piece_base(s, CH, a.seq_q_start) * a.H + h, step = a.H;
     PassOperands<KT> A, B;
-    auto fetch = [&](PassOperands<KT>& o, int ch) {
-        const size_t at = at0 + ch * step;
-        o.g = p.total[at];
-        const float* wp = p.W + (at * CH + r16) * p.dk16 + grp * 4;
-        const float* kp = p.Kt + (at * p.dk16 + r16) * CH + grp * 4;
-        const float* up = p.U0 + (at * p.dv16 + col) * CH + grp * 4;
+    auto fetch_w = [&](PassOperands<KT>& o, size_t at, int rt) {
+        const float* wp = p.W + at * CH * p.dk16 + rt * TILE + lane * 4;
 #pragma unroll
-        for (int rt = 0; rt < 4; ++rt)
+        for (int kt = 0; kt < KT; ++kt) o.W[rt][kt] = *reinterpret_cast<const f32x4*>(wp + kk[kt] * CH);
+    };
+    auto fetch_k = [&](PassOperands<KT>& o, size_t at, int rt) {
+        const float* kp = p.Kt + at * CH * p.dk16 + rt * TILE + lane * 4;
+        o.U[rt] = *reinterpret_cast<const f32x4*>(p.U0 + (at * p.dv16 + n0) * CH + rt * TILE + lane * 4);
 #pragma unroll
-            for (int kt = 0; kt < KT; ++kt) o.W[rt][kt] = *reinterpret_cast<const f32x4*>(wp + (size_t)rt * 16 * p.dk16 + kk[kt]);
-#pragma unroll
-        for (int rt = 0; rt < 4; ++rt) {
-            o.U[rt] = *reinterpret_cast<const f32x4*>(up + rt * 16);
-#pragma unroll
-            for (int kt = 0; kt < KT; ++kt) o.K[kt][rt] = *reinterpret_cast<const f32x4*>(kp + (size_t)kk[kt] * CH + rt * 16);
-        }
+        for (int kt = 0; kt < KT; ++kt) o.K[kt][rt] = *reinterpret_cast<const f32x4*>(kp + kk[kt] * CH);
     };
     auto chunk = [&](PassOperands<KT>& cur, PassOperands<KT>& next, int ch, int buf) {
-        const size_t at = at0 + ch * step;
-        fetch(next, min(ch + 1, nch - 1));
-        __builtin_amdgcn_sched_barrier(0);  // the loads go out ahead of the products, not among them
+        const size_t at = at0 + ch * step, then = at0 + min(ch + 1, nch - 1) * step;
+        next.g = p.total[then];
 #pragma unroll
-        for (int rt = 0; rt < 4; ++rt) {
-            f32x4 ws = (f32x4){0.f, 0.f, 0.f, 0.f};
+        for (int r2 = 0; r2 < 4; r2 += 2) {
+            fetch_w(next, then, r2);
+            fetch_w(next, then, r2 + 1);
+            __builtin_amdgcn_sched_barrier(0);
+            f32x4 ws[2] = {(f32x4){0.f, 0.f, 0.f, 0.f}, (f32x4){0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
             for (int kt = 0; kt < KT; ++kt)
 #pragma unroll
-                for (int i = 0; i < 4; ++i) ws = mfma_f32(cur.W[rt][kt][i], S[kt][i], ws);
-            part[buf][wave][rt][lane] = ws;
+                for (int i = 0; i < 4; ++i)
+#pragma unroll
+                    for (int u = 0; u < 2; ++u) ws[u] = mfma_f32(cur.W[r2 + u][kt][i], S[kt][i], ws[u]);
+#pragma unroll
+            for (int u = 0; u < 2; ++u) part[buf][wave][r2 + u][lane] = ws[u];
+            __builtin_amdgcn_sched_barrier(0);
         }
         // the state before the chunk, for the kernel that makes the outputs
 #pragma unroll
         for (int kt = 0; kt < KT; ++kt)
-            if (FULL || k0[kt] < p.dk16) *reinterpret_cast<f32x4*>(p.Sb + (at * p.dv16 + col) * p.dk16 + k0[kt] + grp * 4) = S[kt];
+            if (FULL || k0[kt] < p.dk16) *reinterpret_cast<f32x4*>(p.Sb + (at * p.dv16 + n0) * p.dk16 + k0[kt] * 16 + lane * 4) = S[kt];
         __syncthreads();  // the waves' shares of W S are in LDS (the other half was read before they were written)
-        f32x4 own = cur.U[0];
+        f32x4 share[4][4], own = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int rt = 0; rt < 4; ++rt) {
-            f32x4 ws = part[buf][0][rt][lane];
+        for (int rt = 0; rt < 4; ++rt)
 #pragma unroll
-            for (int w = 1; w < 4; ++w) ws += part[buf][w][rt][lane];
-            cur.U[rt] -= ws;
-            own = rt == wave ? cur.U[rt] : own;
-        }
-        *reinterpret_cast<f32x4*>(p.U + (at * p.dv16 + col) * CH + wave * 16 + grp * 4) = own;  // a wave leaves a quarter
+            for (int w = 0; w < 4; ++w) share[rt][w] = part[buf][w][rt][lane];
 #pragma unroll
         for (int kt = 0; kt < KT; ++kt) {
             S[kt] *= cur.g;
@@ -472,18 +503,33 @@ __global__ __launch_bounds__(256) void delta_pass_kernel(DeltaChunkArgs p) {
                 for (int rt = 0; rt < 4; ++rt) cur.K[kt][rt] = (f32x4){0.f, 0.f, 0.f, 0.f};
         }
 #pragma unroll
-        for (int rt = 0; rt < 4; ++rt)
+        for (int rt = 0; rt < 4; ++rt) {
+            f32x4 ws = share[rt][0];
+#pragma unroll
+            for (int w = 1; w < 4; ++w) ws += share[rt][w];
+            cur.U[rt] -= ws;
+            own = rt == wave ? cur.U[rt] : own;
+            fetch_k(next, then, rt);
+            if (rt == 3) *reinterpret_cast<f32x4*>(p.U + (at * p.dv16 + n0) * CH + wave * TILE + lane * 4) = own;  // a wave leaves a quarter
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int i = 0; i < 4; ++i)
 #pragma unroll
                 for (int kt = 0; kt < KT; ++kt) S[kt] = mfma_f32(cur.K[kt][rt][i], cur.U[rt][i], S[kt]);
+            __builtin_amdgcn_sched_barrier(0);
+        }
     };
-    fetch(A, 0);
-    for (int ch = 0; ch < nch; ch += 2) {
+    A.g = p.total[at0];
+#pragma unroll
+    for (int rt = 0; rt < 4; ++rt) fetch_w(A, at0, rt);
+#pragma unroll
+    for (int rt = 0; rt < 4; ++rt) fetch_k(A, at0, rt);
+    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the loop's own waits count from here, not in the order of these first loads
+    for (int ch = 0; ch + 1 < nch; ch += 2) {  // (one straight block: with an exit between the two the compiler's waits were for loads just sent)
         chunk(A, B, ch, 0);
-        if (ch + 1 >= nch) break;
         chunk(B, A, ch + 1, 1);
     }
+    if (nch & 1) chunk(A, B, nch - 1, 0);
 #pragma unroll
     for (int kt = 0; kt < KT; ++kt)
 #pragma unroll
@@ -526,8 +572,8 @@ __global__ __launch_bounds__(256) void delta_out_kernel(DeltaChunkArgs p) {
         for (int kk = 0; kk < SL / 16; ++kk)
 #pragma unroll
             for (int c = 0; c < CT; ++c)
-                B[kk][c] = *reinterpret_cast<const f32x4*>(p.Sb + (at * p.dv16 + min((wave + 4 * c) * 16, p.dv16 - 16) + r16) * p.dk16 +
-                                                           min(c0 + kk * 16, p.dk16 - 16) + grp * 4);
+                B[kk][c] = *reinterpret_cast<const f32x4*>(p.Sb + (at * p.dv16 + min((wave + 4 * c) * 16, p.dv16 - 16)) * p.dk16 +
+                                                           min(c0 + kk * 16, p.dk16 - 16) * 16 + lane * 4);
         if (c0) __syncthreads();
         put_slice(Qs, qs, c0, n, a.d);
         put_slice(Ks, ks, c0, n, a.d);
@@ -587,7 +633,7 @@ __global__ __launch_bounds__(256) void delta_out_kernel(DeltaChunkArgs p) {
     for (int jt = 0; jt < 4; ++jt)
 #pragma unroll
         for (int c = 0; c < CT; ++c)
-            Uf[jt][c] = *reinterpret_cast<const f32x4*>(p.U + (at * p.dv16 + min((wave + 4 * c) * 16, p.dv16 - 16) + r16) * CH + jt * 16 + grp * 4);
+            Uf[jt][c] = *reinterpret_cast<const f32x4*>(p.U + (at * p.dv16 + min((wave + 4 * c) * 16, p.dv16 - 16)) * CH + jt * TILE + lane * 4);
     __syncthreads();
 #pragma unroll
     for (int rt = 0; rt < 4; ++rt) {
