@@ -38,7 +38,7 @@ struct RouteSums {
 // for together, V columns a lane; a logit is the sum of a lane's columns, then of the lanes, whatever R and EW.  The choice and all that follows are a wave's a row.
 // An output at a time was a trip to memory for every fourth, and with one row a block every row brought the weights from the L2 again
 // (us, warm: four rows of 2,048 over 9 outputs 7.1 -> 5.1, 2,048 rows 14.7 -> 8.5; 64 rows over 64 outputs 25.2 -> 17.6, 2,048 72.8 -> 33.2).
-template <int R, int V, int EW>
+template <int R, int V, int EW, int AHEAD>
 __global__ __launch_bounds__(256) void route_kernel(const elem_t* __restrict__ x, const float* __restrict__ w,
                                                     const float* __restrict__ bias, float* __restrict__ gates, int d, int E, int top,
                                                     int scoring, const float* __restrict__ correction, int extra, RouteSums rs) {
@@ -58,7 +58,6 @@ __global__ __launch_bounds__(256) void route_kernel(const elem_t* __restrict__ x
             for (int r = 0; r < R; ++r) v[k][r] = 0.f;
         // AHEAD steps' loads on one straight path: left to the compiler, the unrolled loop asked for a step or two at a time.  us, warm, the same sums: four rows of 2,048 over
         // 9 outputs 5.7 -> 5.4, 64 rows over 64 outputs 24.7 -> 16.5, 2,048 rows 8.8 -> 8.5 and 46 -> 30 (four steps ahead of one row: 5.7 and 18.9; of four rows 9.2 and 30.7).
-        constexpr int AHEAD = R == 1 ? 8 : 2;
         for (int c0 = lane * V; c0 < d; c0 += 64 * V * AHEAD) {
             float we[AHEAD][EW][V], xr[AHEAD][R][V];
 #pragma unroll
@@ -663,8 +662,8 @@ extern "C" int ms_route(const void* x, const float* w, const float* bias, float*
     MS_REQUIRE(top >= 1 && top <= E && top <= 64, "route: %d of %d experts a row (at most 64)", top, E);
     MS_REQUIRE((plane == nullptr) == (sums == nullptr) && (!plane || (real > 0 && real <= E)), "route: %d of %d outputs are experts", real, E);
     const RouteSums rs{plane, sums, real, d, T};
-#define MS_ROUTE(R_, V_, EW_)                                                                                                                         \
-    hipLaunchKernelGGL((route_kernel<R_, V_, EW_>), dim3(ceil_div(T, R_)), dim3(256), 0, stream, (const elem_t*)x, w, bias, gates, d, E, top, scoring, \
+#define MS_ROUTE(R_, V_, EW_, A_)                                                                                                                     \
+    hipLaunchKernelGGL((route_kernel<R_, V_, EW_, A_>), dim3(ceil_div(T, R_)), dim3(256), 0, stream, (const elem_t*)x, w, bias, gates, d, E, top, scoring, \
                        correction, extra, rs)
     // four columns a load where every row begins at a multiple of them; four rows a block where that leaves every CU a block
     const bool fours = d % 4 == 0 && (reinterpret_cast<uintptr_t>(w) & 15) == 0 && (reinterpret_cast<uintptr_t>(x) & (4 * sizeof(elem_t) - 1)) == 0;
@@ -672,14 +671,24 @@ extern "C" int ms_route(const void* x, const float* w, const float* bias, float*
     // up to four outputs: one a wave, which asks for nothing twice (four outputs of 2,048, three a wave / one / an output in turn: 16 rows 5.0 / 4.2 / 4.9 us,
     // 1,000 rows 7.8 / 5.6 / 6.6; five outputs, three a wave / in turn: 5.0 / 5.7 and 7.9 / 7.5)
     const bool one = E + extra <= 4;
-    if (one && fours && many) MS_ROUTE(4, 4, 1);
-    else if (one && fours) MS_ROUTE(1, 4, 1);
-    else if (one && many) MS_ROUTE(4, 1, 1);
-    else if (one) MS_ROUTE(1, 1, 1);
-    else if (fours && many) MS_ROUTE(4, 4, 3);
-    else if (fours) MS_ROUTE(1, 4, 3);
-    else if (many) MS_ROUTE(4, 1, 3);
-    else MS_ROUTE(1, 1, 3);
+    // No more steps ahead than a row has: with eight, four rows of 1,024 over 9 outputs took 9.2 us in a decode step and 7.4 in a plain loop.  Warm, plain loop -> now: four rows
+    // over 9 outputs 4.1 -> 3.9 us (512 columns), 4.4 -> 4.2 (1,024), 4.9 -> 4.6 (2,048); over 65 of 1,024 11.9 -> 11.1; 2,048 rows of 1,024 over 9 6.5 -> 6.2.
+    const int steps = ceil_div(d, 64 * 4);
+#define MS_ROUTE_FOURS(EW_)                     \
+    do {                                        \
+        if (many && steps > 1) MS_ROUTE(4, 4, EW_, 2); \
+        else if (many) MS_ROUTE(4, 4, EW_, 1);  \
+        else if (steps > 4) MS_ROUTE(1, 4, EW_, 8); \
+        else if (steps > 2) MS_ROUTE(1, 4, EW_, 4); \
+        else MS_ROUTE(1, 4, EW_, 2);            \
+    } while (0)
+    if (one && fours) MS_ROUTE_FOURS(1);
+    else if (fours) MS_ROUTE_FOURS(3);
+    else if (one && many) MS_ROUTE(4, 1, 1, 2);
+    else if (one) MS_ROUTE(1, 1, 1, 8);
+    else if (many) MS_ROUTE(4, 1, 3, 2);
+    else MS_ROUTE(1, 1, 3, 8);
+#undef MS_ROUTE_FOURS
 #undef MS_ROUTE
     return check_launch("route");
 }

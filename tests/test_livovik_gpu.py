@@ -185,6 +185,23 @@ def test_experts_weighed_at_their_inputs_against_the_plain_feed_forward(dtype, E
     close(out.y, want, dtype, "the sum of the chosen experts and the gated one")
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("T", [3, 1029])
+@pytest.mark.parametrize("extra", [1, 8])
+@pytest.mark.parametrize("width", [8, 256, 264, 512, 520, 1024, 1032, 2048, 2056])
+def test_logits_whatever_the_steps_of_a_row(dtype, T, extra, width):
+    """A row's steps of 256 columns, one to nine, around every number of steps that is asked for at once."""
+    ops = ops_of(dtype)
+    torch.manual_seed(width + extra)
+    h, w = torch.randn(T, width).to(dtype), torch.randn(1 + extra, width) * width ** -0.5
+    got = ops.route(dev(h), dev(w), None, 1, extra_gates=extra)[:, 1:].cpu().double()
+    z, size = h.double() @ w.double().T, h.double().abs() @ w.double().abs().T
+    # a lane adds up to width / 64 + 4 products, the lanes in six sums: each rounds by half a unit of its value, at most `size`; the sigmoid's slope is a quarter and its own error a few units
+    bound = 0.25 * (width / 64 + 10) * 2.0 ** -24 * size[:, 1:] + 4 * 2.0 ** -24
+    err = (got - torch.sigmoid(z[:, 1:])).abs()
+    assert bool((err <= bound).all()), f"error {float(err.max()):.3e}, {float((err / bound).max()):.2f} of the bound"
+
+
 def test_a_gate_of_every_row_goes_with_softmax_weights_too():
     ops, ref = ops_of(torch.float32), EmulatedOps(torch.float32)
     torch.manual_seed(0)
