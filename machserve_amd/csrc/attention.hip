@@ -1382,9 +1382,9 @@ __global__ __launch_bounds__(256) void decode_attention_kernel(DecodeArgs a) {
     }
 
     if constexpr (FUSED) {
-        // The row's own key: one more term of the online softmax, in the last wave of split 0, which has no more tiles than the others (with up to
-        // 192 keys none): in wave 0, behind its tile, it took 1.1 of a block's 7.6 us behind 33 keys.
-        if (sp == 0 && wave == 3) {
+        // The row's own key: one more term of the online softmax, in split 0.  Where the keys are not cut it is the last wave's, which has no more tiles than
+        // the others (with up to 192 keys none): in wave 0, behind its tile, it took 1.1 of a block's 7.6 us behind 33 keys.  Where they are cut every wave has tiles.
+        if (sp == 0 && wave == (a.nsplit == 1 ? 3 : 0)) {
             float dot = 0.f;
 #pragma unroll
             for (int ks = 0; ks < NKS; ++ks) {
