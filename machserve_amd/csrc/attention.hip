@@ -1171,12 +1171,18 @@ __global__ __launch_bounds__(256) void decode_attention_kernel(DecodeArgs a) {
         for (int u = 0; u < COLS; ++u) {
             col_e[u] = column(tid + u * 256);
             bias_e[u] = bias[col_e[u]];
+            if constexpr (!MANY) {  // a column's bias and sums side by side: 8 requests behind 2,048 tokens 0.8851 -> 0.8835 ms a step (24 layers)
+                part_e[0][u] = row0[col_e[u]];
+                part_e[1][u] = row0[(size_t)min(1, a.n_partials - 1) * pstride + col_e[u]];
+            }
         }
+        if constexpr (MANY) {
 #pragma unroll
-        for (int q = 0; q < EARLY; ++q) {
-            const size_t po = (size_t)min(q, a.n_partials - 1) * pstride;
+            for (int q = 0; q < EARLY; ++q) {
+                const size_t po = (size_t)min(q, a.n_partials - 1) * pstride;
 #pragma unroll
-            for (int u = 0; u < COLS; ++u) part_e[q][u] = row0[po + col_e[u]];
+                for (int u = 0; u < COLS; ++u) part_e[q][u] = row0[po + col_e[u]];
+            }
         }
         freq_e = (a.inv_freq ? a.inv_freq : row0)[min(tid, hd / 2 - 1)];
         slot = a.slot_map[s];
