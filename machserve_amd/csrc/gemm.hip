@@ -117,16 +117,18 @@ static bool planned(int M, int K) { return M > 64 && K % 64 == 0 && g_gemm_confi
 
 #ifndef MS_ELEM_HALF
 // Whether a 32-bit product runs in parts of 16 bits (GEMM_SPLIT): whole K steps, an output of at least 4,096 columns whose 64x64 tiles are one and a half a CU, or
-// K in slices.  us, 32-bit instructions and parts: 192 x 9,728 x 896 (1.8 a CU) 33.8 and 30.4, 128 rows (1.2) 27.7 and 28.1, 65 rows 20.7 and 27.7; 512 x 4,096 x 1,024 37.7
-// and 35.3.  Narrower outputs gain no more (1,024 x 2,048 x 2,048 69 and 63) and keep sums that are the same in every batch of more than 64 rows.
+// K in slices.  us, 32-bit instructions and parts: 192 x 9,728 x 896 (1.8 a CU) 38 and 35, 128 rows (1.2) 27 and 32, 65 rows 21 and 32; 320 rows 50 and 50; 512 x 4,096 x 1,024
+// 41 and 40, 512 x 5,632 x 2,048 104 and 100.  The rows' number is part of the rule, as it is of the number of slices: a row's sums are those of other batches to
+// rounding only.
 static bool parted(int M, int N, int K, int slices) {
     return K % 32 == 0 && M > 64 && (slices > 1 || (N >= 4096 && 2L * ceil_div(M, 64) * ceil_div(N, 64) >= 3L * compute_units()));
 }
-// ... in tiles of 128x128, a block a CU, which take 1.45 us a K step and round, or of 64x64, 0.5 us for each that a CU has: 768 x 9,728 x 896 (two rounds, 7.1 a CU) 84 and
-// 98 us, 512 rows (two rounds, 4.8) 75 and 67, 512 x 2,048 x 5,632 in four slices (one round, 4) 69 and 85.
+// ... in tiles of 128x128, a block a CU, which take 1.7 us a K step and round, or of 64x64, 0.55 us for each that a CU has: 768 x 9,728 x 896 (two rounds, 7.1 a CU) 100 and
+// 114 us, 512 rows (two rounds, 4.8) 97 and 79, 1,024 rows (three, 9.5) 137 and 142; 512 x 896 x 4,864 in eight slices (one round, 3.5) 38 and 46, 192 x 2,048 x 5,632 (one, 3)
+// 44 and 42, 512 x 2,048 x 5,632 in four (one, 4) 83 and 102.
 static bool parted_wide(int M, int N, int slices) {
     const long cus = compute_units(), wide = (long)ceil_div(M, 128) * ceil_div(N, 128) * slices, narrow = (long)ceil_div(M, 64) * ceil_div(N, 64) * slices;
-    return 1.45 * (double)ceil_div(wide, cus) < 0.5 * (double)narrow / (double)cus;
+    return 1.7 * (double)ceil_div(wide, cus) < 0.55 * (double)narrow / (double)cus;
 }
 #endif
 
@@ -612,7 +614,7 @@ extern "C" int ms_prefers_tiled(int M, int N, int K) {
 
 // K slices of a product that is added to the residual stream, whose next norm adds them up: those of ms_tiled_partials, and in the 32-bit build those of a long K
 // under a narrow output, whose uncut 32x32 tiles are each a chain of all K steps: slices that fill the chip with 128x128 tiles, eight at most.  us, uncut and in slices:
-// 512 x 896 x 4,864 53.6 and 32.9 (eight), 192 rows 44 and 22.
+// 512 x 896 x 4,864 53 and 38 (eight), 192 rows 43 and 25, 1,024 rows 92 and 66 (four).
 extern "C" int ms_residual_partials(int M, int N, int K) {
 #ifndef MS_ELEM_HALF
     if (M > 64 && N < 4096 && K >= 4096 && K % 32 == 0) {

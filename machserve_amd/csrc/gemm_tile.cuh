@@ -14,8 +14,8 @@
 // two-byte elements, and in 32-bit whatever has a partial last step, go global -> registers -> LDS (padded rows); the other
 // products of the 32-bit build go straight to LDS as well (its K steps of 32 are rows of 128 bytes too).
 // Every output element is the sum over K in steps of 32 in ascending order whatever the
-// tile shape or the number of rows, so a row's result does not depend on its batch (of the 32-bit products with wide outputs
-// those of large batches are worked out in parts, with sums of their own: GEMM_SPLIT).
+// tile shape, so a row's result does not depend on the tile that its batch runs in.  What does go by the number of rows is whether K is cut into slices whose sums the
+// reader adds (the 32-bit build: under a narrow output alone), and which 32-bit products are worked out in parts, with sums of their own (GEMM_SPLIT).
 #pragma once
 #include <type_traits>
 
@@ -297,15 +297,17 @@ __device__ __forceinline__ void gemm_tile(const elem_t* __restrict__ A, const el
     if constexpr (SPLIT) {
 #ifndef MS_ELEM_HALF
         // Numbers of 32 bits in three parts of 16 (bfloat16, which has their exponents): x = x1 + x2 + x3, each the rounding of what the ones before it
-        // leave, so that nothing is lost, and the product's terms x1 y1, x1 y2, x2 y1, x2 y2, x1 y3 and x3 y1 on the 16-bit matrix instructions with their sums in 32
-        // bits; what is left out is below 2^-26 of a product, a quarter of its rounding in 32 bits.  The six take 96 cycles where the 32-bit instructions take 256.  Error
-        // against 64 bits (relative, normal inputs), in those and here: K = 896 5.4e-7 and 4.5e-7, 2,048 8.1e-7 and 7.0e-7, 4,864 in eight slices 4.5e-7 and
-        // 3.8e-7.  (Of numbers below 2^-110 the lowest part falls among the subnormal ones.)
+        // leave, so that nothing is lost, and eight of a product's nine terms on the 16-bit matrix instructions, where each is exact.  |x2| is at most 2^-8 |x| and |x3|
+        // 2^-17 |x|: x3 y3, which is left out, is a thousandth of a product's rounding in 32 bits (x2 y3 and x3 y2 together are as much as that rounding).  x1 y1 has
+        // sums of its own, which a step rounds once; the others, below 2^-6 of them, would round them seven times more.  The eight take 128 cycles where the 32-bit
+        // instructions take 256.  Relative error against 64 bits, in those and here: normal inputs of K = 896 5.4e-7 and 1.7e-7, 2,048 8.1e-7 and 2.7e-7, 4,864 in
+        // eight slices 4.5e-7 and 1.5e-7; positive inputs of K = 896 4.6e-7 and 1.7e-7; a single product at most 5.93e-8 and 5.96e-8 (with the six largest terms in
+        // one set of sums 4.5e-7 and, of a single product, 1.28e-7).
         // The threads hold a step's numbers for two steps, part them two at a time between the matrix instructions, and store each part's rows of 64 bytes for
-        // the next step; two buffers, one barrier a step.  What bounds it (parts left out, 128x128 of K = 4,864, one block a CU, 166 us): parting and storing alone
-        // 115, the matrix instructions and LDS reads 110: a matrix instruction leaves the issue of two others free, and LDS takes stores at a third of the rate of
-        // reads.  Three buffers with the fragments a step ahead, loads of four steps ahead, other groupings: the same.  us, 32-bit instructions and here: 512 x 9,728 x 896 91.6
-        // and 66.6 (64x64), 1,024 x 17,920 x 1,536 460 and 344 (128x128); with K in slices 512 x 896 x 4,864 53.6 (uncut) and 32.9.
+        // the next step; two buffers, one barrier a step.  What bounds it: a matrix instruction leaves the issue of two others free, and LDS takes stores at a third of
+        // the rate of reads (with six terms in one set of sums, 128x128 of K = 4,864, one block a CU, 166 us: parting and storing alone 115, the matrix instructions
+        // and LDS reads 110).  us, 32-bit instructions and here: 512 x 9,728 x 896 93 and 79 (64x64), 1,024 x 17,920 x 1,536 461 and 396 (128x128); with K in
+        // slices 512 x 896 x 4,864 53 (uncut) and 38.  (Six terms: 67, 332 and 31.)
         static_assert(BK == 32 && BM * 4 % NT == 0 && BN * 4 % NT == 0, "four threads a row");
         constexpr int A_ROUNDS = BM * 4 / NT, W_ROUNDS = BN * 4 / NT, ROUNDS = A_ROUNDS + W_ROUNDS;
         // thread t has the eight numbers t % 4 of row t / 4 of every round
@@ -325,9 +327,13 @@ __device__ __forceinline__ void gemm_tile(const elem_t* __restrict__ A, const el
         };
         auto place = [](int row, int chunk) { return row * LDS_LD + (chunk ^ ((row >> 1) & 2)) * 4; };  // in floats; a part's rows are 64 bytes, 192 apart
         u32x4 part[3];
+        float most[ROUNDS];  // the largest size of the thread's numbers of each round
+#pragma unroll
+        for (int i = 0; i < ROUNDS; ++i) most[i] = 0.f;
         auto put = [&](int set, int buf, int unit) {  // two numbers of round unit / 4, and the round's stores behind its last
             const int i = unit / 4, e = unit % 4;
             float x = held[set][i][e / 2][e % 2 * 2], y = held[set][i][e / 2][e % 2 * 2 + 1];
+            asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(most[i]) : "v"(x), "v"(y));
 #pragma unroll
             for (int q = 0; q < 3; ++q) {
                 const uint32_t xy = round_pair(x, y);
@@ -349,6 +355,11 @@ __device__ __forceinline__ void gemm_tile(const elem_t* __restrict__ A, const el
 #pragma unroll
         for (int u = 0; u < UNITS; ++u) put(0, 0, u);
         __syncthreads();
+        f32x4 low[TM][TN];
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j) low[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
         auto step = [&](int kt, int buf) {
             ask(min(kt + 2, nk - 1), buf);
             bf16x8 fa[TM][3], fb[TN][3];
@@ -363,17 +374,18 @@ __device__ __forceinline__ void gemm_tile(const elem_t* __restrict__ A, const el
 #pragma unroll
             for (int u = 0; u < FIRST; ++u) put(buf ^ 1, buf ^ 1, u);  // (behind the last step: a place that nobody reads)
             __builtin_amdgcn_sched_barrier(0);
-            constexpr int GR = TM * TN >= 4 ? 4 : TM * TN, GROUPS = 6 * TM * TN / GR;
+            constexpr int GR = TM * TN >= 4 ? 4 : TM * TN, GROUPS = 8 * TM * TN / GR;
 #pragma unroll
             for (int g = 0; g < GROUPS; ++g) {  // the smallest products first
-                constexpr int qa[6] = {0, 2, 1, 0, 1, 0}, qb[6] = {2, 0, 1, 1, 0, 0};
+                constexpr int qa[8] = {2, 1, 2, 0, 1, 1, 0, 0}, qb[8] = {1, 2, 0, 2, 1, 0, 1, 0};
 #pragma unroll
                 for (int u = FIRST; u < UNITS; ++u)
                     if ((u - FIRST) * GROUPS / (UNITS - FIRST) == g) put(buf ^ 1, buf ^ 1, u);
 #pragma unroll
                 for (int m = g * GR; m < (g + 1) * GR; ++m) {
                     const int t = m / (TM * TN), i = m / TN % TM, j = m % TN;
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[i][qa[t]], fb[j][qb[t]], acc[i][j], 0, 0, 0);
+                    f32x4& sum = t == 7 ? acc[i][j] : low[i][j];
+                    sum = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[i][qa[t]], fb[j][qb[t]], sum, 0, 0, 0);
                 }
                 __builtin_amdgcn_sched_barrier(0);
             }
@@ -385,20 +397,45 @@ __device__ __forceinline__ void gemm_tile(const elem_t* __restrict__ A, const el
             step(kt + 1, 1);
         }
         if (kt < nk) step(kt, 0);
-        // An infinity or a NaN among the numbers (an infinity's second part is NaN), numbers whose first part is rounded up to infinity, and sums beyond the
-        // largest number leave sums that are not finite: such a block is worked out again on the 32-bit matrix instructions.
-        bool finite = true;
+        // Parts lose what is below 2^-133, and 2^-126 if such numbers count as zeros: of a sum K 2^-126 (X + Y) at most, X and Y the largest sizes in its row and its
+        // column of W.  A sum beneath 2^-80 of those is taken from the 32-bit matrix instructions, as is one beneath 2^-100, whose terms may round more often than once,
+        // and one that is not finite (an infinity's second part is NaN, and so are those of a number whose first part rounds up to infinity).  Zeros of a
+        // row or column of zeros are right as they are.  Only these sums are: no other row or column of the block shows what stands beside it.
+        __shared__ float largest[BM + BN];
+#pragma unroll
+        for (int i = 0; i < ROUNDS; ++i) {
+            float v = most[i];
+            v = fmaxf(v, __shfl_xor(v, 1, WAVE));
+            v = fmaxf(v, __shfl_xor(v, 2, WAVE));
+            if (t_chunk == 0) largest[i * (NT / 4) + t_row] = v;
+        }
+        __syncthreads();
+        auto sound = [](float v, float x, float y) {
+            const float least = x == 0.f || y == 0.f ? 0.f : fmaxf(fmaxf(x, y) * 0x1p-80f, 0x1p-100f);
+            return fabsf(v) >= least && fabsf(v) < INFINITY;
+        };
+        float row_max[TM][4], col_max[TN];
+        bool again = false;
+#pragma unroll
+        for (int j = 0; j < TN; ++j) col_max[j] = largest[BM + wn * (BN / WN) + j * 16 + r16];
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) row_max[i][e] = largest[wm * (BM / WM) + i * 16 + grp * 4 + e];
 #pragma unroll
         for (int i = 0; i < TM; ++i)
 #pragma unroll
             for (int j = 0; j < TN; ++j)
 #pragma unroll
-                for (int e = 0; e < 4; ++e) finite &= __builtin_isfinite(acc[i][j][e]);
-        if (__syncthreads_or(!finite)) {
+                for (int e = 0; e < 4; ++e) {
+                    acc[i][j][e] += low[i][j][e];
+                    again |= !sound(acc[i][j][e], row_max[i][e], col_max[j]);
+                }
+        if (__syncthreads_or(again)) {
 #pragma unroll
             for (int i = 0; i < TM; ++i)
 #pragma unroll
-                for (int j = 0; j < TN; ++j) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+                for (int j = 0; j < TN; ++j) low[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll 1
             for (int k = k_begin; k < k_end; k += 32) {
                 Frag ra_[TM];
@@ -409,9 +446,16 @@ __device__ __forceinline__ void gemm_tile(const elem_t* __restrict__ A, const el
                 for (int j = 0; j < TN; ++j) {
                     const Frag rb = frag_load(W + (size_t)min(n0 + wn * (BN / WN) + j * 16 + r16, N - 1) * rows.w_pitch(K) + k + grp * 8);
 #pragma unroll
-                    for (int i = 0; i < TM; ++i) mma_16x16x32(acc[i][j], ra_[i], rb);
+                    for (int i = 0; i < TM; ++i) mma_16x16x32(low[i][j], ra_[i], rb);
                 }
             }
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+                for (int j = 0; j < TN; ++j)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        if (!sound(acc[i][j][e], row_max[i][e], col_max[j])) acc[i][j][e] = low[i][j][e];
         }
 #endif
     } else if constexpr (PIPED) {

@@ -122,6 +122,45 @@ def test_32_bit_products_in_parts(M, N, K):
     assert float(err.max()) < 2e-6
 
 
+# ... with nothing lost that the 32-bit products keep: a single product, small numbers of any scale, and rows beside ones that are not finite; both tiles, and K in slices
+@pytest.mark.parametrize("M,N,K", [(193, 8200, 64), (330, 9008, 96), (65, 136, 4128), (513, 896, 4864)])
+def test_32_bit_parts_lose_nothing(M, N, K):
+    ops = ops_for(torch.float32)
+    slices = ops._plan("ms_residual_partials", M, N, K)
+    assert ops._plan("ms_parted", M, N, K, slices) > 0, "the sizes are those of the 32-bit instructions"
+    x = torch.zeros((M, N), device=DEV)
+
+    def product(a, w):
+        return ops.linear(a, w, None, out_f32=True) if N >= 4096 else ops.linear_residual(a, w, x).sum(0)
+
+    # one product a sum: rounded once, half a unit; what its parts add up to first is at most 2^-6 of it and rounded seven times
+    a, w = torch.zeros((M, K), device=DEV), torch.zeros((N, K), device=DEV)
+    a[:, 37], w[:, 37] = 1 + rnd((M,), torch.float32, 41).abs() % 1, 1 + rnd((N,), torch.float32, 42).abs() % 1
+    ref = a.double() @ w.double().T
+    err = float(((product(a, w).double() - ref).abs() / ref).max())
+    assert err <= 2.0 ** -24 * (1 + 7 * 2.0 ** -6), f"a single product is off by {err:.3e}"
+
+    # many: a slice's sum of n terms rounds n times at most, by a quarter of a unit on average, in no direction; sums of numbers of any size alike
+    n, a, w = K // slices, rnd((M, K), torch.float32, 43), rnd((N, K), torch.float32, 44)
+    for ea, ew in [(0, 0), (-118, 0), (-118, 118), (0, -122), (100, -122), (-60, -60), (-104, 4)]:
+        sa, sw = (a.double() * 2.0 ** ea).float(), (w.double() * 2.0 ** ew).float()
+        ref = sa.double() @ sw.double().T
+        err = float((product(sa, sw).double() - ref).norm() / ref.norm())
+        assert err <= n ** 0.5 * 2.0 ** -24, f"numbers of 2^{ea} and 2^{ew}: error {err:.3e}"
+
+    # what stands in other rows of the block, and in other columns' weights, does not show
+    want = product(a, w)
+    odd, odd_w = a.clone(), w.clone()
+    odd[3, 5], odd[20, 1], odd[64, 7], odd[M - 1] = float("inf"), 2.0 ** -120, float("nan"), odd[M - 1] * 2.0 ** -110
+    odd_w[9, 11], odd_w[11] = float("-inf"), 0.0
+    rows, cols = torch.ones(M, dtype=torch.bool, device=DEV), torch.ones(N, dtype=torch.bool, device=DEV)
+    rows[[3, 20, 64, M - 1]], cols[[9, 11]] = False, False
+    got = product(odd, odd_w)
+    assert torch.equal(got[rows][:, cols], want[rows][:, cols])
+    ref = odd.double() @ odd_w.double().T
+    assert torch.equal(torch.isnan(got), torch.isnan(ref)) and bool((got[rows][:, 11] == 0).all())
+
+
 # Around a norm, more than 64 rows: the product that prepares it in every tile, ragged at both edges, a last column of waves that has no columns (widths of 20 and 1,030); what
 # the kernel leaves behind its last part stays untouched.
 @pytest.mark.parametrize("M,N,K,tile", SIZES + [(1030, 1030, 512, None), (65, 20, 64, None), (200, 24, 128, None), (2048, 896, 896, None)])
