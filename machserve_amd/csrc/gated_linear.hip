@@ -44,18 +44,26 @@ __global__ __launch_bounds__(256) void key_decay_kernel(Sums in, int col, const 
 // A thread is a value channel and holds its column of S in registers (DP of them; the rows beyond d stay zero).  Tokens come
 // WALK_BATCH at a time through LDS; the next batch's numbers are asked for before the current batch is walked.  seg_len 0: a
 // block walks all of a request's rows.  Else a request's rows are cut into segments (numbered by piece_of): LOCAL walks
-// each from zero and leaves what it adds (carry [numbers, H, d, dvp]) and the product of its decays (cdec [numbers, H, d]),
+// each from zero and leaves what it adds (carry [places, H, d, dvp]) and the product of its decays (cdec [places, H, d]),
 // the carry kernel replaces what it adds by the state that comes into it, and the second walk makes the outputs.  A request of at most
 // WALK_WHOLE rows is walked by one block all the same, whatever comes with it: its rows take 1.25 us each, three kernels over segments 80 us and more (100 rows alone
 // 131 us walked, 79 in segments of 32; 64 rows 86 and 78; 64 requests of 17 rows 43 and 94), and 60 single rows beside a prompt of 2,000 took 2,468 us while
-// the rows a request had on average decided for all of a step (in segments 188).
+// the rows a request had on average decided for all of a step (in segments 188).  A request of a single segment is walked whole as well.
 constexpr int WALK_BATCH = 8, WALK_WHOLE = 64;
+__host__ __device__ constexpr int whole_rows(int seg_len) { return WALK_WHOLE > seg_len ? WALK_WHOLE : seg_len; }
 struct WalkArgs {
     StateArgs a;
     int seg_len;
     float* carry;
     float* cdec;
 };
+// The place of request s's first segment.  Only requests that are cut have places: such a one has more than whole_rows rows, so that the request cut next begins at
+// least one whole_rows further on, which makes up for the last segment's missing rows.  T / seg_len + min(T / whole_rows, S) places hold all of a step's, however many
+// single rows come with it (a place for each request beside took 0.3 GB for 512 single rows and a portion of 100, 16 heads of 64 x 128).
+__device__ __forceinline__ int carry_base(const WalkArgs& w, int s) {
+    const int q0 = w.a.seq_q_start[s];
+    return q0 / w.seg_len + min(q0 / whole_rows(w.seg_len), s);
+}
 
 template <int DP, int NT, bool LOCAL>
 __global__ __launch_bounds__(NT) void state_walk_kernel(WalkArgs w) {
@@ -68,7 +76,7 @@ __global__ __launch_bounds__(NT) void state_walk_kernel(WalkArgs w) {
     if (w.seg_len) pc = piece_of(blockIdx.x, w.seg_len, a.seq_q_start, a.S);
     const int left = a.seq_q_len[pc.s] - pc.first;
     if (left <= 0) return;  // the same for the whole block
-    const bool whole = w.seg_len == 0 || a.seq_q_len[pc.s] <= WALK_WHOLE;
+    const bool whole = w.seg_len == 0 || a.seq_q_len[pc.s] <= whole_rows(w.seg_len);
     if (whole && pc.first > 0) return;  // its first number's block has all of its rows
     const int n = whole ? left : min(left, w.seg_len);
     const bool last = n == left;
@@ -77,7 +85,8 @@ __global__ __launch_bounds__(NT) void state_walk_kernel(WalkArgs w) {
     const bool live = j < a.dv;
     const size_t head = (size_t)d * a.dvp;
     float* st = a.state + ((size_t)a.seq_slot[pc.s] * a.H + h) * head + j;
-    float* pass = whole ? nullptr : w.carry + ((size_t)blockIdx.x * a.H + h) * head + j;
+    const size_t at = whole ? 0 : (size_t)(carry_base(w, pc.s) + pc.first / w.seg_len) * a.H + h;
+    float* pass = whole ? nullptr : w.carry + at * head + j;
     float S[DP];
     {
         const float* from = whole ? st : pass;
@@ -205,7 +214,7 @@ __global__ __launch_bounds__(NT) void state_walk_kernel(WalkArgs w) {
     if (LOCAL) {
 #pragma unroll
         for (int u = 0; u < (LOCAL ? (DP + NT - 1) / NT : 1); ++u)
-            if (j + u * NT < d) w.cdec[((size_t)blockIdx.x * a.H + h) * d + j + u * NT] = prod[u];
+            if (j + u * NT < d) w.cdec[at * d + j + u * NT] = prod[u];
     }
     if (j >= a.dvp) return;  // the columns that fill dv up hold zeros
     if (LOCAL) {
@@ -225,8 +234,8 @@ constexpr int CARRY_AHEAD = 8;
 __global__ __launch_bounds__(256) void state_carry_kernel(WalkArgs w) {
     const StateArgs& a = w.a;
     const int s = blockIdx.x, h = blockIdx.y, idx = (blockIdx.z * 256 + threadIdx.x) * 4, head = a.d * a.dvp;
-    if (idx >= head || a.seq_q_len[s] <= WALK_WHOLE) return;
-    const int i = idx / a.dvp, base = piece_base(s, w.seg_len, a.seq_q_start);
+    if (idx >= head || a.seq_q_len[s] <= whole_rows(w.seg_len)) return;
+    const int i = idx / a.dvp, base = carry_base(w, s);
     const int nseg = (a.seq_q_len[s] + w.seg_len - 1) / w.seg_len;
     f32x4 Sin = *reinterpret_cast<const f32x4*>(a.state + ((size_t)a.seq_slot[s] * a.H + h) * head + idx);
     for (int seg0 = 0; seg0 < nseg; seg0 += CARRY_AHEAD) {
@@ -270,8 +279,8 @@ extern "C" int ms_key_decay(const float* in, int n_partials, int ld, int col, co
 }
 
 // Gated linear attention.  rows: float [n_partials, T, ld] with q [H, d], k [H, d], v [H, dv] and gate [H, dv] at their columns;
-// alpha float [T, H * d].  single: every request has one row.  seg_len > 0: segments side by side with carry float
-// [T / seg_len + S, H, d, dvp] and cdec float [T / seg_len + S, H, d] as workspace.
+// alpha float [T, H * d].  single: every request has one row.  seg_len > 0: segments side by side with carry float [places, H, d, dvp] and cdec float
+// [places, H, d] as workspace, places = T / seg_len + min(T / max(64, seg_len), S) (carry_base).
 extern "C" int ms_gated_linear(const float* rows, int n_partials, int ld, int q_col, int k_col, int v_col, int g_col, float q_scale,
                                const float* alpha, const float* norm, float eps, float* state, const int* seq_q_start, const int* seq_q_len,
                                const int* seq_slot, int S, void* out, int ld_out, int T, int H, int d, int dv, int dvp, int single,

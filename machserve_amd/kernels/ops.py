@@ -1327,11 +1327,6 @@ class HipOps:
         the step's rows and requests alone."""
         if T < self.SCAN_CHUNK_MIN_ROWS or T // S < self.SCAN_CHUNK_MIN_ROWS // 2:
             return 0, 0
-        return self._cut_rows(T, S, seg, floats_per_segment)
-
-    @staticmethod
-    def _cut_rows(T: int, S: int, seg: int, floats_per_segment: int) -> tuple:
-        """Segments of ``seg`` rows, longer ones where their workspace would pass 256 MiB."""
         n_segs = -(-T // seg)
         while S * n_segs * floats_per_segment * 4 > (256 << 20) and n_segs > 1:
             seg *= 2
@@ -1675,6 +1670,20 @@ class HipOps:
 
     STATE_SEGMENT = 32  # rows of a segment of gated linear attention
     STATE_WHOLE = 64  # ... of requests of more rows than this (WALK_WHOLE in the kernels)
+    STATE_WORKSPACE = 256 << 20  # bytes of states handed from segment to segment; longer segments where they would be more
+
+    @classmethod
+    def _state_segments(cls, T: int, S: int, floats_per_state: int) -> tuple:
+        """``(segment length, places for the states between segments)`` for gated linear attention over ``T`` rows of ``S`` requests, or ``(0, 0)`` where
+        no request can be long enough to be cut: one has at most ``T - S + 1`` rows, and those of at most ``max(STATE_WHOLE, segment)`` rows are walked whole
+        by the kernels themselves, whatever comes with them."""
+        seg = cls.STATE_SEGMENT
+        while T - S >= (whole := max(cls.STATE_WHOLE, seg)):
+            n = T // seg + min(T // whole, S)
+            if (n - 1) * floats_per_state * 4 <= cls.STATE_WORKSPACE:
+                return seg, n
+            seg *= 2
+        return 0, 0
 
     def gated_linear(self, sums: torch.Tensor, alpha: torch.Tensor, norm_w: torch.Tensor, eps: float, q_scale: float, state: torch.Tensor,
                      seq_q_start: torch.Tensor, seq_q_len: torch.Tensor, seq_slot: torch.Tensor, H: int, d: int, dv: int, out_cols: int,
@@ -1693,10 +1702,8 @@ class HipOps:
         seg = n = 0
         carry = cdec = None
         if not single:
-            # a request may have T - S + 1 rows; those of at most 64 are walked whole by the kernels themselves, whatever comes with them
-            seg, n = self._cut_rows(T, 1, self.STATE_SEGMENT, H * d * dvp) if T - S >= self.STATE_WHOLE else (0, 0)
+            seg, n = self._state_segments(T, S, H * d * dvp)
         if seg:
-            n = T // seg + S
             carry = torch.empty((n, H, d, dvp), dtype=torch.float32, device=sums.device)
             cdec = torch.empty((n, H, d), dtype=torch.float32, device=sums.device)
         self._check(lib, lib.ms_gated_linear(

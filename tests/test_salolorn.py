@@ -304,3 +304,26 @@ def test_specs_that_do_not_fit_are_refused():
     spec = config_from_dict(U.CONFIGS["mixed"]).to_spec()
     with pytest.raises(ConfigError, match="passes begin"):
         replace(spec, loop_steps=replace(spec.loop_steps, starts=(1, 99))).validate()
+
+
+def test_places_of_the_states_between_segments():
+    """Every request that is cut has places of its own for its segments, within those that are allocated, whatever comes with it; a request that may be cut is."""
+    import random
+    from machserve_amd.kernels.ops import HipOps
+    rng = random.Random(0)
+    for trial in range(400):
+        lengths = [rng.choice((1, 1, 1, 0, 17, 63, 64, 65, 96, 127, 128, 129, 300, rng.randint(1, 2000))) for _ in range(rng.randint(1, 40))]
+        T, S, state = sum(lengths), len(lengths), rng.choice((100, 1 << 17, 1 << 20, 1 << 22))
+        seg, n = HipOps._state_segments(T, S, state) if T else (0, 0)
+        if not seg:
+            assert all(length <= 64 for length in lengths) or state > 100 or 0 in lengths
+            continue
+        assert (n - 1) * state * 4 <= HipOps.STATE_WORKSPACE
+        whole, used, q0 = max(64, seg), set(), 0
+        for s, length in enumerate(lengths):
+            if length > whole:
+                for k in range(-(-length // seg)):
+                    place = q0 // seg + min(q0 // whole, s) + k
+                    assert place < n and place not in used, (lengths, seg)
+                    used.add(place)
+            q0 += length

@@ -88,6 +88,42 @@ def test_gated_linear_attention(dtype, single, H, d, dv):
             close(got_state, want_state, torch.float32, f"states after {lengths}")
 
 
+# Requests around the rows from which one is cut, single rows between them and 200 behind; `limit` states between segments make segments of 32, 64, 128 and 256 rows, or none.
+@pytest.mark.parametrize("limit,seg", [(56, 32), (40, 64), (17, 128), (8, 256), (0, 0)])
+def test_gated_linear_attention_in_segments(monkeypatch, limit, seg):
+    ops, ref = ops_of(torch.float32), EmulatedOps(torch.float32)
+    torch.manual_seed(limit)
+    H, d, dv = 2, 12, 20
+    lengths = [65, 1, 129, 64, 300, 1, 257, 33, 66, 1, 127] + [1] * 200
+    T, S, cols = sum(lengths), len(lengths), 40
+    monkeypatch.setattr(type(ops), "STATE_WORKSPACE", limit * H * d * dv * 4)
+    assert ops._state_segments(T, S, H * d * dv)[0] == seg
+    sums = torch.randn(2, T, 136) * 0.7
+    alpha, norm = torch.sigmoid(torch.randn(T, H * d) + 3.0), torch.rand(dv) + 0.5
+    seqs = sequences(lengths, list(range(S))[::-1])
+    state = torch.randn(S, H, d, dv)
+    want_state, got_state = state.clone(), dev(state)
+    want = ref.gated_linear(sums, alpha, norm, 1e-5, d ** -0.5, want_state, *seqs, H, d, dv, cols)
+    got = ops.gated_linear(dev(sums), dev(alpha), dev(norm), 1e-5, d ** -0.5, got_state, *[dev(s) for s in seqs], H, d, dv, cols)
+    close(got, want, torch.float32, "outputs")
+    close(got_state, want_state, torch.float32, "states")
+
+
+def test_single_rows_beside_a_portion_take_no_workspace():
+    """500 decoding requests and one portion of 100 rows, 16 heads of 64 x 128 (half a megabyte a state): the portion's four segments, not a state for each request."""
+    ops = ops_of(torch.bfloat16)
+    H, d, dv, lengths = 16, 64, 128, [1] * 250 + [100] + [1] * 250
+    T, S = sum(lengths), len(lengths)
+    sums, alpha = torch.randn(1, T, 2 * H * (d + dv), device=DEV), torch.rand(T, H * d, device=DEV)
+    seqs, state, norm = [dev(s) for s in sequences(lengths, list(range(S)))], torch.zeros(S, H, d, dv, device=DEV), torch.ones(dv, device=DEV)
+    torch.cuda.synchronize()
+    before = torch.cuda.memory_allocated()
+    torch.cuda.reset_peak_memory_stats()
+    ops.gated_linear(sums, alpha, norm, 1e-5, d ** -0.5, state, *seqs, H, d, dv, H * dv)
+    torch.cuda.synchronize()
+    assert torch.cuda.max_memory_allocated() - before < 32 << 20
+
+
 # ------------------------------------------------------------------ the gated delta rule
 SIZES_DELTA = [(4, 2, 16, 24), (5, 1, 10, 13), (2, 2, 9, 6), (4, 2, 32, 32), (2, 1, 64, 128), (2, 2, 96, 48), (4, 2, 128, 128), (2, 1, 64, 256), (1, 1, 256, 64), (2, 1, 200, 130)]
 
