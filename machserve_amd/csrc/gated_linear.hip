@@ -43,12 +43,13 @@ __global__ __launch_bounds__(256) void key_decay_kernel(Sums in, int col, const 
 // ---- gated linear attention over many rows ---------------------------------------------------------------------
 // A thread is a value channel and holds its column of S in registers (DP of them; the rows beyond d stay zero).  Tokens come
 // WALK_BATCH at a time through LDS; the next batch's numbers are asked for before the current batch is walked.  seg_len 0: a
-// block walks all of a request's rows.  Else a request's rows are cut into segments (numbered by piece_of): LOCAL walks
+// block walks all of a request's rows.  Else a request's rows are cut into segments (the requests' first ones are the first S blocks, later_segment has the others): LOCAL walks
 // each from zero and leaves what it adds (carry [places, H, d, dvp]) and the product of its decays (cdec [places, H, d]),
 // the carry kernel replaces what it adds by the state that comes into it, and the second walk makes the outputs.  A request of at most
 // WALK_WHOLE rows is walked by one block all the same, whatever comes with it: its rows take 1.25 us each, three kernels over segments 80 us and more (100 rows alone
 // 131 us walked, 79 in segments of 32; 64 rows 86 and 78; 64 requests of 17 rows 43 and 94), and 60 single rows beside a prompt of 2,000 took 2,468 us while
 // the rows a request had on average decided for all of a step (in segments 188).  A request of a single segment is walked whole as well.
+// (The lengths are on the device: a step that may hold a request to be cut and holds none pays for two launches that find nothing, 5 us: 64 requests of 17 rows 44 and 49.)
 constexpr int WALK_BATCH = 8, WALK_WHOLE = 64;
 __host__ __device__ constexpr int whole_rows(int seg_len) { return WALK_WHOLE > seg_len ? WALK_WHOLE : seg_len; }
 struct WalkArgs {
@@ -65,6 +66,19 @@ __device__ __forceinline__ int carry_base(const WalkArgs& w, int s) {
     return q0 / w.seg_len + min(q0 / whole_rows(w.seg_len), s);
 }
 
+// Segments behind a request's first one, by number: request s's begin at its first row / L, which leaves each of them a number of its own below T / L.  The first segments, and the
+// requests that are walked whole, are numbered by themselves ahead of these: with a request's segments in one row, the blocks of short requests stood between numbers
+// that nobody has, unevenly over the chip (64 requests of 17 rows: the walk 65 us, without them 43).
+__device__ __forceinline__ Piece later_segment(int number, int L, const int* __restrict__ seq_q_start, int S) {
+    int lo = 0, hi = S - 1;
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (seq_q_start[mid] / L <= number) lo = mid;
+        else hi = mid - 1;
+    }
+    return Piece{lo, (number - seq_q_start[lo] / L + 1) * L};
+}
+
 template <int DP, int NT, bool LOCAL>
 __global__ __launch_bounds__(NT) void state_walk_kernel(WalkArgs w) {
     constexpr int TB = WALK_BATCH, NW = NT / 64, KPT = TB * DP / NT;
@@ -73,11 +87,11 @@ __global__ __launch_bounds__(NT) void state_walk_kernel(WalkArgs w) {
     __shared__ float vs[TB][NT], os[LOCAL ? 1 : TB][NT], part[TB][NW];
     const int h = blockIdx.y, j = threadIdx.x, d = a.d;
     Piece pc{(int)blockIdx.x, 0};
-    if (w.seg_len) pc = piece_of(blockIdx.x, w.seg_len, a.seq_q_start, a.S);
+    if (w.seg_len && (int)blockIdx.x >= a.S) pc = later_segment(blockIdx.x - a.S, w.seg_len, a.seq_q_start, a.S);
     const int left = a.seq_q_len[pc.s] - pc.first;
     if (left <= 0) return;  // the same for the whole block
     const bool whole = w.seg_len == 0 || a.seq_q_len[pc.s] <= whole_rows(w.seg_len);
-    if (whole && pc.first > 0) return;  // its first number's block has all of its rows
+    if (whole && pc.first > 0) return;  // its first block has all of its rows
     const int n = whole ? left : min(left, w.seg_len);
     const bool last = n == left;
     if (LOCAL && last) return;  // nobody needs what the last segment passes on
@@ -311,7 +325,7 @@ extern "C" int ms_gated_linear(const float* rows, int n_partials, int ld, int q_
         MS_WALK_D(false, S);
         return check_launch("gated linear");
     }
-    const int numbers = T / seg_len + S;
+    const int numbers = S + T / seg_len;
     MS_WALK_D(true, numbers);
     if (int rc = check_launch("gated linear, segments from zero")) return rc;
     hipLaunchKernelGGL(state_carry_kernel, dim3(S, H, ceil_div(d * dvp, 1024)), dim3(256), 0, stream, w);

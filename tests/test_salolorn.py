@@ -320,6 +320,12 @@ def test_places_of_the_states_between_segments():
             continue
         assert (n - 1) * state * 4 <= HipOps.STATE_WORKSPACE
         whole, used, q0 = max(64, seg), set(), 0
+        starts = [sum(lengths[:i]) for i in range(S)]
+        later = {}  # what the blocks behind the first S walk: (request, segment)
+        for e in range(T // seg):
+            r = max(i for i in range(S) if starts[i] // seg <= e)
+            later[r, e - starts[r] // seg + 1] = e
+        assert all((r, k) in later for r in range(S) if lengths[r] > whole for k in range(1, -(-lengths[r] // seg))), (lengths, seg)
         for s, length in enumerate(lengths):
             if length > whole:
                 for k in range(-(-length // seg)):
