@@ -1052,8 +1052,8 @@ struct DecodeTile {
     Frag vf[DNTP][ND];
 };
 
-// MANY (fused): the q/k/v product left more than two partial sums, of which up to eight are then asked for first of all.
-template <bool FUSED, bool MANY = false>
+// MANY (fused): the q/k/v product left more than two partial sums, of which up to eight are then asked for first of all.  CUT (fused): the keys are cut over several blocks.
+template <bool FUSED, bool MANY = false, bool CUT = false>
 __global__ __launch_bounds__(256) void decode_attention_kernel(DecodeArgs a) {
     arguments_now(a.q, a.kpool, a.vpool, a.out, a.part_o, a.part_ml, a.block_table, a.seq_pos0, a.table_stride, a.H, a.KV, a.hd,
                   a.ps, a.window, a.nsplit, a.scale, a.qkv, a.bias, a.inv_freq, a.slot_map, a.n_partials, a.stride);
@@ -1208,7 +1208,12 @@ __global__ __launch_bounds__(256) void decode_attention_kernel(DecodeArgs a) {
             cs[tid] = c;
             sn[tid] = sv;
         }
-        const int page = slot >= 0 ? slot / ps : 0, off = slot >= 0 ? slot % ps : 0;  // (divisions: while the sums are on their way)
+        int page = 0, off = 0;
+        auto find_slot = [&] {
+            page = slot >= 0 ? slot / ps : 0;
+            off = slot >= 0 ? slot % ps : 0;
+        };
+        if constexpr (!CUT) find_slot();  // (divisions: while the sums are on their way)
         // Further partial sums, eight at a time, all of their loads asked for before the first is added: the
         // sums were written by the kernel before this one, and one load after the other would be as many trips
         // to them (beyond the last partial sum: the last one again, not added).
@@ -1261,6 +1266,7 @@ __global__ __launch_bounds__(256) void decode_attention_kernel(DecodeArgs a) {
         // own key and value are rounded as the page holds them, and one block writes them there (nobody
         // reads them in this launch).
         {
+            if constexpr (CUT) find_slot();
             const bool writes = sp == 0 && slot >= 0;
             elem_t* kdst = const_cast<elem_t*>(a.kpool) + (((size_t)page * a.KV + kvh) * ps + off) * hd;
             elem_t* vdst = const_cast<elem_t*>(a.vpool) + ((size_t)page * a.KV + kvh) * hd * ps + off;
@@ -1389,8 +1395,9 @@ __global__ __launch_bounds__(256) void decode_attention_kernel(DecodeArgs a) {
 
     if constexpr (FUSED) {
         // The row's own key: one more term of the online softmax, in split 0.  Where the keys are not cut it is the last wave's, which has no more tiles than
-        // the others (with up to 192 keys none): in wave 0, behind its tile, it took 1.1 of a block's 7.6 us behind 33 keys.  Where they are cut every wave has tiles.
-        if (sp == 0 && wave == (a.nsplit == 1 ? 3 : 0)) {
+        // the others (with up to 192 keys none): in wave 0, behind its tile, it took 1.1 of a block's 7.6 us behind 33 keys.  Where they are cut the waves' tiles
+        // are many as a rule, and which wave has it made no difference.
+        if (sp == 0 && wave == (CUT ? 0 : 3)) {
             float dot = 0.f;
 #pragma unroll
             for (int ks = 0; ks < NKS; ++ks) {
@@ -1847,8 +1854,10 @@ extern "C" int MS_CAT(ms_decode_attention_fused_nd, MS_ATTN_ND)(
     MS_REQUIRE(slot_map && kpool && vpool, "decode attention: the fused form writes the cache");
     DecodeArgs a{nullptr, (const elem_t*)kpool, (const elem_t*)vpool, (elem_t*)out, part_o, part_ml, block_table, seq_pos0,
                  table_stride, H, KV, hd, ps, window, nsplit, scale, qkv, bias, inv_freq, slot_map, n_partials, stride, nullptr, nullptr};
-    if (n_partials > 2) hipLaunchKernelGGL((decode_attention_kernel<true, true>), dim3((unsigned)S, (unsigned)KV, (unsigned)nsplit), dim3(256), 0, stream, a);
-    else hipLaunchKernelGGL((decode_attention_kernel<true>), dim3((unsigned)S, (unsigned)KV, (unsigned)nsplit), dim3(256), 0, stream, a);
+    const bool many = n_partials > 2, cut = nsplit > 1;
+    auto kernel = many ? (cut ? decode_attention_kernel<true, true, true> : decode_attention_kernel<true, true, false>)
+                       : (cut ? decode_attention_kernel<true, false, true> : decode_attention_kernel<true, false, false>);
+    hipLaunchKernelGGL(kernel, dim3((unsigned)S, (unsigned)KV, (unsigned)nsplit), dim3(256), 0, stream, a);
     int rc = check_launch("decode_attention_fused");
     if (rc || nsplit == 1) return rc;
     hipLaunchKernelGGL(decode_merge_kernel, dim3((unsigned)(S * H)), dim3(64), 0, stream, part_o, part_ml, (elem_t*)out, hd, nsplit, a.sinks, H, a.out_gate);

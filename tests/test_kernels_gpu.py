@@ -629,8 +629,25 @@ def test_decode_attention(dtype, H, KV, hd, ps, window):
 def test_decode_attention_fused(dtype, H, KV, hd, ps, window, P_):
     """Bias, rotation, cache write and attention from partial sums of the projection; twice in a
     row with the same pages, the second time one position on, as decoding does."""
+    _fused_decode_attention(dtype, H, KV, hd, ps, window, P_, [0, 1, ps - 1, ps, 130, 700, 2049, 63, 64])
+
+
+# Three sums to more than the eight that are asked for first, heads of up to 64 and above; keys cut over blocks and (`short`) not, where requests have no key but the row's own,
+# keys for some of the four waves and for all.  28 heads over 4 of 128 and 16 over 1 of 80 are 1,152 and 1,440 columns: those that a thread asks for first, and more behind them.
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("short", [False, True])
+@pytest.mark.parametrize("H,KV,hd,ps,window,P_", [(28, 4, 128, 64, None, 7), (16, 1, 80, 32, 1000, 9), (14, 2, 64, 64, None, 8), (12, 2, 128, 64, None, 3),
+                                                  (12, 2, 128, 64, None, 17), (14, 2, 64, 64, None, 1)])
+def test_decode_attention_fused_of_many_sums(dtype, short, H, KV, hd, ps, window, P_):
+    lens = [0, 1, 17, 31, 32, 33, 64, 95, 96, 126] if short else [0, 1, ps - 1, ps, 130, 700, 2049, 63, 64]
+    ops = ops_for(dtype)
+    splits = ops._decode_splits(len(lens), KV, max(-(-(c + 2) // ps) for c in lens), ps, window, ops._attention_lib(hd)[4], hd)
+    assert (splits == 1) == short, f"{splits} splits: the sizes are those of the other form"
+    _fused_decode_attention(dtype, H, KV, hd, ps, window, P_, lens)
+
+
+def _fused_decode_attention(dtype, H, KV, hd, ps, window, P_, lens):
     ops, emu = ops_for(dtype), EmulatedOps(dtype)
-    lens = [0, 1, ps - 1, ps, 130, 700, 2049, 63, 64]
     S = len(lens)
     gen = torch.Generator().manual_seed(600 + hd)
     n_pages = sum(-(-(c + 2) // ps) for c in lens) + 2
