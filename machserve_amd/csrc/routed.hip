@@ -56,21 +56,69 @@ __global__ __launch_bounds__(256) void route_kernel(const elem_t* __restrict__ x
         for (int k = 0; k < EW; ++k)
 #pragma unroll
             for (int r = 0; r < R; ++r) v[k][r] = 0.f;
-        // AHEAD steps' loads on one straight path: left to the compiler, the unrolled loop asked for a step or two at a time.  us, warm, the same sums: four rows of 2,048 over
-        // 9 outputs 5.7 -> 5.4, 64 rows over 64 outputs 24.7 -> 16.5, 2,048 rows 8.8 -> 8.5 and 46 -> 30 (four steps ahead of one row: 5.7 and 18.9; of four rows 9.2 and 30.7).
-        for (int c0 = lane * V; c0 < d; c0 += 64 * V * AHEAD) {
-            float we[AHEAD][EW][V], xr[AHEAD][R][V];
+        if constexpr (AHEAD > 1) {
+            // The loads of AHEAD steps on one straight path (beyond the row its end, not added).  Left to the compiler, the loop below asks for a step or two at a time: us,
+            // warm, the same sums, that loop and here: four rows of 2,048 over 9 outputs 5.0 and 4.7, 64 rows over 64 outputs 15.9 and 13.3, 2,048 rows 8.0 and 7.7, 30.2 and
+            // 25.6.  (With that loop behind this one, for the steps that fill no round, four rows of 2,048 over 4 outputs 4.4 for 3.7: the code is twice as long.
+            // The loads are written out in both: through a function that both call they took 4 to 15 % longer.)
+            for (int c0 = lane * V; c0 < d; c0 += 64 * V * AHEAD) {
+                float we[AHEAD][EW][V], xr[AHEAD][R][V];
 #pragma unroll
-            for (int u = 0; u < AHEAD; ++u) {
-                const int c = AHEAD == 1 ? c0 : min(c0 + u * 64 * V, d - V);
+                for (int u = 0; u < AHEAD; ++u) {
+                    const int c = min(c0 + u * 64 * V, d - V);
+#pragma unroll
+                    for (int k = 0; k < EW; ++k) {
+                        const float* from = w + (size_t)min(e0 + 4 * k, outputs - 1) * d + c;
+                        if constexpr (V == 4) {
+                            const float4 four = *reinterpret_cast<const float4*>(from);
+                            we[u][k][0] = four.x, we[u][k][1] = four.y, we[u][k][2] = four.z, we[u][k][3] = four.w;
+                        } else {
+                            we[u][k][0] = from[0];
+                        }
+                    }
+#pragma unroll
+                    for (int r = 0; r < R; ++r) {
+                        const elem_t* row = x + (size_t)min(t0 + r, rs.T - 1) * d + c;
+                        if constexpr (V == 4 && sizeof(elem_t) == 2) {
+                            const u32x2 raw = *reinterpret_cast<const u32x2*>(row);
+                            const elem_t* four = reinterpret_cast<const elem_t*>(&raw);
+#pragma unroll
+                            for (int i = 0; i < V; ++i) xr[u][r][i] = to_f32(four[i]);
+                        } else if constexpr (V == 4) {
+                            const float4 four = *reinterpret_cast<const float4*>(row);
+                            xr[u][r][0] = four.x, xr[u][r][1] = four.y, xr[u][r][2] = four.z, xr[u][r][3] = four.w;
+                        } else {
+                            xr[u][r][0] = to_f32(row[0]);
+                        }
+                    }
+                }
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int u = 0; u < AHEAD; ++u) {
+                    const bool in = c0 + u * 64 * V < d;
+#pragma unroll
+                    for (int k = 0; k < EW; ++k)
+#pragma unroll
+                        for (int r = 0; r < R; ++r)
+#pragma unroll
+                            for (int i = 0; i < V; ++i) {
+                                const float sum = v[k][r] + xr[u][r][i] * we[u][k][i];
+                                v[k][r] = in ? sum : v[k][r];
+                            }
+                }
+            }
+        } else {
+#pragma unroll(R == 1 ? 8 : 4)
+            for (int c = lane * V; c < d; c += 64 * V) {
+                float we[EW][V], xr[R][V];
 #pragma unroll
                 for (int k = 0; k < EW; ++k) {
                     const float* from = w + (size_t)min(e0 + 4 * k, outputs - 1) * d + c;
                     if constexpr (V == 4) {
                         const float4 four = *reinterpret_cast<const float4*>(from);
-                        we[u][k][0] = four.x, we[u][k][1] = four.y, we[u][k][2] = four.z, we[u][k][3] = four.w;
+                        we[k][0] = four.x, we[k][1] = four.y, we[k][2] = four.z, we[k][3] = four.w;
                     } else {
-                        we[u][k][0] = from[0];
+                        we[k][0] = from[0];
                     }
                 }
 #pragma unroll
@@ -80,28 +128,20 @@ __global__ __launch_bounds__(256) void route_kernel(const elem_t* __restrict__ x
                         const u32x2 raw = *reinterpret_cast<const u32x2*>(row);
                         const elem_t* four = reinterpret_cast<const elem_t*>(&raw);
 #pragma unroll
-                        for (int i = 0; i < V; ++i) xr[u][r][i] = to_f32(four[i]);
+                        for (int i = 0; i < V; ++i) xr[r][i] = to_f32(four[i]);
                     } else if constexpr (V == 4) {
                         const float4 four = *reinterpret_cast<const float4*>(row);
-                        xr[u][r][0] = four.x, xr[u][r][1] = four.y, xr[u][r][2] = four.z, xr[u][r][3] = four.w;
+                        xr[r][0] = four.x, xr[r][1] = four.y, xr[r][2] = four.z, xr[r][3] = four.w;
                     } else {
-                        xr[u][r][0] = to_f32(row[0]);
+                        xr[r][0] = to_f32(row[0]);
                     }
                 }
-            }
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int u = 0; u < AHEAD; ++u) {
-                const bool in = AHEAD == 1 || c0 + u * 64 * V < d;
 #pragma unroll
                 for (int k = 0; k < EW; ++k)
 #pragma unroll
                     for (int r = 0; r < R; ++r)
 #pragma unroll
-                        for (int i = 0; i < V; ++i) {
-                            const float sum = v[k][r] + xr[u][r][i] * we[u][k][i];
-                            v[k][r] = in ? sum : v[k][r];
-                        }
+                        for (int i = 0; i < V; ++i) v[k][r] += xr[r][i] * we[k][i];
             }
         }
 #pragma unroll
@@ -671,23 +711,32 @@ extern "C" int ms_route(const void* x, const float* w, const float* bias, float*
     // up to four outputs: one a wave, which asks for nothing twice (four outputs of 2,048, three a wave / one / an output in turn: 16 rows 5.0 / 4.2 / 4.9 us,
     // 1,000 rows 7.8 / 5.6 / 6.6; five outputs, three a wave / in turn: 5.0 / 5.7 and 7.9 / 7.5)
     const bool one = E + extra <= 4;
-    // No more steps ahead than a row has: with eight, four rows of 1,024 over 9 outputs took 9.2 us in a decode step and 7.4 in a plain loop.  Warm, plain loop -> now: four rows
-    // over 9 outputs 4.1 -> 3.9 us (512 columns), 4.4 -> 4.2 (1,024), 4.9 -> 4.6 (2,048); over 65 of 1,024 11.9 -> 11.1; 2,048 rows of 1,024 over 9 6.5 -> 6.2.
-    const int steps = ceil_div(d, 64 * 4);
-#define MS_ROUTE_FOURS(EW_)                     \
-    do {                                        \
-        if (many && steps > 1) MS_ROUTE(4, 4, EW_, 2); \
-        else if (many) MS_ROUTE(4, 4, EW_, 1);  \
-        else if (steps > 4) MS_ROUTE(1, 4, EW_, 8); \
-        else if (steps > 2) MS_ROUTE(1, 4, EW_, 4); \
-        else MS_ROUTE(1, 4, EW_, 2);            \
+    // Steps asked for at once: eight, four where a row has four at most, two of two and of four rows, as long as the last round asks for few steps that the row does not have
+    // (us, plain loop and so, 64 rows over 64 outputs: 1,536 columns, two of eight, 14.2 and 13.3; 2,304 columns, seven of sixteen, 17.0 and 18.8): a quarter at most; none of
+    // four rows (2,048 rows of 768 columns over 9 outputs, one of four, 5.8 and 6.1); and one of eight, in one round, where two rows share a CU (300 rows:
+    // 1,792 columns over 64 outputs, one of eight, 17.5 and 15.5; 1,536 over 9, two, 5.4 and 5.7; 3,584 over 9, two of sixteen, 7.2 and 7.6).  With more than two rows a CU
+    // the blocks beside each other hide the loads, and the registers count (1,000 rows over 64 outputs: 1,280 columns 18.4 and 27, 2,048 columns 26.4 and 27.8).
+    const int steps = ceil_div(d, 64 * 4), most = many || steps <= 2 ? 2 : steps <= 4 ? 4 : 8, surplus = ceil_div(steps, most) * most - steps;
+    const bool straight = many                     ? surplus == 0
+                          : T <= compute_units()     ? surplus * 4 <= steps + surplus
+                          : T <= 2 * compute_units() ? surplus * 8 <= most && steps <= 8
+                                                     : false;
+    const int ahead = straight ? most : 1;
+#define MS_ROUTE_FOURS(EW_)                              \
+    do {                                                 \
+        if (many && ahead == 2) MS_ROUTE(4, 4, EW_, 2);  \
+        else if (many) MS_ROUTE(4, 4, EW_, 1);           \
+        else if (ahead == 8) MS_ROUTE(1, 4, EW_, 8);     \
+        else if (ahead == 4) MS_ROUTE(1, 4, EW_, 4);     \
+        else if (ahead == 2) MS_ROUTE(1, 4, EW_, 2);     \
+        else MS_ROUTE(1, 4, EW_, 1);                     \
     } while (0)
     if (one && fours) MS_ROUTE_FOURS(1);
     else if (fours) MS_ROUTE_FOURS(3);
     else if (one && many) MS_ROUTE(4, 1, 1, 2);
-    else if (one) MS_ROUTE(1, 1, 1, 8);
+    else if (one) MS_ROUTE(1, 1, 1, 1);
     else if (many) MS_ROUTE(4, 1, 3, 2);
-    else MS_ROUTE(1, 1, 3, 8);
+    else MS_ROUTE(1, 1, 3, 1);
 #undef MS_ROUTE_FOURS
 #undef MS_ROUTE
     return check_launch("route");

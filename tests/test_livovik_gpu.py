@@ -202,6 +202,15 @@ def test_logits_whatever_the_steps_of_a_row(dtype, T, extra, width):
     assert bool((err <= bound).all()), f"error {float(err.max()):.3e}, {float((err / bound).max()):.2f} of the bound"
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("T", [256, 257, 512, 513])
+@pytest.mark.parametrize("extra", [1, 8])
+@pytest.mark.parametrize("width", [768, 1280, 1536, 1792, 2304, 3072, 3584])
+def test_logits_around_the_rows_of_a_cu(dtype, T, extra, width):
+    """Rows of three to fourteen steps, with a CU of their own, two to a CU and more: in rounds that are full, in rounds that are not, and in the plain loop."""
+    test_logits_whatever_the_steps_of_a_row(dtype, T, extra, width)
+
+
 def test_a_gate_of_every_row_goes_with_softmax_weights_too():
     ops, ref = ops_of(torch.float32), EmulatedOps(torch.float32)
     torch.manual_seed(0)
