@@ -279,7 +279,6 @@ __global__ __launch_bounds__(256) void norm_add_kernel(float* __restrict__ x, co
     for (int c = threadIdx.x; c < d; c += 256) dst[c] += vals[c] * inv * w[c];
 }
 
-// A branch's norm behind it and the next branch's norm ahead of it, in one pass over the row:
 // The same for widths of up to 1,024 GROUPS in whole fours, each branch of at most NP sums: a thread keeps its columns in registers, and all that the row needs from memory is
 // asked for at once.  In the kernel above a row of 2,048 is two rounds of sums and, behind the norm, eight of loads that wait for the stores before them
 // (the stream may be what they write): 16 rows of 2,048 in a decode step, eight sums 6.1 -> 4.5 us, two branches of eight 7.9 -> 4.6.
@@ -339,16 +338,21 @@ static void launch_norm_add(float* x, const float* partials, int n_partials, con
         hipLaunchKernelGGL((norm_add_wide_kernel<G_, NP_, PAIR>), dim3(T), dim3(256), 0, stream, x, partials, n_partials, ps, w, d, eps, bias, fa, pb, nb, fb); \
         return;                                                                                                                                          \
     } while (0)
-    // (registers: 128 of sums at most)
+    // Sums rounded up to two, four or eight, 128 registers of them at most: a sum more is read from the last one's lines again, and not added (three sums, 2,048 rows of
+    // 1,024: the kernel above 6.1 us, as eight sums 6.0, as four 5.1).  More than four sums of wide rows of which more than four a CU come stay above: they
+    // are read from memory, 2,048 rows of 2,048, two branches of eight 48.2 us above and 51.2 here.
     if (aligned && most <= 2 && d <= 1024) MS_NORM_ADD(1, 2);
     if (aligned && most <= 2 && d <= 2048) MS_NORM_ADD(2, 2);
     if (aligned && most <= 2 && d <= 4096) MS_NORM_ADD(4, 2);
+    if (aligned && most <= 4 && d <= 1024) MS_NORM_ADD(1, 4);
+    if (aligned && most <= 4 && d <= 2048) MS_NORM_ADD(2, 4);
     if (aligned && most <= 8 && d <= 1024) MS_NORM_ADD(1, 8);
-    if (aligned && most <= 8 && d <= 2048) MS_NORM_ADD(2, 8);
+    if (aligned && most <= 8 && d <= 2048 && T <= 4 * compute_units()) MS_NORM_ADD(2, 8);
 #undef MS_NORM_ADD
     hipLaunchKernelGGL(norm_add_kernel<PAIR>, dim3(T), dim3(256), (size_t)d * sizeof(float), stream, x, partials, n_partials, ps, w, d, eps, bias, fa, pb, nb, fb);
 }
 
+// A branch's norm behind it and the next branch's norm ahead of it, in one pass over the row:
 // x[t, :] += y / rms(y) * w  with y as norm_add_kernel has it,  then  out[t, :] = x / rms(x) * w2 in the element type.
 // For widths that are a multiple of four and at most 1024 * G, and up to NP sums a branch: a thread owns G groups of four
 // columns and asks for everything the row needs before it uses the first value (sums beyond the last one read the last one

@@ -1084,8 +1084,17 @@ def test_zeroing_a_place_of_several_arrays():
 @pytest.mark.parametrize("na,nb", [(1, 1), (2, 1), (3, 2), (8, 8), (9, 1)])
 def test_normed_branches_added_to_the_stream(d, na, nb):
     """One, two and four groups of 1,024 columns and widths behind them; up to two, up to eight and more sums: a branch, a branch with a bias, two branches weighed."""
-    ops = ops_for(torch.bfloat16)
-    T, eps = 3, 1e-5
+    _normed_branches(3, d, na, nb)
+
+
+@pytest.mark.parametrize("T,d,na,nb", [(3, 1024, 4, 4), (3, 2048, 4, 1), (3, 1028, 5, 3), (1024, 2048, 5, 1), (1025, 2048, 8, 5), (1025, 1028, 6, 1), (1025, 1024, 8, 8)])
+def test_normed_branches_of_four_sums_and_of_many_rows(T, d, na, nb):
+    """Up to four sums, and more than four of wide rows around four rows a CU."""
+    _normed_branches(T, d, na, nb)
+
+
+def _normed_branches(T, d, na, nb):
+    ops, eps = ops_for(torch.bfloat16), 1e-5
     x0, pa, pb = rnd((T, d), torch.float32, 111), rnd((na, T, d), torch.float32, 112), rnd((nb, T, d), torch.float32, 113)
     w, bias = 1 + rnd((d,), torch.float32, 114, 0.2), rnd((d,), torch.float32, 115)
     norm = lambda y: y / torch.sqrt((y * y).mean(-1, keepdim=True) + eps) * w.double()  # noqa: E731
