@@ -8,7 +8,8 @@
 
 namespace ms {
 
-// x[t, :] = float(table[tokens[t], :]) * scale, and the same in the element type in `rounded` if it is given.
+// x[t, :] = float(table[tokens[t], :]) * scale, and with ROUNDED the same in the element type in `rounded`.
+template <bool ROUNDED>
 __global__ __launch_bounds__(256) void embed_kernel(const int* __restrict__ tokens, const elem_t* __restrict__ table,
                                                     float* __restrict__ x, elem_t* __restrict__ rounded, int d, float scale) {
     arguments_now(tokens, table, x, rounded, d, scale);
@@ -17,7 +18,7 @@ __global__ __launch_bounds__(256) void embed_kernel(const int* __restrict__ toke
     for (int c = threadIdx.x; c < d; c += 256) {
         const float v = to_f32(src[c]) * scale;
         x[(size_t)t * d + c] = v;
-        if (rounded) rounded[(size_t)t * d + c] = from_f32<elem_t>(v);
+        if constexpr (ROUNDED) rounded[(size_t)t * d + c] = from_f32<elem_t>(v);
     }
 }
 // The same for widths of up to 1,024 GROUPS in whole fours, 8 or 16 bytes a load, all of a row's asked for at once: an element a load and one after the other the kernel
@@ -791,7 +792,8 @@ extern "C" int ms_embed_rounded(const int* tokens, const void* table, float* x, 
     if (fours && d <= 1024) MS_EMBED(embed_wide_kernel<1>);
     else if (fours && d <= 2048) MS_EMBED(embed_wide_kernel<2>);
     else if (fours && d <= 4096) MS_EMBED(embed_wide_kernel<4>);
-    else MS_EMBED(embed_kernel);
+    else if (rounded) MS_EMBED(embed_kernel<true>);
+    else MS_EMBED(embed_kernel<false>);
 #undef MS_EMBED
     return check_launch("embed");
 }
