@@ -28,9 +28,10 @@ class Embedding(Part):
         return self.rt.ops.embed(tokens, self.weight, getattr(self.spec, "scale", 1.0))
 
     def forward_rounded(self, tokens: torch.Tensor):
-        """The rows, and the same in the element type or None where the kernels do not leave them."""
+        """The rows, and the same in the element type or None where the kernels do not leave them or :meth:`forward` is another's."""
         both = getattr(self.rt.ops, "embed_rounded", None)
-        return (self.forward(tokens), None) if both is None else both(tokens, self.weight, getattr(self.spec, "scale", 1.0))
+        own = getattr(self.forward, "__func__", None) is Embedding.forward
+        return (self.forward(tokens), None) if both is None or not own else both(tokens, self.weight, getattr(self.spec, "scale", 1.0))
 
 
 @register_embedding("pair_embedding")

@@ -627,3 +627,27 @@ def test_toy_model_on_the_cpu_stand_ins():
 @pytest.mark.parametrize("dtype", [torch.float32])
 def test_toy_model_on_the_gpu(dtype):
     _check("cuda:0", None, dtype)
+
+
+def test_an_embedding_of_ones_own_is_the_one_that_blocks_read():
+    """Blocks that read the rows rounded get those of the embedding's own ``forward``, in a class of its own or put in its place, and the kernel's pair only where it is the
+    framework's."""
+    from types import SimpleNamespace
+    from machserve_amd.parts import Embedding
+
+    class Doubled(Embedding):
+        def forward(self, tokens):
+            return 2.0 * super().forward(tokens)
+
+    emu = EmulatedOps(torch.float32)
+    rt = SimpleNamespace(ops=SimpleNamespace(embed=emu.embed, embed_rounded=lambda t, w, s: (emu.embed(t, w, s), emu.embed(t, w, s).bfloat16())))
+    spec, weight, tokens = EmbeddingSpec(VOCAB, WIDTH), torch.randn(VOCAB, WIDTH), torch.tensor([3, 0, 89], dtype=torch.int32)
+    plain, own, placed = Embedding(spec, rt), Doubled(spec, rt), Embedding(spec, rt)
+    for part in (plain, own, placed):
+        part.load({"weight": weight})
+    placed.forward = lambda tokens: -weight[tokens.long()]
+    x, rounded = plain.forward_rounded(tokens)
+    assert torch.equal(x, weight[tokens.long()]) and torch.equal(rounded, x.bfloat16())
+    for part, factor in ((own, 2.0), (placed, -1.0)):
+        x, rounded = part.forward_rounded(tokens)
+        assert torch.equal(x, factor * weight[tokens.long()]) and rounded is None
