@@ -400,6 +400,23 @@ extern "C" int ms_swiglu_scaled_takes(int M, int I, int K) {
 #endif
 }
 
+// ... and whether it pays to hand it rows that lack their norm's division: few rows, or tiles that are at most a round of the chip.  Every tile reads its rows' factors at its start and
+// applies them at its end, which in the first round is less than the norm's kernel, and is paid again in each further one.  us a layer, output projection to gated product, with
+// the norm between them and without: 0.5B sizes 2,048 rows (248 tiles) 48.7 and 48.2, 3,001 (372) 68.6 and 70.2; 1.5B 1,024 (224) 77.6 and 76.6, 1,500 (336) 105.8 and 107.9,
+// 4,096 (896) 232 and 242; 7B 1,024 (476) 287 and 290; width 1,024 and 2,816 in the middle, 3,001 rows (216) 57.0 and 55.8.
+extern "C" int ms_swiglu_scaled_pays(int M, int I, int K) {
+#ifdef MS_ELEM_HALF
+    if (!ms_swiglu_scaled_takes(M, I, K)) return 0;
+    if (!planned(M, K)) return 1;
+    const int n = 2 * ceil_div(I, 16) * 16;
+    const auto& t = kTiles[plan_gemm(M, n, K, 1, false, true).tile];
+    return (long)ceil_div(M, t.bm) * ceil_div(n, t.bn) <= (long)compute_units() * t.per_cu;
+#else
+    (void)M; (void)I; (void)K;
+    return 0;
+#endif
+}
+
 // ms_linear_swiglu for rows that came in multiplied by a norm's weight only: both products of a row are
 // divided by the row's root mean square, 1 / sqrt(sum_p row_ss[p, row] / K + eps), before the activation.
 extern "C" int ms_linear_swiglu_scaled(const void* a, const float* row_ss, int ss_parts, float eps, const void* w, void* out, int M, int I,

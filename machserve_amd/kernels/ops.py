@@ -384,7 +384,7 @@ class HipOps:
         first leaves ``x * norm_w`` and the rows' sums of squares beside the sum, the second divides its
         finished sums by the root mean square (:meth:`linear_residual_prenorm`, :meth:`linear_swiglu_scaled`)."""
         return ((self._plan("ms_prenorm_parts", M, N, K) > 0 or (not self._tiled(M, N, K) and self._plan("ms_skinny_prenorm_parts", M, N, K) > 0))
-                and bool(self._plan("ms_swiglu_scaled_takes", M, n_gate_up // 2, N)
+                and bool(self._plan("ms_swiglu_scaled_pays", M, n_gate_up // 2, N)
                          or self._plan("ms_swiglu_scaled_skinny_takes", M, n_gate_up // 2, N)))
 
     def linear_residual_prenorm(self, a: torch.Tensor, w: torch.Tensor, x: torch.Tensor, norm_w: torch.Tensor):

@@ -197,3 +197,20 @@ def test_gated_products_with_row_factors_of_many_rows(M, I, K, parts):
     assert_close(got, z * torch.sigmoid(z) * u, torch.bfloat16, "gated product with row factors")
     if M > 300:
         assert_close(ops.linear_swiglu_scaled(a[:200].contiguous(), share[:, :200].contiguous(), 1e-5, w, I), got[:200].double(), torch.bfloat16, "a row in another batch")
+
+
+@pytest.mark.parametrize("M,width,I,pays", [(2048, 896, 4864, True), (2049, 896, 4864, False), (1024, 1536, 8960, True), (1500, 1536, 8960, False), (2048, 3584, 18944, False),
+                                            (3001, 1024, 2816, True), (16, 896, 4864, True)])
+def test_a_norm_is_prepared_where_the_gated_product_is_a_round(M, width, I, pays):
+    """Around a round of the gated product's tiles; with either answer the norm between the products is the same."""
+    from machserve_amd.kernels.ops import interleave_gate_up
+    ops = ops_for(torch.bfloat16)
+    assert ops.prenorm_swiglu_takes(M, width, width, 2 * I) == pays
+    if M > 2049:
+        return
+    a, w, x = rnd((M, width), torch.bfloat16, 61), rnd((width, width), torch.bfloat16, 62, width ** -0.5), rnd((M, width), torch.float32, 63)
+    gu, nw = interleave_gate_up(rnd((I, width), torch.bfloat16, 64, width ** -0.5), rnd((I, width), torch.bfloat16, 65, width ** -0.5)), 1 + rnd((width,), torch.float32, 66, 0.1)
+    x1 = x.clone()
+    assert ops._plan("ms_prenorm_parts", M, width, width) > 0
+    want = ops.linear_swiglu(ops.rmsnorm(x1, nw, 1e-6, partials=ops.linear_residual(a, w, x1)), gu, I)
+    assert_close(ops.linear_swiglu_scaled(*ops.linear_residual_prenorm(a, w, x, nw), 1e-6, gu, I), want.float(), torch.bfloat16, "gated product behind a norm")
