@@ -1053,7 +1053,8 @@ struct DecodeTile {
 };
 
 // MANY (fused): the q/k/v product left more than two partial sums, of which up to eight are then asked for first of all.  CUT (fused): the keys are cut over several blocks.
-template <bool FUSED, bool MANY = false, bool CUT = false>
+// WIDE (fused): a KV head's share of the row is more than 1,024 columns, five a thread.
+template <bool FUSED, bool MANY = false, bool CUT = false, bool WIDE = false>
 __global__ __launch_bounds__(256) void decode_attention_kernel(DecodeArgs a) {
     arguments_now(a.q, a.kpool, a.vpool, a.out, a.part_o, a.part_ml, a.block_table, a.seq_pos0, a.table_stride, a.H, a.KV, a.hd,
                   a.ps, a.window, a.nsplit, a.scale, a.qkv, a.bias, a.inv_freq, a.slot_map, a.n_partials, a.stride);
@@ -1148,7 +1149,7 @@ __global__ __launch_bounds__(256) void decode_attention_kernel(DecodeArgs a) {
         }
     };
     // The fused prologue stages this KV head's share of the step's row: its g query heads, its key, its
-    // value, (g + 2) * hd columns, four per thread at a time, with heads of more than 64 five (1,280: seven heads of 128 beside key and value are 1,152).  What the
+    // value, (g + 2) * hd columns, four per thread at a time, of more than 1,024 columns five (1,280: seven heads of 128 beside key and value are 1,152).  What the
     // first of them need from memory (the bias and the first partial sums) is asked for here, before anything else: nothing of it
     // depends on the row's position, and the row's query is what the block waits for in the end.  (Seven sums of 1,152 columns, 28 heads
     // over 4 of 128, 16 requests: two first, five more and the last 128 columns behind them 13.8 us, all at once 11.5.)
@@ -1162,7 +1163,7 @@ __global__ __launch_bounds__(256) void decode_attention_kernel(DecodeArgs a) {
         const int qcol = kvh * g * hd, kcol = a.H * hd + kvh * hd, vcol = (a.H + a.KV) * hd + kvh * hd;
         return c < g * hd ? qcol + c : (c < (g + 1) * hd ? kcol + c - g * hd : vcol + c - (g + 1) * hd);
     };
-    constexpr int COLS = ND > 4 ? 5 : 4, EARLY = MANY ? 8 : 2;
+    constexpr int COLS = WIDE ? 5 : 4, EARLY = MANY ? 8 : 2;
     int col_e[COLS];
     float bias_e[COLS], part_e[EARLY][COLS], freq_e = 0.f;
     int slot = -1;
@@ -1855,8 +1856,15 @@ extern "C" int MS_CAT(ms_decode_attention_fused_nd, MS_ATTN_ND)(
     DecodeArgs a{nullptr, (const elem_t*)kpool, (const elem_t*)vpool, (elem_t*)out, part_o, part_ml, block_table, seq_pos0,
                  table_stride, H, KV, hd, ps, window, nsplit, scale, qkv, bias, inv_freq, slot_map, n_partials, stride, nullptr, nullptr};
     const bool many = n_partials > 2, cut = nsplit > 1;
-    auto kernel = many ? (cut ? decode_attention_kernel<true, true, true> : decode_attention_kernel<true, true, false>)
-                       : (cut ? decode_attention_kernel<true, false, true> : decode_attention_kernel<true, false, false>);
+    auto form = [&](auto wide) {
+        constexpr bool W = decltype(wide)::value;
+        return many ? (cut ? decode_attention_kernel<true, true, true, W> : decode_attention_kernel<true, true, false, W>)
+                    : (cut ? decode_attention_kernel<true, false, true, W> : decode_attention_kernel<true, false, false, W>);
+    };
+    auto kernel = form(std::false_type{});
+    if constexpr (ND > 4)  // (of at most 1,024 columns the fifth is one that nobody uses: us, 12 heads over 2 of 128, one sum, five and four: 8 requests behind 33 keys 8.39 and 8.27,
+                           // behind 2,048 12.62 and 12.45, 64 behind 120 10.53 and 10.43)
+        if ((H / KV + 2) * hd > 1024) kernel = form(std::true_type{});
     hipLaunchKernelGGL(kernel, dim3((unsigned)S, (unsigned)KV, (unsigned)nsplit), dim3(256), 0, stream, a);
     int rc = check_launch("decode_attention_fused");
     if (rc || nsplit == 1) return rc;

@@ -636,7 +636,7 @@ def test_decode_attention_fused(dtype, H, KV, hd, ps, window, P_):
 # keys for some of the four waves and for all.  28 heads over 4 of 128 and 16 over 1 of 80 are 1,152 and 1,440 columns: those that a thread asks for first, and more behind them.
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("short", [False, True])
-@pytest.mark.parametrize("H,KV,hd,ps,window,P_", [(28, 4, 128, 64, None, 7), (16, 1, 80, 32, 1000, 9), (14, 2, 64, 64, None, 8), (12, 2, 128, 64, None, 3),
+@pytest.mark.parametrize("H,KV,hd,ps,window,P_", [(28, 4, 128, 64, None, 7), (28, 4, 128, 64, None, 2), (16, 1, 80, 32, 1000, 9), (14, 2, 64, 64, None, 8), (12, 2, 128, 64, None, 3),
                                                   (12, 2, 128, 64, None, 17), (14, 2, 64, 64, None, 1)])
 def test_decode_attention_fused_of_many_sums(dtype, short, H, KV, hd, ps, window, P_):
     lens = [0, 1, 17, 31, 32, 33, 64, 95, 96, 126] if short else [0, 1, ps - 1, ps, 130, 700, 2049, 63, 64]
