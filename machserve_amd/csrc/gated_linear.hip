@@ -43,40 +43,52 @@ __global__ __launch_bounds__(256) void key_decay_kernel(Sums in, int col, const 
 // ---- gated linear attention over many rows ---------------------------------------------------------------------
 // A thread is a value channel and holds its column of S in registers (DP of them; the rows beyond d stay zero).  Tokens come
 // WALK_BATCH at a time through LDS; the next batch's numbers are asked for before the current batch is walked.  seg_len 0: a
-// block walks all of a request's rows.  Else a request's rows are cut into segments (the requests' first ones are the first S blocks, later_segment has the others): LOCAL walks
-// each from zero and leaves what it adds (carry [places, H, d, dvp]) and the product of its decays (cdec [places, H, d]),
-// the carry kernel replaces what it adds by the state that comes into it, and the second walk makes the outputs.  A request of at most
-// WALK_WHOLE rows is walked by one block all the same, whatever comes with it: its rows take 1.25 us each, three kernels over segments 80 us and more (100 rows alone
-// 131 us walked, 79 in segments of 32; 64 rows 86 and 78; 64 requests of 17 rows 43 and 94), and 60 single rows beside a prompt of 2,000 took 2,468 us while
-// the rows a request had on average decided for all of a step (in segments 188).  A request of a single segment is walked whole as well.
-// (The lengths are on the device: a step that may hold a request to be cut and holds none pays for two launches that find nothing, 5 us: 64 requests of 17 rows 44 and 49.)
-constexpr int WALK_BATCH = 8, WALK_WHOLE = 64;
-__host__ __device__ constexpr int whole_rows(int seg_len) { return WALK_WHOLE > seg_len ? WALK_WHOLE : seg_len; }
+// block walks all of a request's rows.  Else a request of more than `whole` rows is cut into segments (the requests' first ones are the first S blocks, cut_segment has the
+// others): LOCAL walks each from zero and leaves what it adds (carry [places, H, d, dvp]) and the product of its decays (cdec [places, H, d]),
+// the carry kernel replaces what it adds by the state that comes into it, and the second walk makes the outputs.  A request of at most `whole` rows is
+// walked by one block all the same, whatever comes with it: a row takes 1.27 us of a walk (64 x 128), three kernels over segments 78 us and more (100 rows alone
+// 132 us walked, 79 in segments of 32; 64 rows 87 and 78; 60 single rows beside a prompt of 2,000 2,477 and 150) and more than twice the rows' work, which counts where the step's rows fill the
+// chip as they are: `whole` goes by how many come (us, walked and in segments: 16 requests of 70 rows, 8 heads of 128 x 256, 222 and 280, 32 of 100 314 and 621; 64 of 128, 16 heads of
+// 64 x 128, 211 and 401, 16 of 200 258 and 187).
+// (The lengths are on the device: a step that may hold a request to be cut and holds none pays for two launches that find nothing, 4 us: 64 requests of 17 rows 44 and 48, of 2 rows 17.6 and 23.5.)
+constexpr int WALK_BATCH = 8;
 struct WalkArgs {
     StateArgs a;
-    int seg_len;
+    int seg_len, whole;  // (whole >= seg_len)
     float* carry;
     float* cdec;
 };
-// The place of request s's first segment.  Only requests that are cut have places: such a one has more than whole_rows rows, so that the request cut next begins at
-// least one whole_rows further on, which makes up for the last segment's missing rows.  T / seg_len + min(T / whole_rows, S) places hold all of a step's, however many
+// The place of request s's first segment.  Only requests that are cut have places: such a one has more than `whole` rows, so that the request cut next begins at
+// least that many rows further on, which makes up for the last segment's missing rows.  T / seg_len + min(T / whole, S) places hold all of a step's, however many
 // single rows come with it (a place for each request beside took 0.3 GB for 512 single rows and a portion of 100, 16 heads of 64 x 128).
 __device__ __forceinline__ int carry_base(const WalkArgs& w, int s) {
     const int q0 = w.a.seq_q_start[s];
-    return q0 / w.seg_len + min(q0 / whole_rows(w.seg_len), s);
+    return q0 / w.seg_len + min(q0 / w.whole, s);
 }
 
-// Segments behind a request's first one, by number: request s's begin at its first row / L, which leaves each of them a number of its own below T / L.  The first segments, and the
-// requests that are walked whole, are numbered by themselves ahead of these: with a request's segments in one row, the blocks of short requests stood between numbers
-// that nobody has, unevenly over the chip (64 requests of 17 rows: the walk 65 us, without them 43).
-__device__ __forceinline__ Piece later_segment(int number, int L, const int* __restrict__ seq_q_start, int S) {
-    int lo = 0, hi = S - 1;
-    while (lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if (seq_q_start[mid] / L <= number) lo = mid;
-        else hi = mid - 1;
+// Segments of the requests that are cut, by number without gaps, all but the one of each that LOCAL leaves out (the last: nobody needs what it passes on) or that has a block among the first
+// S (the first); requests behind the last number are S.  Every wave adds the requests up for itself, 64 a step.  Numbers with gaps, every request's own from its first row / L on, left the blocks that
+// walk unevenly over the chip's dies, which blocks go to in turn: 64 requests of 128 rows in segments (16 heads of 64 x 128) 504 us, now 401.
+template <bool LOCAL>
+__device__ __forceinline__ Piece cut_segment(const WalkArgs& w, int number) {
+    const int lane = threadIdx.x % WAVE;
+    int before = 0;
+    for (int s0 = 0; s0 < w.a.S; s0 += WAVE) {
+        const int len = s0 + lane < w.a.S ? w.a.seq_q_len[s0 + lane] : 0, own = len > w.whole ? (len - 1) / w.seg_len : 0;
+        int upto = own;
+#pragma unroll
+        for (int o = 1; o < WAVE; o <<= 1) {
+            const int v = __shfl_up(upto, o, WAVE);
+            if (lane >= o) upto += v;
+        }
+        const uint64_t behind = __ballot(before + upto > number);
+        if (behind) {
+            const int at = __builtin_ctzll(behind);
+            return Piece{s0 + at, (number - before - __shfl(upto - own, at, WAVE) + (LOCAL ? 0 : 1)) * w.seg_len};
+        }
+        before += __shfl(upto, WAVE - 1, WAVE);
     }
-    return Piece{lo, (number - seq_q_start[lo] / L + 1) * L};
+    return Piece{w.a.S, 0};
 }
 
 template <int DP, int NT, bool LOCAL>
@@ -85,16 +97,17 @@ __global__ __launch_bounds__(NT) void state_walk_kernel(WalkArgs w) {
     const StateArgs& a = w.a;
     __shared__ __align__(16) float qs[LOCAL ? 1 : TB][DP], ks[TB][DP], ws[TB][DP];
     __shared__ float vs[TB][NT], os[LOCAL ? 1 : TB][NT], part[TB][NW];
-    const int h = blockIdx.y, j = threadIdx.x, d = a.d;
-    Piece pc{(int)blockIdx.x, 0};
-    if (w.seg_len && (int)blockIdx.x >= a.S) pc = later_segment(blockIdx.x - a.S, w.seg_len, a.seq_q_start, a.S);
+    // (heads innermost: the blocks that find nothing are the grid's last)
+    const int number = blockIdx.x / a.H, h = blockIdx.x - number * a.H, j = threadIdx.x, d = a.d;
+    Piece pc{number, 0};
+    if (LOCAL) pc = cut_segment<true>(w, number);
+    else if (w.seg_len && number >= a.S) pc = cut_segment<false>(w, number - a.S);
+    if (pc.s >= a.S) return;  // the same for the whole block
     const int left = a.seq_q_len[pc.s] - pc.first;
-    if (left <= 0) return;  // the same for the whole block
-    const bool whole = w.seg_len == 0 || a.seq_q_len[pc.s] <= whole_rows(w.seg_len);
-    if (whole && pc.first > 0) return;  // its first block has all of its rows
+    if (left <= 0) return;
+    const bool whole = w.seg_len == 0 || a.seq_q_len[pc.s] <= w.whole;
     const int n = whole ? left : min(left, w.seg_len);
     const bool last = n == left;
-    if (LOCAL && last) return;  // nobody needs what the last segment passes on
     const int q0 = a.seq_q_start[pc.s] + pc.first, kh = h / (a.H / a.G);
     const bool live = j < a.dv;
     const size_t head = (size_t)d * a.dvp;
@@ -248,7 +261,7 @@ constexpr int CARRY_AHEAD = 8;
 __global__ __launch_bounds__(256) void state_carry_kernel(WalkArgs w) {
     const StateArgs& a = w.a;
     const int s = blockIdx.x, h = blockIdx.y, idx = (blockIdx.z * 256 + threadIdx.x) * 4, head = a.d * a.dvp;
-    if (idx >= head || a.seq_q_len[s] <= whole_rows(w.seg_len)) return;
+    if (idx >= head || a.seq_q_len[s] <= w.whole) return;
     const int i = idx / a.dvp, base = carry_base(w, s);
     const int nseg = (a.seq_q_len[s] + w.seg_len - 1) / w.seg_len;
     f32x4 Sin = *reinterpret_cast<const f32x4*>(a.state + ((size_t)a.seq_slot[s] * a.H + h) * head + idx);
@@ -293,21 +306,21 @@ extern "C" int ms_key_decay(const float* in, int n_partials, int ld, int col, co
 }
 
 // Gated linear attention.  rows: float [n_partials, T, ld] with q [H, d], k [H, d], v [H, dv] and gate [H, dv] at their columns;
-// alpha float [T, H * d].  single: every request has one row.  seg_len > 0: segments side by side with carry float [places, H, d, dvp] and cdec float
-// [places, H, d] as workspace, places = T / seg_len + min(T / max(64, seg_len), S) (carry_base).
+// alpha float [T, H * d].  single: every request has one row.  seg_len > 0: requests of more than `whole` rows in segments side by side with carry
+// float [places, H, d, dvp] and cdec float [places, H, d] as workspace, places = T / seg_len + min(T / whole, S) (carry_base).
 extern "C" int ms_gated_linear(const float* rows, int n_partials, int ld, int q_col, int k_col, int v_col, int g_col, float q_scale,
                                const float* alpha, const float* norm, float eps, float* state, const int* seq_q_start, const int* seq_q_len,
                                const int* seq_slot, int S, void* out, int ld_out, int T, int H, int d, int dv, int dvp, int single,
-                               int seg_len, float* carry, float* cdec, hipStream_t stream) {
+                               int seg_len, int whole, float* carry, float* cdec, hipStream_t stream) {
     const Sums in{rows, n_partials, (size_t)T * ld, ld};
     const StateArgs a{in, in, in, q_col, k_col, v_col, q_scale, alpha, nullptr, in, g_col, norm, eps, state, seq_q_start, seq_q_len, seq_slot, S,
                       (elem_t*)out, ld_out, T, H, H, d, dv, dvp};
     MS_REQUIRE(n_partials > 0, "gated linear: no rows");
     if (int rc = check_state(a, "gated linear")) return rc;
     if (single) return launch_step<false>(a, stream);
-    MS_REQUIRE(seg_len == 0 || (seg_len > 0 && carry && cdec), "gated linear: segments of %d need their workspace", seg_len);
-    const WalkArgs w{a, seg_len, carry, cdec};
-#define MS_WALK(DP, NT, LOCAL, X) hipLaunchKernelGGL((state_walk_kernel<DP, NT, LOCAL>), dim3(X, H), dim3(NT), 0, stream, w)
+    MS_REQUIRE(seg_len == 0 || (seg_len > 0 && whole >= seg_len && carry && cdec), "gated linear: segments of %d of requests above %d rows need their workspace", seg_len, whole);
+    const WalkArgs w{a, seg_len, whole, carry, cdec};
+#define MS_WALK(DP, NT, LOCAL, X) hipLaunchKernelGGL((state_walk_kernel<DP, NT, LOCAL>), dim3((unsigned)(X) * H), dim3(NT), 0, stream, w)
 #define MS_WALK_N(DP, LOCAL, X)                   \
     do {                                          \
         if (dv <= 64) MS_WALK(DP, 64, LOCAL, X);  \
@@ -325,12 +338,12 @@ extern "C" int ms_gated_linear(const float* rows, int n_partials, int ld, int q_
         MS_WALK_D(false, S);
         return check_launch("gated linear");
     }
-    const int numbers = S + T / seg_len;
-    MS_WALK_D(true, numbers);
+    const int cuts = T / seg_len;  // (a request of n rows has (n - 1) / seg_len of those that are numbered)
+    MS_WALK_D(true, cuts);
     if (int rc = check_launch("gated linear, segments from zero")) return rc;
     hipLaunchKernelGGL(state_carry_kernel, dim3(S, H, ceil_div(d * dvp, 1024)), dim3(256), 0, stream, w);
     if (int rc = check_launch("gated linear, states between segments")) return rc;
-    MS_WALK_D(false, numbers);
+    MS_WALK_D(false, S + cuts);
 #undef MS_WALK_D
 #undef MS_WALK_N
 #undef MS_WALK

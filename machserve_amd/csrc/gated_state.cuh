@@ -16,7 +16,7 @@
 //                               in segments side by side (gated_linear.hip)
 //   delta rule, many rows       chunks of 64 tokens as small matrix products (gated_delta.hip)
 // Decays, their logarithms, step sizes, unit norms, states and every sum and product here are 32-bit in every build; what a
-// token gets depends on the cut of its prompt by rounding only, and on nothing else the step holds.
+// token gets depends on the cut of its prompt and, in gated linear attention, on how many rows its step holds, by rounding only.
 #pragma once
 #include "recurrence.cuh"
 

@@ -1669,21 +1669,22 @@ class HipOps:
         return alpha
 
     STATE_SEGMENT = 32  # rows of a segment of gated linear attention
-    STATE_WHOLE = 64  # ... of requests of more rows than this (WALK_WHOLE in the kernels)
+    STATE_WHOLE = 64  # ... of requests of more rows than this, or more (see _state_segments)
     STATE_WORKSPACE = 256 << 20  # bytes of states handed from segment to segment; longer segments where they would be more
 
     @classmethod
-    def _state_segments(cls, T: int, S: int, floats_per_state: int) -> tuple:
-        """``(segment length, places for the states between segments)`` for gated linear attention over ``T`` rows of ``S`` requests, or ``(0, 0)`` where
-        no request can be long enough to be cut: one has at most ``T - S + 1`` rows, and those of at most ``max(STATE_WHOLE, segment)`` rows are walked whole
-        by the kernels themselves, whatever comes with them."""
+    def _state_segments(cls, T: int, S: int, floats_per_state: int, rows_at_once: float = 0.0) -> tuple:
+        """``(segment length, rows up to which a request is walked whole, places for the states between segments)`` for gated linear attention over
+        ``T`` rows of ``S`` requests, or zeros where no request can be long enough to be cut: one has at most ``T - S + 1`` rows.
+        ``rows_at_once``: what the step's rows, in segments, take a chip full of blocks, in rows of a block alone.  Segments cost that and some 45 rows, a walk is as
+        long as its rows: a request is cut where it has more."""
         seg = cls.STATE_SEGMENT
-        while T - S >= (whole := max(cls.STATE_WHOLE, seg)):
+        while T - S >= (whole := max(cls.STATE_WHOLE, seg, 45 + int(rows_at_once))):
             n = T // seg + min(T // whole, S)
             if (n - 1) * floats_per_state * 4 <= cls.STATE_WORKSPACE:
-                return seg, n
+                return seg, whole, n
             seg *= 2
-        return 0, 0
+        return 0, 0, 0
 
     def gated_linear(self, sums: torch.Tensor, alpha: torch.Tensor, norm_w: torch.Tensor, eps: float, q_scale: float, state: torch.Tensor,
                      seq_q_start: torch.Tensor, seq_q_len: torch.Tensor, seq_slot: torch.Tensor, H: int, d: int, dv: int, out_cols: int,
@@ -1699,17 +1700,18 @@ class HipOps:
         if single and S != T:
             raise KernelError(f"gated linear: {T} rows of {S} requests are not single rows")
         out = torch.empty((T, out_cols), dtype=self.dtype, device=sums.device)
-        seg = n = 0
+        seg = whole = n = 0
         carry = cdec = None
-        if not single:
-            seg, n = self._state_segments(T, S, H * d * dvp)
+        if not single:  # a block is one, two or four waves; rows of a walk that a wave of rows a CU adds to segments: 0.12 (32 x 64, 12 x 20) and 0.15 (32 x 256), else 0.28 to 0.34
+            waves = T * H * (1 if dv <= 64 else 2 if dv <= 128 else 4) / self._cus
+            seg, whole, n = self._state_segments(T, S, H * d * dvp, waves * (0.15 if d <= 32 else 0.3))
         if seg:
             carry = torch.empty((n, H, d, dvp), dtype=torch.float32, device=sums.device)
             cdec = torch.empty((n, H, d), dtype=torch.float32, device=sums.device)
         self._check(lib, lib.ms_gated_linear(
             _ptr(sums), _c_int(P), _c_int(N), _c_int(0), _c_int(H * d), _c_int(2 * H * d), _c_int(2 * H * d + H * dv), _c_float(q_scale), _ptr(alpha),
             _ptr(norm_w), _c_float(eps), _ptr(state), _ptr(seq_q_start), _ptr(seq_q_len), _ptr(seq_slot), _c_int(S), _ptr(out), _c_int(out_cols),
-            _c_int(T), _c_int(H), _c_int(d), _c_int(dv), _c_int(dvp), _c_int(int(single)), _c_int(seg), _ptr(carry), _ptr(cdec), self._stream()))
+            _c_int(T), _c_int(H), _c_int(d), _c_int(dv), _c_int(dvp), _c_int(int(single)), _c_int(seg), _c_int(whole), _ptr(carry), _ptr(cdec), self._stream()))
         return out
 
     def delta_rows(self, sums: torch.Tensor, conv_w: torch.Tensor, conv_state: Optional[torch.Tensor], a_log: torch.Tensor, dt_bias: torch.Tensor,

@@ -307,29 +307,32 @@ def test_specs_that_do_not_fit_are_refused():
 
 
 def test_places_of_the_states_between_segments():
-    """Every request that is cut has places of its own for its segments, within those that are allocated, whatever comes with it; a request that may be cut is."""
+    """Every request that is cut has places of its own for its segments, within those that are allocated, whatever comes with it; every segment has one block that walks it in
+    either walk; a request that may be cut is."""
     import random
     from machserve_amd.kernels.ops import HipOps
     rng = random.Random(0)
     for trial in range(400):
         lengths = [rng.choice((1, 1, 1, 0, 17, 63, 64, 65, 96, 127, 128, 129, 300, rng.randint(1, 2000))) for _ in range(rng.randint(1, 40))]
-        T, S, state = sum(lengths), len(lengths), rng.choice((100, 1 << 17, 1 << 20, 1 << 22))
-        seg, n = HipOps._state_segments(T, S, state) if T else (0, 0)
+        T, S, state, at_once = sum(lengths), len(lengths), rng.choice((100, 1 << 17, 1 << 20, 1 << 22)), rng.choice((0.0, 20.0, 50.0, 300.0))
+        seg, whole, n = HipOps._state_segments(T, S, state, at_once) if T else (0, 0, 0)
         if not seg:
-            assert all(length <= 64 for length in lengths) or state > 100 or 0 in lengths
+            assert all(length <= max(64, 45 + int(at_once)) for length in lengths) or state > 100 or 0 in lengths
             continue
-        assert (n - 1) * state * 4 <= HipOps.STATE_WORKSPACE
-        whole, used, q0 = max(64, seg), set(), 0
-        starts = [sum(lengths[:i]) for i in range(S)]
-        later = {}  # what the blocks behind the first S walk: (request, segment)
-        for e in range(T // seg):
-            r = max(i for i in range(S) if starts[i] // seg <= e)
-            later[r, e - starts[r] // seg + 1] = e
-        assert all((r, k) in later for r in range(S) if lengths[r] > whole for k in range(1, -(-lengths[r] // seg))), (lengths, seg)
+        assert (n - 1) * state * 4 <= HipOps.STATE_WORKSPACE and whole >= max(64, seg)
+        starts, used = [sum(lengths[:i]) for i in range(S)], set()
+        own = [(length - 1) // seg if length > whole else 0 for length in lengths]
+        assert sum(own) <= T // seg, "a block for each numbered segment"
+        for local in (True, False):
+            walked = {(s, 0) for s in range(S) if not local}
+            for number in range(sum(own)):
+                s = next(s for s in range(S) if sum(own[:s + 1]) > number)
+                walked.add((s, number - sum(own[:s]) + (0 if local else 1)))
+            assert walked == {(s, k) for s in range(S) for k in range(own[s] + (0 if local else 1))}
         for s, length in enumerate(lengths):
             if length > whole:
-                for k in range(-(-length // seg)):
-                    place = q0 // seg + min(q0 // whole, s) + k
+                assert own[s] + 1 == -(-length // seg)
+                for k in range(own[s] + 1):
+                    place = starts[s] // seg + min(starts[s] // whole, s) + k
                     assert place < n and place not in used, (lengths, seg)
                     used.add(place)
-            q0 += length

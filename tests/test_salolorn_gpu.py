@@ -109,6 +109,28 @@ def test_gated_linear_attention_in_segments(monkeypatch, limit, seg):
     close(got_state, want_state, torch.float32, "states")
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_gated_linear_attention_beside_many_rows(dtype):
+    """Rows that fill the chip as they are: requests around the length from which one is cut beside them, more than 64 and more than 128 requests."""
+    ops, ref = ops_of(dtype), EmulatedOps(dtype)
+    torch.manual_seed(5)
+    H, d, dv = 16, 10, 130
+    for lengths in ([100] * 3 + [86, 87, 88, 89, 300] + [1] * 80 + [64, 33], [40] * 30 + [0, 130, 290] + [3] * 100 + [600]):
+        T, S, cols, dvp = sum(lengths), len(lengths), H * dv, 132
+        _, whole, _ = ops._state_segments(T, S, H * d * dvp, T * H * 4 / ops._cus * 0.15)
+        assert whole > 64 and max(lengths) > whole and any(64 < n <= whole for n in lengths)
+        sums = torch.randn(1, T, 2 * H * (d + dv)) * 0.7
+        alpha, norm = torch.sigmoid(torch.randn(T, H * d) + 3.0), torch.rand(dv) + 0.5
+        seqs = sequences(lengths, list(range(S))[::-1])
+        state = torch.zeros(S, H, d, dvp)
+        state[..., :dv] = torch.randn(S, H, d, dv)
+        want_state, got_state = state.clone(), dev(state)
+        want = ref.gated_linear(sums, alpha, norm, 1e-5, d ** -0.5, want_state, *seqs, H, d, dv, cols)
+        got = ops.gated_linear(dev(sums), dev(alpha), dev(norm), 1e-5, d ** -0.5, got_state, *[dev(s) for s in seqs], H, d, dv, cols)
+        close(got, want, dtype, "outputs")
+        close(got_state, want_state, torch.float32, "states")
+
+
 def test_single_rows_beside_a_portion_take_no_workspace():
     """500 decoding requests and one portion of 100 rows, 16 heads of 64 x 128 (half a megabyte a state): the portion's four segments, not a state for each request."""
     ops = ops_of(torch.bfloat16)
