@@ -116,13 +116,17 @@ static bool planned(int M, int K) { return M > 64 && K % 64 == 0 && g_gemm_confi
 #endif
 
 #ifndef MS_ELEM_HALF
-// Whether a 32-bit product runs in parts of 16 bits (GEMM_SPLIT): whole K steps, K in slices or an output of at least 4,096 columns whose 64x64 tiles are two a CU, or whose
-// 32x32 tiles, in which it ran else, are six and a half.  us, 32-bit instructions and parts: 192 x 9,728 x 896 (7.1 tiles of 32x32 a CU) 38 and 35, 160 rows (5.9) 32 and 35, 128 x
-// 12,288 x 896 (6) 30 and 34, 65 rows (4.5) 28 and 35; 320 x 9,728 x 896 (three of 64x64 a CU, a full round of either) 48 and 50, 512 rows 90 and 76; 512 x 4,096 x 1,024 (two)
-// 38 and 39, 1,024 rows 94 and 57.  The rows' number is part of the rule, as it is of the number of slices: a row's sums are those of other batches to rounding only.
+// Whether a 32-bit product runs in parts of 16 bits (GEMM_SPLIT): whole K steps, K in slices or an output of at least 4,096 columns in which the 32-bit instructions would fill
+// rounds badly.  Those have 32x32 tiles below two of 64x64 a CU, and parts are faster from six and a half of them on; else three of 64x64 a CU at a time, which take as long with
+// two and a bit as with three, and parts, 0.6 us a step for each that a CU has, are faster behind two up to 2.6 of them, and beyond a round.  us, 32-bit instructions and parts: 192 x
+// 9,728 x 896 (7.1 tiles of 32x32 a CU) 38 and 34, 160 rows (5.9) 32 and 35, 128 x 12,288 x 896 (6) 30 and 34, 65 rows (4.5) 28 and 35; 512 x 4,096 x 1,024 (2 of 64x64) 37.7 and 39.6,
+// 256 x 8,192 x 2,048 (2) 70 and 77, 400 x 4,864 x 896 (2.1) 46 and 42.6, 300 x 8,192 x 2,048 (2.5) 99 and 95, 700 x 4,096 x 1,024 (2.75) 53 and 54, 300 x 9,728 x 896 (2.97) 48.6 and
+// 50.8, 400 rows (4.2) 85 and 73, 1,024 x 4,096 x 1,024 (4) 95 and 57.  The rows' number is part of the rule, as it is of the number of slices: a row's sums are those of other
+// batches to rounding only.
 static bool parted(int M, int N, int K, int slices) {
     const long cus = compute_units(), tiles = (long)ceil_div(M, 64) * ceil_div(N, 64), small = (long)ceil_div(M, 32) * ceil_div(N, 32);
-    return K % 32 == 0 && M > 64 && (slices > 1 || (N >= 4096 && (tiles >= 2 * cus || 2 * small >= 13 * cus)));
+    const bool faster = tiles < 2 * cus ? 2 * small >= 13 * cus : tiles > 3 * cus || (tiles > 2 * cus && 5 * tiles <= 13 * cus);
+    return K % 32 == 0 && M > 64 && (slices > 1 || (N >= 4096 && faster));
 }
 // ... in tiles of 128x128, a block a CU, which take 1.7 us a K step and round, or of 64x64, 0.55 us for each that a CU has: 768 x 9,728 x 896 (two rounds, 7.1 a CU) 100 and
 // 114 us, 512 rows (two rounds, 4.8) 97 and 79, 1,024 rows (three, 9.5) 137 and 142; 512 x 896 x 4,864 in eight slices (one round, 3.5) 38 and 46, 192 x 2,048 x 5,632 (one, 3)

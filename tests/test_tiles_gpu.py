@@ -122,6 +122,14 @@ def test_32_bit_products_in_parts(M, N, K):
     assert float(err.max()) < 2e-6
 
 
+# Below two tiles of 64x64 a CU, at two, behind them, towards three, at a few more: where the 32-bit instructions fill their rounds they stay.
+@pytest.mark.parametrize("M,N,K,parts", [(160, 9728, 896, 0), (192, 9728, 896, 1), (512, 4096, 1024, 0), (400, 4864, 896, 1), (300, 9728, 896, 0), (400, 9728, 896, 1), (64, 9728, 896, 0)])
+def test_which_32_bit_products_are_taken_in_parts(M, N, K, parts):
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the sizes are those of 256 CUs")
+    assert (ops_for(torch.float32)._plan("ms_parted", M, N, K, 1) > 0) == bool(parts)
+
+
 # ... with nothing lost that the 32-bit products keep: a single product, small numbers of any scale, and rows beside ones that are not finite; both tiles, and K in slices
 @pytest.mark.parametrize("M,N,K", [(193, 8200, 64), (330, 9008, 96), (65, 136, 4128), (513, 896, 4864)])
 def test_32_bit_parts_lose_nothing(M, N, K):
