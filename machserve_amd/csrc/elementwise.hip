@@ -331,8 +331,8 @@ template <bool PAIR>
 static void launch_norm_add(float* x, const float* partials, int n_partials, const float* w, int T, int d, float eps, const float* bias, float fa,
                             const float* pb, int nb, float fb, hipStream_t stream) {
     const size_t ps = (size_t)T * d;
-    const bool aligned = d % 4 == 0 && ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(partials) | reinterpret_cast<uintptr_t>(w) |
-                                         reinterpret_cast<uintptr_t>(bias) | reinterpret_cast<uintptr_t>(pb)) & 15) == 0;
+    bool wide = d % 4 == 0 && ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(partials) | reinterpret_cast<uintptr_t>(w) |
+                                reinterpret_cast<uintptr_t>(bias) | reinterpret_cast<uintptr_t>(pb)) & 15) == 0;
     const int most = max(n_partials, nb);
 #define MS_NORM_ADD(G_, NP_)                                                                                                                             \
     do {                                                                                                                                                 \
@@ -341,14 +341,17 @@ static void launch_norm_add(float* x, const float* partials, int n_partials, con
     } while (0)
     // Sums rounded up to two, four or eight, 128 registers of them at most: a sum more is read from the last one's lines again, and not added (three sums, 2,048 rows of
     // 1,024: the kernel above 6.1 us, as eight sums 6.0, as four 5.1).  More than four sums of wide rows of which more than four a CU come stay above: they
-    // are read from memory, 2,048 rows of 2,048, two branches of eight 48.2 us above and 51.2 here.
-    if (aligned && most <= 2 && d <= 1024) MS_NORM_ADD(1, 2);
-    if (aligned && most <= 2 && d <= 2048) MS_NORM_ADD(2, 2);
-    if (aligned && most <= 2 && d <= 4096) MS_NORM_ADD(4, 2);
-    if (aligned && most <= 4 && d <= 1024) MS_NORM_ADD(1, 4);
-    if (aligned && most <= 4 && d <= 2048) MS_NORM_ADD(2, 4);
-    if (aligned && most <= 8 && d <= 1024) MS_NORM_ADD(1, 8);
-    if (aligned && most <= 8 && d <= 2048 && T <= 4 * compute_units()) MS_NORM_ADD(2, 8);
+    // are read from memory, 2,048 rows of 2,048, two branches of eight 48.2 us above and 51.2 here.  So do more than four sums, or more than four rows a CU, where half
+    // of the threads have no columns of their own (us, above and here: 512 columns, two branches of eight, 16 rows 3.0 and 3.4, 2,048 rows 7.2 and 8.9; 100 columns, one sum,
+    // 2,048 rows 3.7 and 4.0; but 512 columns, four sums, 300 rows 3.2 and 2.8).
+    if (d <= 512 && (most > 4 || T > 4 * compute_units())) wide = false;
+    if (wide && most <= 2 && d <= 1024) MS_NORM_ADD(1, 2);
+    if (wide && most <= 2 && d <= 2048) MS_NORM_ADD(2, 2);
+    if (wide && most <= 2 && d <= 4096) MS_NORM_ADD(4, 2);
+    if (wide && most <= 4 && d <= 1024) MS_NORM_ADD(1, 4);
+    if (wide && most <= 4 && d <= 2048) MS_NORM_ADD(2, 4);
+    if (wide && most <= 8 && d <= 1024) MS_NORM_ADD(1, 8);
+    if (wide && most <= 8 && d <= 2048 && T <= 4 * compute_units()) MS_NORM_ADD(2, 8);
 #undef MS_NORM_ADD
     hipLaunchKernelGGL(norm_add_kernel<PAIR>, dim3(T), dim3(256), (size_t)d * sizeof(float), stream, x, partials, n_partials, ps, w, d, eps, bias, fa, pb, nb, fb);
 }

@@ -1087,9 +1087,10 @@ def test_normed_branches_added_to_the_stream(d, na, nb):
     _normed_branches(3, d, na, nb)
 
 
-@pytest.mark.parametrize("T,d,na,nb", [(3, 1024, 4, 4), (3, 2048, 4, 1), (3, 1028, 5, 3), (1024, 2048, 5, 1), (1025, 2048, 8, 5), (1025, 1028, 6, 1), (1025, 1024, 8, 8)])
+@pytest.mark.parametrize("T,d,na,nb", [(3, 1024, 4, 4), (3, 2048, 4, 1), (3, 1028, 5, 3), (1024, 2048, 5, 1), (1025, 2048, 8, 5), (1025, 1028, 6, 1), (1025, 1024, 8, 8),
+                                         (1024, 512, 4, 1), (1025, 512, 4, 2), (3, 512, 5, 1), (3, 516, 5, 5)])
 def test_normed_branches_of_four_sums_and_of_many_rows(T, d, na, nb):
-    """Up to four sums, and more than four of wide rows around four rows a CU."""
+    """Up to four sums, and more than four of wide rows around four rows a CU; widths of which half of the threads have no columns."""
     _normed_branches(T, d, na, nb)
 
 
