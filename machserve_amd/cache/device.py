@@ -32,11 +32,16 @@ class DeviceCache:
         # the states' arrays stay where they are as long as this object has them: one launch zeroes a slot of them all
         self._zero = None
         arrays = [t for tensors in self._states.values() for t in tensors.values() if t.numel()]
-        if arrays and torch.device(device).type == "cuda":
-            from ..kernels import get_ops
-            ops = get_ops(dtype, str(device))
-            places = ops.places_of(arrays)
-            self._zero = lambda slot: ops.zero_places(places, slot)
+        if arrays and arrays[0].is_cuda:
+            from ..kernels import HipOps, get_ops
+            if dtype in HipOps.ELEMS:
+                ops = get_ops(dtype, str(arrays[0].device))
+                places = ops.places_of(arrays)
+
+                def zero(slot: int) -> None:
+                    with torch.cuda.device(arrays[0].device):  # (a request may be admitted by a thread whose device is another)
+                        ops.zero_places(places, slot)
+                self._zero = zero
         # the one-request view
         self.kpools = {i: t for (i, j), t in self._kpools.items() if not manager.layer_requests[i][0]}
         self.vpools = {i: t for (i, j), t in self._vpools.items() if not manager.layer_requests[i][0]}

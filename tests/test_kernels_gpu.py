@@ -1080,6 +1080,20 @@ def test_zeroing_a_place_of_several_arrays():
             ops.zero_places(places, place)
 
 
+@pytest.mark.parametrize("dtype", [torch.float64, torch.bfloat16])
+def test_zeroing_a_slot_of_a_cache(dtype):
+    """Whatever the cache's element type, one that has no kernels included: a slot's states in every layer are zeros, the others stay."""
+    from machserve_amd.cache import CacheManager, DeviceCache
+    from machserve_amd.parts.base import StateRequest
+    cache = DeviceCache(CacheManager([StateRequest({"s": (3, 5), "c": (7,)}), StateRequest({"s": (16, 4)})], 16, 8, 2), dtype, torch.device(DEV))
+    arrays = [t for layer in (0, 1) for t in cache.binding(layer).tensors.values()]
+    for t in arrays:
+        t.fill_(1)
+    cache.zero_state(1)
+    for t in arrays:
+        assert not bool(t[1].any()) and bool((t[[0, 2]] == 1).all())
+
+
 @pytest.mark.parametrize("d", [4, 896, 1024, 1028, 2048, 2052, 4096, 4100])
 @pytest.mark.parametrize("na,nb", [(1, 1), (2, 1), (3, 2), (8, 8), (9, 1)])
 def test_normed_branches_added_to_the_stream(d, na, nb):
