@@ -43,18 +43,19 @@ __global__ __launch_bounds__(256) void key_decay_kernel(Sums in, int col, const 
 // ---- gated linear attention over many rows ---------------------------------------------------------------------
 // A thread is a value channel and holds its column of S in registers (DP of them; the rows beyond d stay zero).  Tokens come
 // WALK_BATCH at a time through LDS; the next batch's numbers are asked for before the current batch is walked.  seg_len 0: a
-// block walks all of a request's rows.  Else a request of more than `whole` rows is cut into segments (the requests' first ones are the first S blocks, cut_segment has the
-// others): LOCAL walks each from zero and leaves what it adds (carry [places, H, d, dvp]) and the product of its decays (cdec [places, H, d]),
-// the carry kernel replaces what it adds by the state that comes into it, and the second walk makes the outputs.  A request of at most `whole` rows is
-// walked by one block all the same, whatever comes with it: a row takes 1.27 us of a walk (64 x 128), three kernels over segments 78 us and more (100 rows alone
+// block walks all of a request's rows.  Else, if any request has more than `least` rows, those of more than `whole` are cut into segments (the requests' first ones are the first S blocks,
+// cut_segment has the others): LOCAL walks each from zero and leaves what it adds (carry [places, H, d, dvp]) and the product of its decays (cdec [places, H, d]),
+// the carry kernel replaces what it adds by the state that comes into it, and the second walk makes the outputs.  The other requests are
+// walked by a block each in that launch, whatever comes with them: a row takes 1.27 us of a walk (64 x 128), three kernels over segments 78 us and more (100 rows alone
 // 132 us walked, 79 in segments of 32; 64 rows 87 and 78; 60 single rows beside a prompt of 2,000 2,477 and 150) and more than twice the rows' work, which counts where the step's rows fill the
-// chip as they are: `whole` goes by how many come (us, walked and in segments: 16 requests of 70 rows, 8 heads of 128 x 256, 222 and 280, 32 of 100 314 and 621; 64 of 128, 16 heads of
-// 64 x 128, 211 and 401, 16 of 200 258 and 187).
+// chip as they are: `least` goes by how many come (us, walked and in segments: 16 requests of 70 rows, 8 heads of 128 x 256, 222 and 280, 32 of 100 314 and 621; 64 of 128, 16 heads of
+// 64 x 128, 211 and 401, 16 of 200 258 and 187).  `whole` is less: beside one that is cut a walk stands behind the other two kernels (953 rows and 71, 16 heads of 64 x 128: the last launch
+// 109 us with the 71 walked whole, 58 in segments).
 // (The lengths are on the device: a step that may hold a request to be cut and holds none pays for two launches that find nothing, 4 us: 64 requests of 17 rows 44 and 48, of 2 rows 17.6 and 23.5.)
 constexpr int WALK_BATCH = 8;
 struct WalkArgs {
     StateArgs a;
-    int seg_len, whole;  // (whole >= seg_len)
+    int seg_len, whole, least;  // (seg_len <= whole <= least)
     float* carry;
     float* cdec;
 };
@@ -66,11 +67,33 @@ __device__ __forceinline__ int carry_base(const WalkArgs& w, int s) {
     return q0 / w.seg_len + min(q0 / w.whole, s);
 }
 
+// Whether a request of the step is long enough for requests to be cut; every wave looks for itself, 64 a step.
+__device__ __forceinline__ bool step_is_cut(const WalkArgs& w) {
+    for (int s0 = threadIdx.x % WAVE; s0 - (int)(threadIdx.x % WAVE) < w.a.S; s0 += WAVE)
+        if (__any(s0 < w.a.S && w.a.seq_q_len[s0] > w.least)) return true;
+    return false;
+}
+__device__ __forceinline__ bool is_whole(const WalkArgs& w, int len) { return len <= w.whole || (len <= w.least && !step_is_cut(w)); }
+
+// The requests that are cut, by number; behind the last S.
+__device__ __forceinline__ int cut_request(const WalkArgs& w, int number) {
+    if (!step_is_cut(w)) return w.a.S;
+    const int lane = threadIdx.x % WAVE;
+    for (int s0 = 0; s0 < w.a.S; s0 += WAVE) {
+        const bool cut = s0 + lane < w.a.S && w.a.seq_q_len[s0 + lane] > w.whole;
+        const uint64_t all = __ballot(cut), it = __ballot(cut && __popcll(all & ((1ull << lane) - 1)) == number);
+        if (it) return s0 + __builtin_ctzll(it);
+        number -= __popcll(all);
+    }
+    return w.a.S;
+}
+
 // Segments of the requests that are cut, by number without gaps, all but the one of each that LOCAL leaves out (the last: nobody needs what it passes on) or that has a block among the first
 // S (the first); requests behind the last number are S.  Every wave adds the requests up for itself, 64 a step.  Numbers with gaps, every request's own from its first row / L on, left the blocks that
 // walk unevenly over the chip's dies, which blocks go to in turn: 64 requests of 128 rows in segments (16 heads of 64 x 128) 504 us, now 401.
 template <bool LOCAL>
 __device__ __forceinline__ Piece cut_segment(const WalkArgs& w, int number) {
+    if (!step_is_cut(w)) return Piece{w.a.S, 0};
     const int lane = threadIdx.x % WAVE;
     int before = 0;
     for (int s0 = 0; s0 < w.a.S; s0 += WAVE) {
@@ -105,7 +128,7 @@ __global__ __launch_bounds__(NT) void state_walk_kernel(WalkArgs w) {
     if (pc.s >= a.S) return;  // the same for the whole block
     const int left = a.seq_q_len[pc.s] - pc.first;
     if (left <= 0) return;
-    const bool whole = w.seg_len == 0 || a.seq_q_len[pc.s] <= w.whole;
+    const bool whole = !LOCAL && (w.seg_len == 0 || (number < a.S && is_whole(w, left)));
     const int n = whole ? left : min(left, w.seg_len);
     const bool last = n == left;
     const int q0 = a.seq_q_start[pc.s] + pc.first, kh = h / (a.H / a.G);
@@ -260,8 +283,8 @@ __global__ __launch_bounds__(NT) void state_walk_kernel(WalkArgs w) {
 constexpr int CARRY_AHEAD = 8;
 __global__ __launch_bounds__(256) void state_carry_kernel(WalkArgs w) {
     const StateArgs& a = w.a;
-    const int s = blockIdx.x, h = blockIdx.y, idx = (blockIdx.z * 256 + threadIdx.x) * 4, head = a.d * a.dvp;
-    if (idx >= head || a.seq_q_len[s] <= w.whole) return;
+    const int s = cut_request(w, blockIdx.x), h = blockIdx.y, idx = (blockIdx.z * 256 + threadIdx.x) * 4, head = a.d * a.dvp;
+    if (s >= a.S || idx >= head) return;
     const int i = idx / a.dvp, base = carry_base(w, s);
     const int nseg = (a.seq_q_len[s] + w.seg_len - 1) / w.seg_len;
     f32x4 Sin = *reinterpret_cast<const f32x4*>(a.state + ((size_t)a.seq_slot[s] * a.H + h) * head + idx);
@@ -306,20 +329,20 @@ extern "C" int ms_key_decay(const float* in, int n_partials, int ld, int col, co
 }
 
 // Gated linear attention.  rows: float [n_partials, T, ld] with q [H, d], k [H, d], v [H, dv] and gate [H, dv] at their columns;
-// alpha float [T, H * d].  single: every request has one row.  seg_len > 0: requests of more than `whole` rows in segments side by side with carry
+// alpha float [T, H * d].  single: every request has one row.  seg_len > 0: requests of more than `whole` rows, if one has more than `least`, in segments side by side with carry
 // float [places, H, d, dvp] and cdec float [places, H, d] as workspace, places = T / seg_len + min(T / whole, S) (carry_base).
 extern "C" int ms_gated_linear(const float* rows, int n_partials, int ld, int q_col, int k_col, int v_col, int g_col, float q_scale,
                                const float* alpha, const float* norm, float eps, float* state, const int* seq_q_start, const int* seq_q_len,
                                const int* seq_slot, int S, void* out, int ld_out, int T, int H, int d, int dv, int dvp, int single,
-                               int seg_len, int whole, float* carry, float* cdec, hipStream_t stream) {
+                               int seg_len, int whole, int least, float* carry, float* cdec, hipStream_t stream) {
     const Sums in{rows, n_partials, (size_t)T * ld, ld};
     const StateArgs a{in, in, in, q_col, k_col, v_col, q_scale, alpha, nullptr, in, g_col, norm, eps, state, seq_q_start, seq_q_len, seq_slot, S,
                       (elem_t*)out, ld_out, T, H, H, d, dv, dvp};
     MS_REQUIRE(n_partials > 0, "gated linear: no rows");
     if (int rc = check_state(a, "gated linear")) return rc;
     if (single) return launch_step<false>(a, stream);
-    MS_REQUIRE(seg_len == 0 || (seg_len > 0 && whole >= seg_len && carry && cdec), "gated linear: segments of %d of requests above %d rows need their workspace", seg_len, whole);
-    const WalkArgs w{a, seg_len, whole, carry, cdec};
+    MS_REQUIRE(seg_len == 0 || (seg_len > 0 && whole >= seg_len && least >= whole && carry && cdec), "gated linear: segments of %d of requests above %d rows need their workspace", seg_len, whole);
+    const WalkArgs w{a, seg_len, whole, least, carry, cdec};
 #define MS_WALK(DP, NT, LOCAL, X) hipLaunchKernelGGL((state_walk_kernel<DP, NT, LOCAL>), dim3((unsigned)(X) * H), dim3(NT), 0, stream, w)
 #define MS_WALK_N(DP, LOCAL, X)                   \
     do {                                          \
@@ -341,7 +364,7 @@ extern "C" int ms_gated_linear(const float* rows, int n_partials, int ld, int q_
     const int cuts = T / seg_len;  // (a request of n rows has (n - 1) / seg_len of those that are numbered)
     MS_WALK_D(true, cuts);
     if (int rc = check_launch("gated linear, segments from zero")) return rc;
-    hipLaunchKernelGGL(state_carry_kernel, dim3(S, H, ceil_div(d * dvp, 1024)), dim3(256), 0, stream, w);
+    hipLaunchKernelGGL(state_carry_kernel, dim3(min(S, T / (whole + 1)), H, ceil_div(d * dvp, 1024)), dim3(256), 0, stream, w);
     if (int rc = check_launch("gated linear, states between segments")) return rc;
     MS_WALK_D(false, S + cuts);
 #undef MS_WALK_D

@@ -230,7 +230,8 @@ extern "C" int ms_latent_query(const float* q, const int* positions, const float
                                int T, int H, int d, int dp, int rot, int rank, int hd, int halves, hipStream_t stream) {
     MS_REQUIRE(T > 0 && H > 0 && d > 0 && dp >= d, "latent query: %d rows, %d heads, plain part %d in %d", T, H, d, dp);
     MS_REQUIRE(rot >= 0 && rot % 2 == 0 && rank + rot <= hd && (rot == 0 || inv_freq), "latent query: latent %d + rotated part %d in a key of %d", rank, rot, hd);
-    // (16 rows of 16 heads of 128 and 64: one block a row 6.9 us in a decode step, eight 3.5)
+    // (16 rows of 16 heads of 128 and 64: one block a row 6.9 us in a decode step, eight 3.5; warm, 1 to 128 rows 4.1 to 4.4 us and 2.5 to 2.8, 32 heads 6.3 to 6.9 and 2.8 to 3.2,
+    // 4 heads of 64 and 32, which fill one block, 2.2 to 2.5)
     const int blocks = T <= 128 ? min(8, ceil_div(H * dp, 256)) : 1;
     hipLaunchKernelGGL(latent_query_kernel, dim3(T, blocks), dim3(256), 0, stream, q, positions, inv_freq, cs_factor, (elem_t*)plain,
                        (elem_t*)att, H, d, dp, rot, rank, hd, halves);

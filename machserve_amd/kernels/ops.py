@@ -1674,17 +1674,20 @@ class HipOps:
 
     @classmethod
     def _state_segments(cls, T: int, S: int, floats_per_state: int, rows_at_once: float = 0.0) -> tuple:
-        """``(segment length, rows up to which a request is walked whole, places for the states between segments)`` for gated linear attention over
-        ``T`` rows of ``S`` requests, or zeros where no request can be long enough to be cut: one has at most ``T - S + 1`` rows.
+        """``(segment length, whole, least, places for the states between segments)`` for gated linear attention over ``T`` rows of ``S`` requests: requests of
+        more than ``whole`` rows are cut if any has more than ``least``; zeros where none can have, one has at most ``T - S + 1`` rows.
         ``rows_at_once``: what the step's rows, in segments, take a chip full of blocks, in rows of a block alone.  Segments cost that and some 45 rows, a walk is as
-        long as its rows: a request is cut where it has more."""
+        long as its rows: the step is cut where a request has more.  Beside one that is cut a walk counts against the second of the segments' two walks."""
         seg = cls.STATE_SEGMENT
-        while T - S >= (whole := max(cls.STATE_WHOLE, seg, 45 + int(rows_at_once))):
+        while True:
+            whole = max(cls.STATE_WHOLE, seg, int(0.6 * rows_at_once))
+            least = max(whole, 45 + int(rows_at_once))
+            if T - S < least:
+                return 0, 0, 0, 0
             n = T // seg + min(T // whole, S)
             if (n - 1) * floats_per_state * 4 <= cls.STATE_WORKSPACE:
-                return seg, whole, n
+                return seg, whole, least, n
             seg *= 2
-        return 0, 0, 0
 
     def gated_linear(self, sums: torch.Tensor, alpha: torch.Tensor, norm_w: torch.Tensor, eps: float, q_scale: float, state: torch.Tensor,
                      seq_q_start: torch.Tensor, seq_q_len: torch.Tensor, seq_slot: torch.Tensor, H: int, d: int, dv: int, out_cols: int,
@@ -1700,18 +1703,18 @@ class HipOps:
         if single and S != T:
             raise KernelError(f"gated linear: {T} rows of {S} requests are not single rows")
         out = torch.empty((T, out_cols), dtype=self.dtype, device=sums.device)
-        seg = whole = n = 0
+        seg = whole = least = n = 0
         carry = cdec = None
         if not single:  # a block is one, two or four waves; rows of a walk that a wave of rows a CU adds to segments: 0.12 (32 x 64, 12 x 20) and 0.15 (32 x 256), else 0.28 to 0.34
             waves = T * H * (1 if dv <= 64 else 2 if dv <= 128 else 4) / self._cus
-            seg, whole, n = self._state_segments(T, S, H * d * dvp, waves * (0.15 if d <= 32 else 0.3))
+            seg, whole, least, n = self._state_segments(T, S, H * d * dvp, waves * (0.15 if d <= 32 else 0.3))
         if seg:
             carry = torch.empty((n, H, d, dvp), dtype=torch.float32, device=sums.device)
             cdec = torch.empty((n, H, d), dtype=torch.float32, device=sums.device)
         self._check(lib, lib.ms_gated_linear(
             _ptr(sums), _c_int(P), _c_int(N), _c_int(0), _c_int(H * d), _c_int(2 * H * d), _c_int(2 * H * d + H * dv), _c_float(q_scale), _ptr(alpha),
             _ptr(norm_w), _c_float(eps), _ptr(state), _ptr(seq_q_start), _ptr(seq_q_len), _ptr(seq_slot), _c_int(S), _ptr(out), _c_int(out_cols),
-            _c_int(T), _c_int(H), _c_int(d), _c_int(dv), _c_int(dvp), _c_int(int(single)), _c_int(seg), _c_int(whole), _ptr(carry), _ptr(cdec), self._stream()))
+            _c_int(T), _c_int(H), _c_int(d), _c_int(dv), _c_int(dvp), _c_int(int(single)), _c_int(seg), _c_int(whole), _c_int(least), _ptr(carry), _ptr(cdec), self._stream()))
         return out
 
     def delta_rows(self, sums: torch.Tensor, conv_w: torch.Tensor, conv_state: Optional[torch.Tensor], a_log: torch.Tensor, dt_bias: torch.Tensor,

@@ -315,13 +315,14 @@ def test_places_of_the_states_between_segments():
     for trial in range(400):
         lengths = [rng.choice((1, 1, 1, 0, 17, 63, 64, 65, 96, 127, 128, 129, 300, rng.randint(1, 2000))) for _ in range(rng.randint(1, 40))]
         T, S, state, at_once = sum(lengths), len(lengths), rng.choice((100, 1 << 17, 1 << 20, 1 << 22)), rng.choice((0.0, 20.0, 50.0, 300.0))
-        seg, whole, n = HipOps._state_segments(T, S, state, at_once) if T else (0, 0, 0)
+        seg, whole, least, n = HipOps._state_segments(T, S, state, at_once) if T else (0, 0, 0, 0)
         if not seg:
             assert all(length <= max(64, 45 + int(at_once)) for length in lengths) or state > 100 or 0 in lengths
             continue
-        assert (n - 1) * state * 4 <= HipOps.STATE_WORKSPACE and whole >= max(64, seg)
+        assert (n - 1) * state * 4 <= HipOps.STATE_WORKSPACE and least >= whole >= max(64, seg)
         starts, used = [sum(lengths[:i]) for i in range(S)], set()
-        own = [(length - 1) // seg if length > whole else 0 for length in lengths]
+        cut = [length > whole and max(lengths) > least for length in lengths]
+        own = [(length - 1) // seg if c else 0 for c, length in zip(cut, lengths)]
         assert sum(own) <= T // seg, "a block for each numbered segment"
         for local in (True, False):
             walked = {(s, 0) for s in range(S) if not local}
@@ -330,7 +331,7 @@ def test_places_of_the_states_between_segments():
                 walked.add((s, number - sum(own[:s]) + (0 if local else 1)))
             assert walked == {(s, k) for s in range(S) for k in range(own[s] + (0 if local else 1))}
         for s, length in enumerate(lengths):
-            if length > whole:
+            if cut[s]:
                 assert own[s] + 1 == -(-length // seg)
                 for k in range(own[s] + 1):
                     place = starts[s] // seg + min(starts[s] // whole, s) + k

@@ -115,10 +115,11 @@ def test_gated_linear_attention_beside_many_rows(dtype):
     ops, ref = ops_of(dtype), EmulatedOps(dtype)
     torch.manual_seed(5)
     H, d, dv = 16, 10, 130
-    for lengths in ([100] * 3 + [86, 87, 88, 89, 300] + [1] * 80 + [64, 33], [40] * 30 + [0, 130, 290] + [3] * 100 + [600]):
+    for lengths, cut in (([100] * 3 + [63, 64, 65, 66, 300] + [1] * 80 + [64, 33], True), ([40] * 30 + [0, 130, 290] + [3] * 100 + [600], True),
+                         ([108] * 15 + [1] * 70, False), ([109] * 15 + [1] * 70, True)):
         T, S, cols, dvp = sum(lengths), len(lengths), H * dv, 132
-        _, whole, _ = ops._state_segments(T, S, H * d * dvp, T * H * 4 / ops._cus * 0.15)
-        assert whole > 64 and max(lengths) > whole and any(64 < n <= whole for n in lengths)
+        _, whole, least, _ = ops._state_segments(T, S, H * d * dvp, T * H * 4 / ops._cus * 0.15)
+        assert least > whole and (max(lengths) > least) == cut and max(lengths) > whole
         sums = torch.randn(1, T, 2 * H * (d + dv)) * 0.7
         alpha, norm = torch.sigmoid(torch.randn(T, H * d) + 3.0), torch.rand(dv) + 0.5
         seqs = sequences(lengths, list(range(S))[::-1])
