@@ -716,8 +716,10 @@ extern "C" int ms_route(const void* x, const float* w, const float* bias, float*
     // four rows (2,048 rows of 768 columns over 9 outputs, one of four, 5.8 and 6.1); and one of eight, in one round, where two rows share a CU (300 rows:
     // 1,792 columns over 64 outputs, one of eight, 17.5 and 15.5; 1,536 over 9, two, 5.4 and 5.7; 3,584 over 9, two of sixteen, 7.2 and 7.6).  With more than two rows a CU
     // the blocks beside each other hide the loads, and the registers count (1,000 rows over 64 outputs: 1,280 columns 18.4 and 27, 2,048 columns 26.4 and 27.8).
+    // An output a wave of four rows has fewer loads a step, of which the loop asks for four: two are enough up to 1,536 columns (2,048 rows over 2 outputs 4.8 and 4.4; one output of 4,096,
+    // 1,024 rows 4.9 and 5.3), and with a column a load nowhere (one output of 3,001 6.6 and 8.6, 128 in 32-bit 137 and 147).
     const int steps = ceil_div(d, 64 * 4), most = many || steps <= 2 ? 2 : steps <= 4 ? 4 : 8, surplus = ceil_div(steps, most) * most - steps;
-    const bool straight = many                     ? surplus == 0
+    const bool straight = many                     ? surplus == 0 && (!one || steps <= 6)
                           : T <= compute_units()     ? surplus * 4 <= steps + surplus
                           : T <= 2 * compute_units() ? surplus * 8 <= most && steps <= 8
                                                      : false;
@@ -733,9 +735,9 @@ extern "C" int ms_route(const void* x, const float* w, const float* bias, float*
     } while (0)
     if (one && fours) MS_ROUTE_FOURS(1);
     else if (fours) MS_ROUTE_FOURS(3);
-    else if (one && many) MS_ROUTE(4, 1, 1, 2);
+    else if (one && many) MS_ROUTE(4, 1, 1, 1);
     else if (one) MS_ROUTE(1, 1, 1, 1);
-    else if (many) MS_ROUTE(4, 1, 3, 2);
+    else if (many) MS_ROUTE(4, 1, 3, 1);
     else MS_ROUTE(1, 1, 3, 1);
 #undef MS_ROUTE_FOURS
 #undef MS_ROUTE
