@@ -12,6 +12,12 @@
 // a load, which the CU's load path takes a quarter as fast as whole lines.  us at 8 rows, cold weights, few-rows / tiled / here: 5,632 x 2,048 with an
 // activation 11.8 / 13.1 / 7.5; 11,264 x 2,048 gated 22.4 / 14.1 / 12.4; 9,728 x 896 gated 9.1 / 7.4 / 6.3; 37,888 x 3,584 gated 72 / 62 / 52;
 // 2,048 x 5,632 in slices 11.3 / 8.4 / 6.9; 896 x 4,864 in slices 5.5 / 6.5 / 4.2; 151,936 x 896 69 / 60 / 54.
+//
+// `past`: the weight's loads are non-temporal ones, which leave nothing in the memory-side cache of 256 MB.  What comes from memory comes a tenth faster so, as the
+// loads alone, cold, us without and with: 37,888 x 3,584 49.9 and 44.8 (6.1 TB/s), 3,584 x 18,944 in four slices 23.8 and 21.3, 152,064 x 896 44.6 and 40.4, 9,728 x 896
+// 5.2 and 4.8; and weights that are read through the cache stay in it, if they fit.  A weight that would still be there from the step before is read slower so (11,264 x 2,048:
+// 8.2 and 9.4), so the weights are marked by what all of a model's come to (engine/loading.py).  Sixteen requests of the 7B sizes, 16 steps and their prompts, 70.0 -> 65.7 ms;
+// one of the 0.5B sizes 11.78 -> 10.98.
 #pragma once
 #include "gemm_tile.cuh"
 
@@ -53,9 +59,15 @@ __device__ __forceinline__ void few_rows_tile(const elem_t* __restrict__ A, cons
     auto ask = [&](int i, int stage) {  // this wave's step i
         const size_t k = (size_t)i * (64 * KW);
         const uint32_t to = own + stage * STEP;
+        if (ep.past) {
 #pragma unroll
-        for (int l = 0; l < 2 * NT; ++l)
-            asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(ow[l]), "s"(base_w + k), "s"(to + l * 1024) : "memory", "m0");
+            for (int l = 0; l < 2 * NT; ++l)
+                asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 nt" ::"v"(ow[l]), "s"(base_w + k), "s"(to + l * 1024) : "memory", "m0");
+        } else {
+#pragma unroll
+            for (int l = 0; l < 2 * NT; ++l)
+                asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(ow[l]), "s"(base_w + k), "s"(to + l * 1024) : "memory", "m0");
+        }
 #pragma unroll
         for (int l = 0; l < 2 * MT; ++l) {
             if constexpr (Rows::GATHERS)

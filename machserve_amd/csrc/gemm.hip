@@ -16,6 +16,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_kernel(const elem_t* __rest
                                                    int M, int N, int K, EpiArgs ep) {
     arguments_now(A, W, M, N, K, ep.out, ep.bias, ep.ldo, ep.n_out, ep.k_per_split, ep.split_stride);
     if constexpr (SCALED) arguments_now(ep.row_ss, ep.ss_parts, ep.ss_eps);
+    if constexpr (STAGES == 4 && BM == 64) arguments_now(ep.past);
     const int tiles_m = ceil_div(M, BM);
     int tile = blockIdx.x;
     // Blocks go to the eight dies in turn, each die with an L2 of its own.  With a multiple of eight row tiles a die gets the same rows under
@@ -64,7 +65,7 @@ static GemmPlan plan_gemm(int M, int N, int K, int splits, bool store32, bool ga
 }
 template <int MT, int NT, int STAGES, int EPI, bool SCALED>
 __global__ __launch_bounds__(64 * FEW_WAVES) void gemm_few_kernel(const elem_t* __restrict__ A, const elem_t* __restrict__ W, int M, int N, int K, EpiArgs ep) {
-    arguments_now(A, W, M, N, K, ep.out, ep.bias, ep.ldo, ep.n_out, ep.k_per_split, ep.split_stride);
+    arguments_now(A, W, M, N, K, ep.out, ep.bias, ep.ldo, ep.n_out, ep.k_per_split, ep.split_stride, ep.past);
     if constexpr (SCALED) arguments_now(ep.row_ss, ep.ss_parts, ep.ss_eps);
     if constexpr (EPI == EPI_PRENORM) arguments_now(ep.norm_w, ep.hn, ep.ss_part);
     few_rows_tile<MT, NT, FEW_WAVES, STAGES, EPI, SCALED>(A, W, M, N, K, ep, 0, blockIdx.x * 16 * NT, blockIdx.y, NoExperts{});
@@ -363,35 +364,68 @@ static int plan_tiled_splits(int M, int N, int K) {
 
 using namespace ms;
 
+// Each product has two entry points: `..._past` reads the weight of up to 64 rows past the last-level cache where few_rows.cuh or 64x64 tiles with four
+// buffers serve it (see few_rows.cuh); the sums are the same.
+
 // out[M, N] = a[M, K] w[N, K]^T (+ bias[N]); out is float when out_f32 != 0, else the element type.
-extern "C" int ms_linear(const void* a, const void* w, const float* bias, void* out, int out_f32, int M, int N, int K,
-                         hipStream_t stream) {
+static int linear(const void* a, const void* w, const float* bias, void* out, int out_f32, int M, int N, int K,
+                         hipStream_t stream, bool past) {
     EpiArgs ep{out, bias, N, N, 0, 0};
+    ep.past = past && M <= 64;
     if (out_f32) return launch_gemm<EPI_STORE_F32>((const elem_t*)a, (const elem_t*)w, M, N, K, ep, stream);
     return launch_gemm<EPI_STORE_ELEM>((const elem_t*)a, (const elem_t*)w, M, N, K, ep, stream);
 }
+extern "C" int ms_linear(const void* a, const void* w, const float* bias, void* out, int out_f32, int M, int N, int K,
+                         hipStream_t stream) {
+    return linear(a, w, bias, out, out_f32, M, N, K, stream, false);
+}
+extern "C" int ms_linear_past(const void* a, const void* w, const float* bias, void* out, int out_f32, int M, int N, int K,
+                         hipStream_t stream) {
+    return linear(a, w, bias, out, out_f32, M, N, K, stream, true);
+}
 
 // x[M, N] += a[M, K] w[N, K]^T, x being the 32-bit residual stream.
-extern "C" int ms_linear_residual(const void* a, const void* w, float* x, int M, int N, int K, hipStream_t stream) {
+static int linear_residual(const void* a, const void* w, float* x, int M, int N, int K, hipStream_t stream, bool past) {
     EpiArgs ep{x, nullptr, N, N, 0, 0};
+    ep.past = past && M <= 64;
     return launch_gemm<EPI_RESIDUAL>((const elem_t*)a, (const elem_t*)w, M, N, K, ep, stream);
+}
+extern "C" int ms_linear_residual(const void* a, const void* w, float* x, int M, int N, int K, hipStream_t stream) {
+    return linear_residual(a, w, x, M, N, K, stream, false);
+}
+extern "C" int ms_linear_residual_past(const void* a, const void* w, float* x, int M, int N, int K, hipStream_t stream) {
+    return linear_residual(a, w, x, M, N, K, stream, true);
 }
 
 // out[M, I] = act(a g^T) * (a u^T) where w holds gate and up rows interleaved in blocks of 16:
 // rows [32 t, 32 t + 16) are gate rows [16 t, 16 t + 16), rows [32 t + 16, 32 t + 32) the same
 // up rows; w has 2 * ceil16(I) rows, the padding rows being zero.
-extern "C" int ms_linear_swiglu(const void* a, const void* w, void* out, int M, int I, int K, int act, hipStream_t stream) {
+static int linear_swiglu(const void* a, const void* w, void* out, int M, int I, int K, int act, hipStream_t stream, bool past) {
     MS_REQUIRE(act >= 0 && act < ACT_COUNT, "gated product: no activation %d", act);
     const int n = 2 * ceil_div(I, 16) * 16;
     EpiArgs ep{out, nullptr, I, I, 0, 0, nullptr, 0, 0.f, act};
+    ep.past = past && M <= 64;
     return launch_gemm<EPI_SWIGLU>((const elem_t*)a, (const elem_t*)w, M, n, K, ep, stream);
+}
+extern "C" int ms_linear_swiglu(const void* a, const void* w, void* out, int M, int I, int K, int act, hipStream_t stream) {
+    return linear_swiglu(a, w, out, M, I, K, act, stream, false);
+}
+extern "C" int ms_linear_swiglu_past(const void* a, const void* w, void* out, int M, int I, int K, int act, hipStream_t stream) {
+    return linear_swiglu(a, w, out, M, I, K, act, stream, true);
 }
 
 // out[M, N] = act(a[M, K] w[N, K]^T) in the element type, the activation (UnaryActivation) in the product's epilogue.
-extern "C" int ms_linear_act(const void* a, const void* w, void* out, int M, int N, int K, int act, hipStream_t stream) {
+static int linear_act(const void* a, const void* w, void* out, int M, int N, int K, int act, hipStream_t stream, bool past) {
     MS_REQUIRE(act >= 0 && act < UNARY_COUNT, "product with an activation: no activation %d", act);
     EpiArgs ep{out, nullptr, N, N, 0, 0, nullptr, 0, 0.f, act};
+    ep.past = past && M <= 64;
     return launch_gemm<EPI_ACT>((const elem_t*)a, (const elem_t*)w, M, N, K, ep, stream);
+}
+extern "C" int ms_linear_act(const void* a, const void* w, void* out, int M, int N, int K, int act, hipStream_t stream) {
+    return linear_act(a, w, out, M, N, K, act, stream, false);
+}
+extern "C" int ms_linear_act_past(const void* a, const void* w, void* out, int M, int N, int K, int act, hipStream_t stream) {
+    return linear_act(a, w, out, M, N, K, act, stream, true);
 }
 
 // Whether ms_linear_swiglu_scaled takes this shape: bfloat16, whole K steps of 64.
@@ -424,8 +458,8 @@ extern "C" int ms_swiglu_scaled_pays(int M, int I, int K) {
 
 // ms_linear_swiglu for rows that came in multiplied by a norm's weight only: both products of a row are
 // divided by the row's root mean square, 1 / sqrt(sum_p row_ss[p, row] / K + eps), before the activation.
-extern "C" int ms_linear_swiglu_scaled(const void* a, const float* row_ss, int ss_parts, float eps, const void* w, void* out, int M, int I,
-                                       int K, int act, hipStream_t stream) {
+static int linear_swiglu_scaled(const void* a, const float* row_ss, int ss_parts, float eps, const void* w, void* out, int M, int I,
+                                       int K, int act, hipStream_t stream, bool past) {
 #ifdef MS_ELEM_HALF
     MS_REQUIRE(act >= 0 && act < ACT_COUNT, "gated product: no activation %d", act);
     MS_REQUIRE(ms_swiglu_scaled_takes(M, I, K), "gated product with row factors: M=%d K=%d is not taken", M, K);
@@ -433,6 +467,7 @@ extern "C" int ms_linear_swiglu_scaled(const void* a, const float* row_ss, int s
     MS_REQUIRE((reinterpret_cast<uintptr_t>(a) & 15) == 0 && (reinterpret_cast<uintptr_t>(w) & 15) == 0, "gemm: operands must be 16-byte aligned");
     const int n = 2 * ceil_div(I, 16) * 16;
     EpiArgs ep{out, nullptr, I, I, K, 0, row_ss, ss_parts, eps, act};
+    ep.past = past && M <= 64;
     if (planned(M, K)) {
         if constexpr (kRoundsBeforeTheNormIsSafe) return launch_around_norm<EPI_SWIGLU, true>((const elem_t*)a, (const elem_t*)w, M, n, K, ep, stream);
     }
@@ -444,6 +479,14 @@ extern "C" int ms_linear_swiglu_scaled(const void* a, const float* row_ss, int s
     (void)a; (void)row_ss; (void)ss_parts; (void)eps; (void)w; (void)out; (void)M; (void)I; (void)K; (void)act; (void)stream;
     MS_REQUIRE(false, "gated product with row factors: built for bfloat16 only");
 #endif
+}
+extern "C" int ms_linear_swiglu_scaled(const void* a, const float* row_ss, int ss_parts, float eps, const void* w, void* out, int M, int I,
+                                       int K, int act, hipStream_t stream) {
+    return linear_swiglu_scaled(a, row_ss, ss_parts, eps, w, out, M, I, K, act, stream, false);
+}
+extern "C" int ms_linear_swiglu_scaled_past(const void* a, const float* row_ss, int ss_parts, float eps, const void* w, void* out, int M, int I,
+                                       int K, int act, hipStream_t stream) {
+    return linear_swiglu_scaled(a, row_ss, ss_parts, eps, w, out, M, I, K, act, stream, true);
 }
 
 // Column tiles of ms_linear_residual_prenorm for this shape (the first size of its ss_part), or 0 if it is not taken: up to 16 rows over whole K steps,
@@ -463,13 +506,14 @@ extern "C" int ms_prenorm_parts(int M, int N, int K) {
 
 // x[M, N] += a w^T, and beside it hn[M, N] = x * norm_w in the element type and ss_part[parts, M], whose sum over parts is the rows' sums of
 // squares of x (parts = ms_prenorm_parts).
-extern "C" int ms_linear_residual_prenorm(const void* a, const void* w, float* x, const float* norm_w, void* hn, float* ss_part, int M, int N, int K,
-                                          hipStream_t stream) {
+static int linear_residual_prenorm(const void* a, const void* w, float* x, const float* norm_w, void* hn, float* ss_part, int M, int N, int K,
+                                          hipStream_t stream, bool past) {
 #ifdef MS_ELEM_HALF
     MS_REQUIRE(ms_prenorm_parts(M, N, K) > 0, "product that prepares the norm: M=%d N=%d K=%d is not taken", M, N, K);
     MS_REQUIRE(norm_w && hn && ss_part, "product that prepares the norm: its outputs are missing");
     MS_REQUIRE((reinterpret_cast<uintptr_t>(a) & 15) == 0 && (reinterpret_cast<uintptr_t>(w) & 15) == 0, "gemm: operands must be 16-byte aligned");
     EpiArgs ep{x, nullptr, N, N, K, 0};
+    ep.past = past && M <= 64;
     ep.norm_w = norm_w;
     ep.hn = (elem_t*)hn;
     ep.ss_part = ss_part;
@@ -481,6 +525,14 @@ extern "C" int ms_linear_residual_prenorm(const void* a, const void* w, float* x
     (void)a; (void)w; (void)x; (void)norm_w; (void)hn; (void)ss_part; (void)M; (void)N; (void)K; (void)stream;
     MS_REQUIRE(false, "product that prepares the norm: built for bfloat16 only");
 #endif
+}
+extern "C" int ms_linear_residual_prenorm(const void* a, const void* w, float* x, const float* norm_w, void* hn, float* ss_part, int M, int N, int K,
+                                          hipStream_t stream) {
+    return linear_residual_prenorm(a, w, x, norm_w, hn, ss_part, M, N, K, stream, false);
+}
+extern "C" int ms_linear_residual_prenorm_past(const void* a, const void* w, float* x, const float* norm_w, void* hn, float* ss_part, int M, int N, int K,
+                                          hipStream_t stream) {
+    return linear_residual_prenorm(a, w, x, norm_w, hn, ss_part, M, N, K, stream, true);
 }
 
 // Whether ms_linear_qkv_rope takes this shape: two-byte elements, more rows than the few-rows kernels take, heads of
@@ -648,15 +700,29 @@ extern "C" int ms_residual_partials(int M, int N, int K) {
 }
 
 // out[slices, M, N] (float) = partial sums of a w^T over that many slices of K.
-extern "C" int ms_linear_slices(const void* a, const void* w, float* out, int M, int N, int K, int slices, hipStream_t stream) {
+static int linear_slices(const void* a, const void* w, float* out, int M, int N, int K, int slices, hipStream_t stream, bool past) {
     EpiArgs ep{out, nullptr, N, N, 0, 0};
+    ep.past = past && M <= 64;
     return launch_gemm<EPI_STORE_F32>((const elem_t*)a, (const elem_t*)w, M, N, K, ep, stream, slices);
+}
+extern "C" int ms_linear_slices(const void* a, const void* w, float* out, int M, int N, int K, int slices, hipStream_t stream) {
+    return linear_slices(a, w, out, M, N, K, slices, stream, false);
+}
+extern "C" int ms_linear_slices_past(const void* a, const void* w, float* out, int M, int N, int K, int slices, hipStream_t stream) {
+    return linear_slices(a, w, out, M, N, K, slices, stream, true);
 }
 
 // out[ks, M, N] (float) = partial sums of a w^T over ms_tiled_partials(M, N, K) slices of K.
-extern "C" int ms_linear_split_tiled(const void* a, const void* w, float* out, int M, int N, int K, hipStream_t stream) {
+static int linear_split_tiled(const void* a, const void* w, float* out, int M, int N, int K, hipStream_t stream, bool past) {
     EpiArgs ep{out, nullptr, N, N, 0, 0};
+    ep.past = past && M <= 64;
     return launch_gemm<EPI_STORE_F32>((const elem_t*)a, (const elem_t*)w, M, N, K, ep, stream, plan_tiled_splits(M, N, K));
+}
+extern "C" int ms_linear_split_tiled(const void* a, const void* w, float* out, int M, int N, int K, hipStream_t stream) {
+    return linear_split_tiled(a, w, out, M, N, K, stream, false);
+}
+extern "C" int ms_linear_split_tiled_past(const void* a, const void* w, float* out, int M, int N, int K, hipStream_t stream) {
+    return linear_split_tiled(a, w, out, M, N, K, stream, true);
 }
 
 // Measurements only: force one tile configuration (0 = choose by shape).

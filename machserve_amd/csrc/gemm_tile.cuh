@@ -73,6 +73,7 @@ struct EpiArgs {
     const float* norm_w;  // [N]
     elem_t* hn;           // [M, N]
     float* ss_part;       // [N / 16, or the columns of a wave, rounded up, M]
+    int past = 0;         // W is read past the last-level cache (see few_rows.cuh): up to 64 rows, where every block reads its own columns of it
 };
 
 // The block of rows m0 .. m0 + BM and columns n0 .. n0 + BN.  `rows` says which row of A the block's row i is and, for the
@@ -224,7 +225,9 @@ __device__ __forceinline__ void gemm_tile(const elem_t* __restrict__ A, const el
             const int i = l - A_CHUNKS;
             const uint32_t to = lds_w + buf * (BN * LDS_LD * (int)sizeof(elem_t)) + (i * (NT / 8) + swave * 8) * (LDS_LD * (int)sizeof(elem_t));
             const elem_t* from = WIDE ? W + (size_t)min(n0 + i * (NT / 8) + swave * 8, N - 8) * rows.w_pitch(K) : base_w;
-            asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(ow[WIDE ? 0 : i]), "s"(from + k0), "s"(to) : "memory", "m0");
+            if (STAGES == 4 && BM == 64 && ep.past)
+                asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 nt" ::"v"(ow[WIDE ? 0 : i]), "s"(from + k0), "s"(to) : "memory", "m0");
+            else asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(ow[WIDE ? 0 : i]), "s"(from + k0), "s"(to) : "memory", "m0");
         }
     };
     auto load_direct = [&](int k0, int buf) {

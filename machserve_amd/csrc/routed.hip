@@ -373,6 +373,7 @@ struct ExpertArgs {
     int ff, shared;       // columns of an expert, and of the one that every row uses (0: there is none)
     int width;            // of the rows
     int shared_gate, weigh_input, act;
+    int past;             // the weights are read past the last-level cache (few_rows.cuh); up to 32 rows
 };
 
 __global__ __launch_bounds__(1024) void expert_rows_kernel(const int* __restrict__ plane, int* __restrict__ rows, int* __restrict__ counts, int T, int E) {
@@ -565,6 +566,7 @@ __global__ __launch_bounds__(64 * FEW_WAVES) void expert_few_kernel(const elem_t
     __syncthreads();
     EpiArgs ep{out, nullptr, DOWN ? g.width : max(g.ff, g.shared), DOWN ? g.width : cols, K, 0};
     ep.k_per_split = K;
+    ep.past = g.past;
     const ExpertRows<!DOWN> rows{g, shared ? nullptr : few, e, shared ? g.routed_slots : tile * g.T, of_row};
     const elem_t* own = W + (size_t)e * g.ff * (DOWN ? 1 : PER * g.width);  // its columns, or its rows
     few_rows_tile<MT, NT, FEW_WAVES, STAGES, EPI, false>(A, own, count, N, K, ep, 0, n0, 0, rows);
@@ -785,20 +787,38 @@ extern "C" int ms_expert_rows(const int* plane, int* rows, int* counts, int T, i
 
 // x [T, width]; w: the experts' matrices one behind the other and then that of the expert every row uses (`shared` columns, 0: none), each
 // [cols, width], or with `gated` [2 cols, width] with gate and up rows interleaved in blocks of 16; out [slots, max(ff, shared)].
-extern "C" int ms_experts_up(const void* x, const void* w, void* out, const int* plane, const float* gates, const int* rows, const int* counts,
+static int experts_up(const void* x, const void* w, void* out, const int* plane, const float* gates, const int* rows, const int* counts,
                              int T, int E, int ld_gates, int top, int ff, int shared, int width, int gated, int shared_gate, int weigh_input,
-                             int act, hipStream_t stream) {
-    const ExpertArgs g{plane, gates, rows, counts, T, E, ld_gates, top, 0, 0, 0, ff, shared, width, shared_gate, weigh_input, act};
+                             int act, hipStream_t stream, int past) {
+    const ExpertArgs g{plane, gates, rows, counts, T, E, ld_gates, top, 0, 0, 0, ff, shared, width, shared_gate, weigh_input, act, past};
     if (int rc = check_experts("experts up", g)) return rc;
     MS_REQUIRE(!weigh_input || gated, "experts up: weights inside experts that are not gated");
     return gated ? launch_experts<EPI_EXPERT_GATED>(x, w, out, g, stream) : launch_experts<EPI_EXPERT_PLAIN>(x, w, out, g, stream);
 }
+extern "C" int ms_experts_up(const void* x, const void* w, void* out, const int* plane, const float* gates, const int* rows, const int* counts,
+                             int T, int E, int ld_gates, int top, int ff, int shared, int width, int gated, int shared_gate, int weigh_input,
+                             int act, hipStream_t stream) {
+    return experts_up(x, w, out, plane, gates, rows, counts, T, E, ld_gates, top, ff, shared, width, gated, shared_gate, weigh_input, act, stream, 0);
+}
+extern "C" int ms_experts_up_past(const void* x, const void* w, void* out, const int* plane, const float* gates, const int* rows, const int* counts,
+                             int T, int E, int ld_gates, int top, int ff, int shared, int width, int gated, int shared_gate, int weigh_input,
+                             int act, hipStream_t stream) {
+    return experts_up(x, w, out, plane, gates, rows, counts, T, E, ld_gates, top, ff, shared, width, gated, shared_gate, weigh_input, act, stream, 1);
+}
 
 // a [slots, max(ff, shared)] as ms_experts_up leaves it; w [width, E * ff + shared]: the experts' down matrices side by side,
 // then the shared one's; sums [top (+ 1), T, width]: plane k of row t is the k-th expert that it uses, the last plane the shared one's.
-extern "C" int ms_experts_down(const void* a, const void* w, float* sums, const int* plane, const float* gates, const int* rows, const int* counts,
-                               int T, int E, int ld_gates, int top, int ff, int shared, int width, hipStream_t stream) {
-    const ExpertArgs g{plane, gates, rows, counts, T, E, ld_gates, top, 0, 0, 0, ff, shared, width, 0, 0, 0};
+static int experts_down(const void* a, const void* w, float* sums, const int* plane, const float* gates, const int* rows, const int* counts,
+                               int T, int E, int ld_gates, int top, int ff, int shared, int width, hipStream_t stream, int past) {
+    const ExpertArgs g{plane, gates, rows, counts, T, E, ld_gates, top, 0, 0, 0, ff, shared, width, 0, 0, 0, past};
     if (int rc = check_experts("experts down", g)) return rc;
     return launch_experts<EPI_EXPERT_DOWN>(a, w, sums, g, stream);
+}
+extern "C" int ms_experts_down(const void* a, const void* w, float* sums, const int* plane, const float* gates, const int* rows, const int* counts,
+                               int T, int E, int ld_gates, int top, int ff, int shared, int width, hipStream_t stream) {
+    return experts_down(a, w, sums, plane, gates, rows, counts, T, E, ld_gates, top, ff, shared, width, stream, 0);
+}
+extern "C" int ms_experts_down_past(const void* a, const void* w, float* sums, const int* plane, const float* gates, const int* rows, const int* counts,
+                               int T, int E, int ld_gates, int top, int ff, int shared, int width, hipStream_t stream) {
+    return experts_down(a, w, sums, plane, gates, rows, counts, T, E, ld_gates, top, ff, shared, width, stream, 1);
 }

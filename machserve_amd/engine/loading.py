@@ -37,6 +37,40 @@ class LoadedModel:
     rt: Runtime
 
 
+# The memory-side cache (256 MB) that every read from memory goes through.  A decode step reads all weights one after the other: what fits in it
+# is still there a step later, and of more than it holds nothing is, because whatever comes later pushes out what came before.  So
+# where the weights are more, the largest are read past it (the loads' non-temporal form, which leaves nothing there) and the smallest, up to this much, stay.
+# A chain of products of eight rows, us each, through the cache and past it: 9,728 x 896 in 60 to 240 MB of weights 4.45 and 4.8 to 5.1, 300 MB 5.04 and 4.82,
+# 400 to 2,000 MB 5.26 to 5.48 and 4.84; 11,264 x 2,048 8.2 and 9.4, 9.3 and 9.4, 10.4 and 9.5.
+CACHED_WEIGHT_BYTES = 192 << 20
+
+
+def mark_weights_past_cache(model: DecoderModel, kept: int = CACHED_WEIGHT_BYTES) -> int:
+    """Marks the weights that steps of few rows read past the last-level cache (``past_cache`` on the tensor): none if all of them
+    fit in ``kept`` bytes, else the largest, so that the others do.  Returns how many bytes are marked.  The mark changes the
+    kind of load and no result; a view of a weight does not carry it."""
+    found = {}
+    again = {id(p) for i, b in enumerate(model.blocks) if model.order.count(i) > 1 for q in b.parts() for p in (q, *getattr(q, "sub_parts", lambda: [])())}
+    for part in model.parts():
+        if part is model.embedding and getattr(model.head, "weight", None) is not None:
+            continue  # rows of a table: not read as a whole
+        if id(part) in again:
+            continue  # a layer that a step runs more than once finds its weights in the cache
+        for value in vars(part).values():
+            for t in value if isinstance(value, (list, tuple)) else (value,):
+                if isinstance(t, torch.Tensor) and t.dim() >= 2 and t.dtype == model.rt.dtype:
+                    found[t.data_ptr()] = t
+    weights = sorted(found.values(), key=lambda t: t.numel())
+    sizes = [t.numel() * t.element_size() for t in weights]
+    fits = sum(sizes) <= kept
+    marked = room = 0
+    for t, size in zip(weights, sizes):
+        t.past_cache = not fits and room + size > kept
+        room += 0 if t.past_cache else size
+        marked += size if t.past_cache else 0
+    return marked
+
+
 def load_model(model_dir: Optional[str] = None, *, dtype="bfloat16", device: str = "cuda:0", page_size: int = 64,
                num_pages=None, max_tokens: Optional[int] = None, max_requests: int = 64,
                config=None, tensors=None, ops=None, use_graphs: bool = True, portion: Optional[int] = None) -> LoadedModel:
@@ -54,6 +88,7 @@ def load_model(model_dir: Optional[str] = None, *, dtype="bfloat16", device: str
     model = DecoderModel(config.to_spec(), rt)
     source = TensorDict(tensors) if tensors is not None else Checkpoint(model_dir)
     load_weights(model, source, rt)
+    mark_weights_past_cache(model)
     if num_pages is None:
         if max_tokens is None:
             max_tokens = 4096

@@ -320,6 +320,11 @@ class HipOps:
         (M, K), N = a.shape, w.shape[0]
         return (self._few(M, N, K, slices, pairs) and self._aligned(a, w)) or self._tiled(M, N, K)
 
+    def _reading(self, lib, name: str, w: torch.Tensor):
+        """The entry point ``name``, or the one that reads few rows' weights past the last-level cache if ``w`` is marked so
+        (``past_cache``, see ``engine/loading.py``)."""
+        return getattr(lib, name + "_past" if getattr(w, "past_cache", False) else name)
+
     def linear_split(self, a: torch.Tensor, w: torch.Tensor, allow_partials: bool = True) -> torch.Tensor:
         """Float32 ``[P, M, N]`` whose sum over P is ``a @ w.T``.  The cut of K depends on N and K only in
         the weight-streaming kernels and, up to 32 rows, in those whose waves share K, so the consumer
@@ -332,8 +337,8 @@ class HipOps:
             if P == 1:
                 return self.linear(a, w, None, out_f32=True).unsqueeze(0)
             out = torch.empty((P, M, N), dtype=torch.float32, device=a.device)
-            self._check(self._core, self._core.ms_linear_split_tiled(_ptr(a), _ptr(w), _ptr(out), _c_int(M), _c_int(N),
-                                                                     _c_int(K), self._stream()))
+            fn = self._reading(self._core, "ms_linear_split_tiled", w)
+            self._check(self._core, fn(_ptr(a), _ptr(w), _ptr(out), _c_int(M), _c_int(N), _c_int(K), self._stream()))
             return out
         P = self._plan("ms_skinny_partials", M, N, K, int(allow_partials))
         out = torch.empty((P, M, N), dtype=torch.float32, device=a.device)
@@ -350,8 +355,8 @@ class HipOps:
         if bias is not None:
             self._want(bias, torch.float32, "linear bias", N)
         out = torch.empty((M, N), dtype=torch.float32 if out_f32 else self.dtype, device=a.device)
-        self._check(self._core, self._core.ms_linear(_ptr(a), _ptr(w), _ptr(bias), _ptr(out), _c_int(int(out_f32)),
-                                                     _c_int(M), _c_int(N), _c_int(K), self._stream()))
+        fn = self._reading(self._core, "ms_linear", w)
+        self._check(self._core, fn(_ptr(a), _ptr(w), _ptr(bias), _ptr(out), _c_int(int(out_f32)), _c_int(M), _c_int(N), _c_int(K), self._stream()))
         return out
 
     def linear_residual(self, a: torch.Tensor, w: torch.Tensor, x: torch.Tensor) -> Optional[torch.Tensor]:
@@ -372,10 +377,11 @@ class HipOps:
         P = self._plan("ms_residual_partials", M, N, K)
         if P > 1:
             out = torch.empty((P, M, N), dtype=torch.float32, device=a.device)
-            self._check(self._core, self._core.ms_linear_slices(_ptr(a), _ptr(w), _ptr(out), _c_int(M), _c_int(N), _c_int(K), _c_int(P), self._stream()))
+            fn = self._reading(self._core, "ms_linear_slices", w)
+            self._check(self._core, fn(_ptr(a), _ptr(w), _ptr(out), _c_int(M), _c_int(N), _c_int(K), _c_int(P), self._stream()))
             return out
-        self._check(self._core, self._core.ms_linear_residual(_ptr(a), _ptr(w), _ptr(x), _c_int(M), _c_int(N), _c_int(K),
-                                                              self._stream()))
+        fn = self._reading(self._core, "ms_linear_residual", w)
+        self._check(self._core, fn(_ptr(a), _ptr(w), _ptr(x), _c_int(M), _c_int(N), _c_int(K), self._stream()))
         return None
 
     def prenorm_swiglu_takes(self, M: int, N: int, K: int, n_gate_up: int) -> bool:
@@ -393,7 +399,7 @@ class HipOps:
         M, N, K = self._mm_operands(a, w, "linear_residual_prenorm")
         self._want(x, torch.float32, "residual stream", M, N)
         self._want(norm_w, torch.float32, "norm weight", N)
-        parts, fn = self._plan("ms_prenorm_parts", M, N, K) if self._aligned(a, w) else 0, self._core.ms_linear_residual_prenorm
+        parts, fn = self._plan("ms_prenorm_parts", M, N, K) if self._aligned(a, w) else 0, self._reading(self._core, "ms_linear_residual_prenorm", w)
         if parts < 1:
             parts, fn = self._plan("ms_skinny_prenorm_parts", M, N, K), self._core.ms_linear_residual_prenorm_skinny
         if parts < 1:
@@ -415,7 +421,7 @@ class HipOps:
         out = torch.empty((M, intermediate), dtype=self.dtype, device=hn.device)
         few_rows = self._few(M, N, K, False, True) and self._aligned(hn, w_gate_up)
         skinny = not few_rows and bool(self._plan("ms_swiglu_scaled_skinny_takes", M, intermediate, K))
-        fn = self._core.ms_linear_swiglu_scaled_skinny if skinny else self._core.ms_linear_swiglu_scaled
+        fn = self._core.ms_linear_swiglu_scaled_skinny if skinny else self._reading(self._core, "ms_linear_swiglu_scaled", w_gate_up)
         self._check(self._core, fn(_ptr(hn), _ptr(row_ss), _c_int(row_ss.shape[0]), _c_float(eps), _ptr(w_gate_up), _ptr(out),
                                    _c_int(M), _c_int(intermediate), _c_int(K), _c_int(act), self._stream()))
         return out
@@ -429,7 +435,7 @@ class HipOps:
         if N != 2 * ((intermediate + 15) // 16) * 16:
             raise KernelError(f"linear_swiglu: interleaved weight has {N} rows for intermediate size {intermediate}")
         out = torch.empty((M, intermediate), dtype=self.dtype, device=a.device)
-        fn = self._core.ms_linear_swiglu if self._through_tiles(a, w_gate_up, False, True) else self._core.ms_linear_swiglu_skinny
+        fn = self._reading(self._core, "ms_linear_swiglu", w_gate_up) if self._through_tiles(a, w_gate_up, False, True) else self._core.ms_linear_swiglu_skinny
         self._check(self._core, fn(_ptr(a), _ptr(w_gate_up), _ptr(out), _c_int(M), _c_int(intermediate), _c_int(K),
                                    _c_int(act), self._stream()))
         return out
@@ -440,7 +446,7 @@ class HipOps:
             raise KernelError(f"linear_act: activation {activation!r} is not built (built: {', '.join(sorted(UNARY_ACTIVATIONS))})")
         M, N, K = self._mm_operands(a, w, "linear_act")
         out = torch.empty((M, N), dtype=self.dtype, device=a.device)
-        fn = self._core.ms_linear_act if self._through_tiles(a, w, False) else self._core.ms_linear_act_skinny
+        fn = self._reading(self._core, "ms_linear_act", w) if self._through_tiles(a, w, False) else self._core.ms_linear_act_skinny
         self._check(self._core, fn(_ptr(a), _ptr(w), _ptr(out), _c_int(M), _c_int(N), _c_int(K), _c_int(UNARY_ACTIVATIONS[activation]),
                                    self._stream()))
         return out
@@ -1457,9 +1463,9 @@ class HipOps:
             self._check(lib, lib.ms_expert_rows(_ptr(plane), _ptr(rows), _ptr(counts), _c_int(T), _c_int(experts), self._stream()))
         a = new((self._plan("ms_experts_slots", T, experts, top, shared, lib=lib), max(ff, shared)), self.dtype)
         sizes = [_ptr(plane), _ptr(gates), _ptr(rows), _ptr(counts)] + [_c_int(v) for v in (T, experts, gates.shape[1], top, ff, shared, d)]
-        self._check(lib, lib.ms_experts_up(_ptr(h), _ptr(w_up), _ptr(a), *sizes, _c_int(int(gated)), _c_int(int(shared_gate)),
+        self._check(lib, self._reading(lib, "ms_experts_up", w_up)(_ptr(h), _ptr(w_up), _ptr(a), *sizes, _c_int(int(gated)), _c_int(int(shared_gate)),
                                            _c_int(int(weigh_input)), _c_int(self.EXPERT_ACTIVATIONS[activation]), self._stream()))
-        self._check(lib, lib.ms_experts_down(_ptr(a), _ptr(w_down), _ptr(sums), *sizes, self._stream()))
+        self._check(lib, self._reading(lib, "ms_experts_down", w_down)(_ptr(a), _ptr(w_down), _ptr(sums), *sizes, self._stream()))
         return sums, gates
 
     def expert_act(self, up: torch.Tensor, gates: torch.Tensor, ff: int, activation: str, experts: Optional[int] = None,
