@@ -11,25 +11,51 @@
 
 namespace ms {
 
+// The order of the tiles.  Blocks go to the eight dies in turn, each die with an L2 of its own, and what a die's blocks read beside one another goes over the
+// fabric once: so a die takes a run of the order in which `group` row tiles stand under every column in turn, K slice by K slice, and what it has in
+// work is nearly a square.  What bounds the tiles' loops is this traffic: W comes from memory, at 23 bytes a clock into a CU whatever is asked for ahead, from
+// the last-level cache at 40, and what the die has already read at 53.  us before (by turns or a run of whole columns, every slice in every die)
+// and so, cold W: 2,048 x 3,584 x 18,944 in two slices 195 -> 182, 3,001 x 11,264 x 2,048 108 -> 101, 2,048 x 2,048 x 5,632 in two 41.6 -> 40.1, 512 x 9,728 x 896
+// (64x64) 23.4 -> 20.9; W in the last-level cache: 181 -> 173, 99 -> 98, 37.8 -> 36.0, 22.6 -> 14.6.
+struct TilePlace {
+    int m, n, split;
+};
+// x / d by a reciprocal: a whole division is twenty instructions one behind the other, four of them 1 us ahead of a block's first load.  With x + 1/2 the quotient is
+// no nearer to a whole number than 1 / 2d, and wrong by 2^-22 of itself.
+__device__ __forceinline__ int quotient(int x, int d) {
+    if (x >= 1 << 20) return x / d;
+    return __builtin_amdgcn_readfirstlane((int)(((float)x + 0.5f) * __builtin_amdgcn_rcpf((float)d)));
+}
+__device__ __forceinline__ TilePlace tile_of_block(int tiles_m, int group) {
+    const int tiles = gridDim.x, all = tiles * gridDim.y, id = blockIdx.x + tiles * blockIdx.y;
+    const int per = all / 8, rest = all % 8, die = id % 8;
+    int at = die * per + min(die, rest) + id / 8, split = 0;
+    if (gridDim.y > 1) {
+        split = quotient(at, tiles);
+        at -= split * tiles;
+    }
+    const int band = group * quotient(tiles, tiles_m), g = quotient(at, band), in = at - g * band, rows = min(group, tiles_m - g * group), n = quotient(in, rows);
+    return {g * group + in - n * rows, n, split};
+}
+
 template <int BM, int BN, int WM, int WN, int BK, int EPI, int STAGES = 2, bool SCALED = false>
 __global__ __launch_bounds__(64 * WM * WN) void gemm_kernel(const elem_t* __restrict__ A, const elem_t* __restrict__ W,
                                                    int M, int N, int K, EpiArgs ep) {
-    arguments_now(A, W, M, N, K, ep.out, ep.bias, ep.ldo, ep.n_out, ep.k_per_split, ep.split_stride);
+    arguments_now(A, W, M, N, K, ep.out, ep.bias, ep.ldo, ep.n_out, ep.k_per_split, ep.split_stride, ep.group);
     if constexpr (SCALED) arguments_now(ep.row_ss, ep.ss_parts, ep.ss_eps);
     if constexpr (STAGES == 4 && BM == 64) arguments_now(ep.past);
     const int tiles_m = ceil_div(M, BM);
-    int tile = blockIdx.x;
-    // Blocks go to the eight dies in turn, each die with an L2 of its own.  With a multiple of eight row tiles a die gets the same rows under
-    // every column, and all of W; a contiguous run of the order instead gives it all rows under its own columns.  What
-    // the dies read together is the smaller this way where W has more rows than A (and where the row tiles are no multiple of eight a
-    // die would read everything): 2,048 x 37,888 x 3,584 470 -> 453 us, 1,040 rows 289 -> 272; 2,048 x 2,048 x 5,632 the other
-    // way round, 45.7 against 43.7.  (Tiles of 128 rows are taken where W is small beside them.)
-    if (STAGES == GEMM_PIPED && (tiles_m % 8 != 0 || (BM == 256 && N > 2 * M))) {
-        const int per = gridDim.x / 8, rest = gridDim.x % 8, die = tile % 8;
-        tile = die * per + min(die, rest) + tile / 8;
-    }
-    const int tm = tile % tiles_m, tn = tile / tiles_m;
-    gemm_tile<BM, BN, WM, WN, BK, EPI, STAGES, SCALED>(A, W, M, N, K, ep, tm * BM, tn * BN, blockIdx.y, NoExperts{});
+    // (64x64 tiles with four buffers are few, and gain nothing by it: 2,048 x 64 x 2,048 12.0 us by turns, 13.1 so)
+    constexpr bool BY_TURNS = kHalf && STAGES == 4 && EPI != EPI_QKV_ROPE;
+    const TilePlace at = BY_TURNS || tiles_m == 1 ? TilePlace{(int)blockIdx.x % tiles_m, (int)blockIdx.x / tiles_m, (int)blockIdx.y} : tile_of_block(tiles_m, ep.group);
+    gemm_tile<BM, BN, WM, WN, BK, EPI, STAGES, SCALED>(A, W, M, N, K, ep, at.m * BM, at.n * BN, at.split, NoExperts{});
+}
+
+// Row tiles side by side (see tile_of_block): the power of two nearest to what makes the rows and the columns that a die has in work, of which it holds `per_cu`
+// tiles a CU, equally many.
+static int row_group(int bm, int bn, int per_cu, long blocks) {
+    const double run = (double)min(ceil_div(blocks, 8L), (long)max(1, compute_units() / 8) * per_cu);
+    return 1 << max(0, (int)lround(0.5 * log2(run * bn / bm)));
 }
 
 #ifdef MS_MEASURE  // switches for measurements, in no library that serves
@@ -154,6 +180,7 @@ static int launch_gemm(const elem_t* A, const elem_t* W, int M, int N, int K, Ep
 #define MS_GEMM_DEEP(BM_, BN_, WM_, WN_, BK_, ST_)                                                                         \
     do {                                                                                                                  \
         const long nb = (long)ceil_div(M, BM_) * ceil_div(N, BN_);                                                        \
+        ep.group = row_group(BM_, BN_, BM_ >= 256 ? 1 : BM_ == 128 ? 2 : 4, nb * ns);                                     \
         hipLaunchKernelGGL((gemm_kernel<BM_, BN_, WM_, WN_, BK_, EPI, ST_>), dim3((unsigned)nb, ns), dim3(64 * WM_ * WN_), 0, stream, \
                            A, W, M, N, K, ep);                                                                            \
         return check_launch("gemm " #BM_ "x" #BN_ "x" #BK_ " deep");                                                      \
@@ -161,6 +188,7 @@ static int launch_gemm(const elem_t* A, const elem_t* W, int M, int N, int K, Ep
 #define MS_GEMM(BM_, BN_, WM_, WN_, BK_)                                                                              \
     do {                                                                                                              \
         const long nb = (long)ceil_div(M, BM_) * ceil_div(N, BN_);                                                    \
+        ep.group = row_group(BM_, BN_, BM_ >= 256 ? 1 : BM_ == 128 ? 2 : 4, nb * ns);                                 \
         hipLaunchKernelGGL((gemm_kernel<BM_, BN_, WM_, WN_, BK_, EPI>), dim3((unsigned)nb, ns), dim3(64 * WM_ * WN_), 0, stream, \
                            A, W, M, N, K, ep);                                                                        \
         return check_launch("gemm " #BM_ "x" #BN_ "x" #BK_);                                                          \
@@ -268,6 +296,7 @@ static int launch_around_norm(const elem_t* A, const elem_t* W, int M, int N, in
     ep.k_per_split = K;
 #define MS_AROUND(BM_, BN_, WM_, WN_, ST_)                                                                                                                 \
     do {                                                                                                                                                   \
+        ep.group = row_group(BM_, BN_, BM_ >= 256 ? 1 : BM_ == 128 ? 2 : 4, (long)ceil_div(M, BM_) * ceil_div(N, BN_));                                    \
         hipLaunchKernelGGL((gemm_kernel<BM_, BN_, WM_, WN_, 64, EPI, ST_, SCALED>), dim3((unsigned)((long)ceil_div(M, BM_) * ceil_div(N, BN_)), 1),       \
                            dim3(64 * WM_ * WN_), 0, stream, A, W, M, N, K, ep);                                                                            \
         return check_launch("gemm around a norm, " #BM_ "x" #BN_);                                                                                         \
@@ -571,6 +600,7 @@ extern "C" int ms_linear_qkv_rope(const void* a, const void* w, const float* bia
 #define MS_QKV(BM_, BN_)                                                                                                 \
     do {                                                                                                                 \
         const long nb = (long)ceil_div(M, BM_) * (N / BN_);                                                              \
+        ep.group = row_group(BM_, BN_, BM_ == 128 ? 2 : 4, nb);                                                          \
         hipLaunchKernelGGL((gemm_kernel<BM_, BN_, 4, 1, 64, EPI_QKV_ROPE>), dim3((unsigned)nb, 1), dim3(256), 0, stream, \
                            (const elem_t*)a, (const elem_t*)w, M, N, K, ep);                                             \
         return check_launch("gemm q/k/v with rotation " #BM_ "x" #BN_);                                                  \
@@ -583,6 +613,7 @@ extern "C" int ms_linear_qkv_rope(const void* a, const void* w, const float* bia
         // 128x64 take 20.3 (288 blocks, barely one a CU, each step a trip to the L2); four buffers where the blocks are
         // at most two a CU (512 to 1,536 rows: 10.6 -> 10.0, 11.8 -> 11.4 us; at 2,048 rows 13.4 -> 17.9)
         const long nb = (long)ceil_div(M, 64) * (N / 64);
+        ep.group = row_group(64, 64, 4, nb);
         if (nb <= round_blocks) {
             hipLaunchKernelGGL((gemm_kernel<64, 64, 4, 1, 64, EPI_QKV_ROPE, 4>), dim3((unsigned)nb, 1), dim3(256), 0, stream,
                                (const elem_t*)a, (const elem_t*)w, M, N, K, ep);
