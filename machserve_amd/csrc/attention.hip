@@ -97,7 +97,31 @@ struct AttnArgs {
     float softcap;
     // tiles of 32 rows: the reference of a row's exponentials follows its maximum when that has risen by more (in powers of two)
     float rise;
+    // what the kernels behind this one will read from memory (weights), in units of 16 bytes: blocks from `n_blocks` on bring it into the last-level cache
+    int n_blocks;
+    uint32_t n_ahead[2];
+    const u32x4* ahead[2];
 };
+
+// A block beside the attention's own: its share of the bytes that are read ahead.  An attention over a prompt is bound by its instructions and leaves the memory idle, and
+// products in tiles whose weights are in the last-level cache take less of a layer than with weights from memory (the loads of cold weights bound
+// their loops): 2,048 rows, us, 896 x 4,864 in slices 26.6 and 20.5, 9,728 x 896 gated 36.8 and 32.5, 1,536 x 8,960 80 and 58, 2,048 x 2,048 22.8 and 18.6.
+__device__ __forceinline__ void read_ahead(const AttnArgs& a, int block, int blocks) {
+    constexpr uint32_t AT_ONCE = 16;
+    u32x4 seen = {0u, 0u, 0u, 0u};
+#pragma unroll
+    for (int r = 0; r < 2; ++r) {
+        const uint32_t n = a.n_ahead[r], turn = blockDim.x * AT_ONCE;
+        for (uint32_t at = (uint32_t)block * turn + threadIdx.x; at < n; at += (uint32_t)blocks * turn) {
+            u32x4 v[AT_ONCE];
+#pragma unroll
+            for (uint32_t u = 0; u < AT_ONCE; ++u) v[u] = a.ahead[r][min(at + u * blockDim.x, n - 1)];
+#pragma unroll
+            for (uint32_t u = 0; u < AT_ONCE; ++u) seen ^= v[u];
+        }
+    }
+    asm volatile("" ::"v"(seen));
+}
 
 // The first key a row at `pos` sees under a window and a chunked mask (either 0: none).
 __device__ __forceinline__ int first_visible_key(int pos, int window, int chunk) {
@@ -153,6 +177,10 @@ template <int KG> constexpr int attention_waves_per_simd() { return 1; }
 
 template <int KG>
 __global__ __launch_bounds__(256 * KG, attention_waves_per_simd<KG>()) void paged_attention_kernel(AttnArgs a) {
+    if (a.n_blocks > 0 && (int)blockIdx.x >= a.n_blocks) {
+        if (blockIdx.y == 0) read_ahead(a, blockIdx.x - a.n_blocks, gridDim.x - a.n_blocks);
+        return;
+    }
     constexpr int KS_ELEMS = BKV * K_LD, VS_ELEMS = HDT * V_LD;
     constexpr int STAGE_BYTES = (KS_ELEMS + VS_ELEMS) * (int)sizeof(elem_t);
     constexpr int MERGE_FLOATS = 4 * 64 * (4 * ND + 2);  // per group: four waves, per lane the output and (max, sum)
@@ -636,6 +664,10 @@ __device__ __forceinline__ int v_swizzle(int d) { return ((d >> 2) & 1) | (((d >
 // ONE_PAGE: the page size is a multiple of a tile's 32 keys
 template <bool ONE_PAGE>
 __global__ __launch_bounds__(r32::KG * r32::GT, r32::KG * r32::RW * r32::PER_CU / 4) void paged_attention_rows32_kernel(AttnArgs a) {
+    if (a.n_blocks > 0 && (int)blockIdx.x >= a.n_blocks) {
+        if (blockIdx.y == 0) read_ahead(a, blockIdx.x - a.n_blocks, gridDim.x - a.n_blocks);
+        return;
+    }
     using namespace r32;
     static_assert((HDT == 64 || HDT == 128) && TK == 32 && RW == 2 && NS == 2, "the swizzles, the tiles' split over a group's waves and the rounds are written for these shapes");
     __shared__ __attribute__((aligned(1024))) unsigned char smem[SMEM];
@@ -1632,11 +1664,26 @@ extern "C" int MS_CAT(ms_attention_splits_nd, MS_ATTN_ND)(int n_work, int KV, in
 // float [T, H] that the output of each (row, head) is multiplied by.
 // `chunk`, `softcap`: see AttnArgs (0: none).  What a row can reach back (`reach`: the window, the chunk, or the smaller of
 // both) is what the choice of the kernel and of its key groups goes by.
-extern "C" int MS_CAT(ms_paged_attention_mask_nd, MS_ATTN_ND)(
+// How many blocks read `bytes` ahead beside the `blocks` of a kernel of which the chip holds `places`: those that fill the CUs up to equally many, which cost
+// the attention nothing, or if they are too few to be done in its time a block more on every CU; none where the attention is more than a round.  us of an attention over
+// 2,048 tokens (14 over 2 heads of 64, 452 blocks) that reads 26 MB ahead, by blocks beside: none 25.1, 16 40.6, 32 24.8, 48 24.9, 60 25.2, 64 28.6, 96 27.3, 128 26.9, 316 26.7.
+// ms with 32 MB ahead at most and without, 0.5B: 100 tokens 1.14 and 1.20, 400 1.53 and 1.62, 700 1.69 and 1.81, 1,000 2.06 and 2.06, 2,048 3.01 and 3.15; 1.5B: 200
+// tokens 2.31 and 2.48, 500 3.02 and 3.06, 2,000 7.20 and 7.20.
+static int blocks_ahead(long bytes, long blocks, long places, int threads) {
+    constexpr long LEAST = 48, MOST = 256;
+    if (bytes < 16) return 0;
+    const long cus = attention_compute_units();
+    long n = ceil_div(blocks, cus) * cus - blocks;
+    if (n < LEAST) n += cus;
+    return (int)std::max(0L, std::min({n, places - blocks, MOST, ceil_div(bytes, (long)threads * 256)}));
+}
+
+extern "C" int MS_CAT(ms_paged_attention_ahead_nd, MS_ATTN_ND)(
     const void* q, const void* kpool, const void* vpool, void* out, const int* block_table, int table_stride,
     const int* seq_q_start, const int* seq_q_len, const int* seq_pos0, const int* work, int n_work, int H, int KV,
     int hd, int ps, int n_pages, int window_of_mask, float scale, int max_key_groups, int T, int nsplit, float* part_o,
-    float* part_ml, const float* sinks, const float* out_gate, int chunk, float softcap, hipStream_t stream) {
+    float* part_ml, const float* sinks, const float* out_gate, int chunk, float softcap, const void* ahead0, long bytes0, const void* ahead1,
+    long bytes1, hipStream_t stream) {
     MS_REQUIRE(n_work > 0, "attention: no work");
     MS_REQUIRE(chunk >= 0 && softcap >= 0.f && (softcap == 0.f || scale != 0.f), "attention: chunk %d, score cap %g", chunk, (double)softcap);
     const int window = window_of_mask > 0 && chunk > 0 ? (window_of_mask < chunk ? window_of_mask : chunk) : (window_of_mask > 0 ? window_of_mask : chunk);
@@ -1650,6 +1697,11 @@ extern "C" int MS_CAT(ms_paged_attention_mask_nd, MS_ATTN_ND)(
     AttnArgs a{(const elem_t*)q, (const elem_t*)kpool, (const elem_t*)vpool, (elem_t*)out, block_table, seq_q_start,
                seq_q_len, seq_pos0, work, table_stride, H, KV, hd, ps, window_of_mask, scale, n_work, 0, nsplit, part_o, part_ml, sinks, out_gate,
                chunk, softcap};
+    MS_REQUIRE(bytes0 >= 0 && bytes1 >= 0 && bytes0 < 1L << 35 && bytes1 < 1L << 35 && (bytes0 < 16 || ahead0) && (bytes1 < 16 || ahead1) &&
+                   ((reinterpret_cast<uintptr_t>(ahead0) | reinterpret_cast<uintptr_t>(ahead1)) & 15) == 0,
+               "attention: what is read ahead must begin at 16 bytes");
+    a.ahead[0] = (const u32x4*)ahead0, a.ahead[1] = (const u32x4*)ahead1;
+    a.n_ahead[0] = (uint32_t)(bytes0 / 16), a.n_ahead[1] = (uint32_t)(bytes1 / 16);
     // key groups per block by the longest context the block tables allow (the lengths themselves
     // are on the device): short contexts have no chain worth cutting
     const long span = window > 0 ? (long)window + BKV : (long)table_stride * ps;
@@ -1661,7 +1713,7 @@ extern "C" int MS_CAT(ms_paged_attention_mask_nd, MS_ATTN_ND)(
         groups = 1;
     }
     MS_REQUIRE((long)n_work * KV * SUB_BLOCKS < 2147483647L, "attention: %d blocks of rows times %d key/value heads", n_work, KV);
-    const dim3 grid((unsigned)(n_work * KV * SUB_BLOCKS), (unsigned)nsplit);
+    dim3 grid((unsigned)(n_work * KV * SUB_BLOCKS), (unsigned)nsplit);
     // how many blocks of each variant a CU holds, and how many CUs there are: asked once
     static int cus = 0, resident[4] = {0, 0, 0, 0};
     if (cus == 0) {
@@ -1682,7 +1734,10 @@ extern "C" int MS_CAT(ms_paged_attention_mask_nd, MS_ATTN_ND)(
         if (takes_rows32(hd, ps, table_stride, window, max_key_groups)) {
             a.pair_span = r32::PER_CU == 2 ? std::max(cus / (KV * r32::SUB), 1) : 0;
             a.rise = HDT == 64 && span >= 2048 ? 6.0f : 0.0f;  // see the kernel
-            const dim3 grid32((unsigned)(n_work * KV * r32::SUB), (unsigned)nsplit);
+            const long own = (long)n_work * KV * r32::SUB;
+            const int beside = blocks_ahead(bytes0 + bytes1, own * nsplit, (long)cus * r32::PER_CU, r32::KG * r32::GT);
+            if (beside > 0) a.n_blocks = (int)own;
+            const dim3 grid32((unsigned)(own + beside), (unsigned)nsplit);
             if (ps % r32::TK == 0) hipLaunchKernelGGL(paged_attention_rows32_kernel<true>, grid32, dim3(r32::KG * r32::GT), 0, stream, a);
             else hipLaunchKernelGGL(paged_attention_rows32_kernel<false>, grid32, dim3(r32::KG * r32::GT), 0, stream, a);
             int rc32 = check_launch("paged_attention (32-row tiles)");
@@ -1692,6 +1747,11 @@ extern "C" int MS_CAT(ms_paged_attention_mask_nd, MS_ATTN_ND)(
         }
     }
 #endif
+    const int variant = groups >= 4 && MAX_KEY_GROUPS >= 4 ? 2 : groups >= 2 ? 1 : 0;
+    if (const int beside = blocks_ahead(bytes0 + bytes1, (long)grid.x * nsplit, (long)cus * resident[variant], 256 << variant)) {
+        a.n_blocks = (int)grid.x;
+        grid.x += (unsigned)beside;
+    }
     if (groups >= 4 && MAX_KEY_GROUPS >= 4) {
         // sixteen waves leave each 128 registers, which only the small bfloat16 tiles fit into
         a.pair_span = span_for(2);
@@ -1707,6 +1767,17 @@ extern "C" int MS_CAT(ms_paged_attention_mask_nd, MS_ATTN_ND)(
     if (rc || nsplit == 1) return rc;
     hipLaunchKernelGGL(decode_merge_kernel, dim3((unsigned)((size_t)T * H)), dim3(64), 0, stream, part_o, part_ml, (elem_t*)out, hd, nsplit, a.sinks, H, a.out_gate);
     return check_launch("attention_merge");
+}
+
+extern "C" int MS_CAT(ms_paged_attention_mask_nd, MS_ATTN_ND)(
+    const void* q, const void* kpool, const void* vpool, void* out, const int* block_table, int table_stride,
+    const int* seq_q_start, const int* seq_q_len, const int* seq_pos0, const int* work, int n_work, int H, int KV,
+    int hd, int ps, int n_pages, int window, float scale, int max_key_groups, int T, int nsplit, float* part_o,
+    float* part_ml, const float* sinks, const float* out_gate, int chunk, float softcap, hipStream_t stream) {
+    return MS_CAT(ms_paged_attention_ahead_nd, MS_ATTN_ND)(q, kpool, vpool, out, block_table, table_stride, seq_q_start, seq_q_len,
+                                                             seq_pos0, work, n_work, H, KV, hd, ps, n_pages, window, scale,
+                                                             max_key_groups, T, nsplit, part_o, part_ml, sinks, out_gate, chunk, softcap,
+                                                             nullptr, 0, nullptr, 0, stream);
 }
 
 extern "C" int MS_CAT(ms_paged_attention_ex_nd, MS_ATTN_ND)(

@@ -11,6 +11,7 @@ from ..cache import CacheManager, DeviceCache, pages_by_need
 from ..config import load_config
 from ..kernels import get_ops
 from ..parts import DecoderModel, Runtime
+from ..parts.base import Mixer
 from ..weights import Checkpoint, TensorDict, load_weights
 from .step import StepFunction
 
@@ -71,6 +72,20 @@ def mark_weights_past_cache(model: DecoderModel, kept: int = CACHED_WEIGHT_BYTES
     return marked
 
 
+def mark_weights_ahead(model: DecoderModel) -> None:
+    """Tells the mixers which weights come behind their attention: the matrices of the block's feed-forward, the smallest first (a long K under a
+    narrow output gains most by it).  Only where the weights do not all stay in the last-level cache anyway."""
+    if not hasattr(model.rt.ops, "AHEAD_BYTES"):
+        return
+    for block in model.blocks:
+        part = getattr(block, "feed_forward", None)
+        found = [t for t in vars(part).values() if isinstance(t, torch.Tensor) and t.dim() == 2 and t.dtype == model.rt.dtype] if part is not None else []
+        for mixer in block.mixers():
+            for m in (mixer, *getattr(mixer, "sub_parts", lambda: [])()):
+                if isinstance(m, Mixer):
+                    m.ahead = tuple(sorted(found, key=lambda t: t.numel())[:2])
+
+
 def load_model(model_dir: Optional[str] = None, *, dtype="bfloat16", device: str = "cuda:0", page_size: int = 64,
                num_pages=None, max_tokens: Optional[int] = None, max_requests: int = 64,
                config=None, tensors=None, ops=None, use_graphs: bool = True, portion: Optional[int] = None) -> LoadedModel:
@@ -88,7 +103,8 @@ def load_model(model_dir: Optional[str] = None, *, dtype="bfloat16", device: str
     model = DecoderModel(config.to_spec(), rt)
     source = TensorDict(tensors) if tensors is not None else Checkpoint(model_dir)
     load_weights(model, source, rt)
-    mark_weights_past_cache(model)
+    if mark_weights_past_cache(model) > 0:
+        mark_weights_ahead(model)
     if num_pages is None:
         if max_tokens is None:
             max_tokens = 4096

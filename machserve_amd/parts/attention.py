@@ -93,7 +93,7 @@ class Attention(Mixer):
                 q = ops.linear_qkv_rope(h.tensor() if isinstance(h, PendingNorm) else h, self.w_qkv, self.b_qkv, ctx.shared[key],
                                         view.slot_map, self.kpool, self.vpool, s.heads, s.kv_heads, s.head_dim, view.page_size)
                 o = ops.paged_attention(q, self.kpool, self.vpool, view.block_table, ctx.seq_q_start, ctx.seq_q_len, ctx.seq_pos0,
-                                        ctx.attention_work[g], s.heads, s.kv_heads, s.head_dim, view.page_size, s.window, self.scale)
+                                        ctx.attention_work[g], s.heads, s.kv_heads, s.head_dim, view.page_size, s.window, self.scale, **self.reading_ahead())
                 stream.add_linear(o, self.w_o)
                 return
         # [P, T, nq (+ 2 nkv)] partial sums, bias not yet added
@@ -127,5 +127,5 @@ class Attention(Mixer):
         else:
             o = ops.paged_attention(q, self.kpool, self.vpool, view.block_table, ctx.seq_q_start, ctx.seq_q_len,
                                     ctx.seq_pos0, ctx.attention_work[g], s.heads, s.kv_heads, s.head_dim, view.page_size,
-                                    s.window, self.scale)
+                                    s.window, self.scale, **self.reading_ahead())
         stream.add_linear(o, self.w_o)

@@ -341,6 +341,13 @@ class PositionEncoding(Part):
 class Mixer(Part):
     """Mixes information between positions of one request (attention, or a recurrence)."""
 
+    # weights that are read behind the mixer's attention, which that may bring into the last-level cache (``engine/loading.py`` sets them)
+    ahead: tuple = ()
+
+    def reading_ahead(self) -> dict:
+        """The argument of ``ops.paged_attention`` that says so."""
+        return {"ahead": self.ahead} if self.ahead else {}
+
     def cache_request(self):
         """PagedKVRequest, SharedKVRequest, StateRequest, None, or a list of these (pages and state together,
         or several caches of different widths)."""

@@ -142,5 +142,5 @@ class ChunkedAttention(Mixer):
         else:
             o = ops.paged_attention(q, self.kpool, self.vpool, view.block_table, ctx.seq_q_start, ctx.seq_q_len, ctx.seq_pos0,
                                     ctx.attention_work[g], s.heads, s.kv_heads, self.hd, view.page_size, s.window, float(s.scale),
-                                    sinks=self.sinks, out_gate=gate, chunk=chunk, softcap=cap)
+                                    sinks=self.sinks, out_gate=gate, chunk=chunk, softcap=cap, **self.reading_ahead())
         stream.add_linear(o, self.w_o)

@@ -91,5 +91,5 @@ class ConvAttention(Mixer):
         else:
             o = ops.paged_attention(q, self.kpool, self.vpool, view.block_table, ctx.seq_q_start, ctx.seq_q_len, ctx.seq_pos0,
                                     ctx.attention_work[g], s.heads, s.kv_heads, self.hd, view.page_size, None, float(s.scale),
-                                    sinks=None, out_gate=gate)
+                                    sinks=None, out_gate=gate, **self.reading_ahead())
         stream.add_linear(o, self.w_o)

@@ -140,7 +140,7 @@ class DiffAttention(Mixer):
                                      view.page_size, None, float(s.scale))
         else:
             o = ops.paged_attention(q, self.kpool, self.vpool, view.block_table, ctx.seq_q_start, ctx.seq_q_len, ctx.seq_pos0,
-                                    ctx.attention_work[g], self.maps, self.kv_maps, self.hd, view.page_size, None, float(s.scale))
+                                    ctx.attention_work[g], self.maps, self.kv_maps, self.hd, view.page_size, None, float(s.scale), **self.reading_ahead())
         gate = ops.linear(h, self.w_g, None, out_f32=True)
         y = ops.diff_combine(o, gate, self.lam, s.norm_eps, 1.0 - float(s.diff), s.heads, s.kv_heads, self.hd, s.v_head_dim, self.out_cols)
         stream.add_linear(y, self.w_o, self.b_o)

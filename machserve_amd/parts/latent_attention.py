@@ -125,7 +125,7 @@ class LatentAttention(Mixer):
         else:
             o = ops.paged_attention(att.view(att.shape[0], -1), self.kpool, self.vpool, view.block_table, ctx.seq_q_start, ctx.seq_q_len,
                                     ctx.seq_pos0, ctx.attention_work[s.heads], s.heads, 1, self.hd, view.page_size, self.window, float(s.scale),
-                                    sinks=self.sink, out_gate=gate)
+                                    sinks=self.sink, out_gate=gate, **self.reading_ahead())
         y = o.new_zeros((o.shape[0], s.heads, self.vd)) if self.vd != s.v_head_dim else None
         y = ops.heads_linear(o.view(o.shape[0], s.heads, self.hd), self.w_uv, y)
         stream.add_linear(y.view(y.shape[0], -1), self.w_o)

@@ -83,3 +83,43 @@ def test_marked_experts_give_the_same_bits(T):
     plain = run()
     up.past_cache = down.past_cache = True
     assert all(torch.equal(p, q) for p, q in zip(plain, run()))
+
+
+# attention with blocks beside its own that read weights ahead: the 32-row kernel and the general one, whole and cut, one weight and two, of a few bytes, and some that are not taken (too large, beginning anywhere, spread out)
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("hd,before,splits", [(64, 0, 0), (64, 900, 3), (128, 0, 0), (96, 0, 0), (96, 900, 2)])
+def test_an_attention_that_reads_ahead_gives_the_same_bits(dtype, hd, before, splits):
+    from machserve_amd.kernels import get_ops
+    ops = get_ops(dtype, DEV)
+    T, H, KV, ps = 130, 4, 2, 64
+    gen = torch.Generator().manual_seed(hd + before)
+    pages = -(-(T + before) // ps)
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)  # noqa: E731
+    q = torch.randn((T, H * hd), generator=gen).to(DEV, dtype)
+    kp, vp = torch.randn((pages, KV, ps, hd), generator=gen).to(DEV, dtype), torch.randn((pages, KV, hd, ps), generator=gen).to(DEV, dtype)
+    unit = ops.attention_rows_per_block(hd)
+    work = i32([[0, r] for r in range(0, T * (H // KV), unit)])
+    run = lambda **kw: ops.paged_attention(q, kp, vp, i32([list(range(pages))]), i32([0]), i32([T]), i32([before]), work, H, KV, hd, ps, None,  # noqa: E731
+                                           hd ** -0.5, key_splits=splits, **kw)
+    plain = run()
+    small, odd, wide = (torch.zeros(n, dtype=dtype, device=DEV) for n in (4, 40961, (ops.AHEAD_BYTES >> 1) // plain.element_size()))
+    for ahead in ((small,), (odd,), (odd, wide), (wide, wide), (torch.cat([wide, wide, odd]),), (odd[1:], wide[:1].expand(1 << 24))):
+        assert torch.equal(run(ahead=ahead), plain)
+
+
+def test_what_a_mixer_reads_ahead_is_its_feed_forward():
+    from machserve_amd.engine.loading import mark_weights_ahead
+    from machserve_amd.parts.base import Mixer
+    w = lambda n, dt=torch.bfloat16: torch.zeros((n, 8), dtype=dt)  # noqa: E731
+    inner, mixer = Mixer.__new__(Mixer), Mixer.__new__(Mixer)
+    mixer.sub_parts = lambda: [inner]
+    up, down = w(200), w(90)
+    blocks = [SimpleNamespace(feed_forward=SimpleNamespace(up=up, down=down, router=w(4, torch.float32), bias=torch.zeros(8, dtype=torch.bfloat16)), mixers=lambda: [mixer]),
+              SimpleNamespace(feed_forward=None, mixers=lambda: [Mixer.__new__(Mixer)])]
+    model = SimpleNamespace(blocks=blocks, rt=SimpleNamespace(dtype=torch.bfloat16, ops=object()))
+    mark_weights_ahead(model)
+    assert mixer.ahead == () and mixer.reading_ahead() == {}  # stand-ins for the kernels take no such argument
+    model.rt.ops = SimpleNamespace(AHEAD_BYTES=1)
+    mark_weights_ahead(model)
+    assert [t is want for t, want in zip(mixer.ahead, (down, up))] == [True, True] and inner.ahead == mixer.ahead and inner.reading_ahead() == {"ahead": inner.ahead}
