@@ -9,6 +9,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #if (defined(MS_ELEM_BF16) + defined(MS_ELEM_F16) + defined(MS_ELEM_F32)) != 1
 #error "define exactly one of MS_ELEM_BF16, MS_ELEM_F16, MS_ELEM_F32"
 #endif
@@ -183,6 +185,13 @@ __device__ __forceinline__ float gate_activation(float g, int act) {
 #endif
 }
 
+// f with the activation as a constant: in an epilogue of many elements the choice is made once, not as a select behind both formulas an element.
+template <class F>
+__device__ __forceinline__ void with_gate_activation(int act, F f) {
+    if (act == ACT_GELU_TANH) f(std::integral_constant<int, ACT_GELU_TANH>{});
+    else f(std::integral_constant<int, ACT_SILU>{});
+}
+
 // ---- the activation of a feed-forward without a gate branch --------------------------
 enum UnaryActivation { UNARY_RELU2 = 0, UNARY_SILU = 1, UNARY_GELU_TANH = 2, UNARY_COUNT = 3 };
 __device__ __forceinline__ float unary_activation(float v, int act) {
@@ -191,6 +200,13 @@ __device__ __forceinline__ float unary_activation(float v, int act) {
         return r * r;
     }
     return gate_activation(v, act == UNARY_SILU ? ACT_SILU : ACT_GELU_TANH);
+}
+
+template <class F>
+__device__ __forceinline__ void with_unary_activation(int act, F f) {
+    if (act == UNARY_RELU2) f(std::integral_constant<int, UNARY_RELU2>{});
+    else if (act == UNARY_SILU) f(std::integral_constant<int, UNARY_SILU>{});
+    else f(std::integral_constant<int, UNARY_GELU_TANH>{});
 }
 
 // ---- reductions -----------------------------------------------------------------

@@ -681,35 +681,72 @@ __device__ __forceinline__ void gemm_tile(const elem_t* __restrict__ A, const el
             for (int i = 0; i < TM; ++i) over[i * 64] = acc[i][TN - 1];
         __syncthreads();
     }
+    // The gate's activation in tile row i of a wave, in place; the up tiles are multiplied where the product is rounded (one instruction in half precision).
+    auto activate = [&](auto act, int i) {
+        float f[4] = {1.f, 1.f, 1.f, 1.f};  // SCALED: of the rows this lane holds
+        if constexpr (SCALED) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int lr = wm * (BM / WM) + i * 16 + grp * 4 + e;
+                if constexpr (PIPED) {
+                    f[e] = ss_q[0][lr];
+                    continue;
+                }
+                float ssum = 0.f;
+#pragma unroll
+                for (int qq = 0; qq < 256 / BM; ++qq) ssum += ss_q[PIPED ? 0 : qq][lr];
+                f[e] = 1.0f / sqrtf(ssum / (float)K + ep.ss_eps);
+            }
+        }
+        if constexpr (SPLIT_PAIR) {
+            __builtin_amdgcn_sched_barrier(0);
+            if (!second) last_up = over[i * 64];
+        }
+#pragma unroll
+        for (int j = 0; j < TN; j += 2) {
+            if (SPLIT_PAIR && j == TN - 1 && second) continue;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                if constexpr (SCALED) {
+                    acc[i][j][e] *= f[e];
+                    if (SPLIT_PAIR && j == TN - 1) last_up[e] *= f[e];
+                    else acc[i][min(j + 1, TN - 1)][e] *= f[e];
+                }
+                acc[i][j][e] = gate_activation(acc[i][j][e], act);
+            }
+        }
+    };
+    // Activations before the stores and for the one that the product has: their code is there once, not once a kind of store.  As a select an element, behind both
+    // formulas, five of an element's twelve vector instructions were for the one that is not taken.  us from a tile's last step to its last store, before and now: 256x320
+    // 6.3 and 5.4, 256x256 4.3 and 3.3, 256x192 3.2 and 2.6.  (The widest tiles have no registers for sums that come from either formula: there the stores are there twice.)
+    if constexpr (EPI == EPI_SWIGLU && !WIDE) {
+        with_gate_activation(ep.act, [&](auto act) {
+#pragma unroll
+            for (int i = 0; i < TM; ++i) activate(act, i);
+        });
+    } else if constexpr (EPI == EPI_ACT) {
+        with_unary_activation(ep.act, [&](auto act) {
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+                for (int j = 0; j < TN; ++j) {
+                    const float b = ep.bias ? ep.bias[min(col_base + j * 16, N - 1)] : 0.f;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) acc[i][j][e] = unary_activation(acc[i][j][e] + b, act);
+                }
+        });
+    }
     // A tile at the lower edge of an output whose rows come in whole groups of sixteen (a decode step
     // of 48 requests in a 64-row tile) skips the groups beyond the last row and stores the others
     // without checks as well.
-    auto emit = [&](auto checked, auto row_groups) {
+    auto emit = [&](auto checked, auto row_groups, auto act) {
         constexpr bool CHECKED = decltype(checked)::value, ROW_GROUPS = decltype(row_groups)::value;
         if constexpr (EPI == EPI_SWIGLU) {
             elem_t* out = reinterpret_cast<elem_t*>(ep.out);
 #pragma unroll
             for (int i = 0; i < TM; ++i) {
                 if (ROW_GROUPS && m0 + wm * (BM / WM) + i * 16 >= M) continue;
-                float f[4] = {1.f, 1.f, 1.f, 1.f};  // SCALED: of the rows this lane holds
-                if constexpr (SCALED) {
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        const int lr = wm * (BM / WM) + i * 16 + grp * 4 + e;
-                        if constexpr (PIPED) {
-                            f[e] = ss_q[0][lr];
-                            continue;
-                        }
-                        float ssum = 0.f;
-#pragma unroll
-                        for (int qq = 0; qq < 256 / BM; ++qq) ssum += ss_q[PIPED ? 0 : qq][lr];
-                        f[e] = 1.0f / sqrtf(ssum / (float)K + ep.ss_eps);
-                    }
-                }
-                if constexpr (SPLIT_PAIR) {
-                    __builtin_amdgcn_sched_barrier(0);
-                    if (!second) last_up = over[i * 64];
-                }
+                if constexpr (WIDE) activate(act, i);
 #pragma unroll
                 for (int j = 0; j < TN; j += 2) {
                     if (SPLIT_PAIR && j == TN - 1 && second) continue;
@@ -718,12 +755,7 @@ __device__ __forceinline__ void gemm_tile(const elem_t* __restrict__ A, const el
                     for (int e = 0; e < 4; ++e) {
                         const int row = row_base + i * 16 + e;
                         if (CHECKED && !(row < M && col < ep.n_out)) continue;
-                        float gv = acc[i][j][e], uv = SPLIT_PAIR && j == TN - 1 ? last_up[e] : acc[i][min(j + 1, TN - 1)][e];
-                        if constexpr (SCALED) {
-                            gv *= f[e];
-                            uv *= f[e];
-                        }
-                        out[(size_t)row * ep.ldo + col] = from_f32<elem_t>(gate_activation(gv, ep.act) * uv);
+                        out[(size_t)row * ep.ldo + col] = from_f32<elem_t>(acc[i][j][e] * (SPLIT_PAIR && j == TN - 1 ? last_up[e] : acc[i][min(j + 1, TN - 1)][e]));
                     }
                 }
             }
@@ -807,7 +839,7 @@ __device__ __forceinline__ void gemm_tile(const elem_t* __restrict__ A, const el
 #pragma unroll
                 for (int j = 0; j < TN; ++j) {
                     const int col = col_base + j * 16;
-                    const float b = ep.bias ? ep.bias[min(col, N - 1)] : 0.f;
+                    const float b = EPI != EPI_ACT && ep.bias ? ep.bias[min(col, N - 1)] : 0.f;
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
                         const int row = row_base + i * 16 + e;
@@ -816,7 +848,7 @@ __device__ __forceinline__ void gemm_tile(const elem_t* __restrict__ A, const el
                         const float v = acc[i][j][e] + b;
                         if constexpr (EPI == EPI_STORE_F32) reinterpret_cast<float*>(ep.out)[split * ep.split_stride + o] = v;
                         else if constexpr (EPI == EPI_STORE_ELEM) reinterpret_cast<elem_t*>(ep.out)[o] = from_f32<elem_t>(v);
-                        else if constexpr (EPI == EPI_ACT) reinterpret_cast<elem_t*>(ep.out)[o] = from_f32<elem_t>(unary_activation(v, ep.act));
+                        else if constexpr (EPI == EPI_ACT) reinterpret_cast<elem_t*>(ep.out)[o] = from_f32<elem_t>(v);
                         else reinterpret_cast<float*>(ep.out)[o] = prior[i % AHEAD][j][e] + v;  // residual stream, 32-bit
                         if constexpr (EPI == EPI_PRENORM) {
                             const float x = prior[i % AHEAD][j][e] + v;
@@ -882,9 +914,13 @@ __device__ __forceinline__ void gemm_tile(const elem_t* __restrict__ A, const el
         return;
     }
     const bool cols_whole = n0 + BN <= N && (EPI != EPI_SWIGLU || (n0 + BN) / 2 <= ep.n_out);
-    if (whole) emit(std::false_type{}, std::false_type{});
-    else if (cols_whole && M % 16 == 0) emit(std::false_type{}, std::true_type{});
-    else emit(std::true_type{}, std::false_type{});
+    auto finish = [&](auto act) {
+        if (whole) emit(std::false_type{}, std::false_type{}, act);
+        else if (cols_whole && M % 16 == 0) emit(std::false_type{}, std::true_type{}, act);
+        else emit(std::true_type{}, std::false_type{}, act);
+    };
+    if constexpr (EPI == EPI_SWIGLU && WIDE) with_gate_activation(ep.act, finish);
+    else finish(std::integral_constant<int, ACT_SILU>{});  // (not looked at)
 }
 
 
