@@ -18,12 +18,19 @@
 // 5.2 and 4.8; and weights that are read through the cache stay in it, if they fit.  A weight that would still be there from the step before is read slower so (11,264 x 2,048:
 // 8.2 and 9.4), so the weights are marked by what all of a model's come to (engine/loading.py).  Sixteen requests of the 7B sizes, 16 steps and their prompts, 70.0 -> 65.7 ms;
 // one of the 0.5B sizes 11.78 -> 10.98.
+//
+// In 32-bit a step is 32 numbers of K (rows of 128 bytes again), up to 32 rows; the fragments of skinny.hip, which it replaces
+// there, are 64 bytes a row and load, and stream at half the rate.  us, skinny.hip and here, cold weights, 1 and 32 rows: 9,728 x 896 gated 13.0 and 9.1,
+// 22.8 and 13.5; 896 x 4,864 in slices 7.3 and 5.9, 13.9 and 7.3; 11,264 x 2,048 gated 26.5 and 18.4, 47 and 27.6; 2,048 x 5,632 in slices 23.8 and 10.9, 24.9 and 13.5.
+// Over 385 products of 1 to 32 rows, 96 to 40,000 columns and K of 256 to 16,384 1.45 times as fast (geometric mean); decode steps of the further designs' small sizes 1.13 to
+// 1.35 times, of 24 requests of the 0.5B sizes 1.42.  Errors against 64 bits are the same (a pass of three requests 2.1e-6 and 2.0e-6).
 #pragma once
 #include "gemm_tile.cuh"
 
 namespace ms {
 
-#ifdef MS_ELEM_HALF
+constexpr int FEW_STEP = 128 / (int)sizeof(elem_t);  // numbers of K a step
+
 template <int MT, int NT, int KW, int STAGES, int EPI, bool SCALED, class Rows>
 __device__ __forceinline__ void few_rows_tile(const elem_t* __restrict__ A, const elem_t* __restrict__ W, int M, int N, int K, const EpiArgs& ep, int m0,
                                               int n0, int split, const Rows& rows) {
@@ -37,27 +44,27 @@ __device__ __forceinline__ void few_rows_tile(const elem_t* __restrict__ A, cons
     __shared__ float ss_q[SCALED ? KW : 1][SCALED ? 16 * MT : 1];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int r16 = lane & 15, grp = lane >> 4;
-    const int k_begin = split * ep.k_per_split, nk = (min(K, k_begin + ep.k_per_split) - k_begin) / 64;
+    const int k_begin = split * ep.k_per_split, nk = (min(K, k_begin + ep.k_per_split) - k_begin) / FEW_STEP;
     const int mine = (nk - wave + KW - 1) / KW;  // steps of this wave
 
     // lane l of a load: row l / 8 of its eight, the chunk that the swizzle puts at place l % 8
     const int chunk = (lane & 7) ^ (lane >> 3);
-    const elem_t* base_w = W + (size_t)n0 * rows.w_pitch(K) + k_begin + wave * 64;
-    const elem_t* base_a = A + (Rows::GATHERS ? (size_t)0 : (size_t)rows.source(m0) * rows.pitch(K)) + k_begin + wave * 64;
+    const elem_t* base_w = W + (size_t)n0 * rows.w_pitch(K) + k_begin + wave * FEW_STEP;
+    const elem_t* base_a = A + (Rows::GATHERS ? (size_t)0 : (size_t)rows.source(m0) * rows.pitch(K)) + k_begin + wave * FEW_STEP;
     uint32_t ow[2 * NT], oa[2 * MT];
     const elem_t* ga[Rows::GATHERS ? 2 * MT : 1];
 #pragma unroll
     for (int l = 0; l < 2 * NT; ++l)
-        ow[l] = ((uint32_t)(min(n0 + l * 8 + (lane >> 3), N - 1) - n0) * (uint32_t)rows.w_pitch(K) + chunk * 8) * 2u;
+        ow[l] = ((uint32_t)(min(n0 + l * 8 + (lane >> 3), N - 1) - n0) * (uint32_t)rows.w_pitch(K) + chunk * EPC) * (uint32_t)sizeof(elem_t);
 #pragma unroll
     for (int l = 0; l < 2 * MT; ++l) {
         const int m = min(m0 + l * 8 + (lane >> 3), M - 1);
-        if constexpr (Rows::GATHERS) ga[l] = base_a + (size_t)rows.source(m) * rows.pitch(K) + chunk * 8;
-        else oa[l] = ((uint32_t)(m - m0) * (uint32_t)rows.pitch(K) + chunk * 8) * 2u;
+        if constexpr (Rows::GATHERS) ga[l] = base_a + (size_t)rows.source(m) * rows.pitch(K) + chunk * EPC;
+        else oa[l] = ((uint32_t)(m - m0) * (uint32_t)rows.pitch(K) + chunk * EPC) * (uint32_t)sizeof(elem_t);
     }
     const uint32_t own = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)&ring[0][0] + wave * (STAGES * STEP);
     auto ask = [&](int i, int stage) {  // this wave's step i
-        const size_t k = (size_t)i * (64 * KW);
+        const size_t k = (size_t)i * (FEW_STEP * KW);
         const uint32_t to = own + stage * STEP;
         if (ep.past) {
 #pragma unroll
@@ -118,17 +125,29 @@ __device__ __forceinline__ void few_rows_tile(const elem_t* __restrict__ A, cons
         if (i + STAGES - 1 < mine) ask(i + STAGES - 1, last);
         wait_for(min(mine - 1 - i, STAGES - 1));
         const elem_t* t = reinterpret_cast<const elem_t*>(&ring[wave][stage * STEP]);
-        Frag fa[2][MT], fw[2][NT];
+        constexpr int CHUNKS = FEW_STEP / 32;  // of 32 numbers
+        auto fragment = [&](int row, int kk) {
+#ifdef MS_ELEM_HALF
+            return frag_load(t + row * FEW_STEP + ((kk * 4 + grp) ^ (r16 & 7)) * EPC);
+#else
+            Frag f;
+            const f32x4 x = *reinterpret_cast<const f32x4*>(t + row * FEW_STEP + ((2 * grp) ^ (r16 & 7)) * EPC);
+            const f32x4 y = *reinterpret_cast<const f32x4*>(t + row * FEW_STEP + ((2 * grp + 1) ^ (r16 & 7)) * EPC);
 #pragma unroll
-        for (int kk = 0; kk < 2; ++kk) {
-            const int at = ((kk * 4 + grp) ^ (r16 & 7)) * 8;
+            for (int e = 0; e < 4; ++e) { f.v[e] = x[e]; f.v[4 + e] = y[e]; }
+            return f;
+#endif
+        };
+        Frag fa[CHUNKS][MT], fw[CHUNKS][NT];
 #pragma unroll
-            for (int j = 0; j < NT; ++j) fw[kk][j] = frag_load(t + (j * 16 + r16) * 64 + at);
+        for (int kk = 0; kk < CHUNKS; ++kk) {
 #pragma unroll
-            for (int j = 0; j < MT; ++j) fa[kk][j] = frag_load(t + (NT * 16 + j * 16 + r16) * 64 + at);
+            for (int j = 0; j < NT; ++j) fw[kk][j] = fragment(j * 16 + r16, kk);
+#pragma unroll
+            for (int j = 0; j < MT; ++j) fa[kk][j] = fragment(NT * 16 + j * 16 + r16, kk);
         }
 #pragma unroll
-        for (int kk = 0; kk < 2; ++kk)
+        for (int kk = 0; kk < CHUNKS; ++kk)
 #pragma unroll
             for (int m = 0; m < MT; ++m)
 #pragma unroll
@@ -236,6 +255,5 @@ __device__ __forceinline__ void few_rows_tile(const elem_t* __restrict__ A, cons
         }
     }
 }
-#endif
 
 }  // namespace ms

@@ -89,6 +89,7 @@ static GemmPlan plan_gemm(int M, int N, int K, int splits, bool store32, bool ga
     }
     return best;
 }
+#endif
 template <int MT, int NT, int STAGES, int EPI, bool SCALED>
 __global__ __launch_bounds__(64 * FEW_WAVES) void gemm_few_kernel(const elem_t* __restrict__ A, const elem_t* __restrict__ W, int M, int N, int K, EpiArgs ep) {
     arguments_now(A, W, M, N, K, ep.out, ep.bias, ep.ldo, ep.n_out, ep.k_per_split, ep.split_stride, ep.past);
@@ -100,11 +101,11 @@ __global__ __launch_bounds__(64 * FEW_WAVES) void gemm_few_kernel(const elem_t* 
 template <int EPI, bool SCALED = false>
 static int launch_few(const elem_t* A, const elem_t* W, int M, int N, int K, const EpiArgs& ep, hipStream_t stream, int ns) {
     constexpr bool PAIRS = EPI == EPI_SWIGLU;
-    const int rows = few_row_tiles(M), tile = plan_few(M, N, K, ns, PAIRS).tile;
+    const int rows = few_row_tiles(M), tile = plan_few(M, N, K * FEW_BYTES, ns, PAIRS).tile;
 #define MS_FEW(ROWS_, TILE_)                                                                                                                          \
     do {                                                                                                                                              \
         constexpr FewCost t = kFew[ROWS_][TILE_];                                                                                                     \
-        if constexpr (!(PAIRS && t.nt == 1) && !(EPI == EPI_PRENORM && ROWS_ > 0)) {                                                                   \
+        if constexpr (!(PAIRS && t.nt == 1) && !(EPI == EPI_PRENORM && ROWS_ > 0) && !(!kHalf && ROWS_ > 1)) {                                                                   \
             hipLaunchKernelGGL((gemm_few_kernel<1 << ROWS_, t.nt, t.stages, EPI, SCALED>), dim3((unsigned)ceil_div(N, 16 * t.nt), (unsigned)ns),      \
                                dim3(64 * FEW_WAVES), 0, stream, A, W, M, N, K, ep);                                                                   \
             return check_launch("gemm, few rows");                                                                                                    \
@@ -127,17 +128,24 @@ static int launch_few(const elem_t* A, const elem_t* W, int M, int N, int K, con
     MS_REQUIRE(false, "few-rows product: M=%d N=%d K=%d is not taken", M, N, K);
 }
 
-// Whether a product runs in few_rows.cuh, with K cut over several blocks (`slices`) or not: whole K steps, at least one for every wave, up to 16 rows; up to
+// Whether a product runs in few_rows.cuh, with K cut over several blocks (`slices`) or not: whole K steps, at least one for every wave, up to 16 rows, in 32-bit up to 32; in the two-byte builds up to
 // 64 where it is predicted not to be slower than 64x64 tiles.  Their prediction (made for more rows) is an eighth short there: over 240
 // products of 32, 48 and 64 rows, cut and uncut, the choice takes 1.00 to 1.02 times the better of the two, which is 1.08 to 1.6 times as fast as the tiles.
 static bool few_rows(int M, int N, int K, bool slices, bool pairs) {
-    if (M > 64 || K % 64 != 0 || K < 64 * FEW_WAVES || g_gemm_config != 0) return false;
-    if (M <= 16) return true;
+    // (32-bit: a wave of two steps is no better than one of skinny.hip, 40,000 x 256 10.9 us and 10.2)
+    if (M > 64 || K % FEW_STEP != 0 || K < FEW_STEP * FEW_WAVES * (kHalf ? 1 : 3) || g_gemm_config != 0) return false;
+    if (M <= (kHalf ? 16 : 32)) return true;  // (in 32-bit all rows whose sums are those of a row by itself)
+#ifdef MS_ELEM_HALF
     const int ns = slices ? tiled_slices(M, N, K) : 1, per = ceil_div(ceil_div(K, ns), 64) * 64;
     const float tiled = fmaxf(tile_time(kTiles[TILE_64x64_DEEP], (long)ceil_div(N, 64) * ns, per, true), 2.5f + (float)N * (float)K * 4e-7f) +
                         (float)(ns - 1) * (float)M * (float)N * (8.0f / 4.5e6f);
     return plan_few(M, N, K, slices ? 0 : 1, pairs).us < 1.12f * tiled;
+#else
+    (void)N; (void)slices; (void)pairs;
+    return false;
+#endif
 }
+#ifdef MS_ELEM_HALF
 // products of more than 64 rows over whole K steps: what is planned as above
 static bool planned(int M, int K) { return M > 64 && K % 64 == 0 && g_gemm_config == 0; }
 #endif
@@ -193,9 +201,9 @@ static int launch_gemm(const elem_t* A, const elem_t* W, int M, int N, int K, Ep
                            A, W, M, N, K, ep);                                                                        \
         return check_launch("gemm " #BM_ "x" #BN_ "x" #BK_);                                                          \
     } while (0)
+    if (few_rows(M, N, K, ns > 1, EPI == EPI_SWIGLU)) return launch_few<EPI>(A, W, M, N, K, ep, stream, (int)ns);
 #ifdef MS_ELEM_HALF
     const int forced = g_gemm_config;
-    if (few_rows(M, N, K, ns > 1, EPI == EPI_SWIGLU)) return launch_few<EPI>(A, W, M, N, K, ep, stream, (int)ns);
     if (forced == 1) MS_GEMM(128, 128, 2, 2, 32);
     if (forced == 2) MS_GEMM(128, 128, 2, 2, 64);
     if (forced == 5) MS_GEMM(128, 64, 2, 2, 64);
@@ -383,9 +391,7 @@ static int tiled_slices(int M, int N, int K) {
 }
 
 static int plan_tiled_splits(int M, int N, int K) {
-#ifdef MS_ELEM_HALF
-    if (g_force_splits == 0 && few_rows(M, N, K, true, false)) return plan_few(M, N, K, 0, false).splits;
-#endif
+    if (g_force_splits == 0 && few_rows(M, N, K, true, false)) return plan_few(M, N, K * FEW_BYTES, 0, false).splits;
     return tiled_slices(M, N, K);
 }
 
@@ -669,12 +675,7 @@ extern "C" int ms_gated_tile(int M, int N, int K) {
 // Whether the entry points of the tiled products run this product in few_rows.cuh (then they are the ones to call): `slices` if its reader adds up
 // K slices, `pairs` for the gated product.
 extern "C" int ms_few_rows_takes(int M, int N, int K, int slices, int pairs) {
-#ifdef MS_ELEM_HALF
     return M >= 1 && N >= 1 && few_rows(M, N, K, slices != 0, pairs != 0);
-#else
-    (void)M; (void)N; (void)K; (void)slices; (void)pairs;
-    return 0;
-#endif
 }
 
 // Of the products that few_rows.cuh does not take (a K that is no whole number of steps, 17 to 64 rows of some shapes, 32-bit), and of norms that could be

@@ -71,11 +71,15 @@ struct FewPlan {
 // The best tile for `splits` slices, or, with splits == 0, the best tile and number of slices (a plane of sums more is written and read again, and
 // no slice is shorter than a step for every wave).  `pairs`: gate and up columns lie side by side.  Up to 32 rows the slices are those of 16, so that a row's
 // sums do not depend on how many rows come with it.
+// K in numbers of two bytes: one of four counts twice (a slice is a multiple of 64 numbers of either).
+constexpr int FEW_BYTES = (int)sizeof(elem_t) / 2, FEW_SLICE = 64 * FEW_BYTES;
 static inline FewPlan plan_few(int M, int N, int K, int splits, bool pairs) {
     if (splits == 0 && M <= 32 && M != 16) return plan_few(M, N, K, plan_few(16, N, K, 0, pairs).splits, pairs);
     FewPlan best{0, 1, INFINITY};
-    for (int s = splits ? splits : 1; s <= (splits ? splits : 8); ++s) {
-        const int per = ceil_div(ceil_div(K, s), 64) * 64;
+    // (up to sixteen slices only in 32-bit and of very few columns, 128 x 16,384 6.4 us in eight, 4.8 in sixteen: the norm that adds them up takes longer by more than the
+    // prediction knows, a pass of three requests of the 0.5B sizes 20.4 ms and 20.5 with ten of the down projection)
+    for (int s = splits ? splits : 1; s <= (splits ? splits : kHalf || N > 256 ? 8 : 16); ++s) {
+        const int per = ceil_div(ceil_div(K, s), FEW_SLICE) * FEW_SLICE;
         if (splits == 0 && s > 1 && (ceil_div(K, per) != s || per < 64 * FEW_WAVES)) continue;
         for (int i = pairs ? 1 : 0; i < FEW_TILES; ++i) {
             const FewCost& t = kFew[few_row_tiles(M)][i];

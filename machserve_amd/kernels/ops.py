@@ -306,7 +306,7 @@ class HipOps:
 
     def _few(self, M: int, N: int, K: int, slices: bool, pairs: bool = False) -> bool:
         """Whether this product of at most 64 rows runs in ``few_rows.cuh``, through the entry points of the tiled products
-        (two-byte elements, whole K steps, up to 16 rows always)."""
+        (whole K steps, up to 16 rows always; in 32-bit up to 32, and only those)."""
         return M <= self.SKINNY_ROWS and bool(self._plan("ms_few_rows_takes", M, N, K, int(slices), int(pairs)))
 
     @staticmethod
@@ -457,6 +457,11 @@ class HipOps:
         16 rows, and a shape the few-rows kernel would take anyway)."""
         return (not self._tiled(M, N, K)
                 and bool(self._plan("ms_skinny_norm_takes", M, N, K, n_partials)))
+
+    def norm_stands_alone(self, M: int, N: int, K: int, pairs: bool) -> bool:
+        """Whether a product that could apply the norm itself (:meth:`norm_folds_into`) is the faster one behind a norm of its own: in 32-bit, where its waves
+        share out K."""
+        return self.dtype == torch.float32 and self._few(M, N, K, not pairs, pairs)
 
     def _normed_operands(self, x, partials, norm_w, w, what):
         M, K = x.shape

@@ -129,18 +129,21 @@ class PendingRMSNorm(PendingNorm):
     """The RMS norm left to its reader's first product, folded into it where the kernels take the shape.  Where a normed branch
     is still to be added to the stream and the product does not take the norm, the two norms are one kernel."""
 
-    def _post_goes_first(self, n: int) -> bool:
-        stream = self.stream
-        return stream.post is not None and not stream.ops.norm_folds_into(stream.x.shape[0], n, stream.x.shape[1], 0)
+    def _folds(self, n: int, n_partials: int, pairs: bool) -> bool:
+        ops, (T, K) = self.stream.ops, self.stream.x.shape
+        alone = getattr(ops, "norm_stands_alone", None)
+        return ops.norm_folds_into(T, n, K, n_partials) and not (alone is not None and alone(T, n, K, pairs))
+
+    def _post_goes_first(self, n: int, pairs: bool) -> bool:
+        return self.stream.post is not None and not self._folds(n, 0, pairs)
 
     def linear_split(self, w):
         stream, ops, weight, eps = self.stream, self.stream.ops, self.norm.weight, self.norm.spec.eps
-        if self._post_goes_first(w.shape[0]):
+        if self._post_goes_first(w.shape[0], False):
             return ops.linear_split(self.tensor(), w)
         stream.launch_deferred()
-        T, K = stream.x.shape
         P = 0 if stream.pending is None else stream.pending.shape[0]
-        if ops.norm_folds_into(T, w.shape[0], K, P):
+        if self._folds(w.shape[0], P, False):
             out, x_new = ops.linear_split_normed(stream.x, stream.pending, weight, eps, w)
             if x_new is not None:
                 stream.x, stream.pending = x_new, None
@@ -149,7 +152,7 @@ class PendingRMSNorm(PendingNorm):
 
     def linear_swiglu(self, w_gate_up, intermediate, activation="silu"):
         stream, ops, weight, eps = self.stream, self.stream.ops, self.norm.weight, self.norm.spec.eps
-        if self._post_goes_first(w_gate_up.shape[0]):
+        if self._post_goes_first(w_gate_up.shape[0], True):
             return ops.linear_swiglu(self.tensor(), w_gate_up, intermediate, activation)
         if stream.deferred is not None and stream.pending is None:
             # a product that is still to be added: where the kernels can, it leaves what the norm needs beside its
@@ -161,9 +164,8 @@ class PendingRMSNorm(PendingNorm):
                 hn, row_ss = ops.linear_residual_prenorm(a, w, stream.x, weight)
                 return ops.linear_swiglu_scaled(hn, row_ss, eps, w_gate_up, intermediate, activation)
         stream.launch_deferred()
-        T, K = stream.x.shape
         P = 0 if stream.pending is None else stream.pending.shape[0]
-        if ops.norm_folds_into(T, w_gate_up.shape[0], K, P):
+        if self._folds(w_gate_up.shape[0], P, True):
             out, x_new = ops.linear_swiglu_normed(stream.x, stream.pending, weight, eps, w_gate_up, intermediate, activation)
             if x_new is not None:
                 stream.x, stream.pending = x_new, None
