@@ -31,10 +31,17 @@ namespace ms {
 
 constexpr int FEW_STEP = 128 / (int)sizeof(elem_t);  // numbers of K a step
 
-template <int MT, int NT, int KW, int STAGES, int EPI, bool SCALED, class Rows>
+// What a block that norms its one row itself (NORMED) keeps in dynamic LDS: the pending sums, the stream's row and the norm's weight as they come, whole kilobytes each, and the normed row.
+static inline size_t few_normed_lds(int K, int n_pending) {
+    auto whole = [](size_t floats) { return (floats * 4 + 1023) / 1024 * 1024; };
+    return whole((size_t)n_pending * K) + 2 * whole(K) + (size_t)K * sizeof(elem_t);
+}
+
+template <int MT, int NT, int KW, int STAGES, int EPI, bool SCALED, class Rows, bool NORMED = false>
 __device__ __forceinline__ void few_rows_tile(const elem_t* __restrict__ A, const elem_t* __restrict__ W, int M, int N, int K, const EpiArgs& ep, int m0,
                                               int n0, int split, const Rows& rows) {
-    constexpr int STEP = (NT + MT) * 2048, PER_STEP = 2 * (NT + MT);  // bytes and loads of a step: rows of 128 bytes, eight a load
+    constexpr int RING = NT + (NORMED ? 0 : MT);  // tiles of sixteen rows in a ring
+    constexpr int STEP = RING * 2048, PER_STEP = 2 * RING;  // bytes and loads of a step: rows of 128 bytes, eight a load
     constexpr int PAIR = EPI == EPI_SWIGLU || EPI == EPI_EXPERT_GATED ? 2 : 1;
     static_assert(NT % PAIR == 0, "gate and up tiles come in pairs");
     static_assert(PER_STEP * (STAGES - 1) <= 63, "the wait count is a 6-bit field");
@@ -42,6 +49,8 @@ __device__ __forceinline__ void few_rows_tile(const elem_t* __restrict__ A, cons
     static_assert(STAGES * STEP >= MT * NT * 1024, "the waves' sums lie where their rings were");
     __shared__ __attribute__((aligned(16))) char ring[KW][STAGES * STEP];
     __shared__ float ss_q[SCALED ? KW : 1][SCALED ? 16 * MT : 1];
+    static_assert(!NORMED || (MT == 1 && EPI == EPI_STORE_F32 && !SCALED && !Rows::GATHERS), "a block that norms its row: one row, sums");
+    extern __shared__ __attribute__((aligned(16))) char normed[];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int r16 = lane & 15, grp = lane >> 4;
     const int k_begin = split * ep.k_per_split, nk = (min(K, k_begin + ep.k_per_split) - k_begin) / FEW_STEP;
@@ -76,7 +85,7 @@ __device__ __forceinline__ void few_rows_tile(const elem_t* __restrict__ A, cons
                 asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(ow[l]), "s"(base_w + k), "s"(to + l * 1024) : "memory", "m0");
         }
 #pragma unroll
-        for (int l = 0; l < 2 * MT; ++l) {
+        for (int l = 0; l < (NORMED ? 0 : 2 * MT); ++l) {
             if constexpr (Rows::GATHERS)
                 asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(ga[l] + k), "s"(to + (2 * NT + l) * 1024) : "memory", "m0");
             else
@@ -89,9 +98,64 @@ __device__ __forceinline__ void few_rows_tile(const elem_t* __restrict__ A, cons
 #pragma unroll
         for (int j = 0; j < NT; ++j) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
 
+    // NORMED: the row's sources are asked for ahead of the first steps, a kilobyte a load, shared out over the waves
+    const int row4 = K / 4, row_kb = (K + 255) / 256 * 256;
+    float* const src_p = reinterpret_cast<float*>(normed);
+    float* const src_x = src_p + (ep.n_pending * K + 255) / 256 * 256;
+    float* const src_w = src_x + row_kb;
+    elem_t* const row_n = reinterpret_cast<elem_t*>(src_w + row_kb);
+    if constexpr (NORMED) {
+        auto bring = [&](const float* from, int quads, const float* to) {
+            const uint32_t at = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const char*)to;
+            for (int c = wave; c * 64 < quads; c += KW)
+                asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"((uint32_t)min(c * 64 + lane, quads - 1) * 16u), "s"(from),
+                             "s"(__builtin_amdgcn_readfirstlane(at + c * 1024)) : "memory", "m0");
+        };
+        bring(ep.pending, ep.n_pending * row4, src_p);
+        bring(ep.stream, row4, src_x);
+        bring(ep.norm_w, row4, src_w);
+    }
 #pragma unroll
     for (int s = 0; s < STAGES - 1; ++s)
         if (s < mine) ask(s, s);
+    if constexpr (NORMED) {
+        // As the norm's kernel does it, with its numbers: a thread's fours of the row, the sums added in order, squares over the waves in order.
+        auto together = [&] {
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+        };
+        __shared__ float squares[KW];
+        static_assert(KW == 4, "256 threads, as the norm's kernel has");
+        __builtin_amdgcn_sched_barrier(0);
+        if (mine >= STAGES - 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PER_STEP * (STAGES - 1)) : "memory");  // all but the weight's
+        else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        together();
+        const bool writes = blockIdx.x == 0 && blockIdx.y == 0;
+        float ss = 0.f;
+        for (int c = threadIdx.x; c < row4; c += 256) {
+            f32x4* x = reinterpret_cast<f32x4*>(src_x) + c;
+            f32x4 v = *x;
+            for (int p = 0; p < ep.n_pending; ++p) v += reinterpret_cast<const f32x4*>(src_p)[p * row4 + c];
+            *x = v;
+            if (writes) reinterpret_cast<f32x4*>(ep.stream_out)[c] = v;
+            ss += v.x * v.x + v.y * v.y + v.z * v.z + v.w * v.w;
+        }
+        ss = wave_sum(ss);
+        if (lane == 0) squares[wave] = ss;
+        together();
+        ss = 0.f;
+#pragma unroll
+        for (int w = 0; w < KW; ++w) ss += squares[w];
+        const float inv = 1.0f / sqrtf(ss / (float)K + ep.ss_eps);
+        for (int c = threadIdx.x; c < row4; c += 256) {
+            // (with a zero added, as there: one rounding to half precision)
+            const f32x4 o = reinterpret_cast<const f32x4*>(src_x)[c] * reinterpret_cast<const f32x4*>(src_w)[c] * inv + (f32x4){0.f, 0.f, 0.f, 0.f};
+            typedef elem_t four_t __attribute__((ext_vector_type(4)));
+            reinterpret_cast<four_t*>(row_n)[c] = (four_t){from_f32<elem_t>(o.x), from_f32<elem_t>(o.y), from_f32<elem_t>(o.z), from_f32<elem_t>(o.w)};
+        }
+        together();
+    }
     // SCALED: the rows' sums of squares come in parts, shared out over the waves and their four groups of lanes; the first EARLY of each are asked
     // for here, behind the first steps
     constexpr int SHARES = 4 * KW, EARLY = 4;
@@ -144,7 +208,8 @@ __device__ __forceinline__ void few_rows_tile(const elem_t* __restrict__ A, cons
 #pragma unroll
             for (int j = 0; j < NT; ++j) fw[kk][j] = fragment(j * 16 + r16, kk);
 #pragma unroll
-            for (int j = 0; j < MT; ++j) fa[kk][j] = fragment(NT * 16 + j * 16 + r16, kk);
+            for (int j = 0; j < MT; ++j)
+                fa[kk][j] = NORMED ? frag_load(row_n + k_begin + (wave + i * KW) * FEW_STEP + kk * 32 + grp * 8) : fragment(NT * 16 + j * 16 + r16, kk);
         }
 #pragma unroll
         for (int kk = 0; kk < CHUNKS; ++kk)

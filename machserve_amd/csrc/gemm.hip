@@ -98,6 +98,12 @@ __global__ __launch_bounds__(64 * FEW_WAVES) void gemm_few_kernel(const elem_t* 
     few_rows_tile<MT, NT, FEW_WAVES, STAGES, EPI, SCALED>(A, W, M, N, K, ep, 0, blockIdx.x * 16 * NT, blockIdx.y, NoExperts{});
 }
 
+template <int NT, int STAGES>
+__global__ __launch_bounds__(64 * FEW_WAVES) void gemm_few_normed_kernel(const elem_t* __restrict__ W, int M, int N, int K, EpiArgs ep) {
+    arguments_now(W, M, N, K, ep.out, ep.ldo, ep.k_per_split, ep.split_stride, ep.past, ep.stream, ep.pending, ep.n_pending, ep.norm_w, ep.stream_out, ep.ss_eps);
+    few_rows_tile<1, NT, FEW_WAVES, STAGES, EPI_STORE_F32, false, NoExperts, true>(W, W, M, N, K, ep, 0, blockIdx.x * 16 * NT, blockIdx.y, NoExperts{});
+}
+
 template <int EPI, bool SCALED = false>
 static int launch_few(const elem_t* A, const elem_t* W, int M, int N, int K, const EpiArgs& ep, hipStream_t stream, int ns) {
     constexpr bool PAIRS = EPI == EPI_SWIGLU;
@@ -676,6 +682,51 @@ extern "C" int ms_gated_tile(int M, int N, int K) {
 // K slices, `pairs` for the gated product.
 extern "C" int ms_few_rows_takes(int M, int N, int K, int slices, int pairs) {
     return M >= 1 && N >= 1 && few_rows(M, N, K, slices != 0, pairs != 0);
+}
+
+// Whether a product of one row norms it itself, each of its blocks for itself, and how many slices it then leaves: with sums pending, where what a block keeps is within 64 KB
+// and what all blocks read of it within 24 MB.  A kernel of the chain goes, its launch and its trips to memory; the product waits for the row instead.  Passes of one request, us,
+// without and with: 0.5B sizes 8,340 and 8,090 (thirteen steps), 1.5B (23 MB) 16,240 and 16,010, 32-bit 0.5B (13 MB) 8,700 and 8,650; of two to four requests the same.
+extern "C" int ms_few_normed_takes(int M, int N, int K, int n_pending) {
+    if (M != 1 || n_pending < 1 || n_pending > 16 || !few_rows(M, N, K, true, false)) return 0;
+    const FewPlan p = plan_few(M, N, K * FEW_BYTES, 0, false);
+    const size_t lds = few_normed_lds(K, n_pending);
+    return lds <= 64 * 1024 && lds * ceil_div(N, 16 * kFew[0][p.tile].nt) * p.splits <= 24u << 20 ? p.splits : 0;
+}
+
+// out[slices, 1, N] (float) = partial sums of rmsnorm(x + sum pending; norm_w, eps) w^T over ms_few_normed_takes slices of K, x_out = x + sum pending (another buffer than x).
+static int linear_few_normed(const float* x, const float* pending, int n_pending, const float* norm_w, float eps, float* x_out, const void* w, float* out, int M, int N,
+                             int K, hipStream_t stream, bool past) {
+    const int ns = ms_few_normed_takes(M, N, K, n_pending);
+    MS_REQUIRE(ns > 0, "product that norms its row: M=%d N=%d K=%d with %d pending sums is not taken", M, N, K, n_pending);
+    MS_REQUIRE(x && pending && norm_w && x_out && x_out != x, "product that norms its row: a buffer is missing, or the stream would be written where it is read");
+    MS_REQUIRE(((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(pending) | reinterpret_cast<uintptr_t>(norm_w) | reinterpret_cast<uintptr_t>(x_out) |
+                 reinterpret_cast<uintptr_t>(w)) & 15) == 0, "product that norms its row: operands must be 16-byte aligned");
+    EpiArgs ep{out, nullptr, N, N, ceil_div(ceil_div(K, ns), 64) * 64, (size_t)M * N};
+    ep.past = past;
+    ep.norm_w = norm_w, ep.ss_eps = eps;
+    ep.stream = x, ep.pending = pending, ep.n_pending = n_pending, ep.stream_out = x_out;
+    const unsigned lds = (unsigned)few_normed_lds(K, n_pending);
+    const int tile = plan_few(M, N, K * FEW_BYTES, ns, false).tile;
+#define MS_NORMED(TILE_)                                                                                                                                       \
+    do {                                                                                                                                                       \
+        constexpr FewCost t = kFew[0][TILE_];                                                                                                                  \
+        hipLaunchKernelGGL((gemm_few_normed_kernel<t.nt, t.stages>), dim3((unsigned)ceil_div(N, 16 * t.nt), (unsigned)ns), dim3(64 * FEW_WAVES), lds, stream,  \
+                           (const elem_t*)w, M, N, K, ep);                                                                                                     \
+        return check_launch("gemm, few rows, normed");                                                                                                         \
+    } while (0)
+    if (tile == 0) MS_NORMED(0);
+    if (tile == 1) MS_NORMED(1);
+    MS_NORMED(2);
+#undef MS_NORMED
+}
+extern "C" int ms_linear_few_normed(const float* x, const float* pending, int n_pending, const float* norm_w, float eps, float* x_out, const void* w, float* out, int M,
+                                    int N, int K, hipStream_t stream) {
+    return linear_few_normed(x, pending, n_pending, norm_w, eps, x_out, w, out, M, N, K, stream, false);
+}
+extern "C" int ms_linear_few_normed_past(const float* x, const float* pending, int n_pending, const float* norm_w, float eps, float* x_out, const void* w, float* out, int M,
+                                         int N, int K, hipStream_t stream) {
+    return linear_few_normed(x, pending, n_pending, norm_w, eps, x_out, w, out, M, N, K, stream, true);
 }
 
 // Of the products that few_rows.cuh does not take (a K that is no whole number of steps, 17 to 64 rows of some shapes, 32-bit), and of norms that could be

@@ -73,6 +73,11 @@ struct EpiArgs {
     const float* norm_w;  // [N]
     elem_t* hn;           // [M, N]
     float* ss_part;       // [N / 16, or the columns of a wave, rounded up, M]
+    // a row that its product norms: the stream [K], its pending sums [n_pending, K], and where the stream with them goes (norm_w and ss_eps as above)
+    const float* stream = nullptr;
+    const float* pending = nullptr;
+    int n_pending = 0;
+    float* stream_out = nullptr;
     int group = 1;        // row tiles that a run of the tiles' order has side by side (see tile_of_block)
     int past = 0;         // W is read past the last-level cache (see few_rows.cuh): up to 64 rows, where every block reads its own columns of it
 };

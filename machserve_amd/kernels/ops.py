@@ -477,6 +477,23 @@ class HipOps:
         x_new = torch.empty_like(x) if P else None
         return M, w.shape[0], K, P, x_new
 
+    def norms_its_row(self, M: int, N: int, K: int, n_partials: int, x: torch.Tensor, partials: torch.Tensor, w: torch.Tensor) -> bool:
+        """Whether :meth:`linear_split_row_normed` takes these: one row with sums pending, operands that begin at 16 bytes."""
+        return self._plan("ms_few_normed_takes", M, N, K, n_partials) > 0 and (x.data_ptr() | partials.data_ptr() | w.data_ptr()) % 16 == 0
+
+    def linear_split_row_normed(self, x: torch.Tensor, partials: torch.Tensor, norm_w: torch.Tensor, eps: float, w: torch.Tensor):
+        """:meth:`linear_split` of ``rmsnorm(x + sum(partials))``, the norm in the product's kernel: the same numbers as the norm's own kernel
+        and the product; and the stream with the pending sums added (a new tensor)."""
+        M, N, K, P, x_new = self._normed_operands(x, partials, norm_w, w, "linear_split_row_normed")
+        slices = self._plan("ms_few_normed_takes", M, N, K, P)
+        if slices < 1:
+            raise KernelError(f"linear_split_row_normed: M={M} N={N} K={K} with {P} pending sums is not taken")
+        out = torch.empty((slices, M, N), dtype=torch.float32, device=x.device)
+        fn = self._reading(self._core, "ms_linear_few_normed", w)
+        self._check(self._core, fn(_ptr(x), _ptr(partials), _c_int(P), _ptr(norm_w), _c_float(eps), _ptr(x_new), _ptr(w), _ptr(out), _c_int(M), _c_int(N),
+                                   _c_int(K), self._stream()))
+        return out, x_new
+
     def linear_split_normed(self, x: torch.Tensor, partials: Optional[torch.Tensor], norm_w: torch.Tensor, eps: float,
                             w: torch.Tensor):
         """``rmsnorm(x + sum(partials)) @ w.T`` as float32 ``[1, M, N]``, and the stream with the

@@ -148,6 +148,11 @@ class PendingRMSNorm(PendingNorm):
             if x_new is not None:
                 stream.x, stream.pending = x_new, None
             return out
+        takes = getattr(ops, "norms_its_row", None)
+        if P > 0 and takes is not None and takes(stream.x.shape[0], w.shape[0], stream.x.shape[1], P, stream.x, stream.pending, w):
+            out, stream.x = ops.linear_split_row_normed(stream.x, stream.pending, weight, eps, w)
+            stream.pending = None
+            return out
         return ops.linear_split(self.tensor(), w)
 
     def linear_swiglu(self, w_gate_up, intermediate, activation="silu"):
