@@ -44,15 +44,17 @@ static inline float tile_time(const TileCost& t, long blocks, int k_per_split, b
 
 // Products of few rows (few_rows.cuh: four waves that share out K).  A block of `nt` tiles of 16 columns takes `step[n]` us for each of a wave's K steps
 // where n + 1 such blocks share a CU, `slope` more of it in proportion as the chip is full; the product takes `start` and `per_mb` for each MB of the weight.
-// A fit (non-negative least squares, 6 to 9 % off) to 672 products of 1 to 16 rows and 224 each of 32 and 64: 40 weights of 160 to 151,936 columns and
-// K of 320 to 18,944, cold, in one to eight slices.  The choice of tiles and slices takes 1.01 (uncut) and 1.025 times the best measured.
+// A fit (non-negative least squares, 6 to 10 % off) to 1,416 products of 1 to 16 rows, their weights read as a model has them (past the last-level cache or through it), and 224 each of
+// 32 and 64: 37 and 40 weights of 64 to 151,936 columns and K of 320 to 18,944, cold, in one to eight slices.  Up to 16 rows the choice of tiles and slices takes 1.006 times the
+// best measured, where that of a fit to weights through the cache took 1.034: 37,888 x 3,584 gated 48.1 us in 64 columns a block, 43.1 in 32; 17,920 x 1,536 gated 14.4 and
+// 12.2; 2,048 x 2,048 4.35 in eight slices, 3.94 in two.
 struct FewCost {
     int nt, stages, per_cu;
     float step[3], slope, start, per_mb;
 };
 constexpr int FEW_WAVES = 4, FEW_TILES = 3;
 static constexpr FewCost kFew[3][FEW_TILES] = {  // up to 16, 32 and 64 rows
-    {{1, 3, 3, {0.148f, 0.239f, 0.280f}, 0.254f, 2.32f, 0.141f}, {2, 3, 2, {0.212f, 0.374f}, 0.354f, 2.34f, 0.144f}, {4, 2, 2, {0.440f, 0.797f}, 0.344f, 2.28f, 0.136f}},
+    {{1, 3, 3, {0.143f, 0.265f, 0.419f}, 0.194f, 2.49f, 0.085f}, {2, 3, 2, {0.203f, 0.404f}, 0.349f, 2.44f, 0.081f}, {4, 2, 2, {0.387f, 0.733f}, 0.000f, 2.45f, 0.120f}},
     {{1, 3, 2, {0.261f, 0.436f}, 0.557f, 2.21f, 0.149f}, {2, 2, 2, {0.358f, 0.620f}, 0.483f, 2.34f, 0.143f}, {4, 2, 1, {0.646f}, 1.792f, 2.50f, 0.118f}},
     {{1, 2, 2, {0.406f, 0.717f}, 0.604f, 2.26f, 0.167f}, {2, 2, 1, {0.595f}, 1.792f, 2.52f, 0.114f}, {4, 2, 1, {0.935f}, 3.220f, 3.42f, 0.101f}},
 };
@@ -83,7 +85,8 @@ static inline FewPlan plan_few(int M, int N, int K, int splits, bool pairs) {
         if (splits == 0 && s > 1 && (ceil_div(K, per) != s || per < 64 * FEW_WAVES)) continue;
         for (int i = pairs ? 1 : 0; i < FEW_TILES; ++i) {
             const FewCost& t = kFew[few_row_tiles(M)][i];
-            const float us = few_time(t, (long)ceil_div(N, 16 * t.nt) * s, per, N, K) + (float)(s - 1) * (float)M * (float)N * (8.0f / 4.5e6f);
+            // (a plane of sums more: its bytes, and up to 16 rows 0.05 us of the reader's time)
+            const float us = few_time(t, (long)ceil_div(N, 16 * t.nt) * s, per, N, K) + (float)(s - 1) * ((float)M * (float)N * (8.0f / 4.5e6f) + (M <= 16 ? 0.05f : 0.0f));
             if (us < best.us) best = {i, s, us};
         }
     }
