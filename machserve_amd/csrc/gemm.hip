@@ -45,8 +45,9 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_kernel(const elem_t* __rest
     if constexpr (SCALED) arguments_now(ep.row_ss, ep.ss_parts, ep.ss_eps);
     if constexpr (STAGES == 4 && BM == 64) arguments_now(ep.past);
     const int tiles_m = ceil_div(M, BM);
-    // (64x64 tiles with four buffers are few, and gain nothing by it: 2,048 x 64 x 2,048 12.0 us by turns, 13.1 so)
-    constexpr bool BY_TURNS = kHalf && STAGES == 4 && EPI != EPI_QKV_ROPE;
+    // (Tiles with four buffers are few, and gain nothing by it: 2,048 x 64 x 2,048 12.0 us by turns, 13.1 so; 32-bit, 32x32 tiles, prompts of 100 and 250 rows of the
+    // further designs' small sizes 0.6 % by turns, and 1 % the other way round where K is 2,048 and more.)
+    constexpr bool BY_TURNS = STAGES == 4 && EPI != EPI_QKV_ROPE;
     const TilePlace at = BY_TURNS || tiles_m == 1 ? TilePlace{(int)blockIdx.x % tiles_m, (int)blockIdx.x / tiles_m, (int)blockIdx.y} : tile_of_block(tiles_m, ep.group);
     gemm_tile<BM, BN, WM, WN, BK, EPI, STAGES, SCALED>(A, W, M, N, K, ep, at.m * BM, at.n * BN, at.split, NoExperts{});
 }
